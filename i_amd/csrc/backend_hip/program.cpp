@@ -332,6 +332,15 @@ bool bf16_result_in_place(const Run& run, const Recognized& r) {
   return product_dtype(run, r) == DType::BF16 && r.out.kind == BufferRef::Output && run.outputs[r.out.id].dtype == DType::BF16;
 }
 
+// Does any kernel of the program read this output buffer?  (Such a bf16 output keeps its f32 staging, which the reader takes.)
+bool read_back(const Run& run, BufferRef out) {
+  for (const Step& s : run.plan.exec)
+    if (s.kind == Step::Dispatch)
+      for (BufferRef r : s.reads)
+        if (r.kind == out.kind && r.id == out.id) return true;
+  return false;
+}
+
 // An f32 product through the executor: with few output tiles under a long k loop, the loop in parts over
 // workgroups, the partial products in a temporary (no room for it: the unsplit kernel).
 ihip::Err launch_product_f32(Run& run, const void* a, const void* b, void* c, size_t bh, size_t m, size_t n, size_t k,
@@ -601,15 +610,28 @@ ihip::Err launch_hand_noted(Run& run, const Recognized& r, ihip::LaunchNote* not
       size_t rows = 1;
       for (size_t d = 0; d + 1 < x.size(); ++d) rows *= x[d];
       void *in = nullptr, *out = nullptr;
-      if (ihip::Err e = run.read_f32(r.a.buffer, &in); !e.empty()) return e;
-      if (ihip::Err e = run.write_f32(r.out, &out); !e.empty()) return e;
+      // rows that fit the registers of a workgroup are read and written in their own types; longer bf16 rows are
+      // widened into a temporary first, and rounded from one afterwards
+      ihip::DType in_dt = ihip::F32, out_dt = ihip::F32;
+      if (run.dtype_of(r.a.buffer) == DType::BF16 && r.a.buffer.kind == BufferRef::Input && ihip::row_softmax_any_supported(x.back())) {
+        in = run.raw_ptr(r.a.buffer);
+        in_dt = ihip::BF16;
+      } else if (ihip::Err e = run.read_f32(r.a.buffer, &in); !e.empty()) {
+        return e;
+      }
+      if (run.dtype_of(r.out) == DType::BF16 && ihip::row_softmax_any_supported(x.back()) && !read_back(run, r.out)) {
+        out = run.raw_ptr(r.out);
+        out_dt = ihip::BF16;
+      } else if (ihip::Err e = run.write_f32(r.out, &out); !e.empty()) {
+        return e;
+      }
       const int mode = r.kind == Recognized::RowSoftmax ? 0 : r.kind == Recognized::RowMaxShift ? 1 : r.kind == Recognized::RowNormalize ? 2 : 3;
       // a few very long rows: every row in parts over workgroups, the parts' (max, sum) pairs in a small temporary
       unsigned parts = ihip::row_softmax_parts(rows, x.back(), mode);
       void* stats = nullptr;
       if (parts > 1 && !run.alloc(&stats, rows * parts * 8).empty()) parts = 1;
-      return ihip::launch_row_softmax(static_cast<const float*>(in), static_cast<float*>(out), rows, x.back(), run.stream, mode, note,
-                                      nullptr, 1.0f, static_cast<float*>(stats), parts);
+      return ihip::launch_row_softmax(in, out, rows, x.back(), run.stream, mode, note, nullptr, 1.0f, static_cast<float*>(stats), parts,
+                                      in_dt, out_dt);
     }
     default: return "no hand-written kernel";
   }

@@ -166,25 +166,16 @@ extern "C" __global__ void __launch_bounds__(512, 1) gemm_nt_f32_256x256x32_dire
   gemm_nt_f32_direct_body<256, 2, 4, true>(p);
 }
 
-// row_<op>_wave_{v,s}<NV>, row_<op>_sub_{v,s}<G>, row_<op>_group_{v,s}<NV> and row_<op>_block[_v] for op = softmax,
-// shift (x - row max), norm (x / row sum), exp, scaled_softmax
+// row_<op>_wave_v<NV>, row_<op>_sub_{v,s}<G>, row_<op>_group_v<NV>, row_<op>_any_<T>x<NG> and row_<op>_block[_v] for
+// op = softmax, shift (x - row max), norm (x / row sum), exp, scaled_softmax
 #define ROW_WAVE(OP, MODE, NV)                                                                     \
   extern "C" __global__ void __launch_bounds__(256) row_##OP##_wave_v##NV(SoftmaxParams p) {       \
-    row_softmax_wave_body<NV, true, MODE>(p);                                                      \
-  }                                                                                                \
-  extern "C" __global__ void __launch_bounds__(256) row_##OP##_wave_s##NV(SoftmaxParams p) {       \
-    row_softmax_wave_body<NV, false, MODE>(p);                                                     \
+    row_softmax_wave_body<NV, MODE>(p);                                                            \
   }
-// row_<op>_group_{v,s}<NV>: 8192 < cols <= 4096 * NV, one workgroup of 16 wavefronts per row, row in registers
-// (no s16: element-wise loads of 64 values per lane do not fit 128 registers; such rows take the two-pass kernel)
-#define ROW_GROUP_V(OP, MODE, NV)                                                                  \
-  extern "C" __global__ void __launch_bounds__(1024) row_##OP##_group_v##NV(SoftmaxParams p) {     \
-    row_softmax_group_body<NV, true, MODE>(p);                                                     \
-  }
+// row_<op>_group_v<NV>: 8192 < cols <= 4096 * NV, one workgroup of 16 wavefronts per row, row in registers
 #define ROW_GROUP(OP, MODE, NV)                                                                    \
-  ROW_GROUP_V(OP, MODE, NV)                                                                        \
-  extern "C" __global__ void __launch_bounds__(1024) row_##OP##_group_s##NV(SoftmaxParams p) {     \
-    row_softmax_group_body<NV, false, MODE>(p);                                                    \
+  extern "C" __global__ void __launch_bounds__(1024) row_##OP##_group_v##NV(SoftmaxParams p) {     \
+    row_softmax_group_body<NV, MODE>(p);                                                           \
   }
 // row_<op>_sub_{v,s}<G>: cols <= 4 G <= 128, G lanes per row (64 / G rows per wavefront)
 #define ROW_SUB(OP, MODE, G)                                                                       \
@@ -194,12 +185,22 @@ extern "C" __global__ void __launch_bounds__(512, 1) gemm_nt_f32_256x256x32_dire
   extern "C" __global__ void __launch_bounds__(256) row_##OP##_sub_s##G(SoftmaxParams p) {         \
     row_softmax_sub_body<G, false, MODE>(p);                                                       \
   }
+// row_<op>_any_<T>x<NG>: T lanes per row, NG groups of 8 elements each; any alignment, f32 or bf16 on either side
+#define ROW_ANY(OP, MODE, T, NG)                                                                   \
+  extern "C" __global__ void __launch_bounds__(T > 256 ? T : 256) row_##OP##_any_##T##x##NG(SoftmaxParams p) { \
+    row_softmax_any_body<T, NG, MODE>(p);                                                          \
+  }
 #define ROW_OP(OP, MODE)                                                                           \
   ROW_WAVE(OP, MODE, 1) ROW_WAVE(OP, MODE, 2) ROW_WAVE(OP, MODE, 4) ROW_WAVE(OP, MODE, 8)          \
   ROW_WAVE(OP, MODE, 16) ROW_WAVE(OP, MODE, 32)                                                    \
-  ROW_GROUP(OP, MODE, 4) ROW_GROUP(OP, MODE, 8) ROW_GROUP_V(OP, MODE, 16)                           \
+  ROW_GROUP(OP, MODE, 4) ROW_GROUP(OP, MODE, 8) ROW_GROUP(OP, MODE, 16)                             \
   ROW_SUB(OP, MODE, 1) ROW_SUB(OP, MODE, 2) ROW_SUB(OP, MODE, 4) ROW_SUB(OP, MODE, 8)              \
   ROW_SUB(OP, MODE, 16) ROW_SUB(OP, MODE, 32)                                                      \
+  ROW_ANY(OP, MODE, 2, 1) ROW_ANY(OP, MODE, 4, 1) ROW_ANY(OP, MODE, 8, 1) ROW_ANY(OP, MODE, 16, 1) \
+  ROW_ANY(OP, MODE, 32, 1) ROW_ANY(OP, MODE, 64, 1) ROW_ANY(OP, MODE, 64, 2) ROW_ANY(OP, MODE, 64, 3) \
+  ROW_ANY(OP, MODE, 64, 4) ROW_ANY(OP, MODE, 64, 6) ROW_ANY(OP, MODE, 64, 8)                       \
+  ROW_ANY(OP, MODE, 256, 3) ROW_ANY(OP, MODE, 256, 4) ROW_ANY(OP, MODE, 256, 6) ROW_ANY(OP, MODE, 256, 8) \
+  ROW_ANY(OP, MODE, 1024, 3) ROW_ANY(OP, MODE, 1024, 4) ROW_ANY(OP, MODE, 1024, 6) ROW_ANY(OP, MODE, 1024, 9) \
   extern "C" __global__ void __launch_bounds__(1024) row_##OP##_block(SoftmaxParams p) {           \
     row_softmax_block_body<MODE, false>(p);                                                        \
   }                                                                                                \

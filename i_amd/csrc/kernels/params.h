@@ -71,8 +71,8 @@ struct SplitReduceParams {
 };
 
 struct SoftmaxParams {
-  const float* x;
-  float* y;
+  const void* x;  // f32, or bf16 when in_bf16 is set (the row_*_any_* kernels)
+  void* y;
   uint32_t rows, cols;
   // the "softmax of scale * x" kernels only: scale = scale_value * (scale_ptr ? *scale_ptr : 1)
   const float* scale_ptr;
@@ -82,6 +82,9 @@ struct SoftmaxParams {
   // leaves each part's running max and sum of exponentials in stats[row][part][2], the second combines them.
   float* stats;
   uint32_t parts, part_chunks;
+  // the row_*_any_* kernels: types, how many elements x lies past a 16-byte boundary, and whether y's 16-byte
+  // boundaries fall on the same elements as those of the groups of 8 that start on x's
+  uint32_t in_bf16, out_bf16, x_shift, y_wide;
 };
 
 struct ConvertParams {

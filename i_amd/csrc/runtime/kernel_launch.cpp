@@ -625,8 +625,14 @@ unsigned row_softmax_parts(size_t rows, size_t cols, int mode) {
   return parts < 2 ? 1u : (unsigned)parts;
 }
 
-Err launch_row_softmax(const float* x, float* y, size_t rows, size_t cols, hipStream_t stream, int mode,
-                       LaunchNote* note, const float* scale_ptr, float scale, float* stats, unsigned parts) {
+// Groups of 8 elements that a row of the row_*_any_* kernels spans at most, `shift` being where its operand starts
+// (in elements past a 16-byte boundary).
+static size_t row_groups(size_t cols, unsigned shift) { return cols % 8 == 0 && shift == 0 ? cols / 8 : (cols + 14) / 8; }
+
+bool row_softmax_any_supported(size_t cols) { return cols <= 65536; }
+
+Err launch_row_softmax(const void* x, void* y, size_t rows, size_t cols, hipStream_t stream, int mode, LaunchNote* note,
+                       const float* scale_ptr, float scale, float* stats, unsigned parts, DType in_dtype, DType out_dtype) {
   if (rows == 0 || cols == 0) return {};
   if (!fits_u32(rows) || !fits_u32(cols)) return "row_softmax kernel: extent exceeds 32 bits";
   if (!x || !y) return "row_softmax kernel: null device pointer";
@@ -635,8 +641,10 @@ Err launch_row_softmax(const float* x, float* y, size_t rows, size_t cols, hipSt
   static const char* const kOps[5] = {"softmax", "shift", "norm", "exp", "scaled_softmax"};
   SoftmaxParams p{x, y, (uint32_t)rows, (uint32_t)cols, scale_ptr, scale};
   hipFunction_t fn;
-  const bool vec = cols % 4 == 0 && (reinterpret_cast<uintptr_t>(x) % 16 == 0) && (reinterpret_cast<uintptr_t>(y) % 16 == 0);
-  if (parts > 1 && (mode == 0 || mode == 4)) {
+  const bool f32 = in_dtype == F32 && out_dtype == F32;
+  if (!f32 && !row_softmax_any_supported(cols)) return "row_softmax kernel: bf16 rows are too long";
+  const bool vec = f32 && cols % 4 == 0 && (reinterpret_cast<uintptr_t>(x) % 16 == 0) && (reinterpret_cast<uintptr_t>(y) % 16 == 0);
+  if (f32 && parts > 1 && (mode == 0 || mode == 4)) {
     // every row in parts over workgroups: the parts' (max, sum) pairs into `stats`, then a second launch that
     // combines them and writes
     if (!stats) return "row_softmax kernel: rows in parts need their temporary";
@@ -652,7 +660,37 @@ Err launch_row_softmax(const float* x, float* y, size_t rows, size_t cols, hipSt
     if (Err e = builtin_function((base + "apply" + (vec ? "_v" : "")).c_str(), &fn); !e.empty()) return e;
     return launch(fn, (unsigned)(rows * p.parts), 1, 1, 1024, &p, sizeof(p), stream);
   }
-  if (cols <= 128) {
+  // f32 rows whose length is a multiple of 4 and that start on 16-byte boundaries: float4 chunks.  Every other row
+  // that registers hold (odd lengths, other alignments, bf16 on either side): groups of 8 elements; but f32 rows of
+  // at most 128 columns keep the form with few lanes per row (2000000 x 31: 114 against 209 us).
+  if (!vec && row_softmax_any_supported(cols) && !(f32 && cols <= 128)) {
+    const size_t in_elem = in_dtype == BF16 ? 2 : 4, out_elem = out_dtype == BF16 ? 2 : 4;
+    const size_t x_shift = reinterpret_cast<uintptr_t>(x) % 16 / in_elem, y_shift = reinterpret_cast<uintptr_t>(y) % 16 / out_elem;
+    p.in_bf16 = in_dtype == BF16;
+    p.out_bf16 = out_dtype == BF16;
+    p.x_shift = (uint32_t)x_shift;
+    p.y_wide = (8 + x_shift - y_shift) % (16 / out_elem) == 0;
+    const size_t groups = row_groups(cols, p.x_shift);
+    // Lanes per row and groups per lane: one group per lane up to 32 groups, a wavefront up to 512, then workgroups
+    // of 256 and 1024 lanes, with the least number of groups per lane that covers the row.
+    size_t lanes = 2, each = 1;
+    if (groups <= 64) {
+      while (lanes < groups) lanes *= 2;
+    } else {
+      lanes = groups <= 512 ? 64 : groups <= 2048 ? 256 : 1024;
+      for (size_t n : {2, 3, 4, 6, lanes == 1024 ? 9 : 8}) {
+        each = n;
+        if (!(lanes > 64 && n < 3) && lanes * n >= groups) break;
+      }
+    }
+    const std::string name = std::string("row_") + kOps[mode] + "_any_" + std::to_string(lanes) + "x" + std::to_string(each);
+    if (note) *note = LaunchNote{name, 0, 0};
+    if (Err e = builtin_function(name.c_str(), &fn); !e.empty()) return e;
+    const size_t threads = lanes > 256 ? lanes : 256, grid = (rows * lanes + threads - 1) / threads;
+    if (grid > kMaxGrid) return "row_softmax kernel: grid too large";
+    return launch(fn, (unsigned)grid, 1, 1, (unsigned)threads, &p, sizeof(p), stream);
+  }
+  if (f32 && cols <= 128) {
     // G lanes per row, one float4 chunk each: 64 / G rows per wavefront
     size_t g = 1;
     while (4 * g < cols) g *= 2;
@@ -663,10 +701,10 @@ Err launch_row_softmax(const float* x, float* y, size_t rows, size_t cols, hipSt
     if (grid > kMaxGrid) return "row_softmax kernel: grid too large";
     return launch(fn, (unsigned)grid, 1, 1, 256, &p, sizeof(p), stream);
   }
-  if (cols <= 8192) {
+  if (vec && cols <= 8192) {
     int nv = 1;
     while ((size_t)256 * nv < cols) nv *= 2;
-    const std::string name = std::string("row_") + kOps[mode] + "_wave_" + (vec ? "v" : "s") + std::to_string(nv);
+    const std::string name = std::string("row_") + kOps[mode] + "_wave_v" + std::to_string(nv);
     if (note) *note = LaunchNote{name, 0, 0};
     if (Err e = builtin_function(name.c_str(), &fn); !e.empty()) return e;
     const size_t grid = (rows + 3) / 4;  // four wavefronts (rows) per workgroup
@@ -674,10 +712,10 @@ Err launch_row_softmax(const float* x, float* y, size_t rows, size_t cols, hipSt
     return launch(fn, (unsigned)grid, 1, 1, 256, &p, sizeof(p), stream);
   }
   if (rows > kMaxGrid) return "row_softmax kernel: grid too large";
-  if (cols <= 32768 || (cols <= 65536 && vec)) {
+  if (vec && cols <= 65536) {
     // the row still fits the registers of one workgroup of 16 wavefronts: one read and one write per element
     const int nv = cols <= 16384 ? 4 : cols <= 32768 ? 8 : 16;
-    const std::string name = std::string("row_") + kOps[mode] + "_group_" + (vec ? "v" : "s") + std::to_string(nv);
+    const std::string name = std::string("row_") + kOps[mode] + "_group_v" + std::to_string(nv);
     if (note) *note = LaunchNote{name, 0, 0};
     if (Err e = builtin_function(name.c_str(), &fn); !e.empty()) return e;
     return launch(fn, (unsigned)rows, 1, 1, 1024, &p, sizeof(p), stream);

@@ -108,13 +108,15 @@ Err launch_gemm_nt_f32(const float* a, const float* b, float* c, size_t bh, size
 unsigned gemm_nt_f32_split_k(size_t bh, size_t m, size_t n, size_t k, const KernelOptions& knobs = {});
 bool gemm_nt_f32_supported(size_t k);
 
-// y[rows,cols] = row softmax of x, f32
+// y[rows,cols] = row softmax of x, each f32 or bf16 (arithmetic in f32; bf16 on either side for rows that
+// row_softmax_any_supported() takes, up to 65536 columns)
 // mode 0: softmax; 1: y = x - rowmax(x) (row_max_shift); 2: y = x / rowsum(x) (row_normalize); 3: y = exp(x);
 // 4: softmax of s * x with s = scale * (scale_ptr ? *scale_ptr : 1), scale_ptr a rank-0 f32 operand in device memory.
 // y may be x: every kernel has read a row's element before it writes it.
-Err launch_row_softmax(const float* x, float* y, size_t rows, size_t cols, hipStream_t stream, int mode = 0,
+Err launch_row_softmax(const void* x, void* y, size_t rows, size_t cols, hipStream_t stream, int mode = 0,
                        LaunchNote* note = nullptr, const float* scale_ptr = nullptr, float scale = 1.0f,
-                       float* stats = nullptr, unsigned parts = 1);
+                       float* stats = nullptr, unsigned parts = 1, DType in_dtype = F32, DType out_dtype = F32);
+bool row_softmax_any_supported(size_t cols);
 // (parts > 1, softmax modes only: every row in that many parts over workgroups, two launches; `stats` is room for
 // 2 * rows * parts floats; row_softmax_parts says when it pays: fewer rows than half the CUs, 2^17 columns and more)
 unsigned row_softmax_parts(size_t rows, size_t cols, int mode);
