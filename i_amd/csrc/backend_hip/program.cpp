@@ -352,6 +352,15 @@ ihip::Err launch_product_f32(Run& run, const void* a, const void* b, void* c, si
                                   run.stream, note, static_cast<float*>(partial), splits, run.knobs);
 }
 
+// A product with few rows of A on the kernels for those (gemm_narrow_usable has said so).
+ihip::Err launch_product_narrow(Run& run, const void* a, const void* b, void* c, ihip::DType t, bool nn, size_t bh, size_t m, size_t n,
+                                size_t k, ihip::LaunchNote* note, ihip::DType out_dt) {
+  void* partial = nullptr;
+  unsigned splits = ihip::gemm_narrow_parts(nn, bh, m, n, k);
+  if (splits > 1 && !run.alloc_optional(&partial, bh * splits * m * n * 4)) splits = 1;
+  return ihip::launch_gemm_narrow(a, b, c, t, nn, bh, m, n, k, run.stream, note, out_dt, static_cast<float*>(partial), splits);
+}
+
 // Q, K and V in the arithmetic type of the attention: as they are, or read as f32 (bf16 ones widened into temporaries).
 ihip::Err attention_operands(Run& run, const Recognized& r, bool bf16, const void** q, const void** k, const void** v) {
   if (bf16) {
@@ -547,10 +556,13 @@ ihip::Err launch_hand_noted(Run& run, const Recognized& r, ihip::LaunchNote* not
       if (ihip::Err e = product_operands(run, r, t, &pa, &pb); !e.empty()) return e;
       size_t k = a[nb + 1];
       if (ihip::Err e = padded_operands(run, t, &pa, bh * a[nb], &pb, bh * b[nb], &k); !e.empty()) return e;
+      // (the schedule names one of the tiled kernels' own tiles: then that kernel runs as asked)
+      const bool tile_asked = (r.tile_i == 128 && r.tile_j == 128) || (r.tile_i == 256 && r.tile_j == 256);
+      const ihip::DType kernel_t = t == DType::F32 ? ihip::F32 : ihip::BF16;
+      if (!tile_asked && ihip::gemm_narrow_usable(kernel_t, false, bh, a[nb], b[nb], k, run.knobs))
+        return launch_product_narrow(run, pa, pb, out, kernel_t, false, bh, a[nb], b[nb], k, note, out_dt);
       if (t == DType::F32) return launch_product_f32(run, pa, pb, out, bh, a[nb], b[nb], k, note);
       // few output tiles under a long k loop: the loop is split over workgroups, partial products in a temporary
-      // (unless the schedule names one of the kernels' own tiles: then that kernel runs as asked)
-      const bool tile_asked = (r.tile_i == 128 && r.tile_j == 128) || (r.tile_i == 256 && r.tile_j == 256);
       if (const unsigned splits = tile_asked && run.knobs.gemm_k_parts < 2 ? 1u : ihip::gemm_nt_bf16_split_k(bh, a[nb], b[nb], k, run.knobs);
           splits > 1 && (a[nb] * b[nb]) % 4 == 0) {
         void* partial = nullptr;
@@ -583,9 +595,12 @@ ihip::Err launch_hand_noted(Run& run, const Recognized& r, ihip::LaunchNote* not
       }
       const void *pa = nullptr, *pb_rows = nullptr;
       if (ihip::Err e = product_operands(run, r, f32 ? DType::F32 : DType::BF16, &pa, &pb_rows); !e.empty()) return e;
-      if (!f32 && ihip::gemm_nn_bf16_supported(bh, m, n, k, run.knobs) && reinterpret_cast<uintptr_t>(pa) % 16 == 0 &&
-          reinterpret_cast<uintptr_t>(pb_rows) % 16 == 0) {  // the direct kernels read a row-major right operand themselves
-        const bool tile_asked = (r.tile_i == 128 && r.tile_j == 128) || (r.tile_i == 256 && r.tile_j == 256);
+      const bool tile_asked = (r.tile_i == 128 && r.tile_j == 128) || (r.tile_i == 256 && r.tile_j == 256);
+      const bool aligned = reinterpret_cast<uintptr_t>(pa) % 16 == 0 && reinterpret_cast<uintptr_t>(pb_rows) % 16 == 0;
+      const ihip::DType kernel_t = f32 ? ihip::F32 : ihip::BF16;
+      if (aligned && !tile_asked && ihip::gemm_narrow_usable(kernel_t, true, bh, m, n, k, run.knobs))
+        return launch_product_narrow(run, pa, pb_rows, out, kernel_t, true, bh, m, n, k, note, out_dt);
+      if (!f32 && aligned && ihip::gemm_nn_bf16_supported(bh, m, n, k, run.knobs)) {  // the direct kernels read a row-major right operand themselves
         unsigned splits = tile_asked && run.knobs.gemm_k_parts < 2 ? 1u : ihip::gemm_nt_bf16_split_k(bh, m, n, k, run.knobs);
         void* partial = nullptr;
         if (splits > 1 && ((m * n) % 4 != 0 || !run.alloc_optional(&partial, bh * splits * m * n * 4))) splits = 1;

@@ -5,6 +5,7 @@
 #include "attention_bf16_direct.h"
 #include "attention_f32.h"
 #include "attention_f32_direct.h"
+#include "gemm_narrow.h"
 #include "gemm_nt_bf16.h"
 #include "gemm_nt_f32_direct.h"
 #include "gemm_nt_bf16_mfma16.h"
@@ -165,6 +166,21 @@ extern "C" __global__ void __launch_bounds__(256, 2) gemm_nt_f32_128x128x32_dire
 extern "C" __global__ void __launch_bounds__(512, 1) gemm_nt_f32_256x256x32_direct_ktail(GemmParams p) {
   gemm_nt_f32_direct_body<256, 2, 4, true>(p);
 }
+
+// gemm_{nt_bf16,nt_f32,nn_f32}_narrow<M>x<columns per workgroup>: at most M = 16, 32, 64 rows of A
+#define GEMM_NARROW(NAME, F32, NN, M, MT, N, TN, W)                                                           \
+  extern "C" __global__ void __launch_bounds__(W * 64) gemm_##NAME##_narrow##M##x##N(GemmParams p) {          \
+    gemm_narrow_body<F32, NN, MT, TN, W>(p);                                                                  \
+  }
+GEMM_NARROW(nt_bf16, false, false, 16, 1, 16, 1, 16)
+GEMM_NARROW(nt_bf16, false, false, 16, 1, 32, 2, 16)
+GEMM_NARROW(nt_f32, true, false, 16, 1, 16, 1, 16)
+GEMM_NARROW(nt_f32, true, false, 16, 1, 32, 2, 16)
+GEMM_NARROW(nt_f32, true, false, 32, 2, 16, 1, 16)
+GEMM_NARROW(nt_f32, true, false, 32, 2, 32, 2, 16)
+GEMM_NARROW(nn_f32, true, true, 16, 1, 64, 4, 8)
+GEMM_NARROW(nn_f32, true, true, 32, 2, 64, 4, 8)
+GEMM_NARROW(nn_f32, true, true, 64, 4, 64, 4, 8)
 
 // row_<op>_wave_v<NV>, row_<op>_sub_{v,s}<G>, row_<op>_group_v<NV>, row_<op>_any_<T>x<NG> and row_<op>_block[_v] for
 // op = softmax, shift (x - row max), norm (x / row sum), exp, scaled_softmax

@@ -1,5 +1,6 @@
 #include "kernel_launch.h"
 
+#include <algorithm>
 #include <cmath>
 #include <cstdlib>
 #include <initializer_list>
@@ -418,7 +419,7 @@ unsigned gemm_nt_bf16_split_k(size_t bh, size_t m, size_t n, size_t k, const Ker
   // 256 x 256 tile, plus two slabs' worth before and after its loop; the chip holds 512 / 256 of them at a time;
   // the second launch costs 4 us and the pass over the partial products runs at 3 TB/s.  Examples (unsplit ->
   // split): 64 x 8192 x 8192 79 -> 30 us in 8 parts, 512 x 512 x 4096 52 -> 27 in 8, 256 x 4096 x 4096 41 -> 29
-  // in 8, 256 x 256 x 65536 576 -> 49 in 32; left whole: 1024^3 (10 us; 25 in 2 parts), 2048^3 (28; 40).
+  // in 8, 256 x 256 x 65536 576 -> 49 in 32, 29 x 9904 x 7968 39 in 6 (78 tiles; 48 in 4, 51 in 8); left whole: 1024^3 (10 us; 25 in 2 parts), 2048^3 (28; 40).
   if (k > (size_t(1) << 22)) return 1;
   const size_t slabs = (k + 63) / 64;
   const size_t t128 = ((m + 127) / 128) * ((n + 127) / 128) * bh, t256 = ((m + 255) / 256) * ((n + 255) / 256) * bh;
@@ -431,7 +432,7 @@ unsigned gemm_nt_bf16_split_k(size_t bh, size_t m, size_t n, size_t k, const Ker
   best *= 0.85;  // a split has to gain at least 15 %
   const size_t tiles = tile == 256 ? t256 : t128;
   size_t splits = 1;
-  for (size_t s = 2; s <= 32 && k / s >= 512 && bh * s <= 65535; s *= 2) {
+  for (size_t s = 2; s <= 32 && k / s >= 512 && bh * s <= 65535; ++s) {
     const double t = time_of(tile, tiles * s, (slabs + s - 1) / s) + 4.0 + (double)(bh * s * m * n * 4) / 3e6;
     if (t < best) {
       best = t;
@@ -536,6 +537,69 @@ Err launch_gemm_nn_bf16(const void* a, const void* b, void* c, size_t bh, size_t
   if (Err e = builtin_function("splitk_reduce", &fn); !e.empty()) return e;
   size_t rgrid = (bh * m * n / 4 + 255) / 256;
   if (rgrid > 65536) rgrid = 65536;
+  return launch(fn, (unsigned)rgrid, 1, 1, 256, &r, sizeof(r), stream);
+}
+
+// Where B's one pass through registers beats the tiled kernels (us, tiled -> narrow).  f32 NT up to 32 rows: 30 x 4096
+// x 4096 41 -> 28, 16 x 8192 x 8192 128 -> 66; from 33 rows on nothing is gained (64 x 8192 x 8192 130 -> 137).  f32 NN
+// up to 64 rows, where the tiled kernel needs a transposed copy of B: 64 x 1024 x 16384 78 -> 42.  bf16, whose tiled
+// kernel reads a large B at 5 TB/s, only where the tiled form's second launch weighs as much as B: NT, up to 16 rows,
+// B of at most 40 MB and k up to 8192 (4 x 16384 x 1024 17.4 -> 11.8, 15 x 1248 x 4528 14.9 -> 11.8; 8 x 1024 x
+// 16384 would go 16 -> 27).
+bool gemm_narrow_usable(DType dtype, bool nn, size_t bh, size_t m, size_t n, size_t k, const KernelOptions& knobs) {
+  if (knobs.gemm_tile || knobs.gemm_waves || knobs.gemm_k_parts || !knobs.gemm_direct) return false;  // (a tiled kernel is asked for)
+  if (bh == 0 || bh > 65535 / 32 || m == 0 || n < 512 || k < 512 || !fits_u32(n) || k > (size_t(1) << 22)) return false;
+  if (dtype == BF16) return !nn && m <= 16 && k % 8 == 0 && k <= 8192 && n * k * 2 <= size_t(40) * 1000 * 1000;
+  return k % 4 == 0 && (nn ? m <= 64 && n % 4 == 0 : m <= 32);
+}
+
+// NT workgroups take 16 or 32 columns and are as many as n gives; an NN workgroup takes 64, and the k loop is cut into
+// parts of at least 256, added up by a second launch, until there are three workgroups per CU (16 x 9808 x 4288 is
+// 153 column tiles: 50 us in 2 parts, 41 in 6; 20 x 9000 x 6000 108 and 78).
+unsigned gemm_narrow_parts(bool nn, size_t bh, size_t m, size_t n, size_t k) {
+  if (!nn || (m * n) % 4 != 0) return 1;
+  const size_t tiles = (n + 63) / 64 * bh;
+  if (tiles >= 576 || (tiles >= 192 && k < 2048)) return 1;  // (1 x 16384 x 1024: 14 us whole, 17 in 3 parts)
+  const size_t want = std::min<size_t>(std::min<size_t>((768 + tiles - 1) / tiles, k / 256), 32);
+  if (want < 2) return 1;
+  const size_t chunk = (k / want + 63) / 64 * 64;
+  return (unsigned)((k + chunk - 1) / chunk);
+}
+
+Err launch_gemm_narrow(const void* a, const void* b, void* c, DType dtype, bool nn, size_t bh, size_t m, size_t n, size_t k,
+                       hipStream_t stream, LaunchNote* note, DType out_dtype, float* partial, unsigned splits) {
+  if (m > (nn ? 64 : dtype == BF16 ? 16 : 32) || (nn && dtype == BF16) || bh * std::max(splits, 1u) > 65535 || k > (size_t(1) << 22) || !fits_u32(n)) return "narrow gemm kernel: extent too large";
+  if (k % (dtype == BF16 ? 8 : 4) != 0 || (nn && n % 4 != 0)) return "narrow gemm kernel: unsupported extents";
+  if (bh == 0 || m == 0 || n == 0) return {};
+  if (!a || !b || !c) return "narrow gemm kernel: null device pointer";
+  if (!aligned16(a) || !aligned16(b)) return "narrow gemm kernel: operands must be 16-byte aligned";
+  GemmParams p{};
+  p.a = a; p.b = b; p.c = c;
+  p.bh = (uint32_t)bh; p.m = (uint32_t)m; p.n = (uint32_t)n; p.k = (uint32_t)k;
+  p.out_bf16 = out_dtype == BF16 ? 1u : 0u;
+  if (splits > 1) {
+    if (!partial || (m * n) % 4 != 0) return "narrow gemm kernel: a split needs its temporary and m * n a multiple of 4";
+    p.k_chunk = (uint32_t)(((k + splits - 1) / splits + 63) / 64 * 64);
+    splits = (unsigned)((k + p.k_chunk - 1) / p.k_chunk);  // (rounding the parts up may leave fewer of them)
+  }
+  if (splits > 1) {
+    p.splits = splits;
+    p.c = partial;
+    p.out_bf16 = 0;
+  }
+  // 32 columns (A is read half as often) where that leaves 192 workgroups: 16 x 8192 x 8192 f32 79 us with 16, 66 with 32
+  const size_t tile = nn ? 64 : (n + 31) / 32 * bh < 192 ? 16 : 32;
+  const std::string name = std::string(nn ? "gemm_nn_" : "gemm_nt_") + (dtype == BF16 ? "bf16" : "f32") + "_narrow" +
+                           (m <= 16 ? "16x" : m <= 32 ? "32x" : "64x") + std::to_string(tile);
+  if (note) *note = LaunchNote{splits > 1 ? name + " (k in " + std::to_string(splits) + " parts)" : name, 0, 0};
+  hipFunction_t fn;
+  if (Err e = builtin_function(name.c_str(), &fn); !e.empty()) return e;
+  if (Err e = launch(fn, (unsigned)(((n + tile - 1) / tile + 7) / 8 * 8), (unsigned)(bh * std::max(splits, 1u)), 1, tile < 64 ? 1024 : 512, &p, sizeof(p), stream);
+      !e.empty() || splits <= 1)
+    return e;
+  SplitReduceParams r{partial, c, (uint32_t)bh, splits, (uint64_t)m * n, out_dtype == BF16 ? 1u : 0u};
+  if (Err e = builtin_function("splitk_reduce", &fn); !e.empty()) return e;
+  const size_t rgrid = std::min<size_t>((bh * m * n / 4 + 255) / 256, 65536);
   return launch(fn, (unsigned)rgrid, 1, 1, 256, &r, sizeof(r), stream);
 }
 

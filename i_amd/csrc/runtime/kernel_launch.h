@@ -108,6 +108,15 @@ Err launch_gemm_nt_f32(const float* a, const float* b, float* c, size_t bh, size
 unsigned gemm_nt_f32_split_k(size_t bh, size_t m, size_t n, size_t k, const KernelOptions& knobs = {});
 bool gemm_nt_f32_supported(size_t k);
 
+// A product with few rows of A: B straight into registers, read once.  gemm_narrow_usable says when it is taken
+// (f32 NT up to 32 rows, f32 NN up to 64, bf16 NT up to 16 rows of a small B; no tiled kernel asked for),
+// gemm_narrow_parts into how many parts its k loop goes (then `partial` is room for bh * splits * m * n floats);
+// operands 16-byte aligned.
+bool gemm_narrow_usable(DType dtype, bool nn, size_t bh, size_t m, size_t n, size_t k, const KernelOptions& knobs);
+unsigned gemm_narrow_parts(bool nn, size_t bh, size_t m, size_t n, size_t k);
+Err launch_gemm_narrow(const void* a, const void* b, void* c, DType dtype, bool nn, size_t bh, size_t m, size_t n, size_t k,
+                       hipStream_t stream, LaunchNote* note, DType out_dtype, float* partial = nullptr, unsigned splits = 1);
+
 // y[rows,cols] = row softmax of x, each f32 or bf16 (arithmetic in f32; bf16 on either side for rows that
 // row_softmax_any_supported() takes, up to 65536 columns)
 // mode 0: softmax; 1: y = x - rowmax(x) (row_max_shift); 2: y = x / rowsum(x) (row_normalize); 3: y = exp(x);
