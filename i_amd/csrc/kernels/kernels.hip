@@ -182,8 +182,7 @@ GEMM_NARROW(nn_f32, true, true, 16, 1, 64, 4, 8)
 GEMM_NARROW(nn_f32, true, true, 32, 2, 64, 4, 8)
 GEMM_NARROW(nn_f32, true, true, 64, 4, 64, 4, 8)
 
-// row_<op>_wave_v<NV>, row_<op>_sub_{v,s}<G>, row_<op>_group_v<NV>, row_<op>_any_<T>x<NG> and row_<op>_block[_v] for
-// op = softmax, shift (x - row max), norm (x / row sum), exp, scaled_softmax
+// row_<op>_wave_v<NV>, row_<op>_sub_{v,s}<G>, row_<op>_group_v<NV>, row_<op>_block[_v] and ROW_ANY's forms for op = softmax, shift (x - row max), norm (x / row sum), exp, scaled_softmax
 #define ROW_WAVE(OP, MODE, NV)                                                                     \
   extern "C" __global__ void __launch_bounds__(256) row_##OP##_wave_v##NV(SoftmaxParams p) {       \
     row_softmax_wave_body<NV, MODE>(p);                                                            \
@@ -201,9 +200,11 @@ GEMM_NARROW(nn_f32, true, true, 64, 4, 64, 4, 8)
   extern "C" __global__ void __launch_bounds__(256) row_##OP##_sub_s##G(SoftmaxParams p) {         \
     row_softmax_sub_body<G, false, MODE>(p);                                                       \
   }
-// row_<op>_any_<T>x<NG>: T lanes per row, NG groups of 8 elements each; any alignment, f32 or bf16 on either side
-#define ROW_ANY(OP, MODE, T, NG)                                                                   \
-  extern "C" __global__ void __launch_bounds__(T > 256 ? T : 256) row_##OP##_any_##T##x##NG(SoftmaxParams p) { \
+// Rows of any length, alignment and type (row_softmax_any_body: T lanes per row, NG groups of 8 elements each):
+// row_<op>_lanes_s<T>, 8 T columns; row_<op>_wave_s<NV>, a wavefront, 256 NV columns; row_<op>_group_s<NV>, a workgroup,
+// 4096 NV columns (rounded down)
+#define ROW_ANY(OP, MODE, FORM, T, NG)                                                             \
+  extern "C" __global__ void __launch_bounds__(T > 256 ? T : 256) row_##OP##_##FORM(SoftmaxParams p) { \
     row_softmax_any_body<T, NG, MODE>(p);                                                          \
   }
 #define ROW_OP(OP, MODE)                                                                           \
@@ -212,11 +213,12 @@ GEMM_NARROW(nn_f32, true, true, 64, 4, 64, 4, 8)
   ROW_GROUP(OP, MODE, 4) ROW_GROUP(OP, MODE, 8) ROW_GROUP(OP, MODE, 16)                             \
   ROW_SUB(OP, MODE, 1) ROW_SUB(OP, MODE, 2) ROW_SUB(OP, MODE, 4) ROW_SUB(OP, MODE, 8)              \
   ROW_SUB(OP, MODE, 16) ROW_SUB(OP, MODE, 32)                                                      \
-  ROW_ANY(OP, MODE, 2, 1) ROW_ANY(OP, MODE, 4, 1) ROW_ANY(OP, MODE, 8, 1) ROW_ANY(OP, MODE, 16, 1) \
-  ROW_ANY(OP, MODE, 32, 1) ROW_ANY(OP, MODE, 64, 1) ROW_ANY(OP, MODE, 64, 2) ROW_ANY(OP, MODE, 64, 3) \
-  ROW_ANY(OP, MODE, 64, 4) ROW_ANY(OP, MODE, 64, 6) ROW_ANY(OP, MODE, 64, 8)                       \
-  ROW_ANY(OP, MODE, 256, 3) ROW_ANY(OP, MODE, 256, 4) ROW_ANY(OP, MODE, 256, 6) ROW_ANY(OP, MODE, 256, 8) \
-  ROW_ANY(OP, MODE, 1024, 3) ROW_ANY(OP, MODE, 1024, 4) ROW_ANY(OP, MODE, 1024, 6) ROW_ANY(OP, MODE, 1024, 9) \
+  ROW_ANY(OP, MODE, lanes_s2, 2, 1) ROW_ANY(OP, MODE, lanes_s4, 4, 1) ROW_ANY(OP, MODE, lanes_s8, 8, 1)\
+  ROW_ANY(OP, MODE, lanes_s16, 16, 1) ROW_ANY(OP, MODE, lanes_s32, 32, 1) ROW_ANY(OP, MODE, wave_s2, 64, 1)\
+  ROW_ANY(OP, MODE, wave_s4, 64, 2) ROW_ANY(OP, MODE, wave_s6, 64, 3) ROW_ANY(OP, MODE, wave_s8, 64, 4)\
+  ROW_ANY(OP, MODE, wave_s12, 64, 6) ROW_ANY(OP, MODE, wave_s16, 64, 8) ROW_ANY(OP, MODE, group_s1, 256, 3)\
+  ROW_ANY(OP, MODE, group_s2, 256, 4) ROW_ANY(OP, MODE, group_s4, 256, 8) ROW_ANY(OP, MODE, group_s6, 1024, 3)\
+  ROW_ANY(OP, MODE, group_s8, 1024, 4) ROW_ANY(OP, MODE, group_s12, 1024, 6) ROW_ANY(OP, MODE, group_s18, 1024, 9)\
   extern "C" __global__ void __launch_bounds__(1024) row_##OP##_block(SoftmaxParams p) {           \
     row_softmax_block_body<MODE, false>(p);                                                        \
   }                                                                                                \

@@ -738,16 +738,18 @@ Err launch_row_softmax(const void* x, void* y, size_t rows, size_t cols, hipStre
     // Lanes per row and groups per lane: one group per lane up to 32 groups, a wavefront up to 512, then workgroups
     // of 256 and 1024 lanes, with the least number of groups per lane that covers the row.
     size_t lanes = 2, each = 1;
-    if (groups <= 64) {
+    std::string form;
+    if (groups <= 32) {
       while (lanes < groups) lanes *= 2;
     } else {
       lanes = groups <= 512 ? 64 : groups <= 2048 ? 256 : 1024;
-      for (size_t n : {2, 3, 4, 6, lanes == 1024 ? 9 : 8}) {
+      static const size_t kEach[3][6] = {{1, 2, 3, 4, 6, 8}, {3, 4, 8, 8, 8, 8}, {3, 4, 6, 9, 9, 9}};
+      for (size_t n : kEach[lanes == 64 ? 0 : lanes == 256 ? 1 : 2]) {
         each = n;
-        if (!(lanes > 64 && n < 3) && lanes * n >= groups) break;
+        if (lanes * n >= groups) break;
       }
     }
-    const std::string name = std::string("row_") + kOps[mode] + "_any_" + std::to_string(lanes) + "x" + std::to_string(each);
+    const std::string name = std::string("row_") + kOps[mode] + "_" + form;
     if (note) *note = LaunchNote{name, 0, 0};
     if (Err e = builtin_function(name.c_str(), &fn); !e.empty()) return e;
     const size_t threads = lanes > 256 ? lanes : 256, grid = (rows * lanes + threads - 1) / threads;
@@ -763,12 +765,14 @@ Err launch_row_softmax(const void* x, void* y, size_t rows, size_t cols, hipStre
     if (Err e = builtin_function(name.c_str(), &fn); !e.empty()) return e;
     const size_t grid = (rows * g + 255) / 256;
     if (grid > kMaxGrid) return "row_softmax kernel: grid too large";
+      form = "lanes_s" + std::to_string(lanes);
     return launch(fn, (unsigned)grid, 1, 1, 256, &p, sizeof(p), stream);
   }
   if (vec && cols <= 8192) {
     int nv = 1;
     while ((size_t)256 * nv < cols) nv *= 2;
     const std::string name = std::string("row_") + kOps[mode] + "_wave_v" + std::to_string(nv);
+      form = lanes == 64 ? "wave_s" + std::to_string(2 * each) : "group_s" + std::to_string(8 * lanes * each / 4096);
     if (note) *note = LaunchNote{name, 0, 0};
     if (Err e = builtin_function(name.c_str(), &fn); !e.empty()) return e;
     const size_t grid = (rows + 3) / 4;  // four wavefronts (rows) per workgroup
