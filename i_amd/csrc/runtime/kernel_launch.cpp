@@ -741,6 +741,7 @@ Err launch_row_softmax(const void* x, void* y, size_t rows, size_t cols, hipStre
     std::string form;
     if (groups <= 32) {
       while (lanes < groups) lanes *= 2;
+      form = "lanes_s" + std::to_string(lanes);
     } else {
       lanes = groups <= 512 ? 64 : groups <= 2048 ? 256 : 1024;
       static const size_t kEach[3][6] = {{1, 2, 3, 4, 6, 8}, {3, 4, 8, 8, 8, 8}, {3, 4, 6, 9, 9, 9}};
@@ -748,6 +749,7 @@ Err launch_row_softmax(const void* x, void* y, size_t rows, size_t cols, hipStre
         each = n;
         if (lanes * n >= groups) break;
       }
+      form = lanes == 64 ? "wave_s" + std::to_string(2 * each) : "group_s" + std::to_string(8 * lanes * each / 4096);
     }
     const std::string name = std::string("row_") + kOps[mode] + "_" + form;
     if (note) *note = LaunchNote{name, 0, 0};
@@ -765,14 +767,12 @@ Err launch_row_softmax(const void* x, void* y, size_t rows, size_t cols, hipStre
     if (Err e = builtin_function(name.c_str(), &fn); !e.empty()) return e;
     const size_t grid = (rows * g + 255) / 256;
     if (grid > kMaxGrid) return "row_softmax kernel: grid too large";
-      form = "lanes_s" + std::to_string(lanes);
     return launch(fn, (unsigned)grid, 1, 1, 256, &p, sizeof(p), stream);
   }
   if (vec && cols <= 8192) {
     int nv = 1;
     while ((size_t)256 * nv < cols) nv *= 2;
     const std::string name = std::string("row_") + kOps[mode] + "_wave_v" + std::to_string(nv);
-      form = lanes == 64 ? "wave_s" + std::to_string(2 * each) : "group_s" + std::to_string(8 * lanes * each / 4096);
     if (note) *note = LaunchNote{name, 0, 0};
     if (Err e = builtin_function(name.c_str(), &fn); !e.empty()) return e;
     const size_t grid = (rows + 3) / 4;  // four wavefronts (rows) per workgroup
