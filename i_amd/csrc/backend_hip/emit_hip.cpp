@@ -79,6 +79,13 @@ thread_local bool g_checked_accesses = true;
 // variable that stands for every access to that buffer while the loop is being printed.
 thread_local std::map<size_t, std::string> g_held;
 
+// readonlys whose elements are bf16 in the form being printed (GenericPhase::bf16_reads)
+thread_local std::set<size_t> g_bf16_reads;
+// writeables that are work-item-private in the strip form being printed: a Strip per element, "strip<ind>"
+thread_local std::set<size_t> g_strip_privates;
+// accesses that the statement being printed has loaded beforehand (strip forms): the text that stands for each
+thread_local std::map<const MExpr*, std::string> g_loaded;
+
 // `base[idx]` with base = readonlys[b].data or writeables[b].data: fills the capacity variable's name
 bool buffer_access(const MExpr& e, std::string* cap, bool* writeable = nullptr, size_t* ind = nullptr) {
   if (e.kind != MExpr::Index) return false;
@@ -107,9 +114,18 @@ const std::string* held_local(const MExpr& e) {
 std::string expr_text(const MExpr& e) {
   auto b = [&](const char* sym) { return "(" + expr_text(*e.args[0]) + " " + sym + " " + expr_text(*e.args[1]) + ")"; };
   if (const std::string* local = held_local(e)) return *local;
-  if (std::string cap; g_checked_accesses && buffer_access(e, &cap)) {
-    const std::string idx = expr_text(*e.args[1]);
-    return "((" + idx + ") < " + cap + " ? " + expr_text(*e.args[0]) + "[" + idx + "] : 0.0f)";
+  if (auto it = g_loaded.find(&e); it != g_loaded.end()) return it->second;
+  {
+    std::string cap;
+    bool writeable = false;
+    size_t ind = 0;
+    if (buffer_access(e, &cap, &writeable, &ind)) {
+      const std::string idx = expr_text(*e.args[1]);
+      const bool own = writeable && g_strip_privates.count(ind) != 0;
+      const std::string base = own ? "strip" + std::to_string(ind) : expr_text(*e.args[0]);
+      const std::string element = own ? base + "[" + idx + "].v[e]" : !writeable && g_bf16_reads.count(ind) ? "ilang_bf16(" + base + ", " + idx + ")" : base + "[" + idx + "]";
+      return g_checked_accesses ? "((" + idx + ") < " + cap + " ? " + element + " : 0.0f)" : element;
+    }
   }
   switch (e.kind) {
     case MExpr::Usize: return "(size_t)" + std::to_string(e.usize);
@@ -473,6 +489,82 @@ std::vector<std::pair<size_t, size_t>> phase_ranges(const Block<Param>& body) {
   return out;
 }
 
+// ------------------------------------------------------------------ strips of the innermost parallel loop
+const MExpr& without_casts(const MExpr& e) {
+  const MExpr* p = &e;
+  while (p->kind == MExpr::Cast) p = p->args[0].get();
+  return *p;
+}
+bool mentions(const MExpr& e, const std::string& ident) {
+  if (e.kind == MExpr::Ident && e.ident == ident) return true;
+  for (const MExprPtr& a : e.args)
+    if (a && mentions(*a, ident)) return true;
+  return false;
+}
+// an index in which `ident` counts elements: ident itself, or a sum of it and something without it
+bool unit_stride(const MExpr& index, const std::string& ident) {
+  const MExpr& e = without_casts(index);
+  if (e.kind == MExpr::Ident) return e.ident == ident;
+  return e.kind == MExpr::Add && without_casts(*e.args[1]).kind == MExpr::Ident && without_casts(*e.args[1]).ident == ident && !mentions(*e.args[0], ident);
+}
+// every mention of `ident` in a value is in the index of an element access that steps by one with it
+bool strip_value(const MExpr& e, const std::string& ident) {
+  std::string cap;
+  if (buffer_access(e, &cap)) return !mentions(*e.args[1], ident) || unit_stride(*e.args[1], ident);
+  if (e.kind == MExpr::Ident) return e.ident != ident;
+  for (const MExprPtr& a : e.args)
+    if (a && !strip_value(*a, ident)) return false;
+  return true;
+}
+// The strip form of a nest (GenericPhase::strip): a work-item runs four consecutive iterations of the innermost
+// parallel loop.  That loop may appear nowhere but in the indexes of element accesses, where it steps by one, and
+// every statement stores to such an access or to a private buffer (`privates`), of which every iteration has its own.
+bool strip_body(const std::vector<MStmt>& stmts, const std::string& ident, const std::set<size_t>& privates) {
+  for (const MStmt& s : stmts) {
+    if (s.kind == MStmt::Set) {
+      std::string cap;
+      bool writeable = false;
+      size_t ind = 0;
+      if (!buffer_access(*s.dst, &cap, &writeable, &ind) || !strip_value(*s.value, ident)) return false;
+      if (writeable && privates.count(ind) ? mentions(*s.dst->args[1], ident) : !unit_stride(*s.dst->args[1], ident)) return false;
+    } else if (s.kind == MStmt::Loop || s.kind == MStmt::If) {
+      if (mentions(*s.value, ident) || !strip_body(s.body, ident, privates)) return false;
+    } else {
+      return false;
+    }
+  }
+  return true;
+}
+// does a value read readonlys[ind] along `ident`?
+bool reads_along(const std::vector<MStmt>& stmts, size_t ind, const std::string& ident) {
+  std::function<bool(const MExpr&)> in = [&](const MExpr& e) {
+    std::string cap;
+    bool writeable = false;
+    size_t at = 0;
+    if (buffer_access(e, &cap, &writeable, &at) && !writeable && at == ind && mentions(*e.args[1], ident)) return true;
+    for (const MExprPtr& a : e.args)
+      if (a && in(*a)) return true;
+    return false;
+  };
+  for (const MStmt& s : stmts)
+    if ((s.kind == MStmt::Set && in(*s.value)) || reads_along(s.body, ind, ident)) return true;
+  return false;
+}
+bool reads_writeable(const std::vector<MStmt>& stmts, size_t ind) {
+  std::function<bool(const MExpr&)> in = [&](const MExpr& e) {
+    std::string cap;
+    bool writeable = false;
+    size_t at = 0;
+    if (buffer_access(e, &cap, &writeable, &at) && writeable && at == ind) return true;
+    for (const MExprPtr& a : e.args)
+      if (a && in(*a)) return true;
+    return false;
+  };
+  for (const MStmt& s : stmts)
+    if ((s.kind == MStmt::Set && in(*s.value)) || reads_writeable(s.body, ind)) return true;
+  return false;
+}
+
 // ------------------------------------------------------------------ statement printer
 // the first access to writeables[ind] in an expression / a statement list
 const MExpr* find_writeable_access(const MExpr& e, size_t ind) {
@@ -502,6 +594,8 @@ struct Printer {
   const std::map<size_t, std::vector<size_t>>* held = nullptr;  // loop id -> elements to hold in registers (held_elements)
   const std::vector<WaveLoop>* wave = nullptr;  // the wavefront-per-iteration form: loops spread over the lanes
   const GridForm* grid = nullptr;               // the form with a loop in parts: `part` of `parts` takes its share of grid->loop
+  std::string strip;                            // the strip form: the loop of which a work-item runs four iterations
+  size_t loaded = 0;                            // accesses loaded beforehand so far (their variables' numbers)
   int serial_depth = 0;                         // loops being printed as loops around the current statement
   // In the form with a loop in parts every part accumulates into copies of the accumulated buffers that the
   // launcher has filled with the reduction's identity: the nest's own initialisations of those buffers are dropped.
@@ -536,6 +630,110 @@ struct Printer {
     return true;
   }
   void line(int depth, const std::string& s) { os << std::string(2 * depth, ' ') << s << "\n"; }
+  // "data, index, capacity" of an element access, for the strip helpers
+  std::string place(const MExpr& access) const {
+    std::string cap;
+    buffer_access(access, &cap);
+    return expr_text(*access.args[0]) + ", " + expr_text(*access.args[1]) + (g_checked_accesses ? ", " + cap : std::string(", (size_t)-1"));
+  }
+  // Loads what a value reads into variables: accesses along the strip as four elements, others as the one they are.
+  void load_operands(const MExpr& e, int depth, std::vector<const MExpr*>& mine) {
+    std::string cap;
+    bool writeable = false;
+    size_t ind = 0;
+    if (buffer_access(e, &cap, &writeable, &ind)) {
+      if (held_local(e) || g_loaded.count(&e) || (writeable && g_strip_privates.count(ind))) return;
+      const std::string name = "t" + std::to_string(loaded++);
+      if (mentions(*e.args[1], strip)) {
+        const char* helper = !writeable && g_bf16_reads.count(ind) ? "ilang_load_bf16" : "ilang_load";
+        line(depth, "const Strip " + name + " = " + helper + "(" + place(e) + ");");
+        g_loaded[&e] = name + ".v[e]";
+      } else {
+        line(depth, "const float " + name + " = " + expr_text(e) + ";");
+        g_loaded[&e] = name;
+      }
+      mine.push_back(&e);
+      return;
+    }
+    for (const MExprPtr& a : e.args)
+      if (a) load_operands(*a, depth, mine);
+  }
+  void strip_set(const MStmt& s, int depth) {
+    std::string to = "r.v[e]", cap;
+    bool in_register = true, writeable = false;
+    size_t ind = 0;
+    if (const std::string* local = held_local(*s.dst)) {
+      to = *local;
+    } else if (buffer_access(*s.dst, &cap, &writeable, &ind) && writeable && g_strip_privates.count(ind)) {
+      const std::string idx = expr_text(*s.dst->args[1]);
+      to = (g_checked_accesses ? "if ((" + idx + ") < " + cap + ") " : std::string()) + "strip" + std::to_string(ind) + "[" + idx + "].v[e]";
+    } else {
+      in_register = false;
+    }
+    std::vector<const MExpr*> mine;
+    line(depth, "{");
+    load_operands(*s.value, depth + 1, mine);
+    if (!in_register) line(depth + 1, "Strip r;");
+    line(depth + 1, "#pragma unroll");
+    line(depth + 1, "for (int e = 0; e < 4; ++e) " + to + " = " + expr_text(*s.value) + ";");
+    for (const MExpr* e : mine) g_loaded.erase(e);
+    if (!in_register) strip_store(*s.dst, "r", depth + 1);
+    line(depth, "}");
+  }
+  void strip_store(const MExpr& dst, const std::string& value, int depth) {
+    std::string cap;
+    bool writeable = false;
+    size_t ind = 0;
+    buffer_access(dst, &cap, &writeable, &ind);
+    line(depth, "ilang_store(" + place(dst) + ", " + value + ", args.bf16_writes >> " + std::to_string(ind) + " & 1);");
+  }
+  void strip_accesses(const MExpr& e, const std::string& ident, std::vector<const MExpr*>& out) const {
+    std::string cap;
+    if (buffer_access(e, &cap) && !held_local(e) && mentions(*e.args[1], ident)) out.push_back(&e);
+    for (const MExprPtr& a : e.args)
+      if (a) strip_accesses(*a, ident, out);
+  }
+  // The part of a loop over the lanes that goes four consecutive iterations per lane: for a body that only accumulates
+  // into registers and steps through what it reads by one element.  Returns the variable that says where it ends
+  // (nothing: the loop has no such form).
+  std::string spread_in_strips(const MStmt& loop, bool in_parts, int depth) {
+    std::vector<const MExpr*> accesses;
+    for (const MStmt& s : loop.body) {
+      if (s.kind != MStmt::Set || !held_local(*s.dst) || !strip_value(*s.value, loop.ident)) return {};
+      strip_accesses(*s.value, loop.ident, accesses);
+    }
+    for (const MExpr* a : accesses) {
+      std::string cap;
+      bool writeable = false;
+      buffer_access(*a, &cap, &writeable);
+      if (writeable) return {};
+    }
+    if (accesses.empty()) return {};
+    const std::string whole = "whole_" + loop.ident, first = in_parts ? "part * share_" + loop.ident : "(size_t)0";
+    const std::string end = in_parts ? "end_" + loop.ident : expr_text(*loop.value);
+    std::string enough = end + " > " + first;
+    if (g_checked_accesses)
+      for (const MExpr* a : accesses) {
+        std::string cap;
+        buffer_access(*a, &cap);
+        if (enough.find(cap + " >= 4") == std::string::npos) enough += " && " + cap + " >= 4";
+      }
+    line(depth, "const size_t " + whole + " = " + first + " + (" + enough + " ? (" + end + " - " + first + ") / 4 * 4 : 0);");
+    line(depth, "#pragma unroll 4");
+    line(depth, "for (size_t " + loop.ident + " = " + first + " + 4 * lane; " + loop.ident + " < " + whole + "; " + loop.ident + " += 256) {");
+    // (one iteration after the other: a register may carry a value from one statement to the next)
+    strip = loop.ident;
+    std::vector<const MExpr*> mine;
+    for (const MStmt& s : loop.body) load_operands(*s.value, depth + 1, mine);
+    line(depth + 1, "#pragma unroll");
+    line(depth + 1, "for (int e = 0; e < 4; ++e) {");
+    for (const MStmt& s : loop.body) line(depth + 2, *held_local(*s.dst) + " = " + expr_text(*s.value) + ";");
+    line(depth + 1, "}");
+    for (const MExpr* e : mine) g_loaded.erase(e);
+    strip.clear();
+    line(depth, "}");
+    return whole;
+  }
   void block(const std::vector<MStmt>& stmts, int depth) {
     for (const MStmt& s : stmts) stmt(s, depth);
   }
@@ -544,6 +742,10 @@ struct Printer {
       case MStmt::Set: {
         std::string cap;
         if (dropped_initialisation(s)) break;
+        if (!strip.empty()) {
+          strip_set(s, depth);
+          break;
+        }
         if (const std::string* local = held_local(*s.dst)) {
           line(depth, *local + " = " + expr_text(*s.value) + ";");
         } else if (g_checked_accesses && buffer_access(*s.dst, &cap)) {
@@ -592,7 +794,10 @@ struct Printer {
             if (grid && grid->held_accumulators)
               for (const GridAccumulator& acc : grid->accumulators)
                 if (acc.writeable == h.ind) fresh = &acc;
-            if (h.shared) {
+            if (!strip.empty()) {
+              if (fresh) line(d, "Strip " + h.local + " = {{" + identity_text(fresh->op) + ", " + identity_text(fresh->op) + ", " + identity_text(fresh->op) + ", " + identity_text(fresh->op) + "}};");
+              else line(d, "Strip " + h.local + " = ilang_load(" + place(*h.at) + ");");
+            } else if (h.shared) {
               // the element as it is before the loop, and this lane's share of what the loop adds to it
               line(d, "const float before_" + h.local + " = " + (fresh ? std::string(identity_text(fresh->op)) : expr_text(*h.at)) + ";");
               line(d, "float " + h.local + " = " + identity_text(h.op) + ";");
@@ -600,7 +805,7 @@ struct Printer {
               line(d, "float " + h.local + " = " + (fresh ? std::string(identity_text(fresh->op)) : expr_text(*h.at)) + ";");
             }
           }
-          for (const Held& h : mine) g_held[h.ind] = h.local;
+          for (const Held& h : mine) g_held[h.ind] = strip.empty() ? h.local : h.local + ".v[e]";
           bool spread = false;  // this loop's iterations are dealt out over the lanes
           if (wave)
             for (const WaveLoop& wl : *wave) spread |= wl.spread == loop_id;
@@ -614,8 +819,12 @@ struct Printer {
             line(d, "const size_t end_" + s.ident + " = (part + 1) * share_" + s.ident + " < " + expr_text(*s.value) + " ? (part + 1) * share_" +
                         s.ident + " : " + expr_text(*s.value) + ";");
           }
+          // (a wavefront's lanes take four consecutive elements each first, and one each of what is left)
+          const std::string whole = spread ? spread_in_strips(s, in_parts, d) : std::string();
           if ((spread || !mine.empty()) && innermost(s.body)) line(d, "#pragma unroll 8");
-          if (spread && in_parts)
+          if (!whole.empty())
+            line(d, "for (size_t " + s.ident + " = " + whole + " + lane; " + s.ident + " < " + (in_parts ? "end_" + s.ident : expr_text(*s.value)) + "; " + s.ident + " += 64) {");
+          else if (spread && in_parts)
             line(d, "for (size_t " + s.ident + " = part * share_" + s.ident + " + lane; " + s.ident + " < end_" + s.ident + "; " + s.ident + " += 64) {");
           else if (spread)
             line(d, "for (size_t " + s.ident + " = lane; " + s.ident + " < " + expr_text(*s.value) + "; " + s.ident + " += 64) {");
@@ -630,6 +839,10 @@ struct Printer {
           for (const Held& h : mine) g_held.erase(h.ind);
           for (const Held& h : mine) {
             std::string value = h.local;
+            if (!strip.empty()) {
+              strip_store(*h.at, value, d);
+              continue;
+            }
             if (h.shared) {
               line(d, "for (int lane_xor = 32; lane_xor > 0; lane_xor >>= 1) " + h.local + " = " +
                           reduce_text(h.op, h.local, "__shfl_xor(" + h.local + ", lane_xor)") + ";");
@@ -864,6 +1077,9 @@ ExecPlan split_nests(const ExecPlan& plan, std::vector<size_t>* origin) {
 GenericModule emit_generic_hip(const ExecPlan& plan, const Module& module, const std::vector<bool>& emit) {
   const char* unchecked = std::getenv("ILANG_HIP_UNCHECKED");
   g_checked_accesses = !(unchecked && unchecked[0] == '1');
+  g_bf16_reads.clear();
+  g_strip_privates.clear();
+  g_loaded.clear();
   g_held.clear();  // (an error thrown while a loop was being printed must not leave its substitutions behind)
   GenericModule out;
   out.kernels.resize(plan.kernels.size());
@@ -877,6 +1093,33 @@ GenericModule emit_generic_hip(const ExecPlan& plan, const Module& module, const
   bool any = false, any_grid = false;
   src << "// generated by the i gfx950 backend\n#include <hip/hip_runtime.h>\n#include <math.h>\n#include <stddef.h>\n\n";
   src << "#ifndef ILANG_WAVE_SYNC\n#define ILANG_WAVE_SYNC() __builtin_amdgcn_wave_barrier()\n#endif\n\n";
+  src << "static __device__ __forceinline__ float ilang_bf16(const float* data, size_t at) {\n"
+         "  const unsigned bits = (unsigned)((const unsigned short*)data)[at] << 16;\n  float v;\n  __builtin_memcpy(&v, &bits, 4);\n  return v;\n}\n"
+         // four consecutive elements; the launcher has checked that every buffer accessed so has at least four (cap >= 4).
+         // A strip that does not lie inside its buffer reads as zeros: no branch around the load, so that an unrolled loop
+         // has all its loads in flight.
+         "struct Strip { float v[4]; };\n"
+         "static __device__ __forceinline__ Strip ilang_load(const float* data, size_t at, size_t cap) {\n"
+         "  const bool in = at <= cap - 4;\n  Strip r;\n  __builtin_memcpy(r.v, data + (in ? at : 0), 16);\n"
+         "  for (int e = 0; e < 4; ++e) r.v[e] = in ? r.v[e] : 0.0f;\n  return r;\n}\n"
+         "static __device__ __forceinline__ Strip ilang_load_bf16(const float* data, size_t at, size_t cap) {\n"
+         "  const bool in = at <= cap - 4;\n  Strip r;\n  unsigned u[2];\n"
+         "  __builtin_memcpy(u, (const unsigned short*)data + (in ? at : 0), 8);\n"
+         "  const unsigned w[4] = {u[0] << 16, u[0] & 0xffff0000u, u[1] << 16, u[1] & 0xffff0000u};\n"
+         "  __builtin_memcpy(r.v, w, 16);\n"
+         "  for (int e = 0; e < 4; ++e) r.v[e] = in ? r.v[e] : 0.0f;\n  return r;\n}\n"
+         // to nearest, ties to even; a NaN stays one
+         "static __device__ __forceinline__ unsigned ilang_to_bf16(float v) {\n"
+         "  unsigned u;\n  __builtin_memcpy(&u, &v, 4);\n"
+         "  return v != v ? (u >> 16) | 0x40u : (u + 0x7fffu + (u >> 16 & 1u)) >> 16;\n}\n"
+         "static __device__ __forceinline__ void ilang_store(float* data, size_t at, size_t cap, const Strip& r, size_t bf16) {\n"
+         "  if (at > cap - 4) {\n"
+         "    for (int e = 0; e < 4; ++e)\n      if (at + e < cap) {\n"
+         "        if (bf16) ((unsigned short*)data)[at + e] = (unsigned short)ilang_to_bf16(r.v[e]);\n        else data[at + e] = r.v[e];\n      }\n"
+         "  } else if (bf16) {\n"
+         "    const unsigned u[2] = {ilang_to_bf16(r.v[0]) | ilang_to_bf16(r.v[1]) << 16, ilang_to_bf16(r.v[2]) | ilang_to_bf16(r.v[3]) << 16};\n"
+         "    __builtin_memcpy((unsigned short*)data + at, u, 8);\n"
+         "  } else {\n    __builtin_memcpy(data + at, r.v, 16);\n  }\n}\n\n";
   src << "struct View { float* data; size_t shape[" << rank << "]; size_t layout[" << rank << "]; };\n\n";
   for (size_t k = 0; k < plan.kernels.size(); ++k) {
     if (!emit[k]) continue;
@@ -902,15 +1145,50 @@ GenericModule emit_generic_hip(const ExecPlan& plan, const Module& module, const
     wave_plan(body, initialized, held, phase);
     grid_plan(body, initialized, held, phase);
     any_grid = any_grid || phase.grid.available;
+    const Step* dispatch = nullptr;
+    for (const Step& st : plan.exec)
+      if (st.kind == Step::Dispatch && st.id == k) dispatch = &st;
+    std::set<size_t> private_inds;
+    bool small_privates = true;
+    for (const PrivateBuffer& pb : phase.privates) {
+      private_inds.insert(pb.writeable);
+      small_privates = small_privates && pb.is_static && pb.static_size <= 16;  // (four of each, in registers)
+    }
+    if (!phase.parallel_loops.empty() && small_privates) {
+      const std::string inner = "i" + std::to_string(phase.parallel_loops.back());
+      phase.strip = strip_body(stmts, inner, private_inds);
+      std::set<size_t> loops;
+      loop_ids(body, loops);
+      phase.sequential_loops = loops.size() > phase.parallel_loops.size();
+    }
+    // (a rank-0 input stays f32 in the bf16 forms: the launcher widens it)
+    for (size_t b = 0; dispatch && b < dispatch->reads.size(); ++b) {
+      const BufferRef r = dispatch->reads[b];
+      if (r.kind == BufferRef::Input && !plan.inputs.at(r.id).shape.empty()) phase.bf16_reads.push_back(b);
+    }
+    if (phase.strip) {
+      const std::string inner = "i" + std::to_string(phase.parallel_loops.back());
+      for (size_t b = 0; b < info.n_reads; ++b)
+        if (reads_along(stmts, b, inner)) phase.strip_reads.push_back(b);
+    }
+    // (a buffer that the nest also reads, or accumulates into, keeps its f32 copy)
+    for (size_t w = 0; phase.strip && w < info.n_writes; ++w) {
+      bool direct = w < 8 * sizeof(size_t) && (private_inds.count(w) || !reads_writeable(stmts, w));
+      for (const auto& [loop, inds] : held) direct = direct && std::find(inds.begin(), inds.end(), w) == inds.end();
+      if (direct) phase.strip_direct_writes.push_back(w);
+    }
 
     const size_t nr = std::max<size_t>(info.n_reads, 1), nw = std::max<size_t>(info.n_writes, 1);
     src << "struct Args_" << info.name << " { View readonlys[" << nr << "]; View writeables[" << nw << "]; };\n";
     if (phase.grid.available)
       src << "struct Args_" << info.name << "_g { View readonlys[" << nr << "]; View writeables[" << nw << "]; float* partial[" << nw
           << "]; size_t parts; };\n";
-    const Step* dispatch = nullptr;
-    for (const Step& st : plan.exec)
-      if (st.kind == Step::Dispatch && st.id == k) dispatch = &st;
+    if (phase.strip) {
+      src << "struct Args_" << info.name << "_v { View readonlys[" << nr << "]; View writeables[" << nw << "]; size_t bf16_writes; };\n";
+      if (phase.grid.available)
+        src << "struct Args_" << info.name << "_gv { View readonlys[" << nr << "]; View writeables[" << nw << "]; float* partial[" << nw
+            << "]; size_t parts; size_t bf16_writes; };\n";
+    }
     auto rank_of = [&](BufferRef r) {
       return (r.kind == BufferRef::Input ? plan.inputs.at(r.id) : r.kind == BufferRef::Intermediate ? plan.intermediates.at(r.id)
                                                                                                    : plan.outputs.at(r.id)).layout.size();
@@ -944,7 +1222,7 @@ GenericModule emit_generic_hip(const ExecPlan& plan, const Module& module, const
       }
     };
     // the nest spread over the work-items (wi_first, wi_stride); in_parts: over (work-item, part) pairs
-    auto emit_spread = [&](int depth, bool wave, bool in_parts) {
+    auto emit_spread = [&](int depth, bool wave, bool in_parts, bool strips) {
       const std::string pad(2 * depth, ' ');
       Printer pr;
       pr.held = &held;
@@ -952,10 +1230,12 @@ GenericModule emit_generic_hip(const ExecPlan& plan, const Module& module, const
       if (in_parts) pr.grid = &phase.grid;
       std::vector<std::string> iters;
       for (size_t id : phase.parallel_loops) iters.push_back("i" + std::to_string(id));
+      if (strips) pr.strip = iters.back();
       for (const std::string& it : iters) {
         const MStmt* loop = find_loop(stmts, it);
         if (!loop) lower_error("parallel loop " + it + " not found in kernel body");
-        src << pad << "const size_t n_" << it << " = " << expr_text(*loop->value) << ";\n";
+        if (it == pr.strip) src << pad << "const size_t strip_len = " << expr_text(*loop->value) << ";\n" << pad << "const size_t n_" << it << " = (strip_len + 3) / 4;\n";
+        else src << pad << "const size_t n_" << it << " = " << expr_text(*loop->value) << ";\n";
         pr.parallel.insert(it);
       }
       src << pad << "size_t wi_total = 1;\n";
@@ -986,7 +1266,11 @@ GenericModule emit_generic_hip(const ExecPlan& plan, const Module& module, const
         }
       }
       src << pad << "for (size_t wi = wi_first; wi < " << all << "; wi += wi_stride) {\n";
-      for (const std::string& dg : digits) src << pad << "  const size_t " << dg << " = at_" << dg << ";\n";
+      // (the last strip of a length that is no multiple of 4 overlaps the one before it)
+      for (const std::string& dg : digits) {
+        if (dg == pr.strip) src << pad << "  const size_t " << dg << " = 4 * at_" << dg << " < strip_len - 4 ? 4 * at_" << dg << " : strip_len - 4;\n";
+        else src << pad << "  const size_t " << dg << " = at_" << dg << ";\n";
+      }
       if (in_parts)  // this part's copy of every accumulated buffer stands where the buffer stood
         for (const GridAccumulator& acc : phase.grid.accumulators)
           src << pad << "  writeables[" << acc.writeable << "].data = args.partial[" << acc.writeable << "] + part * part_cap"
@@ -1004,13 +1288,19 @@ GenericModule emit_generic_hip(const ExecPlan& plan, const Module& module, const
       }
       src << pad << "}\n";
     };
-    // forms: the nest as it is; _w: a wavefront per work-item; _g / _gw: either with the outermost sequential loop in parts
-    struct Form { bool wave, in_parts; const char* suffix; };
-    for (const Form form : {Form{false, false, ""}, Form{true, false, "_w"}, Form{false, true, "_g"}, Form{true, true, "_gw"}}) {
+    // forms: the nest as it is; _w: a wavefront per work-item; _g / _gw: either with the outermost sequential loop in
+    // parts; _v / _gv: the work-item forms in strips; each once more, _b, with the inputs' elements in bf16
+    struct Form { bool wave, in_parts, strips; const char* suffix; };
+    for (const bool bf16 : {false, true})
+    for (const Form form : {Form{false, false, false, ""}, Form{true, false, false, "_w"}, Form{false, true, false, "_g"},
+                            Form{true, true, false, "_gw"}, Form{false, false, true, "_v"}, Form{false, true, true, "_gv"}}) {
+      if (bf16 && phase.bf16_reads.empty()) continue;
       if (form.wave && !form.in_parts && phase.wave_loops.empty()) continue;
       if (form.in_parts && (!phase.grid.available || (form.wave && !phase.grid.wave))) continue;
+      if (form.strips && (!phase.strip || (form.in_parts && !phase.grid.held_accumulators))) continue;
+      if (bf16) g_bf16_reads.insert(phase.bf16_reads.begin(), phase.bf16_reads.end());
       src << "extern \"C\" __global__ void __launch_bounds__(" << (form.wave ? GenericPhase::kWaveThreads : 64u) << ") " << phase.name
-          << form.suffix << "(Args_" << info.name << (form.in_parts ? "_g" : "") << " args) {\n";
+          << form.suffix << (bf16 ? "_b" : "") << "(Args_" << info.name << (form.strips ? form.suffix : form.in_parts ? "_g" : "") << " args) {\n";
       src << "  const View* readonlys = args.readonlys;\n";
       src << "  View writeables[" << nw << "];\n";
       src << "  for (int b = 0; b < " << nw << "; ++b) writeables[b] = args.writeables[b];\n";
@@ -1023,7 +1313,12 @@ GenericModule emit_generic_hip(const ExecPlan& plan, const Module& module, const
         src << "  const size_t wi_stride = (size_t)gridDim.x * blockDim.x;\n";
       }
       emit_capacities("  ");
-      emit_privates("  ");
+      if (form.strips) {
+        for (const PrivateBuffer& pb : phase.privates) src << "  Strip strip" << pb.writeable << "[" << pb.static_size << "];\n";
+        g_strip_privates = private_inds;
+      } else {
+        emit_privates("  ");
+      }
       if (phase.parallel_loops.empty() && !form.in_parts) {
         src << "  if (wi_first != 0) return;\n";
         Printer pr;
@@ -1032,9 +1327,11 @@ GenericModule emit_generic_hip(const ExecPlan& plan, const Module& module, const
         pr.block(stmts, 1);
         src << pr.os.str();
       } else {
-        emit_spread(1, form.wave, form.in_parts);
+        emit_spread(1, form.wave, form.in_parts, form.strips);
       }
       src << "}\n\n";
+      g_bf16_reads.clear();
+      g_strip_privates.clear();
     }
     info.phases.push_back(std::move(phase));
   }

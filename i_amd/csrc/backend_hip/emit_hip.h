@@ -43,6 +43,15 @@ struct PrivateBuffer {
 // part accumulates into a copy of its own of each accumulated buffer (a temporary that the launcher fills with
 // the reduction's identity first), and a second kernel, ilang_combine, folds the copies into the buffer in part
 // order.  (GridForm below.)
+//
+// A nest whose innermost parallel loop steps through every buffer it indexes by one element has strip forms,
+// <name>_v and <name>_gv: a work-item runs four consecutive iterations of that loop, so that what was four 4-byte
+// accesses is one of 16 bytes (8 in bf16).  (Where the loop's length is no multiple of four, the last strip overlaps the
+// one before it; that is left to nests that do not read what they write.)  The element-wise forms are bound by HBM and the plain ones by the number
+// of accesses in flight: 16384 x 4096 f32 divided by its column sums 213 -> 172 us (the division alone 145 -> 89, 6
+// TB/s), a bias and a threshold 193 -> 102.  And every form that reads program inputs exists once more, <name>..._b, with
+// those inputs' elements in bf16, which would otherwise be widened into temporaries first (16384 x 4096
+// bf16, results in bf16: 450 -> 100 and 447 -> 56 us; row sums 182 -> 32, where a lane takes four elements at a time).
 struct WaveLoop {
   size_t loop = 0;    // a loop of the parallel body: its accumulators are lane shares, combined after it
   size_t spread = 0;  // the loop whose iterations are dealt out over the lanes: `loop`, or one nested perfectly in it
@@ -75,6 +84,11 @@ struct GenericPhase {
   bool wave_contiguous = false;           // consecutive iterations of those loops read consecutive elements
   static constexpr unsigned kWaveThreads = 256;  // work-items per workgroup of that form (4 wavefronts)
   GridForm grid;
+  bool strip = false;                     // <name>_v (and <name>_gv, with grid.held_accumulators) exist
+  bool sequential_loops = false;          // there are loops besides the parallel ones
+  std::vector<size_t> strip_reads;        // readonlys that the strip form reads four elements at a time (and every writeable)
+  std::vector<size_t> strip_direct_writes;  // writeables that the strip form may store in bf16: stored only, never read
+  std::vector<size_t> bf16_reads;         // readonlys that are program inputs of rank 1 and more: bf16 in the forms <name>..._b
 };
 
 struct GenericKernel {

@@ -690,14 +690,17 @@ ihip::Err generic_function(Program& p, const std::string& name, hipFunction_t* f
 // a loop that a work-item runs by itself, 4 rounds of the 64 lanes when the loop in parts is the one over the lanes,
 // one iteration when the lanes run over a loop inside it; at most 4096, from 16 on a multiple of 8 and from 256 on
 // of 32 (the copies of buffers of 64 elements and more are then folded in two passes).
-size_t generated_parts(const ihip::KernelOptions& knobs, const GridForm& grid, bool wave, size_t total, size_t reduced) {
+// `strips`: a work-item takes four iterations of the innermost parallel loop and `total` counts those.
+size_t generated_parts(const ihip::KernelOptions& knobs, const GridForm& grid, bool wave, size_t total, size_t reduced, bool strips) {
   if (!grid.available || (wave && !grid.wave) || knobs.generated_parts == 1 || total == 0) return 1;
   const size_t least = !wave ? 16 : grid.loop_is_spread ? 256 : 1;
   size_t parts;
   if (knobs.generated_parts > 1) {
     parts = (size_t)knobs.generated_parts;
   } else {
-    const size_t target = wave ? 4096 : 262144;  // wavefronts / work-items that fill the chip
+    // (strips have four times the bytes in flight: column sums of 5042 x 2561 24 us with 131072 work-items, 22 with
+    // 82048; of 16384 x 4096 58 with 131072, 55 with 65536)
+    const size_t target = wave ? 4096 : strips ? 98304 : 262144;  // wavefronts / work-items that fill the chip
     if (total * 2 > target) return 1;
     parts = std::min<size_t>(target / total, reduced / least);
   }
@@ -707,6 +710,54 @@ size_t generated_parts(const ihip::KernelOptions& knobs, const GridForm& grid, b
   if (parts >= 256) parts = parts / 32 * 32;
   else if (parts >= 16) parts = parts / 8 * 8;
   return parts < 2 ? 1 : parts;
+}
+
+// Is this output written by one nest only, and read by none?  (Counting the generated forms of every kernel.)
+bool written_once(const Run& run, BufferRef out) {
+  size_t writers = 0;
+  for (const Step& s : run.p.nest_plan.exec) {
+    if (s.kind != Step::Dispatch) continue;
+    for (BufferRef r : s.reads)
+      if (r.kind == out.kind && r.id == out.id) return false;
+    for (BufferRef w : s.writes) writers += w.kind == out.kind && w.id == out.id;
+  }
+  return out.kind == BufferRef::Output && writers == 1;
+}
+
+// May the nest run in strips of four iterations of its innermost loop, and should it?  Every buffer accessed that way
+// needs four elements.  A length that is no multiple of four makes strips overlap: fine as long as the nest computes
+// the same again, i.e. reads nothing that it writes, neither by name nor because the caller passes one memory as input
+// and output.  Nests without sequential loops and those with their loop in parts are bound by memory and always
+// gain; a nest that loops in its work-items needs enough of them left.
+bool strips_usable(const Run& run, const GenericPhase& ph, const Step& dispatch, size_t total, size_t inner) {
+  if (!ph.strip || inner < 4) return false;
+  for (size_t r : ph.strip_reads)
+    if (product(run.layout_of(dispatch.reads[r])) < 4) return false;
+  auto is_private = [&](size_t w) {
+    for (const PrivateBuffer& pb : ph.privates)
+      if (pb.writeable == w) return true;
+    return false;
+  };
+  for (size_t w = 0; w < dispatch.writes.size(); ++w)
+    if (!is_private(w) && product(run.layout_of(dispatch.writes[w])) < 4) return false;
+  const bool in_parts = ph.grid.available && ph.grid.held_accumulators && run.knobs.generated_parts != 1;
+  if (ph.sequential_loops && !in_parts && total < size_t(4) * 65536) return false;
+  if (inner % 4 == 0) return true;
+  bool fresh = in_parts && ph.privates.empty();  // (sums that the nest starts itself: the same again, too)
+  for (const GridAccumulator& acc : ph.grid.accumulators) fresh = fresh && acc.init_here;
+  if (!(fresh && ph.grid.accumulators.size() == dispatch.writes.size()) &&
+      (ph.sequential_loops || ph.strip_direct_writes.size() != dispatch.writes.size()))
+    return false;
+  for (BufferRef w : dispatch.writes)
+    for (BufferRef r : dispatch.reads) {
+      if (w.kind != BufferRef::Output || r.kind != BufferRef::Input) continue;
+      const char* out = static_cast<const char*>(run.raw_ptr(w));
+      const char* in = static_cast<const char*>(run.raw_ptr(r));
+      const size_t out_bytes = product(run.layout_of(w)) * (run.dtype_of(w) == DType::BF16 ? 2 : 4);
+      const size_t in_bytes = product(run.layout_of(r)) * (run.dtype_of(r) == DType::BF16 ? 2 : 4);
+      if (in < out + out_bytes && out < in + in_bytes) return false;
+    }
+  return true;
 }
 
 ihip::Err launch_generic(Run& run, size_t k, const Step& dispatch) {
@@ -727,17 +778,16 @@ ihip::Err launch_generic(Run& run, size_t k, const Step& dispatch) {
     for (size_t d = 0; d < shape.size() && d < R; ++d) std::memcpy(v + 8 + 8 * d, &shape[d], 8);
     for (size_t d = 0; d < layout.size() && d < R; ++d) std::memcpy(v + 8 + 8 * R + 8 * d, &layout[d], 8);
   };
+  // inputs that are all bf16 (rank 0 aside) are read as they are, by the _b forms
+  bool bf16_inputs = !ph.bf16_reads.empty();
+  for (size_t i : ph.bf16_reads) bf16_inputs = bf16_inputs && run.dtype_of(dispatch.reads[i]) == DType::BF16;
   for (size_t i = 0; i < dispatch.reads.size(); ++i) {
     void* ptr = nullptr;
-    if (ihip::Err e = run.read_f32(dispatch.reads[i], &ptr); !e.empty()) return e;
+    if (bf16_inputs && std::find(ph.bf16_reads.begin(), ph.bf16_reads.end(), i) != ph.bf16_reads.end()) ptr = run.raw_ptr(dispatch.reads[i]);
+    else if (ihip::Err e = run.read_f32(dispatch.reads[i], &ptr); !e.empty()) return e;
     fill(i, ptr, dispatch.reads[i]);
   }
-  std::vector<void*> write_ptrs(dispatch.writes.size(), nullptr);
-  for (size_t i = 0; i < dispatch.writes.size(); ++i) {
-    if (!gk.is_private(i))
-      if (ihip::Err e = run.write_f32(dispatch.writes[i], &write_ptrs[i]); !e.empty()) return e;
-    fill(nr + i, write_ptrs[i], dispatch.writes[i]);
-  }
+  const std::string twin = bf16_inputs ? "_b" : "";
   auto extent_of = [&](const Extent<Param>& e) {
     const BufferRef src = e.source.buffer.writeable ? dispatch.writes.at(e.source.buffer.ind) : dispatch.reads.at(e.source.buffer.ind);
     return run.extent(Extent<size_t>{plan_buffer(run.plan, src).shape.at(e.source.dim), e.kind});
@@ -745,7 +795,7 @@ ihip::Err launch_generic(Run& run, size_t k, const Step& dispatch) {
   run.notes.push_back("generated kernel " + gk.name);
   size_t total = 1;
   for (const auto& e : ph.parallel_extents) total *= extent_of(e);
-  if (total == 0) return {};
+  const size_t inner = ph.parallel_extents.empty() ? 0 : extent_of(ph.parallel_extents.back());
   // The wavefront-per-iteration form (reduction loops spread over 64 lanes), when the nest has one: taken when
   // the reduction is long enough to occupy the lanes and either consecutive lanes read consecutive elements
   // or there are too few iterations to fill the chip with one work-item each.  Option generated.wave = 0 | 1 overrides.
@@ -756,9 +806,26 @@ ihip::Err launch_generic(Run& run, size_t k, const Step& dispatch) {
     wave = reduced >= 128 && (ph.wave_contiguous || (total < 65536 && !ph.grid.available));
     if (run.knobs.generated_wave >= 0) wave = run.knobs.generated_wave == 1;
   }
+  const bool strips = !wave && strips_usable(run, ph, dispatch, total, inner);
+  // the outputs that a strip form stores in bf16 itself; any other bf16 output goes through an f32 temporary
+  size_t bf16_writes = 0;
+  std::vector<void*> write_ptrs(dispatch.writes.size(), nullptr);
+  for (size_t i = 0; i < dispatch.writes.size(); ++i) {
+    const BufferRef w = dispatch.writes[i];
+    if (strips && run.dtype_of(w) == DType::BF16 && written_once(run, w) &&
+        std::find(ph.strip_direct_writes.begin(), ph.strip_direct_writes.end(), i) != ph.strip_direct_writes.end()) {
+      write_ptrs[i] = run.raw_ptr(w);
+      bf16_writes |= size_t(1) << i;
+    } else if (!gk.is_private(i)) {
+      if (ihip::Err e = run.write_f32(w, &write_ptrs[i]); !e.empty()) return e;
+    }
+    fill(nr + i, write_ptrs[i], w);
+  }
+  if (total == 0) return {};
+  const size_t items = strips ? total / inner * ((inner + 3) / 4) : total;  // work-items
   bool dynamic_private = false;  // (per-work-item slices of a device buffer are sized for the plain form's grid)
   for (const PrivateBuffer& pb : ph.privates) dynamic_private = dynamic_private || !pb.is_static;
-  const size_t parts = dynamic_private ? 1 : generated_parts(run.knobs, ph.grid, wave, total, ph.grid.available ? extent_of(ph.grid.extent) : 0);
+  const size_t parts = dynamic_private ? 1 : generated_parts(run.knobs, ph.grid, wave, items, ph.grid.available ? extent_of(ph.grid.extent) : 0, strips);
   hipFunction_t fn;
   if (parts > 1) {
     // every part accumulates into a copy of its own of each accumulated buffer (filled with the reduction's
@@ -780,9 +847,10 @@ ihip::Err launch_generic(Run& run, size_t k, const Step& dispatch) {
     const bool two_passes = width != 0 && most != 0;
     if (two_passes) floats += width * most;
     void* partial = nullptr;
+    const bool in_strips = strips && ph.grid.held_accumulators;
     if (run.alloc_optional(&partial, floats * 4)) {
       std::vector<unsigned char> gargs(args);
-      gargs.resize(args.size() + 8 * nw + 8, 0);
+      gargs.resize(args.size() + 8 * nw + 8 + (in_strips ? 8 : 0), 0);  // (the strip form's bf16_writes: none, the copies are f32)
       float* at = static_cast<float*>(partial);
       struct FillArgs { float* data; size_t count; float value; };
       struct CombineArgs { const float* partial; float* data; size_t parts; size_t count; int op; int keep; };
@@ -817,11 +885,11 @@ ihip::Err launch_generic(Run& run, size_t k, const Step& dispatch) {
         at += counts[a] * parts;
       }
       std::memcpy(gargs.data() + args.size() + 8 * nw, &parts, 8);
-      const std::string name = ph.name + (wave ? "_gw" : "_g");
+      const std::string name = ph.name + (wave ? "_gw" : in_strips ? "_gv" : "_g") + twin;
       if (ihip::Err e = generic_function(p, name, &fn); !e.empty()) return e;
       run.notes.back() += ", as " + name + ": the outermost sequential loop in " + std::to_string(parts) + " parts over " +
                           (wave ? "wavefronts" : "work-items") + ", combined by " + kCombineKernel;
-      const size_t units = total * parts;
+      const size_t units = (in_strips ? items : total) * parts;
       const unsigned per_group = wave ? GenericPhase::kWaveThreads / 64 : 64;
       const size_t groups = std::min<size_t>((units + per_group - 1) / per_group, size_t(1) << 20);
       if (ihip::Err e = ihip::launch(fn, (unsigned)groups, 1, 1, wave ? GenericPhase::kWaveThreads : 64, gargs.data(), gargs.size(), run.stream);
@@ -840,12 +908,12 @@ ihip::Err launch_generic(Run& run, size_t k, const Step& dispatch) {
     const size_t waves = std::min<size_t>(total, size_t(1) << 16);
     const unsigned per_group = GenericPhase::kWaveThreads / 64;
     for (const PrivateBuffer& pb : ph.privates) fill(nr + pb.writeable, nullptr, dispatch.writes[pb.writeable]);
-    if (ihip::Err err = generic_function(p, ph.name + "_w", &fn); !err.empty()) return err;
-    run.notes.back() += ", as " + ph.name + "_w: one wavefront per iteration of the parallel loops";
+    if (ihip::Err err = generic_function(p, ph.name + "_w" + twin, &fn); !err.empty()) return err;
+    run.notes.back() += ", as " + ph.name + "_w" + twin + ": one wavefront per iteration of the parallel loops";
     return ihip::launch(fn, (unsigned)((waves + per_group - 1) / per_group), 1, 1, GenericPhase::kWaveThreads, args.data(), args.size(),
                         run.stream);
   }
-  size_t threads = ph.parallel_loops.empty() ? 1 : total;
+  size_t threads = ph.parallel_loops.empty() ? 1 : items;
   // dynamic private buffers cost memory per work-item slot: cap the slots
   size_t slot_elems = 0;
   for (const PrivateBuffer& pb : ph.privates)
@@ -863,7 +931,13 @@ ihip::Err launch_generic(Run& run, size_t k, const Step& dispatch) {
     }
     fill(nr + pb.writeable, ptr, dispatch.writes[pb.writeable]);
   }
-  if (ihip::Err e = generic_function(p, ph.name, &fn); !e.empty()) return e;
+  const std::string name = ph.name + (strips ? "_v" : "") + twin;
+  if (ihip::Err e = generic_function(p, name, &fn); !e.empty()) return e;
+  if (strips) {
+    args.resize(args.size() + 8, 0);
+    std::memcpy(args.data() + args.size() - 8, &bf16_writes, 8);
+  }
+  if (name != ph.name) run.notes.back() += ", as " + name + (strips ? ": strips of four" : "");
   return ihip::launch(fn, grid, 1, 1, 64, args.data(), args.size(), run.stream);
 }
 
