@@ -343,13 +343,14 @@ bool read_back(const Run& run, BufferRef out) {
 
 // An f32 product through the executor: with few output tiles under a long k loop, the loop in parts over
 // workgroups, the partial products in a temporary (no room for it: the unsplit kernel).
+// b_cols != 0: the right operand is row-major with rows of b_cols elements.
 ihip::Err launch_product_f32(Run& run, const void* a, const void* b, void* c, size_t bh, size_t m, size_t n, size_t k,
-                             ihip::LaunchNote* note) {
+                             ihip::LaunchNote* note, size_t b_cols = 0) {
   void* partial = nullptr;
   unsigned splits = ihip::gemm_nt_f32_split_k(bh, m, n, k, run.knobs);
   if (splits > 1 && ((m * n) % 4 != 0 || !run.alloc_optional(&partial, bh * splits * m * n * 4))) splits = 1;
   return ihip::launch_gemm_nt_f32(static_cast<const float*>(a), static_cast<const float*>(b), static_cast<float*>(c), bh, m, n, k,
-                                  run.stream, note, static_cast<float*>(partial), splits, run.knobs);
+                                  run.stream, note, static_cast<float*>(partial), splits, run.knobs, b_cols);
 }
 
 // A product with few rows of A on the kernels for those (gemm_narrow_usable has said so).
@@ -428,6 +429,8 @@ ihip::Err attention_in_parts(Run& run, const Recognized& r, bool bf16, size_t bh
           !e.empty())
         return e;
     }
+  } else if (dv % 4 == 0 && dv <= (size_t(1) << 24)) {
+    if (ihip::Err e = launch_product_f32(run, s, v, out, bh, nq, dv, nk, &last, dv); !e.empty()) return e;
   } else {
     void* vt = nullptr;
     if (ihip::Err e = run.alloc(&vt, bh * dv * nk * 4); !e.empty()) return e;
@@ -438,23 +441,43 @@ ihip::Err attention_in_parts(Run& run, const Recognized& r, bool bf16, size_t bh
   return {};
 }
 
-// The two operands of an NT product ([rows_a, k] and [rows_b, k], dense) as the matrix-instruction kernels can
-// read them: untouched when k is a multiple of their quantum and both are 16-byte aligned, otherwise
-// copied into stream-ordered temporaries with every row padded with zeros up to the next multiple; *k becomes the
-// padded extent.
-ihip::Err padded_operands(Run& run, DType t, const void** a, size_t rows_a, const void** b, size_t rows_b, size_t* k) {
-  const size_t q = product_k_quantum(t), kp = (*k + q - 1) / q * q, elem = t == DType::BF16 ? 2 : 4;
+// The two operands of a product as the matrix-instruction kernels can read them: untouched when the extents are
+// multiples of their quantum and both are 16-byte aligned, otherwise copied, in one launch, into temporaries padded with
+// zeros.  a is [bh, m, k]; b is [bh, n, k], or [bh, k, n] (nn).  *k becomes the padded extent, *b_cols (nn) that of n.
+ihip::Err padded_operands(Run& run, DType t, bool nn, size_t bh, const void** a, size_t m, const void** b, size_t n, size_t* k, size_t* b_cols) {
+  const size_t q = product_k_quantum(t), kp = (*k + q - 1) / q * q, np = (n + q - 1) / q * q, elem = t == DType::BF16 ? 2 : 4;
   const bool misaligned = reinterpret_cast<uintptr_t>(*a) % 16 != 0 || reinterpret_cast<uintptr_t>(*b) % 16 != 0;
-  if (kp == *k && !misaligned) return {};
+  if (b_cols) *b_cols = nn ? n : 0;
+  if (kp == *k && !misaligned && (!nn || np == n)) return {};
   void *ta = nullptr, *tb = nullptr;
-  if (ihip::Err e = run.alloc(&ta, std::max<size_t>(rows_a * kp * elem, 16)); !e.empty()) return e;
-  if (ihip::Err e = run.alloc(&tb, std::max<size_t>(rows_b * kp * elem, 16)); !e.empty()) return e;
-  if (ihip::Err e = ihip::launch_pad_rows(*a, ta, rows_a, *k, kp, elem, run.stream); !e.empty()) return e;
-  if (ihip::Err e = ihip::launch_pad_rows(*b, tb, rows_b, *k, kp, elem, run.stream); !e.empty()) return e;
+  const size_t bytes_a = bh * m * kp * elem, bytes_b = bh * (nn ? kp * np : n * kp) * elem;
+  if (ihip::Err e = run.alloc(&ta, std::max<size_t>(bytes_a, 16)); !e.empty()) return e;
+  if (ihip::Err e = run.alloc(&tb, std::max<size_t>(bytes_b, 16)); !e.empty()) return e;
+  if (bytes_a != 0 && bytes_b != 0) {
+    if (std::max(bytes_a, bytes_b) / 16 < (size_t(1) << 31)) {
+      const ihip::PadPair pair{{*a, *b}, {ta, tb}, {m, nn ? *k : n}, {m, nn ? kp : n}, {*k, nn ? n : *k}, {kp, nn ? np : kp}};
+      if (ihip::Err e = ihip::launch_pad_pair(pair, bh, elem, run.stream); !e.empty()) return e;
+    } else if (!nn) {
+      if (ihip::Err e = ihip::launch_pad_rows(*a, ta, bh * m, *k, kp, elem, run.stream); !e.empty()) return e;
+      if (ihip::Err e = ihip::launch_pad_rows(*b, tb, bh * n, *k, kp, elem, run.stream); !e.empty()) return e;
+    } else {
+      return "operands too large to be padded";  // (padded_nn_usable has kept such a call away)
+    }
+  }
   *a = ta;
   *b = tb;
   *k = kp;
+  if (b_cols) *b_cols = nn ? np : 0;
   return {};
+}
+
+// May a product with a row-major right operand run on the kernels that read it as it is, after padding if need be?
+bool padded_nn_usable(const Run& run, DType t, size_t bh, size_t m, size_t n, size_t k) {
+  const size_t q = product_k_quantum(t), kp = (k + q - 1) / q * q, np = (n + q - 1) / q * q;
+  if (bh == 0 || m == 0 || n == 0 || k == 0 || bh > 65535 || np > (size_t(1) << 24)) return false;
+  if (bh * std::max(m, np) * kp >= (size_t(1) << 33)) return false;
+  if (t == DType::F32) return ihip::gemm_nt_f32_supported(kp);
+  return ihip::gemm_nn_bf16_supported(bh, m, np, kp, run.knobs);
 }
 
 // The operands of a product in its arithmetic type: as they are, or widened to f32 where the other one is f32.
@@ -555,7 +578,7 @@ ihip::Err launch_hand_noted(Run& run, const Recognized& r, ihip::LaunchNote* not
       const void *pa = nullptr, *pb = nullptr;
       if (ihip::Err e = product_operands(run, r, t, &pa, &pb); !e.empty()) return e;
       size_t k = a[nb + 1];
-      if (ihip::Err e = padded_operands(run, t, &pa, bh * a[nb], &pb, bh * b[nb], &k); !e.empty()) return e;
+      if (ihip::Err e = padded_operands(run, t, false, bh, &pa, a[nb], &pb, b[nb], &k, nullptr); !e.empty()) return e;
       // (the schedule names one of the tiled kernels' own tiles: then that kernel runs as asked)
       const bool tile_asked = (r.tile_i == 128 && r.tile_j == 128) || (r.tile_i == 256 && r.tile_j == 256);
       const ihip::DType kernel_t = t == DType::F32 ? ihip::F32 : ihip::BF16;
@@ -600,20 +623,25 @@ ihip::Err launch_hand_noted(Run& run, const Recognized& r, ihip::LaunchNote* not
       const ihip::DType kernel_t = f32 ? ihip::F32 : ihip::BF16;
       if (aligned && !tile_asked && ihip::gemm_narrow_usable(kernel_t, true, bh, m, n, k, run.knobs))
         return launch_product_narrow(run, pa, pb_rows, out, kernel_t, true, bh, m, n, k, note, out_dt);
-      if (!f32 && aligned && ihip::gemm_nn_bf16_supported(bh, m, n, k, run.knobs)) {  // the direct kernels read a row-major right operand themselves
-        unsigned splits = tile_asked && run.knobs.gemm_k_parts < 2 ? 1u : ihip::gemm_nt_bf16_split_k(bh, m, n, k, run.knobs);
+      const DType t = f32 ? DType::F32 : DType::BF16;
+      size_t kp = k;
+      if (padded_nn_usable(run, t, bh, m, n, k)) {  // the direct kernels read a row-major right operand themselves
+        const void* pb = pb_rows;
+        size_t b_cols = n;
+        if (ihip::Err e = padded_operands(run, t, true, bh, &pa, m, &pb, n, &kp, &b_cols); !e.empty()) return e;
+        if (f32) return launch_product_f32(run, pa, pb, out, bh, m, n, kp, note, b_cols);
+        unsigned splits = tile_asked && run.knobs.gemm_k_parts < 2 ? 1u : ihip::gemm_nt_bf16_split_k(bh, m, n, kp, run.knobs);
         void* partial = nullptr;
         if (splits > 1 && ((m * n) % 4 != 0 || !run.alloc_optional(&partial, bh * splits * m * n * 4))) splits = 1;
-        return ihip::launch_gemm_nn_bf16(pa, pb_rows, out, bh, m, n, k, run.stream, r.tile_i, r.tile_j, note, out_dt,
-                                         static_cast<float*>(partial), splits, run.knobs);
+        return ihip::launch_gemm_nn_bf16(pa, pb, out, bh, m, n, kp, run.stream, r.tile_i, r.tile_j, note, out_dt,
+                                         static_cast<float*>(partial), splits, run.knobs, b_cols);
       }
       const size_t elem = f32 ? 4 : 2;
       void* bt = nullptr;
       if (ihip::Err e = run.alloc(&bt, bh * n * k * elem); !e.empty()) return e;
       if (ihip::Err e = ihip::launch_transpose(pb_rows, bt, bh, k, n, elem, run.stream); !e.empty()) return e;
       const void* pb = bt;
-      size_t kp = k;
-      if (ihip::Err e = padded_operands(run, f32 ? DType::F32 : DType::BF16, &pa, bh * m, &pb, bh * n, &kp); !e.empty()) return e;
+      if (ihip::Err e = padded_operands(run, t, false, bh, &pa, m, &pb, n, &kp, nullptr); !e.empty()) return e;
       if (f32) return launch_product_f32(run, pa, pb, out, bh, m, n, kp, note);
       return ihip::launch_gemm_nt_bf16(pa, pb, out, bh, m, n, kp, run.stream, r.tile_i, r.tile_j, note, out_dt, run.knobs);
     }

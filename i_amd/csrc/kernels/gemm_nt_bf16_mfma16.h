@@ -41,8 +41,8 @@
 // such reads (k0 = 32 ks + 8 (lane / 16) and + 4) complete the lane's 8 k.  Two 16-lane blocks read 8 rows x
 // 32 bytes at a time (rows 0-3 and 8-11 of a k-step, then 4-7 and 12-15, ...), so the 32-byte unit index of a
 // row is XOR-ed, on the global side, with f(row) = row % 4 + 4 ((row / 8) % 2), which sends those 8 rows to 8
-// different bank groups.  Requires n % 8 == 0 as well; 16-byte chunks that start past n re-read the row's last
-// chunk (their columns are not stored).
+// different bank groups.  Requires rows of B of a multiple of 8 elements (b_cols) as well; 16-byte chunks that start
+// past a row re-read its last chunk (their columns are not stored).
 //
 // KTAIL = true is the same kernel for k that is a multiple of 8 but not of 64: the last slab is partial.  The lanes
 // whose 16-byte chunk (NN: whose slab row of B) lies past k transfer nothing and clear their LDS slot instead, so
@@ -84,9 +84,10 @@ __device__ __forceinline__ void gemm_nt_mfma16_tile(const GemmParams& p, char* s
   const uint32_t c16 = lane & 15, g = lane >> 4;
 
   const size_t row_bytes = (size_t)p.k * 2;
+  const size_t brow_bytes = (size_t)p.b_cols * 2;  // NN: a row of B
   const char* __restrict__ A = reinterpret_cast<const char*>(p.a) + (size_t)batch * p.m * row_bytes + (size_t)k_first * 2;
-  const char* __restrict__ B = reinterpret_cast<const char*>(p.b) + (size_t)batch * p.n * row_bytes +
-                               (NN ? (size_t)k_first * p.n * 2 : (size_t)k_first * 2);  // (NN: rows of B are k)
+  const char* __restrict__ B = reinterpret_cast<const char*>(p.b) +  // (NN: rows of B are k)
+                               (NN ? ((size_t)batch * p.k + k_first) * brow_bytes : (size_t)batch * p.n * row_bytes + (size_t)k_first * 2);
   char* __restrict__ C = reinterpret_cast<char*>(p.c) + (size_t)blockIdx.y * p.m * p.n * (p.out_bf16 ? 2 : 4);
   const uint32_t m0 = tm * BTM, n0 = tn * BTN;
 
@@ -124,10 +125,9 @@ __device__ __forceinline__ void gemm_nt_mfma16_tile(const GemmParams& p, char* s
   // round to the next: two offsets, by the parity of the round)
   constexpr int NN_ROUND = NWAVES * RPWN;  // slab rows per round of the workgroup's wave-loads
   static_assert(!NN || NN_ROUND == 16 || NN_ROUND == 8, "NN slab rounds");
-  const size_t brow_bytes = (size_t)p.n * 2;  // NN: a row of B is n elements
   uint32_t boff_nn[2] = {0, 0};
   if constexpr (NN) {
-    const uint32_t last_chunk = (p.n - n0) / 8 - 1;  // n % 8 == 0 and n0 < n
+    const uint32_t last_chunk = (p.b_cols - n0) / 8 - 1;  // b_cols % 8 == 0 and n0 < n
 #pragma unroll
     for (int parity = 0; parity < 2; ++parity) {
       const uint32_t r = wave * RPWN + lane / CHN + (NN_ROUND == 8 ? 8 * parity : 0);
@@ -314,9 +314,12 @@ __device__ __forceinline__ void gemm_nt_mfma16_tile(const GemmParams& p, char* s
   }
 
   // ---- store.  acc[i][j][r] is C[m0 + 16 (wm TM + i) + c16][n0 + 16 (wn TN + j) + 4 g + r]: a lane writes four
-  // consecutive columns at once, a quarter-wave 16 rows of them.  Columns come in fours, so a C whose n is not
-  // a multiple of 4 (or whose base is not 16-byte aligned) is stored element by element.
+  // consecutive columns at once, a quarter-wave 16 rows of them.  A C whose n is not a multiple of 4 (or whose base
+  // is not 16-byte aligned) takes the same wide stores on the alignment of its elements, and only the columns of a
+  // last, partial four go one by one (2047 x 3001 x 777, f32 result: 31 -> 22 us).
   const bool n4 = p.n % 4 == 0 && reinterpret_cast<uintptr_t>(C) % 16 == 0;
+  typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+  typedef __bf16 bf16x4_any __attribute__((ext_vector_type(4), aligned(2)));
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
     const uint32_t row = m0 + (wm * TM + i) * 16 + c16;
@@ -333,10 +336,19 @@ __device__ __forceinline__ void gemm_nt_mfma16_tile(const GemmParams& p, char* s
         } else {
           *reinterpret_cast<f32x4*>(C + 4 * at) = acc[i][j];
         }
-      } else if (!EDGE || row < p.m) {
+      } else if (!EDGE || (row < p.m && col + 4 <= p.n)) {
+        if (p.out_bf16) {
+          bf16x4_any v;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) v[r] = (bf16_t)acc[i][j][r];
+          *reinterpret_cast<bf16x4_any*>(C + 2 * at) = v;
+        } else {
+          *reinterpret_cast<f32x4_any*>(C + 4 * at) = acc[i][j];
+        }
+      } else if (row < p.m) {
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-          if (!EDGE || col + r < p.n) {
+          if (col + r < p.n) {
             if (p.out_bf16) reinterpret_cast<bf16_t*>(C + 2 * at)[r] = (bf16_t)acc[i][j][r];
             else reinterpret_cast<float*>(C + 4 * at)[r] = acc[i][j][r];
           }

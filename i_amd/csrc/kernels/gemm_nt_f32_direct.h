@@ -21,18 +21,24 @@
 //               16-byte operand read covers k = 4 (2 ks + h) .. + 3, and element e of it feeds MFMA e of the k-step.
 //   L2          the workgroup ids that land on one XCD (id % 8) walk blocks of 4 x 8
 //               tiles, so at any time an XCD streams 1024 rows of A and 2048 rows of B
+//   NN          (row-major right operand, C[m,n] = sum_k A[m,k] * B[k,n]) the B slab is [32 k][BT n]: a lane's operand
+//               for element e of a k-step is the one value of row 4 (2 ks + h) + e, column c, four ds_read_b32 for
+//               the ds_read_b128 of the NT form, which the 64 cycles of a matrix instruction hide.  The half-waves
+//               read rows four apart, the same banks, so the 128-byte unit of a row is XOR-ed with (row / 4) % 2.
 //   M, N edges  rows past the end re-read the last valid row and are not stored
-// Requires k % 32 == 0, or k % 4 == 0 with KTAIL.
+// Requires k % 32 == 0, or k % 4 == 0 with KTAIL; NN: rows of B of a multiple of 4 elements (b_cols).
 #pragma once
 
 #include "common.h"
 #include "params.h"
 
 // BT x BT output tile per workgroup of WM x WN waves: 256 with 2 x 4 waves (one workgroup per CU) for large
-// problems, 128 with 2 x 2 waves (two workgroups per CU) for problems with too few 256-tiles to fill the chip.
+// problems, 128 with 2 x 2 waves (two workgroups per CU) for problems with too few 256-tiles to fill the chip, 64 with
+// 2 x 2 waves of one accumulator where 128-tiles leave CUs idle: the f32 matrix rate is so low that operand traffic does
+// not bound the small tile either (see the launcher's model).
 // KTAIL: k is a multiple of 4 but not of 32, the last slab is partial: a lane whose 16-byte chunk lies past k
 // transfers nothing and clears its LDS slot instead, so the slab reads as zeros there.
-template <int BT, int WM, int WN, bool KTAIL = false>
+template <int BT, int WM, int WN, bool KTAIL = false, bool NN = false>
 __device__ __forceinline__ void gemm_nt_f32_direct_body(const GemmParams& p) {
   constexpr int BMT = BT, BNT = BT;
   constexpr int ELEM = 4;            // bytes per operand element
@@ -68,7 +74,9 @@ __device__ __forceinline__ void gemm_nt_f32_direct_body(const GemmParams& p) {
 
   const size_t row_bytes = (size_t)p.k * ELEM;
   const char* __restrict__ A = reinterpret_cast<const char*>(p.a) + (size_t)batch * p.m * row_bytes + (size_t)k_first * ELEM;
-  const char* __restrict__ B = reinterpret_cast<const char*>(p.b) + (size_t)batch * p.n * row_bytes + (size_t)k_first * ELEM;
+  const size_t brow_bytes = (size_t)p.b_cols * ELEM;  // NN: a row of B
+  const char* __restrict__ B = reinterpret_cast<const char*>(p.b) +
+                               (NN ? ((size_t)batch * p.k + k_first) * brow_bytes : (size_t)batch * p.n * row_bytes + (size_t)k_first * ELEM);
   float* __restrict__ C = reinterpret_cast<float*>(p.c) + (size_t)blockIdx.y * p.m * p.n;
   const uint32_t m0 = tm * BMT, n0 = tn * BNT;
 
@@ -78,6 +86,9 @@ __device__ __forceinline__ void gemm_nt_f32_direct_body(const GemmParams& p) {
   const uint32_t lrow = lane / CH, lch = lane % CH;
   const uint32_t gch = lch ^ ((4 * (wave & 1) + lane / 16) % CH);
   const uint32_t smem0 = lds_address(&smem[0][0][0]);
+  // NN: rows of k of 4 BT bytes
+  constexpr int RBN = ELEM * BNT, CHN = RBN / 16, RPWN = 1024 / RBN;
+  auto nn_row = [&](int it) { return (wave + NWAVES * it) * RPWN + lane / CHN; };
   // per-lane byte offsets from the slab's first row of this wave-load; edge tiles clamp the row
   uint32_t aoff[WLW], boff[WLW];
 #pragma unroll
@@ -87,16 +98,23 @@ __device__ __forceinline__ void gemm_nt_f32_direct_body(const GemmParams& p) {
     const uint32_t rb = n0 + r < p.n ? n0 + r : p.n - 1;
     aoff[it] = (ra - m0) * (uint32_t)row_bytes + 16 * gch;
     boff[it] = (rb - n0) * (uint32_t)row_bytes + 16 * gch;
+    if constexpr (NN) {
+      const uint32_t row = nn_row(it), last_chunk = (p.b_cols - n0) / 4 - 1;
+      uint32_t ch = (lane % CHN) ^ (8 * ((row >> 2) & 1));
+      ch = ch < last_chunk ? ch : last_chunk;
+      boff[it] = row * (uint32_t)brow_bytes + 16 * ch;
+    }
   }
   const char* a_tile = A + (size_t)m0 * row_bytes;
-  const char* b_tile = B + (size_t)n0 * row_bytes;
-  const size_t b_slab_step = (size_t)RB;  // bytes from one k slab of B to the next
+  const char* b_tile = NN ? B + (size_t)n0 * ELEM : B + (size_t)n0 * row_bytes;
+  const size_t b_slab_step = NN ? (size_t)BK * brow_bytes : (size_t)RB;  // bytes from one k slab of B to the next
   const uint32_t nslabs = KTAIL ? (kk + BK - 1) / BK : kk / BK;
   const uint32_t tail_chunks = (kk - (nslabs - 1) * BK) / 4;  // KTAIL: 16-byte chunks per row of the last slab
   // one transfer of 16 bytes per lane of slab s; KTAIL: nothing to fetch for this lane: its slot is cleared
-  auto move = [&](const void* base, uint32_t voff, uint32_t lds_base, uint32_t s) {
+  // (`past`: how many chunks or, NN, rows of k of a partial slab lie before this lane's)
+  auto move = [&](const void* base, uint32_t voff, uint32_t lds_base, uint32_t s, uint32_t past, uint32_t limit) {
     if constexpr (KTAIL) {
-      if (s + 1 < nslabs || gch < tail_chunks) dma16(base, voff, lds_base);
+      if (s + 1 < nslabs || past < limit) dma16(base, voff, lds_base);
       else *reinterpret_cast<u32x4*>(&smem[0][0][0] + (lds_base - smem0) + 16 * lane) = u32x4{0, 0, 0, 0};
     } else {
       dma16(base, voff, lds_base);
@@ -107,8 +125,8 @@ __device__ __forceinline__ void gemm_nt_f32_direct_body(const GemmParams& p) {
 #pragma unroll
     for (int it = 0; it < WLW; ++it) {
       const uint32_t w = wave + NWAVES * it;
-      move(a_tile + k_byte, aoff[it], smem0 + (2 * buf + 0) * SLAB + w * 1024, s);
-      move(b_tile + s * b_slab_step, boff[it], smem0 + (2 * buf + 1) * SLAB + w * 1024, s);
+      move(a_tile + k_byte, aoff[it], smem0 + (2 * buf + 0) * SLAB + w * 1024, s, gch, tail_chunks);
+      move(b_tile + s * b_slab_step, boff[it], smem0 + (2 * buf + 1) * SLAB + w * 1024, s, NN ? nn_row(it) : gch, NN ? 4 * tail_chunks : tail_chunks);
     }
   };
 
@@ -117,7 +135,7 @@ __device__ __forceinline__ void gemm_nt_f32_direct_body(const GemmParams& p) {
   uint32_t addr[KS];
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks) addr[ks] = c * RB + 16 * ((2 * ks + h) ^ fr);
-  const uint32_t a_rows = wm * TM * 32 * RB, b_rows = wn * TN * 32 * RB;
+  const uint32_t a_rows = wm * TM * 32 * RB, b_rows = NN ? 0 : wn * TN * 32 * RB;
   f32x16 acc[TM][TN];
 #pragma unroll
   for (int i = 0; i < TM; ++i)
@@ -144,7 +162,15 @@ __device__ __forceinline__ void gemm_nt_f32_direct_body(const GemmParams& p) {
 #pragma unroll
     for (int i = 0; i < TM; ++i) f.a[i] = *reinterpret_cast<const f32x4*>(sa + i * 32 * RB + addr[ks]);
 #pragma unroll
-    for (int j = 0; j < TN; ++j) f.b[j] = *reinterpret_cast<const f32x4*>(sb + j * 32 * RB + addr[ks]);
+    for (int j = 0; j < TN; ++j) {
+      if constexpr (NN) {
+        const char* at = sb + 4 * (2 * ks + h) * RBN + (((wn * TN + j) * 128 + 4 * c) ^ (128 * h));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) f.b[j][e] = *reinterpret_cast<const float*>(at + e * RBN);
+      } else {
+        f.b[j] = *reinterpret_cast<const f32x4*>(sb + j * 32 * RB + addr[ks]);
+      }
+    }
   };
   auto mfma = [&](const Frags& f, int i, int j) {
 #pragma unroll
@@ -171,8 +197,8 @@ __device__ __forceinline__ void gemm_nt_f32_direct_body(const GemmParams& p) {
         for (int r = slot * NREQ / (TM * TN); r < (slot + 1) * NREQ / (TM * TN); ++r) {
           const int it = r % WLW;
           const uint32_t w = wave + NWAVES * it;
-          if (r < WLW) move(a_tile + k_byte, aoff[it], smem0 + (2 * (buf ^ 1) + 0) * SLAB + w * 1024, s_req);
-          else move(b_tile + s_req * b_slab_step, boff[it], smem0 + (2 * (buf ^ 1) + 1) * SLAB + w * 1024, s_req);
+          if (r < WLW) move(a_tile + k_byte, aoff[it], smem0 + (2 * (buf ^ 1) + 0) * SLAB + w * 1024, s_req, gch, tail_chunks);
+          else move(b_tile + s_req * b_slab_step, boff[it], smem0 + (2 * (buf ^ 1) + 1) * SLAB + w * 1024, s_req, NN ? nn_row(it) : gch, NN ? 4 * tail_chunks : tail_chunks);
         }
         __builtin_amdgcn_sched_barrier(0);
       }

@@ -152,20 +152,24 @@ extern "C" __global__ void __launch_bounds__(256, 2) gemm_nt_bf16_128x128x64_dir
 extern "C" __global__ void __launch_bounds__(256, 2) gemm_nn_bf16_128x128x64_direct_ktail(GemmParams p) {
   gemm_nt_mfma16_body<128, 2, 2, true, true>(p);
 }
-extern "C" __global__ void __launch_bounds__(256, 2) gemm_nt_f32_128x128x32_direct(GemmParams p) {
-  gemm_nt_f32_direct_body<128, 2, 2>(p);
-}
-// f32 operands, f32 MFMA: the arithmetic type of the reference
-extern "C" __global__ void __launch_bounds__(512, 1) gemm_nt_f32_256x256x32_direct(GemmParams p) {
-  gemm_nt_f32_direct_body<256, 2, 4>(p);
-}
-// k that is a multiple of 4 but not of 32: the last slab partial
-extern "C" __global__ void __launch_bounds__(256, 2) gemm_nt_f32_128x128x32_direct_ktail(GemmParams p) {
-  gemm_nt_f32_direct_body<128, 2, 2, true>(p);
-}
-extern "C" __global__ void __launch_bounds__(512, 1) gemm_nt_f32_256x256x32_direct_ktail(GemmParams p) {
-  gemm_nt_f32_direct_body<256, 2, 4, true>(p);
-}
+// f32 operands, f32 MFMA: the arithmetic type of the reference.  _ktail: k a multiple of 4 but not of 32, the last
+// slab partial; _brow: row-major right operand
+#define GEMM_F32(BT, WM, WN, OCC)                                                                                   \
+  extern "C" __global__ void __launch_bounds__(WM * WN * 64, OCC) gemm_nt_f32_##BT##x##BT##x32_direct(GemmParams p) {       \
+    gemm_nt_f32_direct_body<BT, WM, WN>(p);                                                                         \
+  }                                                                                                                 \
+  extern "C" __global__ void __launch_bounds__(WM * WN * 64, OCC) gemm_nt_f32_##BT##x##BT##x32_direct_ktail(GemmParams p) { \
+    gemm_nt_f32_direct_body<BT, WM, WN, true>(p);                                                                   \
+  }                                                                                                                 \
+  extern "C" __global__ void __launch_bounds__(WM * WN * 64, OCC) gemm_nt_f32_##BT##x##BT##x32_direct_brow(GemmParams p) {       \
+    gemm_nt_f32_direct_body<BT, WM, WN, false, true>(p);                                                            \
+  }                                                                                                                 \
+  extern "C" __global__ void __launch_bounds__(WM * WN * 64, OCC) gemm_nt_f32_##BT##x##BT##x32_direct_ktail_brow(GemmParams p) { \
+    gemm_nt_f32_direct_body<BT, WM, WN, true, true>(p);                                                             \
+  }
+GEMM_F32(64, 2, 2, 4)
+GEMM_F32(128, 2, 2, 2)
+GEMM_F32(256, 2, 4, 1)
 
 // gemm_{nt_bf16,nt_f32,nn_f32}_narrow<M>x<columns per workgroup>: at most M = 16, 32, 64 rows of A
 #define GEMM_NARROW(NAME, F32, NN, M, MT, N, TN, W)                                                           \
@@ -344,6 +348,41 @@ __device__ __forceinline__ void pad_rows_body(const PadParams& p) {
     dst[at] = c < p.cols ? src[r * p.cols + c] : T(0);
   }
 }
+// Two operands padded in one launch (blockIdx.y says which): a work-item writes 16 bytes of the copy and reads the
+// elements they come from in one access on the alignment of the elements, or one by one at the end of a row.  Bound by
+// its launch at the sizes it meets: 2047 x 777 and 777 x 3001 bf16 in 5 us, where pad_rows, an element per
+// work-item, took 7 and 8 in a launch each.
+template <class T>
+__device__ __forceinline__ void pad_pair_body(const PadPairParams& p) {
+  constexpr uint32_t V = 16 / sizeof(T);
+  typedef T wide __attribute__((ext_vector_type(V), aligned(sizeof(T))));
+  const uint32_t o = blockIdx.y;
+  const T* src = reinterpret_cast<const T*>(o ? p.src[1] : p.src[0]);
+  T* dst = reinterpret_cast<T*>(o ? p.dst[1] : p.dst[0]);
+  const uint32_t rows = o ? p.rows[1] : p.rows[0], padded = o ? p.rows_padded[1] : p.rows_padded[0];
+  const uint32_t cols = o ? p.cols[1] : p.cols[0], width = o ? p.cols_padded[1] : p.cols_padded[0];
+  const uint32_t chunks = width / V, total_rows = p.batches * padded;  // (the launcher keeps the product below 2^32)
+  const uint32_t total = chunks * total_rows;
+  for (uint32_t at = blockIdx.x * blockDim.x + threadIdx.x; at < total; at += gridDim.x * blockDim.x) {
+    const uint32_t row = at / chunks, col = (at - row * chunks) * V;
+    const uint32_t batch = row / padded, r = row - batch * padded;
+    wide v = {};
+    if (r < rows) {
+      const T* from = src + ((size_t)batch * rows + r) * cols + col;
+      if (col + V <= cols) {
+        v = *reinterpret_cast<const wide*>(from);
+      } else {
+#pragma unroll
+        for (uint32_t e = 0; e < V; ++e)
+          if (col + e < cols) v[e] = from[e];
+      }
+    }
+    typedef T wide_aligned __attribute__((ext_vector_type(V)));
+    *reinterpret_cast<wide_aligned*>(dst + (size_t)row * width + col) = v;
+  }
+}
+extern "C" __global__ void __launch_bounds__(256) pad_pair_b16(PadPairParams p) { pad_pair_body<uint16_t>(p); }
+extern "C" __global__ void __launch_bounds__(256) pad_pair_b32(PadPairParams p) { pad_pair_body<uint32_t>(p); }
 extern "C" __global__ void __launch_bounds__(256) pad_rows_b16(PadParams p) { pad_rows_body<uint16_t>(p); }
 extern "C" __global__ void __launch_bounds__(256) pad_rows_b32(PadParams p) { pad_rows_body<uint32_t>(p); }
 

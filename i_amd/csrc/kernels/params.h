@@ -59,6 +59,7 @@ struct GemmParams {
   // writes its f32 partial products to c[(batch * splits + s)][m][n], a temporary that splitk_reduce adds up.
   uint32_t splits;
   uint32_t k_chunk;   // a multiple of 64
+  uint32_t b_cols;    // row-major right operand (NN): elements per row of B, at least n (n, or n rounded up by a padded copy)
 };
 
 // out[b][i] = sum over s < splits of partial[b][s][i], i < count (count a multiple of 4); out f32 or bf16
@@ -93,7 +94,6 @@ struct ConvertParams {
   uint64_t n;
 };
 
-// dst[b][c][r] = src[b][r][c] for b < bh, r < rows, c < cols; elements of 2 or 4 bytes
 // dst[r][c] = c < cols ? src[r][c] : 0 for r < rows, c < cols_padded; elements of 2 or 4 bytes
 struct PadParams {
   const void* src;
@@ -102,6 +102,15 @@ struct PadParams {
   uint32_t cols, cols_padded;
 };
 
+// Two operands at once, each batches x [rows, cols] copied into batches x [rows_padded, cols_padded], zeros beyond; dst
+// 16-byte aligned, cols_padded a multiple of 16 bytes, src at any alignment of its elements
+struct PadPairParams {
+  const void* src[2];
+  void* dst[2];
+  uint32_t batches, rows[2], rows_padded[2], cols[2], cols_padded[2];
+};
+
+// dst[b][c][r] = src[b][r][c] for b < bh, r < rows, c < cols; elements of 2 or 4 bytes
 struct TransposeParams {
   const void* src;
   void* dst;

@@ -477,8 +477,8 @@ Err launch_gemm_nt_bf16_split_k(const void* a, const void* b, void* c, float* pa
   return launch(fn, (unsigned)rgrid, 1, 1, 256, &r, sizeof(r), stream);
 }
 
-static unsigned gemm_nn_tile(size_t bh, size_t m, size_t n, size_t k, size_t tile_m, size_t tile_n, const KernelOptions& knobs) {
-  if (k == 0 || k % 8 != 0 || n % 8 != 0 || k > (size_t(1) << 22) || n > (size_t(1) << 24) || bh > 65535) return 0;
+static unsigned gemm_nn_tile(size_t bh, size_t m, size_t n, size_t k, size_t tile_m, size_t tile_n, const KernelOptions& knobs, size_t b_cols) {
+  if (k == 0 || k % 8 != 0 || b_cols % 8 != 0 || b_cols < n || b_cols > (size_t(1) << 24) || k > (size_t(1) << 22) || n > (size_t(1) << 24) || bh > 65535) return 0;
   if (!fits_u32(m) || !fits_u32(n)) return 0;
   const size_t t256 = ((m + 255) / 256) * ((n + 255) / 256) * bh, t128 = ((m + 127) / 128) * ((n + 127) / 128) * bh;
   unsigned tile = t256 >= 128 ? pick_direct_tile(t256, t128) : 128;
@@ -490,14 +490,15 @@ static unsigned gemm_nn_tile(size_t bh, size_t m, size_t n, size_t k, size_t til
 }
 
 bool gemm_nn_bf16_supported(size_t bh, size_t m, size_t n, size_t k, const KernelOptions& knobs) {
-  return gemm_nn_tile(bh, m, n, k, 0, 0, knobs) != 0;
+  return gemm_nn_tile(bh, m, n, k, 0, 0, knobs, n) != 0;
 }
 
 Err launch_gemm_nn_bf16(const void* a, const void* b, void* c, size_t bh, size_t m, size_t n, size_t k,
                         hipStream_t stream, size_t tile_m, size_t tile_n, LaunchNote* note, DType out_dtype, float* partial,
-                        unsigned splits, const KernelOptions& knobs) {
-  unsigned tile = gemm_nn_tile(bh, m, n, k, tile_m, tile_n, knobs);
-  if (tile == 0) return "gemm_nn kernel: needs k % 8 == 0 and n % 8 == 0 (and extents within its offset range)";
+                        unsigned splits, const KernelOptions& knobs, size_t b_cols) {
+  if (b_cols == 0) b_cols = n;
+  unsigned tile = gemm_nn_tile(bh, m, n, k, tile_m, tile_n, knobs, b_cols);
+  if (tile == 0) return "gemm_nn kernel: needs k % 8 == 0 and rows of B of a multiple of 8 elements (and extents within its offset range)";
   if (bh == 0 || m == 0 || n == 0) return {};
   if (!a || !b || !c) return "gemm_nn kernel: null device pointer";
   if (!aligned16(a) || !aligned16(b)) return "gemm_nn kernel: operands must be 16-byte aligned";
@@ -505,6 +506,7 @@ Err launch_gemm_nn_bf16(const void* a, const void* b, void* c, size_t bh, size_t
   p.a = a; p.b = b; p.c = c;
   p.bh = (uint32_t)bh; p.m = (uint32_t)m; p.n = (uint32_t)n; p.k = (uint32_t)k;
   p.out_bf16 = out_dtype == BF16 ? 1u : 0u;
+  p.b_cols = (uint32_t)b_cols;
   // the k loop in parts over workgroups (gemm_nt_bf16_split_k says when, for this form too): f32 partial products
   // in the caller's temporary, added up by splitk_reduce
   if (splits > 1) {
@@ -605,50 +607,70 @@ Err launch_gemm_narrow(const void* a, const void* b, void* c, DType dtype, bool 
 
 bool gemm_nt_f32_supported(size_t k) { return k > 0 && k % 4 == 0 && k <= (size_t(1) << 21); }
 
-unsigned gemm_nt_f32_split_k(size_t bh, size_t m, size_t n, size_t k, const KernelOptions& knobs) {
-  if (bh == 0 || m == 0 || n == 0 || !gemm_nt_f32_supported(k) || knobs.gemm_k_parts == 1) return 1;
+// Tile and parts of k of an f32 product, by a model of the time in us.  Its matrix instructions are the bound (157
+// TFLOP/s, a sixteenth of bf16) and the workgroups of a CU share them, so the time is what the fullest CU has to do: 1.7
+// per 32-wide slab of a 128 x 128 tile, a quarter of it, 0.46, of a 64 x 64 one, plus two slabs' worth before and after
+// the loop.  A workgroup has one slab in flight, though, and operands beyond the 32 MB of the L2s take 0.7 to arrive: a
+// CU with a single small tile waits for them.  A split costs 4 for the second launch and the pass over the partial
+// products at 3 TB/s, parts have at least 64 of k, and a split has to gain 15 %.  256 x 256 tiles where they fill at
+// least half of the CUs.  Measured (128 x 128 tiles in parts -> this rule): 1000 x 1500 x 700 34 -> 26 us, 1024^3 27 ->
+// 18 (118 TFLOP/s), 128 x 128 x 4096 28 -> 16 in 32 parts, 777 x 999 x 1001 with a row-major right operand, padded
+// copies included, 88 -> 30; 100 x 8000 x 8000 takes 176 on whole 64-tiles, a CU each, and 129 on 128-tiles in 4
+// parts; 64 x 8192 x 8192 105 on 64-tiles in 2 parts, 88 in 4.
+struct F32Plan {
+  unsigned tile, splits;
+};
+static F32Plan f32_plan(size_t bh, size_t m, size_t n, size_t k, const KernelOptions& knobs, bool whole) {
+  const size_t t256 = ((m + 255) / 256) * ((n + 255) / 256) * bh;
   auto parts_of = [&](size_t want) -> unsigned {
-    if (want < 2 || bh * want > 65535) return 1;
+    if (whole || want < 2 || bh * want > 65535) return 1;
     const size_t chunk = (k / want + 63) / 64 * 64;  // what one split contracts: whole slabs
     return (unsigned)((k + chunk - 1) / chunk);
   };
-  if (knobs.gemm_k_parts > 1) return parts_of(std::min<size_t>((size_t)knobs.gemm_k_parts, k / 64));
-  // The model of gemm_nt_bf16_split_k with this kernel's figures: 1.7 us per 32-wide slab for a workgroup on a
-  // 128 x 128 tile, 256 of them at a time (the 256 x 256 tile only takes grids that fill the chip), parts of at
-  // least 64 of k.  Unsplit -> split, us: 128 x 128 x 8192 444 -> 36 (32 parts), 512 x 512 x 4096 227 -> 31 (16),
-  // 1024 x 1024 x 1024 60 -> 27 (4), 8192 x 128 x 8192 (the probabilities times the values of a naive attention)
-  // 451 -> 128 (4), 512 x 64 x 512 34 -> 15 (8); left whole: 2048^3 (120 us; 130 in two parts).
-  const size_t t128 = ((m + 127) / 128) * ((n + 127) / 128) * bh, t256 = ((m + 255) / 256) * ((n + 255) / 256) * bh;
-  if (t256 >= 128) return 1;  // (the large tile's grids fill the chip)
+  const unsigned asked = knobs.gemm_tile == 0 ? 0u : knobs.gemm_tile == 192 ? 256u : (unsigned)knobs.gemm_tile;  // (192 x 256 exists for bf16 NT products only)
+  if (knobs.gemm_k_parts > 1) return {asked ? asked : t256 >= 128 ? 256u : 128u, parts_of(std::min<size_t>((size_t)knobs.gemm_k_parts, k / 64))};
+  if (asked == 256 || (!asked && t256 >= 128)) return {256, 1};
   const size_t slabs = (k + 31) / 32;
-  auto time_of = [](size_t workgroups, size_t slabs_) { return (double)((workgroups + 255) / 256) * (double)(slabs_ + 2) * 1.7; };
-  double best = 0.85 * time_of(t128, slabs);
-  size_t splits = 1;
-  for (size_t s = 2; s <= 32 && k / s >= 64 && bh * s <= 65535; s *= 2) {
-    const double t = time_of(t128 * s, (slabs + s - 1) / s) + 4.0 + (double)(bh * s * m * n * 4) / 3e6;
-    if (t < best) {
-      best = t;
-      splits = s;
+  const bool far = bh * (m + n) * k * 4 > (size_t(32) << 20);
+  F32Plan best{asked ? asked : 128u, 1};
+  double best_time = 1e30;
+  for (unsigned tile : {128u, 64u}) {
+    if (asked && tile != asked) continue;
+    const size_t tiles = ((m + tile - 1) / tile) * ((n + tile - 1) / tile) * bh;
+    for (size_t s = 1; s <= 32 && (s == 1 || (!whole && knobs.gemm_k_parts != 1 && k / s >= 64 && bh * s <= 65535)); ++s) {
+      const double resident = (double)((tiles * s + 255) / 256);
+      double t = (double)((slabs + s - 1) / s + 2) * std::max(resident * (tile == 128 ? 1.7 : 0.46), far ? 0.7 : 0.0);
+      if (s > 1) t = (t + 4.0 + (double)(bh * s * m * n * 4) / 3e6) / 0.85;
+      if (t < best_time) {
+        best_time = t;
+        best = {tile, (unsigned)s};
+      }
     }
   }
-  return parts_of(splits);
+  best.splits = parts_of(best.splits);
+  return best;
+}
+
+unsigned gemm_nt_f32_split_k(size_t bh, size_t m, size_t n, size_t k, const KernelOptions& knobs) {
+  if (bh == 0 || m == 0 || n == 0 || !gemm_nt_f32_supported(k) || knobs.gemm_k_parts == 1) return 1;
+  return f32_plan(bh, m, n, k, knobs, false).splits;
 }
 
 Err launch_gemm_nt_f32(const float* a, const float* b, float* c, size_t bh, size_t m, size_t n, size_t k,
-                       hipStream_t stream, LaunchNote* note, float* partial, unsigned splits, const KernelOptions& knobs) {
+                       hipStream_t stream, LaunchNote* note, float* partial, unsigned splits, const KernelOptions& knobs, size_t b_cols) {
   if (!gemm_nt_f32_supported(k)) return "gemm_nt f32 kernel: k must be a positive multiple of 4 (at most 2^21)";
   if (reinterpret_cast<uintptr_t>(a) % 16 != 0 || reinterpret_cast<uintptr_t>(b) % 16 != 0)
     return "gemm_nt f32 kernel: operands must be 16-byte aligned";
   if (bh == 0 || m == 0 || n == 0) return {};
   if (!fits_u32(m) || !fits_u32(n) || bh > 65535) return "gemm_nt f32 kernel: extent too large";
   if (!a || !b || !c) return "gemm_nt f32 kernel: null device pointer";
+  const bool nn = b_cols != 0;
+  if (nn && (b_cols % 4 != 0 || b_cols < n || b_cols > (size_t(1) << 24))) return "gemm_nn f32 kernel: needs rows of B of a multiple of 4 elements (at most 2^24)";
   GemmParams p{};
   p.a = a; p.b = b; p.c = c;
   p.bh = (uint32_t)bh; p.m = (uint32_t)m; p.n = (uint32_t)n; p.k = (uint32_t)k;
-  // 256 x 256 tiles when they fill at least half of the CUs, 128 x 128 tiles otherwise
-  const size_t t256 = ((m + 255) / 256) * ((n + 255) / 256) * bh;
-  unsigned tile = t256 >= 128 ? 256 : 128;
-  if (knobs.gemm_tile) tile = knobs.gemm_tile == 192 ? 256u : (unsigned)knobs.gemm_tile;  // (192 x 256 exists for bf16 NT products only)
+  p.b_cols = (uint32_t)b_cols;
+  const unsigned tile = f32_plan(bh, m, n, k, knobs, splits <= 1).tile;
   // the k loop in parts over workgroups (gemm_nt_f32_split_k says when): partial products in the caller's temporary
   if (splits > 1) {
     if (!partial) return "gemm_nt f32 kernel: a split needs its temporary";
@@ -666,8 +688,9 @@ Err launch_gemm_nt_f32(const float* a, const float* b, float* c, size_t bh, size
   const size_t grid = (size_t(p.tiles_m) * p.tiles_n + 7) / 8 * 8;  // the tiles in 8 equal runs, one per XCD
   if (grid > kMaxGrid) return "gemm_nt f32 kernel: grid too large";
   hipFunction_t fn;
-  const std::string name = std::string(tile == 256 ? "gemm_nt_f32_256x256x32_direct" : "gemm_nt_f32_128x128x32_direct") +
-                           (k % 32 != 0 ? "_ktail" : "");  // (a partial last slab of 32 k; of the last part, when split)
+  const std::string edge = std::to_string(tile);
+  const std::string name = "gemm_nt_f32_" + edge + "x" + edge + "x32_direct" + (k % 32 != 0 ? "_ktail" : "") + (nn ? "_brow" : "");
+  // (_ktail: a partial last slab of 32 k; of the last part, when split)
   if (note) *note = LaunchNote{splits > 1 ? name + " (k in " + std::to_string(splits) + " parts)" : name, tile, tile};
   if (Err e = builtin_function(name.c_str(), &fn); !e.empty()) return e;
   if (Err e = launch(fn, (unsigned)grid, (unsigned)(bh * (splits > 1 ? splits : 1)), 1, tile == 256 ? 512 : 256, &p, sizeof(p), stream);
@@ -836,6 +859,33 @@ Err launch_pad_rows(const void* src, void* dst, size_t rows, size_t cols, size_t
   size_t grid = (rows * cols_padded + 255) / 256;
   if (grid > 65536) grid = 65536;
   return launch(fn, (unsigned)grid, 1, 1, 256, &p, sizeof(p), stream);
+}
+
+Err launch_pad_pair(const PadPair& pair, size_t batches, size_t elem_bytes, hipStream_t stream) {
+  if (elem_bytes != 2 && elem_bytes != 4) return "pad kernel: element size must be 2 or 4 bytes";
+  PadPairParams p{};
+  p.batches = (uint32_t)batches;
+  size_t most = 0;
+  for (int o = 0; o < 2; ++o) {
+    if (pair.cols[o] > pair.cols_padded[o] || pair.rows[o] > pair.rows_padded[o] || pair.cols_padded[o] * elem_bytes % 16 != 0) return "pad kernel: bad extents";
+    const size_t chunks = batches * pair.rows_padded[o] * (pair.cols_padded[o] * elem_bytes / 16);
+    if (chunks == 0) return "pad kernel: bad extents";
+    if (chunks >= (size_t(1) << 31) || !fits_u32(pair.cols_padded[o])) return "pad kernel: extent too large";
+    if (!pair.src[o] || !pair.dst[o]) return "pad kernel: null device pointer";
+    if (!aligned16(pair.dst[o])) return "pad kernel: the copies must be 16-byte aligned";
+    most = std::max(most, chunks);
+    p.src[o] = pair.src[o];
+    p.dst[o] = pair.dst[o];
+    p.rows[o] = (uint32_t)pair.rows[o];
+    p.rows_padded[o] = (uint32_t)pair.rows_padded[o];
+    p.cols[o] = (uint32_t)pair.cols[o];
+    p.cols_padded[o] = (uint32_t)pair.cols_padded[o];
+  }
+  hipFunction_t fn;
+  if (Err e = builtin_function(elem_bytes == 2 ? "pad_pair_b16" : "pad_pair_b32", &fn); !e.empty()) return e;
+  // (index arithmetic in 32 bits: at most 2^31 chunks and 2^24 work-items past them)
+  const size_t grid = std::min<size_t>((most + 255) / 256, 65536);
+  return launch(fn, (unsigned)grid, 2, 1, 256, &p, sizeof(p), stream);
 }
 
 }  // namespace ihip

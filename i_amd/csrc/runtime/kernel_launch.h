@@ -96,13 +96,16 @@ Err launch_gemm_nt_bf16_split_k(const void* a, const void* b, void* c, float* pa
 // `partial` is room for bh * splits * m * n floats)
 Err launch_gemm_nn_bf16(const void* a, const void* b, void* c, size_t bh, size_t m, size_t n, size_t k,
                         hipStream_t stream, size_t tile_m = 0, size_t tile_n = 0, LaunchNote* note = nullptr,
-                        DType out_dtype = F32, float* partial = nullptr, unsigned splits = 1, const KernelOptions& knobs = {});
+                        DType out_dtype = F32, float* partial = nullptr, unsigned splits = 1, const KernelOptions& knobs = {},
+                        size_t b_cols = 0);
+// (b_cols: elements per row of b, a multiple of 8 and at least n, 0 for n itself; then n may be anything)
 bool gemm_nn_bf16_supported(size_t bh, size_t m, size_t n, size_t k, const KernelOptions& knobs = {});
 
 // c[bh,m,n] = a[bh,m,k] b[bh,n,k]^T, all f32, products and sums in f32 (f32 MFMA); needs k % 4 == 0 and 16-byte aligned operands
 Err launch_gemm_nt_f32(const float* a, const float* b, float* c, size_t bh, size_t m, size_t n, size_t k,
                        hipStream_t stream, LaunchNote* note = nullptr, float* partial = nullptr, unsigned splits = 1,
-                       const KernelOptions& knobs = {});
+                       const KernelOptions& knobs = {}, size_t b_cols = 0);
+// (b_cols != 0: b is row-major, [bh, k, b_cols] with b_cols % 4 == 0 and at least n, and c = a b)
 // (splits > 1: the k loop in that many parts over workgroups, as launch_gemm_nt_bf16_split_k does it; `partial` is
 // room for bh * splits * m * n floats, and gemm_nt_f32_split_k says into how many parts, 1: do not split)
 unsigned gemm_nt_f32_split_k(size_t bh, size_t m, size_t n, size_t k, const KernelOptions& knobs = {});
@@ -139,5 +142,14 @@ Err launch_convert(const void* src, void* dst, DType from, DType to, size_t n, h
 // dst[r][c] = c < cols ? src[r][c] : 0 for c < cols_padded; elem_bytes is 2 or 4
 Err launch_pad_rows(const void* src, void* dst, size_t rows, size_t cols, size_t cols_padded, size_t elem_bytes,
                     hipStream_t stream);
+
+// Two operands, batches x [rows, cols] each, copied into zero-padded batches x [rows_padded, cols_padded] in one launch;
+// rows of the copies are multiples of 16 bytes and the copies 16-byte aligned, src at any alignment of its elements.
+struct PadPair {
+  const void* src[2];
+  void* dst[2];
+  size_t rows[2], rows_padded[2], cols[2], cols_padded[2];
+};
+Err launch_pad_pair(const PadPair& pair, size_t batches, size_t elem_bytes, hipStream_t stream);
 
 }  // namespace ihip
