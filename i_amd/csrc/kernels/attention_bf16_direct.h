@@ -84,12 +84,18 @@
 // the first transfer, so the columns d .. DPAD - 1 of K and dv .. DPAD - 1 of V read as zeros for the whole kernel
 // (Q is padded with zeros in its registers; the output columns past dv are not stored).  Global rows of Q and K are
 // 2 p.d bytes apart, those of V 2 p.dv (and those of O p.dv elements).
-template <int DPAD, int BN, int NWAVES, bool PRECISE = false, bool PADDED = false, int QB = 1>
+//
+// DUSE: how many of a row's DPAD columns the matrix instructions work on, a multiple of 32 that covers d and dv: the rest
+// of a padded row is zeros on either side of the products (96 of 128 columns: 2 x 12 heads of 1000 x 1000, d = 80, 22.0 ->
+// 20.0 us; 8 x 16 heads of 2048, d = 96, 232 -> 205; a kernel of its own, since the choice inside the kernel cost the
+// larger head sizes 2 %).
+template <int DPAD, int BN, int NWAVES, bool PRECISE = false, bool PADDED = false, int QB = 1, int DUSE = DPAD>
 __device__ __forceinline__ void attn_fwd_bf16_direct_body(const AttnParams& p) {
+  static_assert(DUSE == DPAD || (PADDED && DUSE < DPAD && DUSE % 32 == 0), "columns in use");
   constexpr int BM = 32 * QB * NWAVES;
-  constexpr int KSTEPS = DPAD / 16;       // k-steps of the QK^T contraction
+  constexpr int KSTEPS = DUSE / 16;       // k-steps of the QK^T contraction
   constexpr int KT = BN / 32;             // 32-key accumulator tiles
-  constexpr int DT = DPAD / 32;           // 32-column output tiles
+  constexpr int DT = DUSE / 32;           // 32-column output tiles
   constexpr int RB = 2 * DPAD;            // bytes per K/V row
   constexpr int CH = RB / 16;             // 16-byte chunks per row (= lanes per row of a wave-load)
   constexpr int RPB = RB >= 256 ? 1 : 256 / RB;  // rows per 256 bytes (1 for longer rows, which start at the same banks)
@@ -860,9 +866,9 @@ __device__ __forceinline__ void attn_fwd_bf16_direct_body(const AttnParams& p) {
         const uint32_t rows_valid = row0 < p.nq ? (p.nq - row0 < 32u ? p.nq - row0 : 32u) : 0u;
         float* O = reinterpret_cast<float*>(p.o) + ((size_t)head * p.nq + row0) * dv;
 #pragma unroll
-        for (int half = 0; half < DT / 2; ++half) {
+        for (int half = 0; half < (DT + 1) / 2; ++half) {
 #pragma unroll
-          for (int tt = 0; tt < 2; ++tt)
+          for (int tt = 0; tt < 2 && 2 * half + tt < DT; ++tt)
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
               f32x4 w;

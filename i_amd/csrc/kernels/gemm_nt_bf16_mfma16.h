@@ -317,43 +317,65 @@ __device__ __forceinline__ void gemm_nt_mfma16_tile(const GemmParams& p, char* s
   // consecutive columns at once, a quarter-wave 16 rows of them.  A C whose n is not a multiple of 4 (or whose base
   // is not 16-byte aligned) takes the same wide stores on the alignment of its elements, and only the columns of a
   // last, partial four go one by one (2047 x 3001 x 777, f32 result: 31 -> 22 us).
-  const bool n4 = p.n % 4 == 0 && reinterpret_cast<uintptr_t>(C) % 16 == 0;
+  // One loop per kind of store, chosen once, where a workgroup's tile is small: with the choice inside, the code that is
+  // stepped over between the stores cost a product of few tiles half a microsecond (3352 x 184 x 1280: 17.5 against
+  // 16.4 us).  The 256-accumulator forms keep the choice inside, which spaces their stores: 4096^3 takes 114 us so and
+  // 117 in one loop per kind.
   typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
   typedef __bf16 bf16x4_any __attribute__((ext_vector_type(4), aligned(2)));
-#pragma unroll
-  for (int i = 0; i < TM; ++i) {
+  const bool n4 = p.n % 4 == 0 && reinterpret_cast<uintptr_t>(C) % 16 == 0;
+  auto store_one = [&](int i, int j, auto bf16_tag, auto aligned_tag) {
+    constexpr bool BF16 = decltype(bf16_tag)::value, ALIGNED = decltype(aligned_tag)::value;
     const uint32_t row = m0 + (wm * TM + i) * 16 + c16;
+    const uint32_t col = n0 + (wn * TN + j) * 16 + 4 * g;
+    const size_t at = (size_t)row * p.n + col;
+    if (!EDGE || (row < p.m && (ALIGNED ? col < p.n : col + 4 <= p.n))) {
+      if constexpr (BF16) {
+        bf16x4 v;
 #pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      const uint32_t col = n0 + (wn * TN + j) * 16 + 4 * g;
-      const size_t at = (size_t)row * p.n + col;
-      if (n4 && (!EDGE || (row < p.m && col < p.n))) {
-        if (p.out_bf16) {
-          bf16x4 v;
-#pragma unroll
-          for (int r = 0; r < 4; ++r) v[r] = (bf16_t)acc[i][j][r];
-          *reinterpret_cast<bf16x4*>(C + 2 * at) = v;
-        } else {
-          *reinterpret_cast<f32x4*>(C + 4 * at) = acc[i][j];
-        }
-      } else if (!EDGE || (row < p.m && col + 4 <= p.n)) {
-        if (p.out_bf16) {
-          bf16x4_any v;
-#pragma unroll
-          for (int r = 0; r < 4; ++r) v[r] = (bf16_t)acc[i][j][r];
-          *reinterpret_cast<bf16x4_any*>(C + 2 * at) = v;
-        } else {
-          *reinterpret_cast<f32x4_any*>(C + 4 * at) = acc[i][j];
-        }
-      } else if (row < p.m) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (col + r < p.n) {
-            if (p.out_bf16) reinterpret_cast<bf16_t*>(C + 2 * at)[r] = (bf16_t)acc[i][j][r];
-            else reinterpret_cast<float*>(C + 4 * at)[r] = acc[i][j][r];
-          }
+        for (int r = 0; r < 4; ++r) v[r] = (bf16_t)acc[i][j][r];
+        if constexpr (ALIGNED) *reinterpret_cast<bf16x4*>(C + 2 * at) = v;
+        else *reinterpret_cast<bf16x4_any*>(C + 2 * at) = v;
+      } else {
+        if constexpr (ALIGNED) *reinterpret_cast<f32x4*>(C + 4 * at) = acc[i][j];
+        else *reinterpret_cast<f32x4_any*>(C + 4 * at) = acc[i][j];
       }
+    } else if (!ALIGNED && row < p.m) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (col + r < p.n) {
+          if constexpr (BF16) reinterpret_cast<bf16_t*>(C + 2 * at)[r] = (bf16_t)acc[i][j][r];
+          else reinterpret_cast<float*>(C + 4 * at)[r] = acc[i][j][r];
+        }
     }
+  };
+  auto store_all = [&](auto bf16_tag, auto aligned_tag) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) store_one(i, j, bf16_tag, aligned_tag);
+  };
+  using Yes = std::true_type;
+  using No = std::false_type;
+  if constexpr (ASM_MFMA) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        if (n4) {
+          if (p.out_bf16) store_one(i, j, Yes{}, Yes{});
+          else store_one(i, j, No{}, Yes{});
+        } else {
+          if (p.out_bf16) store_one(i, j, Yes{}, No{});
+          else store_one(i, j, No{}, No{});
+        }
+      }
+  } else if (n4) {
+    if (p.out_bf16) store_all(Yes{}, Yes{});
+    else store_all(No{}, Yes{});
+  } else {
+    if (p.out_bf16) store_all(Yes{}, No{});
+    else store_all(No{}, No{});
   }
 }
 

@@ -59,6 +59,15 @@ ATTN_BF16_DIRECT_PAD(128, 64, 4, 2, _f32scale, true)
 ATTN_BF16_DIRECT_PAD(128, 64, 8, 1, _w8_f32scale, true)
 ATTN_BF16_DIRECT_PAD(64, 64, 4, 2, _f32scale, true)
 ATTN_BF16_DIRECT_PAD(64, 64, 8, 1, _w8_f32scale, true)
+// ... of which at most 96 columns are in use
+#define ATTN_BF16_DIRECT_PAD96(BN, NW, OCC, SUFFIX, PRECISE)                                                     \
+  extern "C" __global__ void __launch_bounds__(NW * 64, OCC) attn_fwd_bf16_d128_bn##BN##_direct##SUFFIX##_pad96(AttnParams p) { \
+    attn_fwd_bf16_direct_body<128, BN, NW, PRECISE, true, 1, 96>(p);                                              \
+  }
+ATTN_BF16_DIRECT_PAD96(64, 4, 2, , false)
+ATTN_BF16_DIRECT_PAD96(64, 8, 1, _w8, false)
+ATTN_BF16_DIRECT_PAD96(64, 4, 2, _f32scale, true)
+ATTN_BF16_DIRECT_PAD96(64, 8, 1, _w8_f32scale, true)
 // head sizes above 128 up to 256: one wave per SIMD (all its registers), 128 query rows per workgroup, 32-key tiles
 ATTN_BF16_DIRECT(256, 32, 4, 1, , false)
 ATTN_BF16_DIRECT_PAD(256, 32, 4, 1, , false)

@@ -241,7 +241,10 @@ Err launch_attention(const void* q, const void* k, const void* v, void* o, DType
     else name = dmax <= 32 ? "attn_fwd_f32_d32_bn32" : dmax <= 64 ? "attn_fwd_f32_d64_bn32" : "attn_fwd_f32_d128_bn32";
     bn = 32;
   }
-  if (note) *note = LaunchNote{splits > 1 ? name + " (keys in " + std::to_string(splits) + " parts)" : name, bm, bn};
+  // padded head sizes of which 96 columns cover d and dv: the form that computes no more (its report names it so)
+  const bool columns96 = in_dtype == BF16 && direct && padded && !wide && dmax > 64 && dmax <= 96;
+  if (note) *note = LaunchNote{name + (columns96 ? " (96 columns)" : "") + (splits > 1 ? " (keys in " + std::to_string(splits) + " parts)" : ""), bm, bn};
+  if (columns96) name += "96";
 
   const size_t grid = (size_t(p.bh) * p.nqt + 7) / 8 * 8;  // the query tiles of all heads in 8 equal runs, one per XCD
   if (grid > kMaxGrid) return "attention kernel: grid too large";
