@@ -426,9 +426,11 @@ unsigned gemm_nt_bf16_split_k(size_t bh, size_t m, size_t n, size_t k, const Ker
   if (k > (size_t(1) << 22)) return 1;
   const size_t slabs = (k + 63) / 64;
   const size_t t128 = ((m + 127) / 128) * ((n + 127) / 128) * bh, t256 = ((m + 255) / 256) * ((n + 255) / 256) * bh;
-  auto time_of = [](unsigned tile_, size_t workgroups, size_t slabs_) {
+  // (operands beyond the 32 MB of the L2s come from HBM, whose latency a CU's only workgroup waits for: 1.1 us then, too)
+  const bool far = bh * (m + n) * k * 2 > (size_t(32) << 20);
+  auto time_of = [far](unsigned tile_, size_t workgroups, size_t slabs_) {
     const double rounds = (double)((workgroups + (tile_ == 128 ? 511 : 255)) / (tile_ == 128 ? 512 : 256));
-    return rounds * (double)(slabs_ + 2) * (tile_ == 128 ? (workgroups <= 256 ? 0.7 : 1.1) : 1.3);
+    return rounds * (double)(slabs_ + 2) * (tile_ == 128 ? (workgroups <= 256 && !far ? 0.7 : 1.1) : 1.3);
   };
   double best = time_of(128, t128, slabs);
   if (t256 >= 64) best = std::min(best, time_of(256, t256, slabs));
