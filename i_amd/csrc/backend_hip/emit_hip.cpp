@@ -687,6 +687,18 @@ struct Printer {
     buffer_access(dst, &cap, &writeable, &ind);
     line(depth, "ilang_store(" + place(dst) + ", " + value + ", args.bf16_writes >> " + std::to_string(ind) + " & 1);");
   }
+  // A held element of a work-item-private buffer moves between its register and the strip's own array: the buffer
+  // behind it does not exist in this form.
+  void strip_private(const std::string& local, const MExpr& at, bool load, int depth) {
+    std::string cap;
+    bool writeable = false;
+    size_t ind = 0;
+    buffer_access(at, &cap, &writeable, &ind);
+    const std::string idx = expr_text(*at.args[1]), element = "strip" + std::to_string(ind) + "[" + idx + "]";
+    const std::string inside = "(" + idx + ") < " + cap;
+    if (load) line(depth, "Strip " + local + " = " + (g_checked_accesses ? inside + " ? " + element + " : Strip{};" : element + ";"));
+    else line(depth, (g_checked_accesses ? "if (" + inside + ") " : std::string()) + element + " = " + local + ";");
+  }
   void strip_accesses(const MExpr& e, const std::string& ident, std::vector<const MExpr*>& out) const {
     std::string cap;
     if (buffer_access(e, &cap) && !held_local(e) && mentions(*e.args[1], ident)) out.push_back(&e);
@@ -796,6 +808,7 @@ struct Printer {
                 if (acc.writeable == h.ind) fresh = &acc;
             if (!strip.empty()) {
               if (fresh) line(d, "Strip " + h.local + " = {{" + identity_text(fresh->op) + ", " + identity_text(fresh->op) + ", " + identity_text(fresh->op) + ", " + identity_text(fresh->op) + "}};");
+              else if (g_strip_privates.count(h.ind)) strip_private(h.local, *h.at, true, d);
               else line(d, "Strip " + h.local + " = ilang_load(" + place(*h.at) + ");");
             } else if (h.shared) {
               // the element as it is before the loop, and this lane's share of what the loop adds to it
@@ -840,7 +853,8 @@ struct Printer {
           for (const Held& h : mine) {
             std::string value = h.local;
             if (!strip.empty()) {
-              strip_store(*h.at, value, d);
+              if (g_strip_privates.count(h.ind)) strip_private(h.local, *h.at, false, d);
+              else strip_store(*h.at, value, d);
               continue;
             }
             if (h.shared) {

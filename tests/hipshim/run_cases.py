@@ -105,6 +105,17 @@ CASES = {
     "sum over the two last axes": (lambda: i("+bij~b"), [(3, 9, 70)]),
 }
 
+# nests with a fused temporary (a work-item-private buffer) in their strip forms: products summed without being stored,
+# over the rows and over the columns of the second operand, with innermost extents on either side of four, a strip that
+# straddles work-groups of 64, and enough elements (300 x 1000) for the strip form of a nest whose loop is whole
+for _n in (4, 64, 70, 72):
+    CASES[f"staged column sum 37x{_n}"] = (lambda: i("ij*i~ij||ji") >> i("+ij~j||ji0"), [(37, _n), (37,)])
+    CASES[f"staged column sum of exponentials 37x{_n}"] = (lambda: i("^ij~ij||ji") >> i("+ij~j||ji0"), [(37, _n)])
+    CASES[f"staged matmul 9x70x{_n}"] = (lambda: i("ik*kj~ikj||ijk") >> i("+ikj~ij||ijk0"), [(9, 70), (70, _n)])
+    CASES[f"staged matmul, k third 9x70x{_n}"] = (lambda: i("ik*kj~ijk||ijk") >> i("+ijk~ij||ijk0"), [(9, 70), (70, _n)])
+CASES["staged matmul 300x5x1000"] = (lambda: i("ik*kj~ijk||ijk") >> i("+ijk~ij||ijk0"), [(300, 5), (5, 1000)])
+STAGED_CASES = [name for name in CASES if name.startswith("staged ")]
+
 # the cases with a nest that has a wavefront-per-iteration form (reduction loops spread over 64 lanes)
 WAVE_CASES = ["naive attention ragged", "batched naive attention", "mm_t", "mm_t empty", "matmul unfused",
               "matmul fused init site", "row sum", "column max", "total", "fanout two outputs", "swapped fanout",
@@ -153,7 +164,7 @@ def main():
 
     noalloc = os.environ.get("ILANG_SHIM_NOALLOC") == "1"
     which = os.environ.get("ILANG_SHIM_CASES")
-    names = sys.argv[1:] or (WAVE_CASES if which == "wave" else SAMPLE_CASES if which == "sample" else list(CASES))
+    names = sys.argv[1:] or {"wave": WAVE_CASES, "sample": SAMPLE_CASES, "staged": STAGED_CASES}.get(which, list(CASES))
     tolerance = float(os.environ.get("ILANG_SHIM_TOLERANCE", "1e-5"))
     failed = []
     for name in names:

@@ -58,6 +58,18 @@ def test_reduction_nests_with_their_outer_loop_in_parts_match_too(shim_lib):
     run_cases(shim_lib, {"ILANG_SHIM_PARTS": "4", "ILANG_SHIM_ORDER": "reverse", "ILANG_SHIM_TOLERANCE": "1e-4"}, names=few)
 
 
+def test_strip_forms_with_fused_temporaries_match_too(shim_lib):
+    """A strip of four iterations keeps a fused temporary in a local array of its own, also where the loop being summed
+    over holds that temporary in a register: the buffer behind it does not exist (a null pointer, which faults here).
+    With the loop in the parts that the launcher picks, in three and whole; checked and unchecked; last to first."""
+    loose = {"ILANG_SHIM_TOLERANCE": "1e-4", "ILANG_SHIM_CASES": "staged"}
+    run_cases(shim_lib, loose)
+    run_cases(shim_lib, {**loose, "ILANG_HIP_UNCHECKED": "0"})
+    run_cases(shim_lib, {**loose, "ILANG_SHIM_PARTS": "3", "ILANG_HIP_UNCHECKED": "0"})
+    run_cases(shim_lib, {**loose, "ILANG_SHIM_PARTS": "1", "ILANG_HIP_UNCHECKED": "0"})
+    run_cases(shim_lib, {**loose, "ILANG_SHIM_ORDER": "reverse"})
+
+
 def test_generated_kernels_do_not_depend_on_work_item_order(shim_lib):
     """Work-items run last to first: a dependency between work-items would change the result."""
     run_cases(shim_lib, {"ILANG_SHIM_ORDER": "reverse", "ILANG_SHIM_CASES": "sample"})
