@@ -597,15 +597,19 @@ struct Printer {
   std::string strip;                            // the strip form: the loop of which a work-item runs four iterations
   size_t loaded = 0;                            // accesses loaded beforehand so far (their variables' numbers)
   int serial_depth = 0;                         // loops being printed as loops around the current statement
+  // accumulators whose registers start as the reduction's identity, not as what memory holds
+  const std::vector<GridAccumulator>* fresh = nullptr;
   // In the form with a loop in parts every part accumulates into copies of the accumulated buffers that the
   // launcher has filled with the reduction's identity: the nest's own initialisations of those buffers are dropped.
+  // So they are where the accumulators start fresh: the registers' stores are the only ones.
   bool dropped_initialisation(const MStmt& s) const {
-    if (!grid || s.kind != MStmt::Set || !s.value || s.value->kind != MExpr::Scalar) return false;
+    const std::vector<GridAccumulator>* accumulators = grid ? &grid->accumulators : fresh;
+    if (!accumulators || s.kind != MStmt::Set || !s.value || s.value->kind != MExpr::Scalar) return false;
     std::string cap;
     bool writeable = false;
     size_t ind = 0;
     if (!buffer_access(*s.dst, &cap, &writeable, &ind) || !writeable) return false;
-    for (const GridAccumulator& acc : grid->accumulators)
+    for (const GridAccumulator& acc : *accumulators)
       if (acc.writeable == ind) return true;
     return false;
   }
@@ -800,22 +804,23 @@ struct Printer {
           const int d = mine.empty() ? depth : depth + 1;
           if (!mine.empty()) line(depth, "{");
           for (const Held& h : mine) {
-            // (in the form with a loop in parts an accumulated element starts as the reduction's identity: what its
-            // copy holds is not read, so the copies need no filling when every accumulator is held this way)
-            const GridAccumulator* fresh = nullptr;
-            if (grid && grid->held_accumulators)
-              for (const GridAccumulator& acc : grid->accumulators)
-                if (acc.writeable == h.ind) fresh = &acc;
+            // (an accumulated element that starts as the reduction's identity: what memory holds is not read, so in the
+            // form with a loop in parts the copies need no filling when every accumulator is held this way)
+            const GridAccumulator* starts = nullptr;
+            if (fresh)
+              for (const GridAccumulator& acc : *fresh)
+                if (acc.writeable == h.ind) starts = &acc;
+            const std::string identity = starts ? identity_text(starts->op) : "";
             if (!strip.empty()) {
-              if (fresh) line(d, "Strip " + h.local + " = {{" + identity_text(fresh->op) + ", " + identity_text(fresh->op) + ", " + identity_text(fresh->op) + ", " + identity_text(fresh->op) + "}};");
+              if (starts) line(d, "Strip " + h.local + " = {{" + identity + ", " + identity + ", " + identity + ", " + identity + "}};");
               else if (g_strip_privates.count(h.ind)) strip_private(h.local, *h.at, true, d);
               else line(d, "Strip " + h.local + " = ilang_load(" + place(*h.at) + ");");
             } else if (h.shared) {
               // the element as it is before the loop, and this lane's share of what the loop adds to it
-              line(d, "const float before_" + h.local + " = " + (fresh ? std::string(identity_text(fresh->op)) : expr_text(*h.at)) + ";");
+              line(d, "const float before_" + h.local + " = " + (starts ? identity : expr_text(*h.at)) + ";");
               line(d, "float " + h.local + " = " + identity_text(h.op) + ";");
             } else {
-              line(d, "float " + h.local + " = " + (fresh ? std::string(identity_text(fresh->op)) : expr_text(*h.at)) + ";");
+              line(d, "float " + h.local + " = " + (starts ? identity : expr_text(*h.at)) + ";");
             }
           }
           for (const Held& h : mine) g_held[h.ind] = strip.empty() ? h.local : h.local + ".v[e]";
@@ -993,6 +998,8 @@ void grid_plan(const Block<Param>& body, const std::set<Param>& accumulating, co
   for (const auto& [w, op] : ops)
     phase.grid.held_accumulators = phase.grid.held_accumulators &&
                                    std::find(held_by_g->second.begin(), held_by_g->second.end(), w.ind) != held_by_g->second.end();
+  phase.grid.starts_fresh = phase.grid.held_accumulators;
+  for (const GridAccumulator& acc : phase.grid.accumulators) phase.grid.starts_fresh = phase.grid.starts_fresh && acc.init_here;
   // the wavefront form of the same: when the nest has one and G is its loop over (or around) the lanes
   for (const WaveLoop& wl : phase.wave_loops)
     if (wl.loop == g->id && !wl.accumulators.empty()) {
@@ -1242,6 +1249,7 @@ GenericModule emit_generic_hip(const ExecPlan& plan, const Module& module, const
       pr.held = &held;
       if (wave) pr.wave = &phase.wave_loops;
       if (in_parts) pr.grid = &phase.grid;
+      if (in_parts ? phase.grid.held_accumulators : strips && phase.grid.starts_fresh) pr.fresh = &phase.grid.accumulators;
       std::vector<std::string> iters;
       for (size_t id : phase.parallel_loops) iters.push_back("i" + std::to_string(id));
       if (strips) pr.strip = iters.back();

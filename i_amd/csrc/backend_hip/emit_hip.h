@@ -46,8 +46,10 @@ struct PrivateBuffer {
 //
 // A nest whose innermost parallel loop steps through every buffer it indexes by one element has strip forms,
 // <name>_v and <name>_gv: a work-item runs four consecutive iterations of that loop, so that what was four 4-byte
-// accesses is one of 16 bytes (8 in bf16).  (Where the loop's length is no multiple of four, the last strip overlaps the
-// one before it; that is left to nests that do not read what they write.)  The element-wise forms are bound by HBM and the plain ones by the number
+// accesses is one of 16 bytes (8 in bf16).  Where the loop's length is no multiple of four, the last strip overlaps the
+// one before it, and two work-items store the same elements: that is left to nests that read nothing of what they
+// write.  Sums that the nest starts itself are such nests, since their registers start as the reduction's identity
+// (GridForm::starts_fresh; started through memory, a sum could be read back by the neighbour and counted twice).  The element-wise forms are bound by HBM and the plain ones by the number
 // of accesses in flight: 16384 x 4096 f32 divided by its column sums 213 -> 172 us (the division alone 145 -> 89, 6
 // TB/s), a bias and a threshold 193 -> 102.  And every form that reads program inputs exists once more, <name>..._b, with
 // those inputs' elements in bf16, which would otherwise be widened into temporaries first (16384 x 4096
@@ -72,6 +74,7 @@ struct GridForm {
   bool loop_is_spread = false;          // ... and in it the same loop also runs over the lanes
   bool held_accumulators = false;       // every accumulated element lives in a register across the loop: the parts only
                                         // store into their copies, which therefore need not start as the identity
+  bool starts_fresh = false;            // ... and the nest initialises every one of them itself: nothing it writes is read
 };
 struct GenericPhase {
   std::string name;                       // f<k>

@@ -771,9 +771,8 @@ bool strips_usable(const Run& run, const GenericPhase& ph, const Step& dispatch,
   const bool in_parts = ph.grid.available && ph.grid.held_accumulators && run.knobs.generated_parts != 1;
   if (ph.sequential_loops && !in_parts && total < size_t(4) * 65536) return false;
   if (inner % 4 == 0) return true;
-  bool fresh = in_parts && ph.privates.empty();  // (sums that the nest starts itself: the same again, too)
-  for (const GridAccumulator& acc : ph.grid.accumulators) fresh = fresh && acc.init_here;
-  if (!(fresh && ph.grid.accumulators.size() == dispatch.writes.size()) &&
+  // (sums that the nest starts itself, in registers, are the same again in every strip form)
+  if (!(ph.grid.starts_fresh && ph.grid.accumulators.size() == dispatch.writes.size()) &&
       (ph.sequential_loops || ph.strip_direct_writes.size() != dispatch.writes.size()))
     return false;
   for (BufferRef w : dispatch.writes)

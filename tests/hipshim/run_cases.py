@@ -114,6 +114,12 @@ for _n in (4, 64, 70, 72):
     CASES[f"staged matmul 9x70x{_n}"] = (lambda: i("ik*kj~ikj||ijk") >> i("+ikj~ij||ijk0"), [(9, 70), (70, _n)])
     CASES[f"staged matmul, k third 9x70x{_n}"] = (lambda: i("ik*kj~ijk||ijk") >> i("+ijk~ij||ijk0"), [(9, 70), (70, _n)])
 CASES["staged matmul 300x5x1000"] = (lambda: i("ik*kj~ijk||ijk") >> i("+ijk~ij||ijk0"), [(300, 5), (5, 1000)])
+# sums over fewer rows than are dealt out in parts, of lengths whose last strip overlaps one of the work-group before
+for _op in "+*><":
+    CASES[f"short column reduction {_op} 20x257"] = (lambda op=_op: i(f"{op}ij~j"), [(20, 257)])
+CASES["short column reduction 31x515"] = (lambda: i("+ij~j"), [(31, 515)])
+CASES["short column reduction 5x3x255"] = (lambda: i("+bij~bj"), [(5, 3, 255)])
+SHORT_CASES = [name for name in CASES if name.startswith("short ")]
 STAGED_CASES = [name for name in CASES if name.startswith("staged ")]
 
 # the cases with a nest that has a wavefront-per-iteration form (reduction loops spread over 64 lanes)
@@ -164,7 +170,7 @@ def main():
 
     noalloc = os.environ.get("ILANG_SHIM_NOALLOC") == "1"
     which = os.environ.get("ILANG_SHIM_CASES")
-    names = sys.argv[1:] or {"wave": WAVE_CASES, "sample": SAMPLE_CASES, "staged": STAGED_CASES}.get(which, list(CASES))
+    names = sys.argv[1:] or {"wave": WAVE_CASES, "sample": SAMPLE_CASES, "staged": STAGED_CASES, "short": SHORT_CASES}.get(which, list(CASES))
     tolerance = float(os.environ.get("ILANG_SHIM_TOLERANCE", "1e-5"))
     failed = []
     for name in names:

@@ -70,6 +70,23 @@ def test_strip_forms_with_fused_temporaries_match_too(shim_lib):
     run_cases(shim_lib, {**loose, "ILANG_SHIM_ORDER": "reverse"})
 
 
+def test_overlapping_strips_of_sums_read_nothing_that_they_write(shim_lib):
+    """Two strips that share elements may sit in different work-groups: a sum that starts through memory could load what
+    the other one has already added up.  So the strip form of a sum that the nest starts itself holds no load of the
+    result, and no store but the one behind the loop."""
+    env = dict(os.environ, ILANG_NO_TORCH="1", ILANG_CORE_LIB=str(shim_lib))
+    for expression in ("+ij~j", "*ij~j", ">ij~j", "<ij~j", "+bij~bj"):
+        code = subprocess.run([sys.executable, "-c", f"from i_amd import Component as i\nprint(i('{expression}')._code())"], env=env,
+                              capture_output=True, text=True, cwd=ROOT, timeout=300).stdout
+        for form in ("f0_v(", "f0_v_b(", "f0_gv(", "f0_gv_b("):
+            start = code.index(form)
+            body = code[start:code.index('extern "C"', start)]
+            assert "ilang_load(writeables" not in body and body.count("ilang_store(") == 1, (expression, form)
+    run_cases(shim_lib, {"ILANG_SHIM_CASES": "short", "ILANG_HIP_UNCHECKED": "0"})
+    run_cases(shim_lib, {"ILANG_SHIM_CASES": "short", "ILANG_SHIM_ORDER": "reverse"})
+    run_cases(shim_lib, {"ILANG_SHIM_CASES": "short", "ILANG_SHIM_PARTS": "3", "ILANG_SHIM_TOLERANCE": "1e-4"})
+
+
 def test_generated_kernels_do_not_depend_on_work_item_order(shim_lib):
     """Work-items run last to first: a dependency between work-items would change the result."""
     run_cases(shim_lib, {"ILANG_SHIM_ORDER": "reverse", "ILANG_SHIM_CASES": "sample"})

@@ -45,6 +45,25 @@ def test_reductions_and_their_quotients(name, types):
             assert bool(t.isnan(out_buf[:off]).all()) and bool(t.isnan(out_buf[off + ref.numel():]).all()), what
 
 
+@pytest.mark.parametrize("src", ["f32", "bf16"])
+def test_sums_of_few_rows_whose_strips_overlap(src):
+    """Columns that are no multiple of four, too few rows for parts: neighbouring work-items, in other workgroups too,
+    store the same sums of the columns they share.  Whole numbers: every sum is exact."""
+    from i_amd import Component as i
+
+    dtype = {"f32": t.float32, "bf16": t.bfloat16}[src]
+    for expression, shapes in {"+ij~j": [(20, 257), (31, 515), (3, 5), (1, 1023), (20, 300001), (2, 1048579)],
+                               "+bij~bj": [(5, 3, 255), (7, 20, 1021), (300, 4, 1001)]}.items():
+        for shape in shapes:
+            x = t.randint(-8, 9, shape, device="cuda").to(dtype)
+            component = i(expression)
+            ref = x.double().sum(-2).float()
+            out = t.full_like(ref, float("nan"))
+            for _ in range(3):
+                component.into(out, x)
+                assert t.equal(out, ref), dict(src=src, shape=shape, report=component.report())
+
+
 @pytest.mark.parametrize("types", ["f32-f32", "bf16-f32", "bf16-bf16"])
 def test_elementwise_with_a_broadcast_operand_and_a_scalar(types):
     from i_amd import Component as i
