@@ -535,6 +535,33 @@ bool strip_body(const std::vector<MStmt>& stmts, const std::string& ident, const
   }
   return true;
 }
+// GenericPhase::same_element_reads
+std::vector<size_t> same_element_reads(const Block<Param>& body, const GenericPhase& phase) {
+  const Block<Param>* block = &body;
+  while (block->size() == 1 && (*block)[0].kind == PAct::Loop) block = &(*block)[0].body;
+  auto is_private = [&](const Param& w) {
+    for (const PrivateBuffer& pb : phase.privates)
+      if (pb.writeable == w.ind) return true;
+    return false;
+  };
+  for (size_t n = 0; n < block->size(); ++n)
+    if ((*block)[n].kind == PAct::Loop || is_private((*block)[n].write.buffer) != (n + 1 < block->size())) return {};
+  if (phase.sequential_loops || block->empty()) return {};
+  const Access<Param>& write = block->back().write;
+  Uses u;
+  collect(body, u);
+  std::map<size_t, bool> same;
+  for (const Access<Param>* a : u.all) {
+    if (a->buffer.writeable) continue;
+    bool& ok = same.emplace(a->buffer.ind, true).first->second;
+    ok = ok && a->index.size() == write.index.size();
+    for (size_t d = 0; ok && d < write.index.size(); ++d) ok = same_iter(a->index[d], write.index[d]);
+  }
+  std::vector<size_t> out;
+  for (const auto& [ind, ok] : same)
+    if (ok) out.push_back(ind);
+  return out;
+}
 // does a value read readonlys[ind] along `ident`?
 bool reads_along(const std::vector<MStmt>& stmts, size_t ind, const std::string& ident) {
   std::function<bool(const MExpr&)> in = [&](const MExpr& e) {
@@ -1178,10 +1205,11 @@ GenericModule emit_generic_hip(const ExecPlan& plan, const Module& module, const
     if (!phase.parallel_loops.empty() && small_privates) {
       const std::string inner = "i" + std::to_string(phase.parallel_loops.back());
       phase.strip = strip_body(stmts, inner, private_inds);
-      std::set<size_t> loops;
-      loop_ids(body, loops);
-      phase.sequential_loops = loops.size() > phase.parallel_loops.size();
     }
+    std::set<size_t> loops;
+    loop_ids(body, loops);
+    phase.sequential_loops = loops.size() > phase.parallel_loops.size();
+    phase.same_element_reads = same_element_reads(body, phase);
     // (a rank-0 input stays f32 in the bf16 forms: the launcher widens it)
     for (size_t b = 0; dispatch && b < dispatch->reads.size(); ++b) {
       const BufferRef r = dispatch->reads[b];

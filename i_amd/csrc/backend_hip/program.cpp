@@ -341,6 +341,39 @@ bool read_back(const Run& run, BufferRef out) {
   return false;
 }
 
+// Do an output and an input share memory (the caller passes one buffer, or a part of it, as both)?
+bool overlap(const Run& run, size_t output, size_t input) {
+  auto end = [](const void* data, size_t elements, DType t) { return static_cast<const char*>(data) + elements * (t == DType::BF16 ? 2 : 4); };
+  const DeviceTensor &out = run.outputs[output], &in = run.inputs[input];
+  return in.data < end(out.data, product(run.shape_of({BufferRef::Output, output})), out.dtype) &&
+         out.data < end(in.data, product(in.shape), in.dtype);
+}
+
+// May kernels read this bf16 input where it lies?  Not where an f32 output shares its memory: read through a copy that is
+// made once, it stays what it was while that output is written.
+bool read_in_place(const Run& run, size_t input) {
+  for (size_t o = 0; o < run.outputs.size(); ++o)
+    if (run.outputs[o].dtype == DType::F32 && overlap(run, o, input)) return false;
+  return true;
+}
+
+// May dispatch `at` of `plan` store this bf16 output itself, while the program runs, instead of through an f32 copy that
+// is rounded at the program's end?  Where an input shares the output's memory, only if no later dispatch reads that input
+// and this one, if it does, reads every element just where it writes it (same_element(n) says so of at.reads[n]).
+template <class F>
+bool store_in_place(const Run& run, const ExecPlan& plan, const Step& at, size_t output, F same_element) {
+  for (size_t i = 0; i < run.inputs.size() && i < plan.inputs.size(); ++i) {
+    if (!overlap(run, output, i)) continue;
+    auto is_it = [&](BufferRef r) { return r.kind == BufferRef::Input && r.id == i; };
+    for (const Step* s = &at + 1; s < plan.exec.data() + plan.exec.size(); ++s)
+      if (s->kind == Step::Dispatch && std::any_of(s->reads.begin(), s->reads.end(), is_it)) return false;
+    for (size_t n = 0; n < at.reads.size(); ++n)
+      if (is_it(at.reads[n]) && !(same_element(n) && run.inputs[i].dtype == DType::BF16 && run.inputs[i].data == run.outputs[output].data))
+        return false;
+  }
+  return true;
+}
+
 // An f32 product through the executor: with few output tiles under a long k loop, the loop in parts over
 // workgroups, the partial products in a temporary (no room for it: the unsplit kernel).
 // b_cols != 0: the right operand is row-major with rows of b_cols elements.
@@ -495,7 +528,7 @@ ihip::Err product_operands(Run& run, const Recognized& r, DType t, const void** 
   return {};
 }
 
-ihip::Err launch_hand_noted(Run& run, const Recognized& r, ihip::LaunchNote* note) {
+ihip::Err launch_hand_noted(Run& run, const Recognized& r, const Step& step, ihip::LaunchNote* note) {
   switch (r.kind) {
     case Recognized::Attention: {
       const auto q = run.shape_of(r.a.buffer), k = run.shape_of(r.b.buffer), v = run.shape_of(r.c.buffer);
@@ -656,13 +689,16 @@ ihip::Err launch_hand_noted(Run& run, const Recognized& r, ihip::LaunchNote* not
       // rows that fit the registers of a workgroup are read and written in their own types; longer bf16 rows are
       // widened into a temporary first, and rounded from one afterwards
       ihip::DType in_dt = ihip::F32, out_dt = ihip::F32;
-      if (run.dtype_of(r.a.buffer) == DType::BF16 && r.a.buffer.kind == BufferRef::Input && ihip::row_softmax_any_supported(x.back())) {
+      if (run.dtype_of(r.a.buffer) == DType::BF16 && r.a.buffer.kind == BufferRef::Input && ihip::row_softmax_any_supported(x.back()) &&
+          read_in_place(run, r.a.buffer.id)) {
         in = run.raw_ptr(r.a.buffer);
         in_dt = ihip::BF16;
       } else if (ihip::Err e = run.read_f32(r.a.buffer, &in); !e.empty()) {
         return e;
       }
-      if (run.dtype_of(r.out) == DType::BF16 && ihip::row_softmax_any_supported(x.back()) && !read_back(run, r.out)) {
+      // (a row's lanes have read all of it before they store any)
+      if (run.dtype_of(r.out) == DType::BF16 && ihip::row_softmax_any_supported(x.back()) && !read_back(run, r.out) &&
+          store_in_place(run, run.plan, step, r.out.id, [](size_t) { return true; })) {
         out = run.raw_ptr(r.out);
         out_dt = ihip::BF16;
       } else if (ihip::Err e = run.write_f32(r.out, &out); !e.empty()) {
@@ -680,9 +716,9 @@ ihip::Err launch_hand_noted(Run& run, const Recognized& r, ihip::LaunchNote* not
   }
 }
 
-ihip::Err launch_hand(Run& run, const Recognized& r) {
+ihip::Err launch_hand(Run& run, const Recognized& r, const Step& step) {
   ihip::LaunchNote note;
-  const ihip::Err err = launch_hand_noted(run, r, &note);
+  const ihip::Err err = launch_hand_noted(run, r, step, &note);
   if (err.empty()) run.notes.push_back(note.kernel.empty() ? "nothing to do (empty operands)" : describe_launch(note, r));
   return err;
 }
@@ -776,14 +812,8 @@ bool strips_usable(const Run& run, const GenericPhase& ph, const Step& dispatch,
       (ph.sequential_loops || ph.strip_direct_writes.size() != dispatch.writes.size()))
     return false;
   for (BufferRef w : dispatch.writes)
-    for (BufferRef r : dispatch.reads) {
-      if (w.kind != BufferRef::Output || r.kind != BufferRef::Input) continue;
-      const char* out = static_cast<const char*>(run.raw_ptr(w));
-      const char* in = static_cast<const char*>(run.raw_ptr(r));
-      const size_t out_bytes = product(run.layout_of(w)) * (run.dtype_of(w) == DType::BF16 ? 2 : 4);
-      const size_t in_bytes = product(run.layout_of(r)) * (run.dtype_of(r) == DType::BF16 ? 2 : 4);
-      if (in < out + out_bytes && out < in + in_bytes) return false;
-    }
+    for (BufferRef r : dispatch.reads)
+      if (w.kind == BufferRef::Output && r.kind == BufferRef::Input && overlap(run, w.id, r.id)) return false;
   return true;
 }
 
@@ -807,7 +837,8 @@ ihip::Err launch_generic(Run& run, size_t k, const Step& dispatch) {
   };
   // inputs that are all bf16 (rank 0 aside) are read as they are, by the _b forms
   bool bf16_inputs = !ph.bf16_reads.empty();
-  for (size_t i : ph.bf16_reads) bf16_inputs = bf16_inputs && run.dtype_of(dispatch.reads[i]) == DType::BF16;
+  for (size_t i : ph.bf16_reads)
+    bf16_inputs = bf16_inputs && run.dtype_of(dispatch.reads[i]) == DType::BF16 && read_in_place(run, dispatch.reads[i].id);
   for (size_t i = 0; i < dispatch.reads.size(); ++i) {
     void* ptr = nullptr;
     if (bf16_inputs && std::find(ph.bf16_reads.begin(), ph.bf16_reads.end(), i) != ph.bf16_reads.end()) ptr = run.raw_ptr(dispatch.reads[i]);
@@ -839,8 +870,10 @@ ihip::Err launch_generic(Run& run, size_t k, const Step& dispatch) {
   std::vector<void*> write_ptrs(dispatch.writes.size(), nullptr);
   for (size_t i = 0; i < dispatch.writes.size(); ++i) {
     const BufferRef w = dispatch.writes[i];
+    auto same_element = [&](size_t r) { return std::find(ph.same_element_reads.begin(), ph.same_element_reads.end(), r) != ph.same_element_reads.end(); };
     if (strips && run.dtype_of(w) == DType::BF16 && written_once(run, w) &&
-        std::find(ph.strip_direct_writes.begin(), ph.strip_direct_writes.end(), i) != ph.strip_direct_writes.end()) {
+        std::find(ph.strip_direct_writes.begin(), ph.strip_direct_writes.end(), i) != ph.strip_direct_writes.end() &&
+        store_in_place(run, run.p.nest_plan, dispatch, w.id, same_element)) {
       write_ptrs[i] = run.raw_ptr(w);
       bf16_writes |= size_t(1) << i;
     } else if (!gk.is_private(i)) {
@@ -1290,7 +1323,7 @@ std::string execute(Program& p, const std::vector<DeviceTensor>& inputs, const s
     } else if (step.kind == Step::Dispatch) {
       ihip::Err e;
       if (hand[step.id]) {
-        e = launch_hand(run, p.recognized[step.id]);
+        e = launch_hand(run, p.recognized[step.id], step);
       } else {
         // the generated form: the kernel's loop nests one after the other, each a kernel of its own (one line of the report)
         std::string lines;
