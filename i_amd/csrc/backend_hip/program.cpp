@@ -349,6 +349,11 @@ bool overlap(const Run& run, size_t output, size_t input) {
          out.data < end(in.data, product(in.shape), in.dtype);
 }
 
+// The same for a product's result and an operand read at `ptr` (an intermediate or a copy shares nothing).
+bool result_over(const Run& run, BufferRef out, BufferRef in, const void* ptr) {
+  return out.kind == BufferRef::Output && in.kind == BufferRef::Input && ptr == run.raw_ptr(in) && overlap(run, out.id, in.id);
+}
+
 // May kernels read this bf16 input where it lies?  Not where an f32 output shares its memory: read through a copy that is
 // made once, it stays what it was while that output is written.
 bool read_in_place(const Run& run, size_t input) {
@@ -462,7 +467,7 @@ ihip::Err attention_in_parts(Run& run, const Recognized& r, bool bf16, size_t bh
           !e.empty())
         return e;
     }
-  } else if (dv % 4 == 0 && dv <= (size_t(1) << 24)) {
+  } else if (dv % 4 == 0 && dv <= (size_t(1) << 24) && !result_over(run, r.out, r.c.buffer, v)) {
     if (ihip::Err e = launch_product_f32(run, s, v, out, bh, nq, dv, nk, &last, dv); !e.empty()) return e;
   } else {
     void* vt = nullptr;
@@ -654,11 +659,13 @@ ihip::Err launch_hand_noted(Run& run, const Recognized& r, const Step& step, ihi
       const bool tile_asked = (r.tile_i == 128 && r.tile_j == 128) || (r.tile_i == 256 && r.tile_j == 256);
       const bool aligned = reinterpret_cast<uintptr_t>(pa) % 16 == 0 && reinterpret_cast<uintptr_t>(pb_rows) % 16 == 0;
       const ihip::DType kernel_t = f32 ? ihip::F32 : ihip::BF16;
-      if (aligned && !tile_asked && ihip::gemm_narrow_usable(kernel_t, true, bh, m, n, k, run.knobs))
+      // (an f32 result in the memory of B: the kernels that read B as it is would read it while they write)
+      const bool over_b = f32 && result_over(run, r.out, r.b.buffer, pb_rows);
+      if (aligned && !tile_asked && !over_b && ihip::gemm_narrow_usable(kernel_t, true, bh, m, n, k, run.knobs))
         return launch_product_narrow(run, pa, pb_rows, out, kernel_t, true, bh, m, n, k, note, out_dt);
       const DType t = f32 ? DType::F32 : DType::BF16;
       size_t kp = k;
-      if (padded_nn_usable(run, t, bh, m, n, k)) {  // the direct kernels read a row-major right operand themselves
+      if (!over_b && padded_nn_usable(run, t, bh, m, n, k)) {  // the direct kernels read a row-major right operand themselves
         const void* pb = pb_rows;
         size_t b_cols = n;
         if (ihip::Err e = padded_operands(run, t, true, bh, &pa, m, &pb, n, &kp, &b_cols); !e.empty()) return e;

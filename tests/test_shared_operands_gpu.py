@@ -73,3 +73,32 @@ def test_bf16_rows_over_themselves_and_over_other_rows(cols, shift):
     component = _softmax()
     component.into(out, x)
     assert bool(((out - ref).abs() <= ref * ((cols + 32) * 2.0 ** -24 + 2.0 ** -8)).all()), component.report()
+
+
+@pytest.mark.parametrize("m, n, k", [(96, 100, 96), (600, 512, 600), (16, 1000, 512), (50, 4096, 1024)])
+def test_an_f32_product_over_its_row_major_right_operand(m, n, k):
+    i, _ = _i()
+    component = i("ik*kj~ijk | i:16,j:16 | jii'j'k") >> i("+ijk~ij | i:16,j:16 | jii'j'k0")
+    a = t.randint(-4, 5, (m, k), device="cuda").float()
+    b = t.randint(-4, 5, (k, n), device="cuda").float()
+    ref = (a.double() @ b.double()).float()
+    out = b.view(-1)[:m * n].view(m, n)
+    component.into(out, a, b)
+    assert t.equal(out, ref), component.report()
+
+
+def test_an_f32_attention_of_large_heads_over_its_values():
+    i, I = _i()
+    s = "i:16,j:16"
+    n, d = 700, 132
+    mm_t = i(f"ik*jk~ijk | {s} | jii'j'k") >> i(f"+ijk~ij | {s} | jii'j'k0")
+    row_max_shift = (I & i(f">ij~i | {s} | ji0i'j'")) >> i(f"ij-i~ij | {s} | ji01i'j'")
+    exp = i(f"^ij~ij | {s} | ji0i'j'")
+    row_normalize = (I & i(f"+ij~i | {s} | ji0i'j'")) >> i(f"ij/i~ij | {s} | ji01i'j'")
+    mm = i(f"ij*jk~ikj | {s} | ji0i'kj'") >> i(f"+ikj~ik | {s} | jii'kj'0")
+    component = mm_t >> row_max_shift >> exp >> row_normalize >> mm
+    q, k, v = ((t.rand(n, d, device="cuda") - 0.5) for _ in range(3))
+    ref = t.softmax(q.double() @ k.double().t(), 1) @ v.double()
+    component.into(v, q, k, v)
+    # scores up to 3 in f32 products of 132 terms, probabilities within as much, averages of values up to 1/2
+    assert float((v - ref).abs().max()) <= (132 + 700 + 32) * 2.0 ** -24, component.report()
