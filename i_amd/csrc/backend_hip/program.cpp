@@ -479,43 +479,71 @@ ihip::Err attention_in_parts(Run& run, const Recognized& r, bool bf16, size_t bh
   return {};
 }
 
-// The two operands of a product as the matrix-instruction kernels can read them: untouched when the extents are
-// multiples of their quantum and both are 16-byte aligned, otherwise copied, in one launch, into temporaries padded with
-// zeros.  a is [bh, m, k]; b is [bh, n, k], or [bh, k, n] (nn).  *k becomes the padded extent, *b_cols (nn) that of n.
+// Which operands of a product the matrix-instruction kernels cannot read as they are, and the padded extents: k and,
+// where b is row-major (nn), n rounded up to the kernels' quantum.  Zeros past k are needed on both sides (beside them
+// may lie anything); of a row-major b alone when only n is ragged.
+struct Padding {
+  size_t k, n;
+  bool a, b;
+};
+Padding padding_of(DType t, bool nn, const void* a, const void* b, size_t n, size_t k) {
+  const size_t q = product_k_quantum(t);
+  Padding p{(k + q - 1) / q * q, nn ? (n + q - 1) / q * q : n, false, false};
+  const bool off_a = reinterpret_cast<uintptr_t>(a) % 16 != 0, off_b = reinterpret_cast<uintptr_t>(b) % 16 != 0;
+  p.a = p.k != k || off_a || (!nn && off_b);
+  p.b = p.k != k || off_b || p.n != n || (!nn && off_a);
+  return p;
+}
+
+// The two operands of a product as those kernels can read them: untouched, or copied, in one launch, into temporaries
+// padded with zeros.  a is [bh, m, k]; b is [bh, n, k], or [bh, k, n] (nn).  *k becomes the padded extent, *b_cols (nn) that of n.
 ihip::Err padded_operands(Run& run, DType t, bool nn, size_t bh, const void** a, size_t m, const void** b, size_t n, size_t* k, size_t* b_cols) {
-  const size_t q = product_k_quantum(t), kp = (*k + q - 1) / q * q, np = (n + q - 1) / q * q, elem = t == DType::BF16 ? 2 : 4;
-  const bool misaligned = reinterpret_cast<uintptr_t>(*a) % 16 != 0 || reinterpret_cast<uintptr_t>(*b) % 16 != 0;
-  if (b_cols) *b_cols = nn ? n : 0;
-  if (kp == *k && !misaligned && (!nn || np == n)) return {};
-  void *ta = nullptr, *tb = nullptr;
-  const size_t bytes_a = bh * m * kp * elem, bytes_b = bh * (nn ? kp * np : n * kp) * elem;
-  if (ihip::Err e = run.alloc(&ta, std::max<size_t>(bytes_a, 16)); !e.empty()) return e;
-  if (ihip::Err e = run.alloc(&tb, std::max<size_t>(bytes_b, 16)); !e.empty()) return e;
-  if (bytes_a != 0 && bytes_b != 0) {
-    if (std::max(bytes_a, bytes_b) / 16 < (size_t(1) << 31)) {
-      const ihip::PadPair pair{{*a, *b}, {ta, tb}, {m, nn ? *k : n}, {m, nn ? kp : n}, {*k, nn ? n : *k}, {kp, nn ? np : kp}};
-      if (ihip::Err e = ihip::launch_pad_pair(pair, bh, elem, run.stream); !e.empty()) return e;
-    } else if (!nn) {
-      if (ihip::Err e = ihip::launch_pad_rows(*a, ta, bh * m, *k, kp, elem, run.stream); !e.empty()) return e;
-      if (ihip::Err e = ihip::launch_pad_rows(*b, tb, bh * n, *k, kp, elem, run.stream); !e.empty()) return e;
-    } else {
-      return "operands too large to be padded";  // (padded_nn_usable has kept such a call away)
-    }
+  const Padding pad = padding_of(t, nn, *a, *b, n, *k);
+  const size_t elem = t == DType::BF16 ? 2 : 4;
+  if (b_cols) *b_cols = nn ? pad.n : 0;
+  ihip::PadPair pair{};
+  unsigned count = 0;
+  auto copy = [&](const void** operand, size_t rows, size_t rows_padded, size_t cols, size_t cols_padded) -> ihip::Err {
+    void* to = nullptr;
+    if (ihip::Err e = run.alloc(&to, std::max<size_t>(bh * rows_padded * cols_padded * elem, 16)); !e.empty()) return e;
+    const unsigned o = count;
+    pair.src[o] = *operand;
+    pair.dst[o] = to;
+    pair.rows[o] = rows;
+    pair.rows_padded[o] = rows_padded;
+    pair.cols[o] = cols;
+    pair.cols_padded[o] = cols_padded;
+    *operand = to;
+    ++count;
+    return {};
+  };
+  if (pad.a)
+    if (ihip::Err e = copy(a, m, m, *k, pad.k); !e.empty()) return e;
+  if (pad.b)
+    if (ihip::Err e = nn ? copy(b, *k, pad.k, n, pad.n) : copy(b, n, n, *k, pad.k); !e.empty()) return e;
+  *k = pad.k;
+  size_t least = SIZE_MAX, most = 0;
+  for (unsigned o = 0; o < count; ++o) {
+    const size_t bytes = bh * pair.rows_padded[o] * pair.cols_padded[o] * elem;
+    least = std::min(least, bytes);
+    most = std::max(most, bytes);
   }
-  *a = ta;
-  *b = tb;
-  *k = kp;
-  if (b_cols) *b_cols = nn ? np : 0;
+  if (count == 0 || least == 0) return {};
+  if (most / 16 < (size_t(1) << 31)) return ihip::launch_pad_pair(pair, count, bh, elem, run.stream);
+  if (nn) return "operands too large to be padded";  // (padded_nn_usable has kept such a call away)
+  for (unsigned o = 0; o < count; ++o)
+    if (ihip::Err e = ihip::launch_pad_rows(pair.src[o], pair.dst[o], bh * pair.rows[o], pair.cols[o], pair.cols_padded[o], elem, run.stream); !e.empty()) return e;
   return {};
 }
 
 // May a product with a row-major right operand run on the kernels that read it as it is, after padding if need be?
-bool padded_nn_usable(const Run& run, DType t, size_t bh, size_t m, size_t n, size_t k) {
-  const size_t q = product_k_quantum(t), kp = (k + q - 1) / q * q, np = (n + q - 1) / q * q;
-  if (bh == 0 || m == 0 || n == 0 || k == 0 || bh > 65535 || np > (size_t(1) << 24)) return false;
-  if (bh * std::max(m, np) * kp >= (size_t(1) << 33)) return false;
-  if (t == DType::F32) return ihip::gemm_nt_f32_supported(kp);
-  return ihip::gemm_nn_bf16_supported(bh, m, np, kp, run.knobs);
+// (The padding copies at most 2^31 chunks of 16 bytes; beyond that a row-major operand is transposed, as beyond the kernels' offsets.)
+bool padded_nn_usable(const Run& run, DType t, const void* a, const void* b, size_t bh, size_t m, size_t n, size_t k) {
+  const Padding pad = padding_of(t, true, a, b, n, k);
+  if (bh == 0 || m == 0 || n == 0 || k == 0 || bh > 65535 || pad.n > (size_t(1) << 24)) return false;
+  if (bh * std::max(m, pad.n) * pad.k >= (size_t(1) << 33)) return false;
+  if (t == DType::F32) return ihip::gemm_nt_f32_supported(pad.k);
+  return ihip::gemm_nn_bf16_supported(bh, m, pad.n, pad.k, run.knobs);
 }
 
 // The operands of a product in its arithmetic type: as they are, or widened to f32 where the other one is f32.
@@ -665,7 +693,7 @@ ihip::Err launch_hand_noted(Run& run, const Recognized& r, const Step& step, ihi
         return launch_product_narrow(run, pa, pb_rows, out, kernel_t, true, bh, m, n, k, note, out_dt);
       const DType t = f32 ? DType::F32 : DType::BF16;
       size_t kp = k;
-      if (!over_b && padded_nn_usable(run, t, bh, m, n, k)) {  // the direct kernels read a row-major right operand themselves
+      if (!over_b && padded_nn_usable(run, t, pa, pb_rows, bh, m, n, k)) {  // the direct kernels read a row-major right operand themselves
         const void* pb = pb_rows;
         size_t b_cols = n;
         if (ihip::Err e = padded_operands(run, t, true, bh, &pa, m, &pb, n, &kp, &b_cols); !e.empty()) return e;

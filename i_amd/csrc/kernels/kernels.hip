@@ -357,7 +357,7 @@ __device__ __forceinline__ void pad_rows_body(const PadParams& p) {
     dst[at] = c < p.cols ? src[r * p.cols + c] : T(0);
   }
 }
-// Two operands padded in one launch (blockIdx.y says which): a work-item writes 16 bytes of the copy and reads the
+// One operand or two padded in one launch (blockIdx.y says which): a work-item writes 16 bytes of the copy and reads the
 // elements they come from in one access on the alignment of the elements, or one by one at the end of a row.  2047 x 777
 // and 777 x 3001 bf16 take 8 us together, where pad_rows, an element per work-item, took 7 and 8 in a launch each, after a
 // transpose of 9.

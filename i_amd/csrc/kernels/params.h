@@ -102,7 +102,7 @@ struct PadParams {
   uint32_t cols, cols_padded;
 };
 
-// Two operands at once, each batches x [rows, cols] copied into batches x [rows_padded, cols_padded], zeros beyond; dst
+// One operand or two at once, each batches x [rows, cols] copied into batches x [rows_padded, cols_padded], zeros beyond; dst
 // 16-byte aligned, cols_padded a multiple of 16 bytes, src at any alignment of its elements
 struct PadPairParams {
   const void* src[2];

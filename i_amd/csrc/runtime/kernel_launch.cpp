@@ -866,12 +866,13 @@ Err launch_pad_rows(const void* src, void* dst, size_t rows, size_t cols, size_t
   return launch(fn, (unsigned)grid, 1, 1, 256, &p, sizeof(p), stream);
 }
 
-Err launch_pad_pair(const PadPair& pair, size_t batches, size_t elem_bytes, hipStream_t stream) {
+Err launch_pad_pair(const PadPair& pair, unsigned count, size_t batches, size_t elem_bytes, hipStream_t stream) {
+  if (count < 1 || count > 2) return "pad kernel: one operand or two";
   if (elem_bytes != 2 && elem_bytes != 4) return "pad kernel: element size must be 2 or 4 bytes";
   PadPairParams p{};
   p.batches = (uint32_t)batches;
   size_t most = 0;
-  for (int o = 0; o < 2; ++o) {
+  for (unsigned o = 0; o < count; ++o) {
     if (pair.cols[o] > pair.cols_padded[o] || pair.rows[o] > pair.rows_padded[o] || pair.cols_padded[o] * elem_bytes % 16 != 0) return "pad kernel: bad extents";
     const size_t chunks = batches * pair.rows_padded[o] * (pair.cols_padded[o] * elem_bytes / 16);
     if (chunks == 0) return "pad kernel: bad extents";
@@ -890,7 +891,7 @@ Err launch_pad_pair(const PadPair& pair, size_t batches, size_t elem_bytes, hipS
   if (Err e = builtin_function(elem_bytes == 2 ? "pad_pair_b16" : "pad_pair_b32", &fn); !e.empty()) return e;
   // (index arithmetic in 32 bits: at most 2^31 chunks and 2^24 work-items past them)
   const size_t grid = std::min<size_t>((most + 255) / 256, 65536);
-  return launch(fn, (unsigned)grid, 2, 1, 256, &p, sizeof(p), stream);
+  return launch(fn, (unsigned)grid, count, 1, 256, &p, sizeof(p), stream);
 }
 
 }  // namespace ihip

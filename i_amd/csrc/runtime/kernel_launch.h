@@ -143,13 +143,13 @@ Err launch_convert(const void* src, void* dst, DType from, DType to, size_t n, h
 Err launch_pad_rows(const void* src, void* dst, size_t rows, size_t cols, size_t cols_padded, size_t elem_bytes,
                     hipStream_t stream);
 
-// Two operands, batches x [rows, cols] each, copied into zero-padded batches x [rows_padded, cols_padded] in one launch;
+// One operand or two (count), batches x [rows, cols] each, copied into zero-padded batches x [rows_padded, cols_padded] in one launch;
 // rows of the copies are multiples of 16 bytes and the copies 16-byte aligned, src at any alignment of its elements.
 struct PadPair {
   const void* src[2];
   void* dst[2];
   size_t rows[2], rows_padded[2], cols[2], cols_padded[2];
 };
-Err launch_pad_pair(const PadPair& pair, size_t batches, size_t elem_bytes, hipStream_t stream);
+Err launch_pad_pair(const PadPair& pair, unsigned count, size_t batches, size_t elem_bytes, hipStream_t stream);
 
 }  // namespace ihip

@@ -76,3 +76,16 @@ def test_batched_row_major_right_operands_of_odd_extents():
             component.into(c, x, y)
             ref = t.stack([x[s].double() @ y[s].double() for s in range(b)]).float()
             assert t.equal(c, ref), dict(dtype=dtype, b=b, m=m, n=n, k=k, report=component.report())
+
+
+def test_only_the_operand_that_needs_padding_is_copied():
+    """n alone is ragged: the right operand is copied, the left one, larger than the fixed workspace, is read as it is."""
+    component = _component(True)
+    for dtype, m, n, k in [(t.bfloat16, 8192, 1001, 8192), (t.float32, 8192, 333, 4096)]:
+        a = t.randint(-4, 5, (m, k), device="cuda").to(dtype)
+        b = t.randint(-4, 5, (k, n), device="cuda").to(dtype)
+        c = t.full((m, n), float("nan"), device="cuda")
+        component.into(c, a, b, static_workspace=True)
+        rows = t.arange(0, m, 37, device="cuda")
+        assert t.equal(c[rows], (a[rows].double() @ b.double()).float()), component.report()
+        assert not bool(t.isnan(c).any())
