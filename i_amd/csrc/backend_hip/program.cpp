@@ -541,7 +541,7 @@ ihip::Err padded_operands(Run& run, DType t, bool nn, size_t bh, const void** a,
 bool padded_nn_usable(const Run& run, DType t, const void* a, const void* b, size_t bh, size_t m, size_t n, size_t k) {
   const Padding pad = padding_of(t, true, a, b, n, k);
   if (bh == 0 || m == 0 || n == 0 || k == 0 || bh > 65535 || pad.n > (size_t(1) << 24)) return false;
-  if (bh * std::max(m, pad.n) * pad.k >= (size_t(1) << 33)) return false;
+  if (bh * std::max(pad.a ? m : 0, pad.b ? pad.n : 0) * pad.k >= (size_t(1) << 33)) return false;
   if (t == DType::F32) return ihip::gemm_nt_f32_supported(pad.k);
   return ihip::gemm_nn_bf16_supported(bh, m, pad.n, pad.k, run.knobs);
 }

@@ -89,3 +89,13 @@ def test_only_the_operand_that_needs_padding_is_copied():
         rows = t.arange(0, m, 37, device="cuda")
         assert t.equal(c[rows], (a[rows].double() @ b.double()).float()), component.report()
         assert not bool(t.isnan(c).any())
+
+
+def test_a_row_major_operand_of_more_elements_than_padding_can_copy_is_read_as_it_is():
+    component = _component(True)
+    m, n, k = 8, 16384, 1 << 19  # 2^33 elements
+    a = t.randint(-4, 5, (m, k), device="cuda").bfloat16()
+    b = t.ones(k, n, device="cuda", dtype=t.bfloat16)
+    c = t.full((m, n), float("nan"), device="cuda")
+    component.into(c, a, b, static_workspace=True)
+    assert t.equal(c, a.double().sum(1).float()[:, None].expand(m, n)), component.report()
