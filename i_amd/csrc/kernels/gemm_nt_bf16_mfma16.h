@@ -319,8 +319,9 @@ __device__ __forceinline__ void gemm_nt_mfma16_tile(const GemmParams& p, char* s
   // last, partial four go one by one (2047 x 3001 x 777, f32 result: 31 -> 22 us).
   // One loop per kind of store, chosen once, where a workgroup's tile is small: with the choice inside, the code that is
   // stepped over between the stores cost a product of few tiles half a microsecond (3352 x 184 x 1280: 17.5 against
-  // 16.4 us).  The 256-accumulator forms keep the choice inside, which spaces their stores: 4096^3 takes 114 us so and
-  // 117 in one loop per kind.
+  // 16.4 us).  The 256-accumulator forms keep the choice inside on whole tiles, which spaces their stores: 4096^3 takes 114
+  // us so and 117 in one loop per kind; on tiles at the edges one loop per kind is the faster one there too (row-major right
+  // operand: 64 x 16 x 2128 x 304 52.8 -> 45.1, 5000 x 5000 x 520 53.4 -> 49.1, 2584 x 3800 x 112 18.9 -> 15.8).
   typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
   typedef __bf16 bf16x4_any __attribute__((ext_vector_type(4), aligned(2)));
   const bool n4 = p.n % 4 == 0 && reinterpret_cast<uintptr_t>(C) % 16 == 0;
@@ -357,7 +358,7 @@ __device__ __forceinline__ void gemm_nt_mfma16_tile(const GemmParams& p, char* s
   };
   using Yes = std::true_type;
   using No = std::false_type;
-  if constexpr (ASM_MFMA) {
+  if constexpr (ASM_MFMA && !EDGE) {
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
