@@ -860,7 +860,9 @@ struct Printer {
           // part p takes a run of consecutive iterations of this loop (consecutive rows stay within a page)
           const bool in_parts = grid && grid->loop == loop_id;
           if (in_parts) {
-            line(d, "const size_t share_" + s.ident + " = (" + expr_text(*s.value) + " + parts - 1) / parts;");
+            // (strips, whose loop has eight loads of 16 bytes in flight: shares of whole rounds of eight)
+            const std::string share = "(" + expr_text(*s.value) + " + parts - 1) / parts";
+            line(d, "const size_t share_" + s.ident + " = " + (strip.empty() ? share : "(" + share + " + 7) / 8 * 8") + ";");
             line(d, "const size_t end_" + s.ident + " = (part + 1) * share_" + s.ident + " < " + expr_text(*s.value) + " ? (part + 1) * share_" +
                         s.ident + " : " + expr_text(*s.value) + ";");
           }

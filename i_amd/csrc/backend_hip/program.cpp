@@ -797,17 +797,26 @@ size_t generated_parts(const ihip::KernelOptions& knobs, const GridForm& grid, b
   if (knobs.generated_parts > 1) {
     parts = (size_t)knobs.generated_parts;
   } else {
-    // (strips have four times the bytes in flight: column sums of 5042 x 2561 24 us with 131072 work-items, 22 with
-    // 82048; of 16384 x 4096 58 with 131072, 55 with 65536)
     const size_t target = wave ? 4096 : strips ? 98304 : 262144;  // wavefronts / work-items that fill the chip
     if (total * 2 > target) return 1;
-    parts = std::min<size_t>(target / total, reduced / least);
+    // (strips have four times the bytes in flight, and three wavefronts of them per CU read fastest: with 49152 and 98304
+    // work-items, and in the form without strips, column sums of 16384 x 4096 take 46.3, 49.0 and 46.4 us, of 4096 x 4096
+    // 18.9, 20.5 and 19.4, of 65536 x 1024 51.4, 54.2 and 52.1, of 5042 x 2561 18.2, 20.7 and 22.1; short loops are bound by
+    // their rounds of loads instead, 64 batches of 64 x 1024 10.7 us in 4 parts, 11.6 in 3)
+    parts = std::min<size_t>(strips && reduced > 256 ? std::max<size_t>(49152 / total, 2) : target / total, reduced / least);
   }
   // (at most 4096 parts; 2048 of wavefronts when left to this rule: the pass over the parts of a sum to one element
   // is one wavefront's work and grows with their number, 4096^2 to one element 29.7 us in 4096 parts, 23.8 in 2048)
   parts = std::min<size_t>(std::min<size_t>(parts, wave && knobs.generated_parts <= 1 ? 2048 : 4096), std::max<size_t>(reduced, 1));
   if (parts >= 256) parts = parts / 32 * 32;
   else if (parts >= 16) parts = parts / 8 * 8;
+  if (strips && knobs.generated_parts <= 1 && parts >= 2) {
+    // (their shares are multiples of eight iterations, whole rounds of the loads in flight: no more parts than that leaves;
+    // 100000 x 64 30.6 -> 24.1 us, 4096 x 1024 13.9 -> 12.7)
+    const size_t share = (reduced + parts - 1) / parts, needed = (reduced + (share + 7) / 8 * 8 - 1) / ((share + 7) / 8 * 8);
+    const size_t step = needed >= 256 ? 32 : needed >= 16 ? 8 : 1;
+    parts = std::min(parts, (needed + step - 1) / step * step);
+  }
   return parts < 2 ? 1 : parts;
 }
 
@@ -823,24 +832,25 @@ bool written_once(const Run& run, BufferRef out) {
   return out.kind == BufferRef::Output && writers == 1;
 }
 
-// May the nest run in strips of four iterations of its innermost loop, and should it?  Every buffer accessed that way
-// needs four elements.  A length that is no multiple of four makes strips overlap: fine as long as the nest computes
+// May the nest run in strips of four iterations of its innermost loop?  Every buffer accessed that way needs four
+// elements.  A length that is no multiple of four makes strips overlap: fine as long as the nest computes
 // the same again, i.e. reads nothing that it writes, neither by name nor because the caller passes one memory as input
-// and output.  Nests without sequential loops and those with their loop in parts are bound by memory and always
-// gain; a nest that loops in its work-items needs enough of them left.
-bool strips_usable(const Run& run, const GenericPhase& ph, const Step& dispatch, size_t total, size_t inner) {
-  if (!ph.strip || inner < 4) return false;
+// and output.
+bool strips_usable(const Run& run, const GenericPhase& ph, const Step& dispatch, size_t inner) {
+  auto elements = [&](BufferRef r) {
+    size_t n = 1;
+    for (const auto& e : plan_buffer(run.plan, r).layout) n *= run.extent(e);
+    return n;
+  };
   for (size_t r : ph.strip_reads)
-    if (product(run.layout_of(dispatch.reads[r])) < 4) return false;
+    if (elements(dispatch.reads[r]) < 4) return false;
   auto is_private = [&](size_t w) {
     for (const PrivateBuffer& pb : ph.privates)
       if (pb.writeable == w) return true;
     return false;
   };
   for (size_t w = 0; w < dispatch.writes.size(); ++w)
-    if (!is_private(w) && product(run.layout_of(dispatch.writes[w])) < 4) return false;
-  const bool in_parts = ph.grid.available && ph.grid.held_accumulators && run.knobs.generated_parts != 1;
-  if (ph.sequential_loops && !in_parts && total < size_t(4) * 65536) return false;
+    if (!is_private(w) && elements(dispatch.writes[w]) < 4) return false;
   if (inner % 4 == 0) return true;
   // (sums that the nest starts itself, in registers, are the same again in every strip form)
   if (!(ph.grid.starts_fresh && ph.grid.accumulators.size() == dispatch.writes.size()) &&
@@ -852,6 +862,18 @@ bool strips_usable(const Run& run, const GenericPhase& ph, const Step& dispatch,
   return true;
 }
 
+// Nests without sequential loops and those with their loop in parts are bound by memory and always gain by strips.  A
+// nest whose work-items loop to the end needs enough of them left; and where f32 rows start on 128-byte lines, a
+// wavefront's 4-byte accesses are whole lines already and four times the wavefronts hide more: 200000 columns by 64 rows
+// take 9.2 us and 10.4 in strips, by 1000 rows 127 and 132, 300000 by 64 12.6 and 13.6; off those lines 230000 by 64 11.8
+// and 11.2, by 1000 164 and 146, 2000 batches of 100 by 300 60 and 42.
+bool strips_pay(const GenericPhase& ph, size_t parts, size_t total, size_t inner, bool bf16_inputs) {
+  if (!ph.sequential_loops) return true;
+  if (parts > 1) return ph.grid.held_accumulators;  // (there is no such form otherwise)
+  if (!ph.grid.available || !ph.grid.held_accumulators) return total >= size_t(4) * 65536;
+  return total >= size_t(4) * 49152 && (bf16_inputs || inner % 32 != 0);
+}
+
 ihip::Err launch_generic(Run& run, size_t k, const Step& dispatch) {
   Program& p = run.p;
   const GenericKernel& gk = p.generic.kernels[k];
@@ -860,7 +882,9 @@ ihip::Err launch_generic(Run& run, size_t k, const Step& dispatch) {
   const size_t R = p.generic.rank;
   const size_t view_bytes = 8 + 16 * R;
   const size_t nr = std::max<size_t>(gk.n_reads, 1), nw = std::max<size_t>(gk.n_writes, 1);
-  std::vector<unsigned char> args((nr + nw) * view_bytes, 0);
+  std::vector<unsigned char> args;
+  args.reserve((nr + nw) * view_bytes + 8);
+  args.resize((nr + nw) * view_bytes, 0);
   if (args.size() + 8 * nw + 8 > 4000) return "kernel " + std::to_string(k) + " takes too many buffers for one launch";
 
   auto fill = [&](size_t slot, void* data, BufferRef r) {
@@ -899,7 +923,16 @@ ihip::Err launch_generic(Run& run, size_t k, const Step& dispatch) {
     wave = reduced >= 128 && (ph.wave_contiguous || (total < 65536 && !ph.grid.available));
     if (run.knobs.generated_wave >= 0) wave = run.knobs.generated_wave == 1;
   }
-  const bool strips = !wave && strips_usable(run, ph, dispatch, total, inner);
+  const size_t reduced = ph.grid.available ? extent_of(ph.grid.extent) : 0;
+  auto parts_for = [&](bool in_strips) {
+    return generated_parts(run.knobs, ph.grid, wave, in_strips ? total / inner * ((inner + 3) / 4) : total, reduced, in_strips);
+  };
+  bool strips = !wave && ph.strip && inner >= 4;
+  size_t parts = parts_for(strips && ph.grid.held_accumulators);
+  if (strips && (!strips_pay(ph, parts, total, inner, bf16_inputs) || !strips_usable(run, ph, dispatch, inner))) {
+    strips = false;
+    parts = parts_for(false);
+  }
   // the outputs that a strip form stores in bf16 itself; any other bf16 output goes through an f32 temporary
   size_t bf16_writes = 0;
   std::vector<void*> write_ptrs(dispatch.writes.size(), nullptr);
@@ -920,7 +953,7 @@ ihip::Err launch_generic(Run& run, size_t k, const Step& dispatch) {
   const size_t items = strips ? total / inner * ((inner + 3) / 4) : total;  // work-items
   bool dynamic_private = false;  // (per-work-item slices of a device buffer are sized for the plain form's grid)
   for (const PrivateBuffer& pb : ph.privates) dynamic_private = dynamic_private || !pb.is_static;
-  const size_t parts = dynamic_private ? 1 : generated_parts(run.knobs, ph.grid, wave, items, ph.grid.available ? extent_of(ph.grid.extent) : 0, strips);
+  if (dynamic_private) parts = 1;
   hipFunction_t fn;
   if (parts > 1) {
     // every part accumulates into a copy of its own of each accumulated buffer (filled with the reduction's
@@ -942,10 +975,9 @@ ihip::Err launch_generic(Run& run, size_t k, const Step& dispatch) {
     const bool two_passes = width != 0 && most != 0;
     if (two_passes) floats += width * most;
     void* partial = nullptr;
-    const bool in_strips = strips && ph.grid.held_accumulators;
     if (run.alloc_optional(&partial, floats * 4)) {
       std::vector<unsigned char> gargs(args);
-      gargs.resize(args.size() + 8 * nw + 8 + (in_strips ? 8 : 0), 0);  // (the strip form's bf16_writes: none, the copies are f32)
+      gargs.resize(args.size() + 8 * nw + 8 + (strips ? 8 : 0), 0);  // (the strip form's bf16_writes: none, the copies are f32)
       float* at = static_cast<float*>(partial);
       struct FillArgs { float* data; size_t count; float value; };
       struct CombineArgs { const float* partial; float* data; size_t parts; size_t count; int op; int keep; };
@@ -980,11 +1012,11 @@ ihip::Err launch_generic(Run& run, size_t k, const Step& dispatch) {
         at += counts[a] * parts;
       }
       std::memcpy(gargs.data() + args.size() + 8 * nw, &parts, 8);
-      const std::string name = ph.name + (wave ? "_gw" : in_strips ? "_gv" : "_g") + twin;
+      const std::string name = ph.name + (wave ? "_gw" : strips ? "_gv" : "_g") + twin;
       if (ihip::Err e = generic_function(p, name, &fn); !e.empty()) return e;
       run.notes.back() += ", as " + name + ": the outermost sequential loop in " + std::to_string(parts) + " parts over " +
                           (wave ? "wavefronts" : "work-items") + ", combined by " + kCombineKernel;
-      const size_t units = (in_strips ? items : total) * parts;
+      const size_t units = items * parts;
       const unsigned per_group = wave ? GenericPhase::kWaveThreads / 64 : 64;
       const size_t groups = std::min<size_t>((units + per_group - 1) / per_group, size_t(1) << 20);
       if (ihip::Err e = ihip::launch(fn, (unsigned)groups, 1, 1, wave ? GenericPhase::kWaveThreads : 64, gargs.data(), gargs.size(), run.stream);

@@ -117,6 +117,7 @@ CASES["staged matmul 300x5x1000"] = (lambda: i("ik*kj~ijk||ijk") >> i("+ijk~ij||
 # sums over fewer rows than are dealt out in parts, of lengths whose last strip overlaps one of the work-group before
 for _op in "+*><":
     CASES[f"short column reduction {_op} 20x257"] = (lambda op=_op: i(f"{op}ij~j"), [(20, 257)])
+CASES["short column reduction 3x196611"] = (lambda: i("+ij~j"), [(3, 196611)])
 CASES["short column reduction 31x515"] = (lambda: i("+ij~j"), [(31, 515)])
 CASES["short column reduction 5x3x255"] = (lambda: i("+bij~bj"), [(5, 3, 255)])
 SHORT_CASES = [name for name in CASES if name.startswith("short ")]
