@@ -416,29 +416,33 @@ unsigned gemm_nt_bf16_split_k(size_t bh, size_t m, size_t n, size_t k, const Ker
     const size_t chunk = (k / want + 63) / 64 * 64;
     return (unsigned)((k + chunk - 1) / chunk);
   }
-  // A model of the time in us, fitted to products from 32 x 4096 x 4096 to 2048 x 2048 x 8192 enqueued back to back
-  // (it picks the measured best number of parts, or one within a few per cent of it, on 14 of 16 of them): a
-  // workgroup spends 0.7 us per 64-wide slab on a 128 x 128 tile (1.1 us when two share a CU), 1.3 us on a
-  // 256 x 256 tile, plus two slabs' worth before and after its loop; the chip holds 512 / 256 of them at a time;
-  // the second launch costs 4 us and the pass over the partial products runs at 3 TB/s.  Examples (unsplit ->
-  // split): 64 x 8192 x 8192 79 -> 30 us in 8 parts, 512 x 512 x 4096 52 -> 27 in 8, 256 x 4096 x 4096 41 -> 29
-  // in 8, 256 x 256 x 65536 576 -> 49 in 32, 29 x 9904 x 7968 39 in 6 (78 tiles; 48 in 4, 51 in 8); left whole: 1024^3 (10 us; 25 in 2 parts), 2048^3 (28; 40).
+  // A model of the time in us: a workgroup spends 0.7 us per 64-wide slab on a 128 x 128 tile (0.9 when the operands, beyond
+  // the 32 MB of the L2s, come from HBM, whose latency a CU's only workgroup waits for; 1.1 when two share a CU), 1.4 us on
+  // a 256 x 256 tile, plus two slabs' worth before and after its loop; the chip holds 512 / 256 of them at a time; the
+  // second launch costs 4 us and the pass over the partial products runs at 3 TB/s.  The workgroups that count are those
+  // launched, the tiles of a batch and part rounded up to one per XCD (fewer than four small ones: to four): the empty ones
+  // leave at once but leave holes (8 x 27 x 704 x 7960, 6 tiles a batch: 25 us in 8 parts = 512 workgroups, 34 in 9; 64 x 16 x 512 x
+  // 1024, 4 tiles: 16 whole, 22 in 2).  On 150 products of either layout from 16 x 1072 x 48 to 4 x 88 x 6504 x 6904 the
+  // choice is 3.9 % behind the best of all parts in the mean (10 % with tiles counted instead of workgroups, and 10 % with
+  // parts that are powers of two only).  Examples (unsplit -> split): 64 x 8192 x 8192 79 -> 30 us in 8 parts, 512 x 512 x
+  // 4096 52 -> 27 in 8, 256 x 4096 x 4096 41 -> 29 in 8, 256 x 256 x 65536 576 -> 49 in 32, 2 x 9304 x 2904 37 -> 17 in 5;
+  // left whole: 1024^3 (10 us; 25 in 2 parts), 2048^3 (28; 40).
   if (k > (size_t(1) << 22)) return 1;
   const size_t slabs = (k + 63) / 64;
-  const size_t t128 = ((m + 127) / 128) * ((n + 127) / 128) * bh, t256 = ((m + 255) / 256) * ((n + 255) / 256) * bh;
-  // (operands beyond the 32 MB of the L2s come from HBM, whose latency a CU's only workgroup waits for: 1.1 us then, too)
+  const size_t t128 = ((m + 127) / 128) * ((n + 127) / 128), t256 = ((m + 255) / 256) * ((n + 255) / 256);  // of a batch
   const bool far = bh * (m + n) * k * 2 > (size_t(32) << 20);
-  auto time_of = [far](unsigned tile_, size_t workgroups, size_t slabs_) {
+  auto time_of = [far, bh](unsigned tile_, size_t tiles_, size_t parts, size_t slabs_) {
+    const size_t workgroups = (tile_ == 128 && tiles_ < 4 ? 4 : (tiles_ + 7) / 8 * 8) * bh * parts;
     const double rounds = (double)((workgroups + (tile_ == 128 ? 511 : 255)) / (tile_ == 128 ? 512 : 256));
-    return rounds * (double)(slabs_ + 2) * (tile_ == 128 ? (workgroups <= 256 && !far ? 0.7 : 1.1) : 1.3);
+    return rounds * (double)(slabs_ + 2) * (tile_ == 256 ? 1.4 : workgroups > 256 ? 1.1 : far ? 0.9 : 0.7);
   };
-  double best = time_of(128, t128, slabs);
-  if (t256 >= 64) best = std::min(best, time_of(256, t256, slabs));
-  best *= 0.85;  // a split has to gain at least 15 %
-  const size_t tiles = tile == 256 ? t256 : t128;
+  double best = time_of(128, t128, 1, slabs);
+  if (t256 * bh >= 64) best = std::min(best, time_of(256, t256, 1, slabs));
+  best *= 0.9;  // a split has to gain at least 10 %
   size_t splits = 1;
   for (size_t s = 2; s <= 32 && k / s >= 512 && bh * s <= 65535; ++s) {
-    const double t = time_of(tile, tiles * s, (slabs + s - 1) / s) + 4.0 + (double)(bh * s * m * n * 4) / 3e6;
+    const size_t chunk = (k / s + 63) / 64 * 64, parts = (k + chunk - 1) / chunk;
+    const double t = time_of(tile, tile == 256 ? t256 : t128, parts, chunk / 64) + 4.0 + (double)(bh * parts * m * n * 4) / 3e6;
     if (t < best) {
       best = t;
       splits = s;
