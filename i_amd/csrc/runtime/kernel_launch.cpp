@@ -560,7 +560,19 @@ Err launch_gemm_nn_bf16(const void* a, const void* b, void* c, size_t bh, size_t
 bool gemm_narrow_usable(DType dtype, bool nn, size_t bh, size_t m, size_t n, size_t k, const KernelOptions& knobs) {
   if (knobs.gemm_tile || knobs.gemm_waves || knobs.gemm_k_parts || !knobs.gemm_direct) return false;  // (a tiled kernel is asked for)
   if (bh == 0 || bh > 65535 / 32 || m == 0 || n < 512 || k < 512 || !fits_u32(n) || k > (size_t(1) << 22)) return false;
-  if (dtype == BF16) return !nn && m <= 16 && k % 8 == 0 && k <= 8192 && n * k * 2 <= size_t(40) * 1000 * 1000;
+  if (dtype == BF16) {
+    // Batches of whole 64-wide slabs with many columns in all, or whose 128-tiles make one full round of workgroups: the
+    // tiled kernels fill the chip then, unsplit, and read A once for 128 or 256 columns where this kernel reads it for every 32 (tiled -> narrow, us: 64
+    // batches of 16 x 4096 x 512 66 -> 85, of 16 x 512 x 512 9.9 -> 11.5, 512 of 16 x 1024 x 1024 255 -> 284; but 64 of 1 x 4096
+    // x 2048 255 -> 194, of 8 x 768 x 1024 41 -> 23, and off the slabs of 16 x 4096 x 520 91 -> 75).
+    if (bh > 1 && k % 64 == 0) {
+      const size_t t128 = bh * ((n + 127) / 128);
+      if (n >= 2048 && bh * n >= 32768 && (k <= 1024 || m > 8)) return false;
+      if (n >= 1024 && bh * n >= 262144 && k <= 1024 && m > 8) return false;
+      if (m > 4 && t128 > 192 && t128 <= 256) return false;
+    }
+    return !nn && m <= 16 && k % 8 == 0 && k <= 8192 && n * k * 2 <= size_t(40) * 1000 * 1000;
+  }
   return k % 4 == 0 && (nn ? m <= 64 && n % 4 == 0 : m <= 32);
 }
 

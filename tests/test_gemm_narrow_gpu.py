@@ -7,20 +7,16 @@ import torch as t
 pytestmark = pytest.mark.gpu
 
 
-def _component(nn):
+def _component(nn, b=""):
     from i_amd import Component as i
 
-    if nn:
-        return i("ik*kj~ijk | i:16,j:16 | jii'j'k") >> i("+ijk~ij | i:16,j:16 | jii'j'k0")
-    return i("ik*jk~ijk | i:16,j:16 | jii'j'k") >> i("+ijk~ij | i:16,j:16 | jii'j'k0")
+    right = f"{b}kj" if nn else f"{b}jk"
+    return i(f"{b}ik*{right}~{b}ijk | i:16,j:16 | {b}jii'j'k") >> i(f"+{b}ijk~{b}ij | i:16,j:16 | {b}jii'j'k0")
 
 
-@pytest.mark.parametrize("out", ["bf16", "f32"])
-@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+@pytest.mark.parametrize("dtype, out", [("bf16", "bf16"), ("bf16", "f32"), ("f32", "f32")])
 @pytest.mark.parametrize("nn", [False, True])
 def test_products_of_few_rows(nn, dtype, out):
-    if dtype == "f32" and out == "bf16":
-        pytest.skip("an f32 product of this program has an f32 result")
     types = {"bf16": t.bfloat16, "f32": t.float32}
     component = _component(nn)
     g = t.Generator(device="cuda").manual_seed(3)
@@ -54,3 +50,23 @@ def test_values_of_b_that_no_row_of_the_tail_may_touch():
     c = t.empty(3, n, device="cuda")
     component.into(c, a, b)
     assert t.equal(c, t.full_like(c, float(k)))
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+@pytest.mark.parametrize("nn", [False, True])
+def test_batches_of_few_rows(nn, dtype):
+    """Every batch reads its own operands, k whole and in parts (f32, row-major right operand); batches of whole slabs with
+    many columns stay on the tiled kernels in bf16."""
+    types = {"bf16": t.bfloat16, "f32": t.float32}
+    component = _component(nn, "b")
+    q = 8 if dtype == "bf16" else 4
+    for b, m, n, k in [(2, 16, 512, 512), (3, 5, 516, 512 + q), (5, 12, 1000, 1000), (2, 31, 640, 2048 + 3 * q), (16, 16, 2048, 1024), (9, 1, 600, 4104)]:
+        x = t.randint(-4, 5, (b, m, k), device="cuda").to(types[dtype])
+        y = t.randint(-4, 5, (b, k, n) if nn else (b, n, k), device="cuda").to(types[dtype])
+        c = t.full((b, m, n), float("nan"), device="cuda")
+        component.into(c, x, y)
+        ref = t.stack([x[s].double() @ (y[s].double() if nn else y[s].double().t()) for s in range(b)]).float()
+        what = dict(nn=nn, dtype=dtype, b=b, m=m, n=n, k=k, report=component.report())
+        assert t.equal(c, ref), what
+        narrow = m <= 32 if dtype == "f32" else not nn and m <= 16 and not (b == 16 and n == 2048)
+        assert ("_narrow" in component.report()) == narrow, what
