@@ -1139,7 +1139,8 @@ GenericModule emit_generic_hip(const ExecPlan& plan, const Module& module, const
   for (const auto& b : plan.outputs) rank = std::max({rank, b.shape.size(), b.layout.size()});
   out.rank = rank;
 
-  std::ostringstream src;
+  std::ostringstream prelude, plain, twins;
+  std::ostream src(prelude.rdbuf());  // (switched between the three)
   bool any = false, any_grid = false;
   src << "// generated by the i gfx950 backend\n#include <hip/hip_runtime.h>\n#include <math.h>\n#include <stddef.h>\n\n";
   src << "#ifndef ILANG_WAVE_SYNC\n#define ILANG_WAVE_SYNC() __builtin_amdgcn_wave_barrier()\n#endif\n\n";
@@ -1230,6 +1231,7 @@ GenericModule emit_generic_hip(const ExecPlan& plan, const Module& module, const
     }
 
     const size_t nr = std::max<size_t>(info.n_reads, 1), nw = std::max<size_t>(info.n_writes, 1);
+    src.rdbuf(prelude.rdbuf());
     src << "struct Args_" << info.name << " { View readonlys[" << nr << "]; View writeables[" << nw << "]; };\n";
     if (phase.grid.available)
       src << "struct Args_" << info.name << "_g { View readonlys[" << nr << "]; View writeables[" << nw << "]; float* partial[" << nw
@@ -1350,6 +1352,7 @@ GenericModule emit_generic_hip(const ExecPlan& plan, const Module& module, const
       if (form.wave && !form.in_parts && phase.wave_loops.empty()) continue;
       if (form.in_parts && (!phase.grid.available || (form.wave && !phase.grid.wave))) continue;
       if (form.strips && (!phase.strip || (form.in_parts && !phase.grid.held_accumulators))) continue;
+      src.rdbuf(bf16 ? twins.rdbuf() : plain.rdbuf());
       if (bf16) g_bf16_reads.insert(phase.bf16_reads.begin(), phase.bf16_reads.end());
       src << "extern \"C\" __global__ void __launch_bounds__(" << (form.wave ? GenericPhase::kWaveThreads : 64u) << ") " << phase.name
           << form.suffix << (bf16 ? "_b" : "") << "(Args_" << info.name << (form.strips ? form.suffix : form.in_parts ? "_g" : "") << " args) {\n";
@@ -1387,6 +1390,7 @@ GenericModule emit_generic_hip(const ExecPlan& plan, const Module& module, const
     }
     info.phases.push_back(std::move(phase));
   }
+  src.rdbuf(plain.rdbuf());
   if (any_grid) {
     // the two helpers of the form with a loop in parts: the parts' copies start as the reduction's identity, and
     // fold into the accumulated buffer in part order (op: 0 +, 1 *, 2 max, 3 min; keep: the buffer's own value
@@ -1432,7 +1436,11 @@ GenericModule emit_generic_hip(const ExecPlan& plan, const Module& module, const
     src << "    if (lane == 0) args.data[e] = acc;\n";
     src << "  }\n}\n\n";
   }
-  if (any) out.source = src.str();
+  if (any) {
+    out.prelude = prelude.str();
+    out.source = plain.str();
+    out.bf16_source = twins.str();
+  }
   return out;
 }
 

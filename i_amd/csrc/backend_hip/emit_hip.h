@@ -109,8 +109,11 @@ struct GenericKernel {
 };
 
 struct GenericModule {
-  std::string source;                // full HIP translation unit ("" when no kernel needs it)
-  size_t rank = 1;                   // R of the View structs in the kernel argument block
+  // Two translation units: the forms that read f32 inputs, with the helper kernels, and the forms <name>..._b.  Compiling a
+  // program builds the first one only; the second is built by the first call whose inputs are bf16.
+  std::string prelude;                 // what both start with ("" when no kernel is emitted)
+  std::string source, bf16_source;     // what follows it
+  size_t rank = 1;                     // R of the View structs in the kernel argument block
   std::vector<GenericKernel> kernels;  // one entry per plan kernel; name empty when not emitted
 };
 

@@ -759,25 +759,28 @@ ihip::Err launch_hand(Run& run, const Recognized& r, const Step& step) {
 }
 
 // ---------------------------------------------------------------- generated kernels
-ihip::Err ensure_image(Program& p) {
+ihip::Err ensure_image(Program& p, bool bf16 = false) {
   std::lock_guard<std::mutex> lock(p.mu);
-  if (p.image_built) return {};
-  if (p.generic.source.empty()) return "program has no generated kernels";
-  if (std::string e = hipcc_build(p.generic.source, &p.image); !e.empty()) return e;
-  p.image_built = true;
+  Program::CodeObject& object = bf16 ? p.generated_bf16 : p.generated;
+  if (object.built) return {};
+  if (p.generic.prelude.empty()) return "program has no generated kernels";
+  if (std::string e = hipcc_build(p.generic.prelude + (bf16 ? p.generic.bf16_source : p.generic.source), &object.image); !e.empty()) return e;
+  object.built = true;
   return {};
 }
 
-ihip::Err generic_function(Program& p, const std::string& name, hipFunction_t* fn) {
-  if (ihip::Err e = ensure_image(p); !e.empty()) return e;
+// (`bf16`: one of the forms that read bf16 inputs)
+ihip::Err generic_function(Program& p, const std::string& name, hipFunction_t* fn, bool bf16 = false) {
+  if (ihip::Err e = ensure_image(p, bf16); !e.empty()) return e;
   std::lock_guard<std::mutex> lock(p.mu);
+  Program::CodeObject& object = bf16 ? p.generated_bf16 : p.generated;
   int dev = 0;
   if (ihip::Err e = ihip::check(hipGetDevice(&dev), "hipGetDevice"); !e.empty()) return e;
-  auto it = p.modules.find(dev);
-  if (it == p.modules.end()) {
+  auto it = object.modules.find(dev);
+  if (it == object.modules.end()) {
     hipModule_t mod = nullptr;
-    if (ihip::Err e = ihip::load_module(p.image.data(), &mod); !e.empty()) return e;
-    it = p.modules.emplace(dev, mod).first;
+    if (ihip::Err e = ihip::load_module(object.image.data(), &mod); !e.empty()) return e;
+    it = object.modules.emplace(dev, mod).first;
   }
   return ihip::module_function(it->second, name.c_str(), fn);
 }
@@ -1013,7 +1016,7 @@ ihip::Err launch_generic(Run& run, size_t k, const Step& dispatch) {
       }
       std::memcpy(gargs.data() + args.size() + 8 * nw, &parts, 8);
       const std::string name = ph.name + (wave ? "_gw" : strips ? "_gv" : "_g") + twin;
-      if (ihip::Err e = generic_function(p, name, &fn); !e.empty()) return e;
+      if (ihip::Err e = generic_function(p, name, &fn, bf16_inputs); !e.empty()) return e;
       run.notes.back() += ", as " + name + ": the outermost sequential loop in " + std::to_string(parts) + " parts over " +
                           (wave ? "wavefronts" : "work-items") + ", combined by " + kCombineKernel;
       const size_t units = items * parts;
@@ -1035,7 +1038,7 @@ ihip::Err launch_generic(Run& run, size_t k, const Step& dispatch) {
     const size_t waves = std::min<size_t>(total, size_t(1) << 16);
     const unsigned per_group = GenericPhase::kWaveThreads / 64;
     for (const PrivateBuffer& pb : ph.privates) fill(nr + pb.writeable, nullptr, dispatch.writes[pb.writeable]);
-    if (ihip::Err err = generic_function(p, ph.name + "_w" + twin, &fn); !err.empty()) return err;
+    if (ihip::Err err = generic_function(p, ph.name + "_w" + twin, &fn, bf16_inputs); !err.empty()) return err;
     run.notes.back() += ", as " + ph.name + "_w" + twin + ": one wavefront per iteration of the parallel loops";
     return ihip::launch(fn, (unsigned)((waves + per_group - 1) / per_group), 1, 1, GenericPhase::kWaveThreads, args.data(), args.size(),
                         run.stream);
@@ -1059,7 +1062,7 @@ ihip::Err launch_generic(Run& run, size_t k, const Step& dispatch) {
     fill(nr + pb.writeable, ptr, dispatch.writes[pb.writeable]);
   }
   const std::string name = ph.name + (strips ? "_v" : "") + twin;
-  if (ihip::Err e = generic_function(p, name, &fn); !e.empty()) return e;
+  if (ihip::Err e = generic_function(p, name, &fn, bf16_inputs); !e.empty()) return e;
   if (strips) {
     args.resize(args.size() + 8, 0);
     std::memcpy(args.data() + args.size() - 8, &bf16_writes, 8);
@@ -1173,7 +1176,8 @@ bool row_slices_of(const Graph<Node>& graph, std::vector<char>* sliced) {
 }  // namespace
 
 Program::~Program() {
-  for (auto& kv : modules) ihip::unload_module(kv.second);
+  for (CodeObject* object : {&generated, &generated_bf16})
+    for (auto& kv : object->modules) ihip::unload_module(kv.second);
 }
 
 std::string compile_program(const Component& component, Program** out) {
@@ -1268,7 +1272,7 @@ std::string program_code(const Component& component) {
     }
     os << "\n";
   }
-  os << "\n" << gen.source;
+  os << "\n" << gen.prelude << gen.source << gen.bf16_source;
   return os.str();
 }
 

@@ -44,10 +44,14 @@ struct Program {
   ic::ExecPlan nest_plan;
   std::vector<std::vector<size_t>> nests_of;
   GenericModule generic;               // source for every kernel of nest_plan (hand-written ones keep a generated twin)
-  std::vector<char> image;             // built lazily unless some kernel can only run generated
-  bool image_built = false;
+  struct CodeObject {
+    std::vector<char> image;
+    bool built = false;
+    std::map<int, hipModule_t> modules;  // per device
+  };
+  CodeObject generated;                // built lazily unless some kernel can only run generated
+  CodeObject generated_bf16;           // (GenericModule::bf16_source) built by the first call that needs it
   std::mutex mu;
-  std::map<int, hipModule_t> modules;  // per device
   // what set_option / set_clock_probe have stored (kernel choices that the caller takes from the launchers, and where
   // the attention kernels count their clocks); guarded by mu, copied by every execute() when it starts
   ihip::KernelOptions options;
@@ -57,7 +61,7 @@ struct Program {
   ~Program();
 };
 
-// Lower, recognise, emit; builds the generated code object right away when a
+// Lower, recognise, emit; builds the generated code object (that of the f32 forms) right away when a
 // kernel has no hand-written form.  Throws ic::CompileError / returns error text.
 std::string compile_program(const ic::Component& component, Program** out);
 

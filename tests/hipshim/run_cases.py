@@ -3,7 +3,8 @@ emulation of the HIP runtime (shim.cpp), and compares with the C the oracle back
 component.  Started as a subprocess by tests/test_generated_kernels_cpu.py with
 ILANG_CORE_LIB, ILANG_HIPCC, ILANG_NO_TORCH and ILANG_NO_DISK_CACHE set; ILANG_SHIM_WAVE=1 asks for the
 wavefront-per-iteration form of reduction nests (the program option generated.wave), ILANG_SHIM_PARTS=n for
-reduction nests with their outermost sequential loop in n parts (generated.parts).
+reduction nests with their outermost sequential loop in n parts (generated.parts); ILANG_SHIM_BF16=in|all passes the
+operands (and takes the results) as bf16 device tensors.
 Prints the case name before running it, so a crash (a guard page hit = out-of-bounds access) names its case."""
 import sys
 from pathlib import Path
@@ -123,6 +124,11 @@ CASES["short column reduction 5x3x255"] = (lambda: i("+bij~bj"), [(5, 3, 255)])
 SHORT_CASES = [name for name in CASES if name.startswith("short ")]
 STAGED_CASES = [name for name in CASES if name.startswith("staged ")]
 
+# programs whose kernels store bf16 results themselves (element-wise nests in strips)
+CASES["bias and threshold 21x35"] = (lambda: i("ij+j~ij||ij") >> i("ij>.~ij||ij0"), [(21, 35), (35,), ()])
+CASES["column normalize 37x72"] = (lambda: (I & i("+ij~j||ij")) >> i("ij/j~ij||1ij"), [(37, 72)])
+BF16_RESULT_CASES = ["pointwise chain", "scalar operand", "column normalize 37x72", "bias and threshold 21x35"]
+
 # the cases with a nest that has a wavefront-per-iteration form (reduction loops spread over 64 lanes)
 WAVE_CASES = ["naive attention ragged", "batched naive attention", "mm_t", "mm_t empty", "matmul unfused",
               "matmul fused init site", "row sum", "column max", "total", "fanout two outputs", "swapped fanout",
@@ -150,28 +156,45 @@ CLOSED_FORMS = {
 }
 
 
-def run_without_allocating(comp, inputs):
-    """The same call through i_exec_into_device_noalloc: on the emulated runtime device memory is host memory, so
-    NumPy buffers stand in for device tensors.  Temporaries then come out of the fixed workspace."""
-    import ctypes
+def to_bf16(x):
+    """The bit patterns of the nearest bf16 values (ties to even), as an array of 16-bit words."""
+    u = np.ascontiguousarray(x, dtype=np.float32).view(np.uint32)
+    return ((u + np.uint32(0x7fff) + (u >> 16 & 1)) >> 16).astype(np.uint16)
 
+
+def from_bf16(words):
+    return (words.astype(np.uint32) << 16).view(np.float32)
+
+
+def run_on_device_records(comp, inputs, entry, bf16=False, bf16_out=False):
+    """The same call through i_exec_into_device[_noalloc]: on the emulated runtime device memory is host memory, so NumPy
+    buffers stand in for device tensors.  (noalloc: temporaries come out of the fixed workspace.)  `bf16`: operands of
+    rank 1 and more are passed as bf16; `bf16_out`: so are the outputs, for programs whose kernels store them themselves."""
     from i_amd import _native as nat, ilang
 
-    operands = [ilang._operand(x, "input") for x in inputs]
-    outs = [np.full(shape, np.nan, dtype=np.float32) for shape in comp.output_shapes(*inputs)]
-    targets = [ilang._operand(o, "output") for o in outs]
+    def record(x, words):
+        return ilang._Operand(x.ctypes.data, x.shape, nat.BF16 if words else nat.F32, None, x)
+
+    shapes = comp.output_shapes(*inputs)
+    operands = [record(to_bf16(x), True) if bf16 and x.ndim else record(np.asarray(x, dtype=np.float32), False) for x in inputs]
+    outs = [np.full(shape, 0xffff, dtype=np.uint16) if bf16_out else np.full(shape, np.nan, dtype=np.float32) for shape in shapes]
+    targets = [record(o, bf16_out) for o in outs]
     in_records, keep_in = ilang._pack(operands, on_device=True)
     out_records, keep_out = ilang._pack(targets, on_device=True)
-    nat.check(nat.core.i_exec_into_device_noalloc(comp._compile(), in_records, len(operands), out_records, len(targets), None))
+    nat.check(entry(comp._compile(), in_records, len(operands), out_records, len(targets), None))
+    outs = [from_bf16(o) if bf16_out else o for o in outs]
     return outs[0] if len(outs) == 1 else tuple(outs)
 
 
 def main():
     import os
 
+    from i_amd import _native as nat
+
     noalloc = os.environ.get("ILANG_SHIM_NOALLOC") == "1"
+    bf16 = os.environ.get("ILANG_SHIM_BF16", "")  # "in": bf16 operands, "all": bf16 results too
     which = os.environ.get("ILANG_SHIM_CASES")
-    names = sys.argv[1:] or {"wave": WAVE_CASES, "sample": SAMPLE_CASES, "staged": STAGED_CASES, "short": SHORT_CASES}.get(which, list(CASES))
+    names = sys.argv[1:] or {"wave": WAVE_CASES, "sample": SAMPLE_CASES, "staged": STAGED_CASES, "short": SHORT_CASES, "bf16 results": BF16_RESULT_CASES}.get(which, list(CASES))
     tolerance = float(os.environ.get("ILANG_SHIM_TOLERANCE", "1e-5"))
     failed = []
     for name in names:
@@ -184,7 +207,13 @@ def main():
         if os.environ.get("ILANG_SHIM_PARTS") is not None:
             comp.option("generated.parts", int(os.environ["ILANG_SHIM_PARTS"]))
         inputs = [rnd(s, k + 1) for k, s in enumerate(shapes)]
-        got = run_without_allocating(comp, inputs) if noalloc else comp.exec_numpy(*inputs)
+        if bf16:
+            inputs = [from_bf16(to_bf16(x)) if x.ndim else x for x in inputs]
+            got = run_on_device_records(comp, inputs, nat.core.i_exec_into_device, True, bf16 == "all")
+        elif noalloc:
+            got = run_on_device_records(comp, inputs, nat.core.i_exec_into_device_noalloc)
+        else:
+            got = comp.exec_numpy(*inputs)
         ref = oracle.compile_component(comp.handle).run(*inputs)
         got = got if isinstance(got, tuple) else (got,)
         ref = ref if isinstance(ref, tuple) else (ref,)

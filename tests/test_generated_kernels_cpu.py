@@ -79,8 +79,7 @@ def test_overlapping_strips_of_sums_read_nothing_that_they_write(shim_lib):
         code = subprocess.run([sys.executable, "-c", f"from i_amd import Component as i\nprint(i('{expression}')._code())"], env=env,
                               capture_output=True, text=True, cwd=ROOT, timeout=300).stdout
         for form in ("f0_v(", "f0_v_b(", "f0_gv(", "f0_gv_b("):
-            start = code.index(form)
-            body = code[start:code.index('extern "C"', start)]
+            body = code[code.index(form):].split('extern "C"')[0]
             assert "ilang_load(writeables" not in body and body.count("ilang_store(") == 1, (expression, form)
     run_cases(shim_lib, {"ILANG_SHIM_CASES": "short", "ILANG_HIP_UNCHECKED": "0"})
     run_cases(shim_lib, {"ILANG_SHIM_CASES": "short", "ILANG_SHIM_ORDER": "reverse"})
@@ -142,6 +141,34 @@ def test_fixed_workspace_entry_matches_on_the_cpu(shim_lib):
     emitted C as through the allocating entry."""
     run_cases(shim_lib, {"ILANG_SHIM_NOALLOC": "1"})
     run_cases(shim_lib, {"ILANG_SHIM_NOALLOC": "1", "ILANG_SHIM_PARTS": "3", "ILANG_SHIM_TOLERANCE": "1e-4", "ILANG_SHIM_CASES": "sample"})
+
+
+def test_forms_that_read_bf16_operands_match_too(shim_lib):
+    """bf16 device tensors are read (and, by element-wise nests in strips, written) as they are by forms of their own: work-items,
+    strips, loops in parts and wavefronts, against the emitted C on the same rounded values."""
+    loose = {"ILANG_SHIM_BF16": "in", "ILANG_SHIM_TOLERANCE": "1e-4"}
+    run_cases(shim_lib, {**loose, "ILANG_SHIM_CASES": "sample", "ILANG_HIP_UNCHECKED": "0"})
+    run_cases(shim_lib, {**loose, "ILANG_SHIM_CASES": "staged"})
+    run_cases(shim_lib, {**loose, "ILANG_SHIM_CASES": "short", "ILANG_SHIM_PARTS": "3"})
+    run_cases(shim_lib, {**loose, "ILANG_SHIM_WAVE": "1", "ILANG_HIP_UNCHECKED": "0"}, names=["row sum 5x300", "fused matrix-vector product", "column max", "mlp with pair"])
+    # (a result off by one rounding to 8 bits)
+    run_cases(shim_lib, {"ILANG_SHIM_BF16": "all", "ILANG_SHIM_TOLERANCE": str(2.0 ** -8), "ILANG_SHIM_CASES": "bf16 results", "ILANG_HIP_UNCHECKED": "0"})
+
+
+def test_forms_that_read_bf16_operands_are_built_when_they_are_called(shim_lib, tmp_path):
+    """Compiling a program and running it on f32 operands builds none of them."""
+    logger = tmp_path / "hipcc"
+    logger.write_text(f"#!/bin/sh\nfor a in \"$@\"; do case $a in *.hip) cp \"$a\" {tmp_path}/source_$$.txt;; esac; done\nexec {sys.executable} {SHIM / 'hostcc.py'} \"$@\"\n")
+    logger.chmod(0o755)
+    env = {"ILANG_HIPCC": str(logger)}
+
+    def sources():
+        return [p.read_text() for p in tmp_path.glob("source_*.txt")]
+
+    run_cases(shim_lib, env, names=["column max"])
+    assert len(sources()) == 1 and "f0_v(" in sources()[0] and "f0_v_b(" not in sources()[0]
+    run_cases(shim_lib, {**env, "ILANG_SHIM_BF16": "in"}, names=["column max"])
+    assert len(sources()) == 3 and sum("f0_v_b(" in s for s in sources()) == 1
 
 
 def test_operands_that_disagree_on_a_shared_index_are_refused_before_any_launch(shim_lib):
