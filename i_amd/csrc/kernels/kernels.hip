@@ -195,7 +195,8 @@ GEMM_NARROW(nn_f32, true, true, 16, 1, 64, 4, 8)
 GEMM_NARROW(nn_f32, true, true, 32, 2, 64, 4, 8)
 GEMM_NARROW(nn_f32, true, true, 64, 4, 64, 4, 8)
 
-// row_<op>_wave_v<NV>, row_<op>_sub_{v,s}<G>, row_<op>_group_v<NV>, row_<op>_block[_v] and ROW_ANY's forms for op = softmax, shift (x - row max), norm (x / row sum), exp, scaled_softmax
+// row_<op>_wave_v<NV>, row_<op>_sub_{v,s}<G>, row_<op>_group_v<NV> and row_<op>_block[_v] for op = softmax, shift (x - row
+// max), norm (x / row sum), exp, scaled_softmax; ROW_ANY's forms for the first four
 #define ROW_WAVE(OP, MODE, NV)                                                                     \
   extern "C" __global__ void __launch_bounds__(256) row_##OP##_wave_v##NV(SoftmaxParams p) {       \
     row_softmax_wave_body<NV, MODE>(p);                                                            \
@@ -226,18 +227,19 @@ GEMM_NARROW(nn_f32, true, true, 64, 4, 64, 4, 8)
   ROW_GROUP(OP, MODE, 4) ROW_GROUP(OP, MODE, 8) ROW_GROUP(OP, MODE, 16)                             \
   ROW_SUB(OP, MODE, 1) ROW_SUB(OP, MODE, 2) ROW_SUB(OP, MODE, 4) ROW_SUB(OP, MODE, 8)              \
   ROW_SUB(OP, MODE, 16) ROW_SUB(OP, MODE, 32)                                                      \
-  ROW_ANY(OP, MODE, lanes_s2, 2, 1) ROW_ANY(OP, MODE, lanes_s4, 4, 1) ROW_ANY(OP, MODE, lanes_s8, 8, 1)\
-  ROW_ANY(OP, MODE, lanes_s16, 16, 1) ROW_ANY(OP, MODE, lanes_s32, 32, 1) ROW_ANY(OP, MODE, wave_s2, 64, 1)\
-  ROW_ANY(OP, MODE, wave_s4, 64, 2) ROW_ANY(OP, MODE, wave_s6, 64, 3) ROW_ANY(OP, MODE, wave_s8, 64, 4)\
-  ROW_ANY(OP, MODE, wave_s12, 64, 6) ROW_ANY(OP, MODE, wave_s16, 64, 8) ROW_ANY(OP, MODE, group_s1, 256, 3)\
-  ROW_ANY(OP, MODE, group_s2, 256, 4) ROW_ANY(OP, MODE, group_s4, 256, 8) ROW_ANY(OP, MODE, group_s6, 1024, 3)\
-  ROW_ANY(OP, MODE, group_s8, 1024, 4) ROW_ANY(OP, MODE, group_s12, 1024, 6) ROW_ANY(OP, MODE, group_s18, 1024, 9)\
   extern "C" __global__ void __launch_bounds__(1024) row_##OP##_block(SoftmaxParams p) {           \
     row_softmax_block_body<MODE, false>(p);                                                        \
   }                                                                                                \
   extern "C" __global__ void __launch_bounds__(1024) row_##OP##_block_v(SoftmaxParams p) {         \
     row_softmax_block_body<MODE, true>(p);                                                         \
   }
+#define ROW_ANYS(OP, MODE)                                                                         \
+  ROW_ANY(OP, MODE, lanes_s2, 2, 1) ROW_ANY(OP, MODE, lanes_s4, 4, 1) ROW_ANY(OP, MODE, lanes_s8, 8, 1)\
+  ROW_ANY(OP, MODE, lanes_s16, 16, 1) ROW_ANY(OP, MODE, lanes_s32, 32, 1) ROW_ANY(OP, MODE, wave_s2, 64, 1)\
+  ROW_ANY(OP, MODE, wave_s4, 64, 2) ROW_ANY(OP, MODE, wave_s6, 64, 3) ROW_ANY(OP, MODE, wave_s8, 64, 4)\
+  ROW_ANY(OP, MODE, wave_s12, 64, 6) ROW_ANY(OP, MODE, wave_s16, 64, 8) ROW_ANY(OP, MODE, group_s1, 256, 3)\
+  ROW_ANY(OP, MODE, group_s2, 256, 4) ROW_ANY(OP, MODE, group_s4, 256, 8) ROW_ANY(OP, MODE, group_s6, 1024, 3)\
+  ROW_ANY(OP, MODE, group_s8, 1024, 4) ROW_ANY(OP, MODE, group_s12, 1024, 6) ROW_ANY(OP, MODE, group_s18, 1024, 9)
 #define ROW_PARTS(OP, MODE)                                                                                   \
   extern "C" __global__ void __launch_bounds__(1024) row_##OP##_parts_stats(SoftmaxParams p) {                \
     row_softmax_parts_body<MODE, false, 0>(p);                                                                \
@@ -252,12 +254,17 @@ GEMM_NARROW(nn_f32, true, true, 64, 4, 64, 4, 8)
     row_softmax_parts_body<MODE, true, 1>(p);                                                                 \
   }
 ROW_OP(softmax, 0)
+ROW_ANYS(softmax, 0)
 ROW_PARTS(softmax, 0)
 ROW_PARTS(scaled_softmax, 4)
 ROW_OP(shift, 1)
+ROW_ANYS(shift, 1)
 ROW_OP(norm, 2)
+ROW_ANYS(norm, 2)
 ROW_OP(exp, 3)
-ROW_OP(scaled_softmax, 4)  // the middle kernel of attention in three kernels (head sizes above 128)
+ROW_ANYS(exp, 3)
+// the middle kernel of attention in three kernels: f32 rows of a multiple of 4 elements in an aligned temporary
+ROW_OP(scaled_softmax, 4)
 
 extern "C" __global__ void __launch_bounds__(256) convert_f32_to_bf16(ConvertParams p) {
   const float* s = reinterpret_cast<const float*>(p.src);

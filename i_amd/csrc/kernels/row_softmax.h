@@ -276,6 +276,7 @@ __device__ __forceinline__ void row_softmax_sub_body(const SoftmaxParams& p) {
 // then workgroups of 256 and 1024 lanes, whose reductions cross the wavefronts through LDS.
 template <int T, int NG, int MODE>
 __device__ __forceinline__ void row_softmax_any_body(const SoftmaxParams& p) {
+  static_assert(MODE < 4, "scaled rows are always f32 and aligned");
   constexpr int NW = T > 64 ? T / 64 : 1;  // wavefronts per row
   __shared__ float red[2][NW];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -339,15 +340,6 @@ __device__ __forceinline__ void row_softmax_any_body(const SoftmaxParams& p) {
         if (c + e < 0 || c + e >= cols) r[i][e] = pad;
     }
   }
-  if constexpr (MODE == 4) {  // softmax(scale * x); the padding stays what it is whatever the scale's sign
-    const float sc = load_scale(p.scale_ptr, p.scale_value);
-#pragma unroll
-    for (int i = 0; i < NG; ++i)
-#pragma unroll
-      for (int e = 0; e < 8; ++e)
-        if (column(i) + e >= 0 && column(i) + e < cols) r[i][e] *= sc;
-  }
-
   auto store_as = [&](auto bf16_tag, auto value) {
     constexpr bool BF16 = decltype(bf16_tag)::value;
 #pragma unroll

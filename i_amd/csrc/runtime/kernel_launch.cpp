@@ -750,7 +750,7 @@ Err launch_row_softmax(const void* x, void* y, size_t rows, size_t cols, hipStre
   SoftmaxParams p{x, y, (uint32_t)rows, (uint32_t)cols, scale_ptr, scale};
   hipFunction_t fn;
   const bool f32 = in_dtype == F32 && out_dtype == F32;
-  if (!f32 && !row_softmax_any_supported(cols)) return "row_softmax kernel: bf16 rows are too long";
+  if (!f32 && (!row_softmax_any_supported(cols) || mode == 4)) return "row_softmax kernel: bf16 rows are too long (or scaled)";
   const bool vec = f32 && cols % 4 == 0 && (reinterpret_cast<uintptr_t>(x) % 16 == 0) && (reinterpret_cast<uintptr_t>(y) % 16 == 0);
   if (f32 && parts > 1 && (mode == 0 || mode == 4)) {
     // every row in parts over workgroups: the parts' (max, sum) pairs into `stats`, then a second launch that
@@ -771,7 +771,7 @@ Err launch_row_softmax(const void* x, void* y, size_t rows, size_t cols, hipStre
   // f32 rows whose length is a multiple of 4 and that start on 16-byte boundaries: float4 chunks.  Every other row
   // that registers hold (odd lengths, other alignments, bf16 on either side): groups of 8 elements; but f32 rows of
   // at most 128 columns keep the form with few lanes per row (2000000 x 31: 114 against 209 us).
-  if (!vec && row_softmax_any_supported(cols) && !(f32 && cols <= 128)) {
+  if (!vec && mode != 4 && row_softmax_any_supported(cols) && !(f32 && cols <= 128)) {
     const size_t in_elem = in_dtype == BF16 ? 2 : 4, out_elem = out_dtype == BF16 ? 2 : 4;
     const size_t x_shift = reinterpret_cast<uintptr_t>(x) % 16 / in_elem, y_shift = reinterpret_cast<uintptr_t>(y) % 16 / out_elem;
     p.in_bf16 = in_dtype == BF16;
