@@ -650,17 +650,17 @@ static F32Plan f32_plan(size_t bh, size_t m, size_t n, size_t k, const KernelOpt
   };
   const unsigned asked = knobs.gemm_tile == 0 ? 0u : knobs.gemm_tile == 192 ? 256u : (unsigned)knobs.gemm_tile;  // (192 x 256 exists for bf16 NT products only)
   if (knobs.gemm_k_parts > 1) return {asked ? asked : t256 >= 128 ? 256u : 128u, parts_of(std::min<size_t>((size_t)knobs.gemm_k_parts, k / 64))};
-  if (asked == 256 || (!asked && t256 >= 128)) return {256, 1};
+  if ((asked == 256 || !asked) && t256 >= 128) return {256, 1};
   const size_t slabs = (k + 31) / 32;
   const bool far = bh * (m + n) * k * 4 > (size_t(32) << 20);
   F32Plan best{asked ? asked : 128u, 1};
   double best_time = 1e30;
-  for (unsigned tile : {128u, 64u}) {
-    if (asked && tile != asked) continue;
+  for (unsigned tile : {256u, 128u, 64u}) {
+    if (asked ? tile != asked : tile == 256) continue;
     const size_t tiles = ((m + tile - 1) / tile) * ((n + tile - 1) / tile) * bh;
     for (size_t s = 1; s <= 32 && (s == 1 || (!whole && knobs.gemm_k_parts != 1 && k / s >= 64 && bh * s <= 65535)); ++s) {
       const double resident = (double)((tiles * s + 255) / 256);
-      double t = (double)((slabs + s - 1) / s + 2) * std::max(resident * (tile == 128 ? 1.7 : 0.46), far ? 0.7 : 0.0);
+      double t = (double)((slabs + s - 1) / s + 2) * std::max(resident * (tile == 256 ? 6.8 : tile == 128 ? 1.7 : 0.46), far ? 0.7 : 0.0);
       if (s > 1) t = (t + 4.0 + (double)(bh * s * m * n * 4) / 3e6) / 0.85;
       if (t < best_time) {
         best_time = t;

@@ -51,7 +51,8 @@ def test_products_of_odd_extents(nn, types):
 
 @pytest.mark.parametrize("nn", [False, True])
 def test_every_f32_tile_and_parts(nn):
-    """The three tiles, whole and partial slabs, k whole and in parts, at the edges of a tile and of a half of it."""
+    """The tiles that can be asked for, whole and partial slabs, k whole and in parts, at the edges of a tile and of a half
+    of it.  (The 64 x 64 tile is the rule's own choice only: the tests below.)"""
     for tile in (0, 128, 256):
         for parts in (1, 3):
             for m, n, k in [(64, 64, 32), (63, 68, 36), (257, 260, 416), (129, 384, 1024), (128, 128, 256)]:
@@ -62,6 +63,19 @@ def test_every_f32_tile_and_parts(nn):
 def test_small_f32_tiles_are_reached():
     assert "64x64x32" in _check(True, "f32", "f32", 1000, 1500, 700)
     assert "64x64x32" in _check(False, "f32", "f32", 1000, 1500, 700)
+
+
+@pytest.mark.parametrize("nn", [False, True])
+def test_small_f32_tiles_in_parts(nn):
+    """Few tiles under a long k: the rule takes 64-tiles in parts, whole and partial slabs in the last one."""
+    for m, n, k in [(128, 128, 4096), (126, 132, 4092), (129, 68, 4100), (512, 64, 512), (500, 64, 516), (65, 100, 1288)]:
+        report = _check(nn, "f32", "f32", m, n, k)
+        assert "64x64x32" in report and "parts" in report and ("_brow" in report) == nn and ("_ktail" in report) == (k % 32 != 0), (m, n, k, report)
+
+
+def test_an_f32_tile_that_is_asked_for_goes_in_parts_too():
+    assert "256x256x32_direct (k in" in _check(False, "f32", "f32", 256, 256, 8192, options=(("gemm.tile", 256),))
+    assert "128x128x32_direct (k in" in _check(False, "f32", "f32", 256, 256, 8192, options=(("gemm.tile", 128),))
 
 
 def test_batched_row_major_right_operands_of_odd_extents():
