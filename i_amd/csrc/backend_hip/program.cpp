@@ -802,11 +802,12 @@ size_t generated_parts(const ihip::KernelOptions& knobs, const GridForm& grid, b
   } else {
     const size_t target = wave ? 4096 : strips ? 98304 : 262144;  // wavefronts / work-items that fill the chip
     if (total * 2 > target) return 1;
-    // (strips have four times the bytes in flight, and three wavefronts of them per CU read fastest: with 49152 and 98304
-    // work-items, and in the form without strips, column sums of 16384 x 4096 take 46.3, 49.0 and 46.4 us, of 4096 x 4096
-    // 18.9, 20.5 and 19.4, of 65536 x 1024 51.4, 54.2 and 52.1, of 5042 x 2561 18.2, 20.7 and 22.1; short loops are bound by
-    // their rounds of loads instead, 64 batches of 64 x 1024 10.7 us in 4 parts, 11.6 in 3)
-    parts = std::min<size_t>(strips && reduced > 256 ? std::max<size_t>(49152 / total, 2) : target / total, reduced / least);
+    // (strips have four times the bytes in flight: long loops read fastest with 49152 to 65536 of them.  65536 makes as many
+    // parts as the form without strips has, so that no sum is longer.  Column sums with 65536 and 98304 work-items, and without
+    // strips: 16384 x 4096 47.8, 49.0 and 46.4 us, 4096 x 4096 19.5, 20.5 and 19.4, 65536 x 1024 51.3, 54.2 and 52.1, 5042 x
+    // 2561 19.4, 20.7 and 22.1, 1000 x 50000 33.9, 34.8 and 39.2; short loops are bound by their rounds of loads instead, 64
+    // batches of 64 x 1024 10.7 us in 4 parts, 11.6 in 3)
+    parts = std::min<size_t>(strips && reduced > 256 ? std::max<size_t>(65536 / total, 2) : target / total, reduced / least);
   }
   // (at most 4096 parts; 2048 of wavefronts when left to this rule: the pass over the parts of a sum to one element
   // is one wavefront's work and grows with their number, 4096^2 to one element 29.7 us in 4096 parts, 23.8 in 2048)
@@ -814,11 +815,11 @@ size_t generated_parts(const ihip::KernelOptions& knobs, const GridForm& grid, b
   if (parts >= 256) parts = parts / 32 * 32;
   else if (parts >= 16) parts = parts / 8 * 8;
   if (strips && knobs.generated_parts <= 1 && parts >= 2) {
-    // (their shares are multiples of eight iterations, whole rounds of the loads in flight: no more parts than that leaves;
-    // 100000 x 64 30.6 -> 24.1 us, 4096 x 1024 13.9 -> 12.7)
-    const size_t share = (reduced + parts - 1) / parts, needed = (reduced + (share + 7) / 8 * 8 - 1) / ((share + 7) / 8 * 8);
+    // (their shares are multiples of eight iterations, whole rounds of the loads in flight, and no longer than these parts
+    // would have: 100000 x 64 30.6 -> 24.1 us, 4096 x 1024 13.9 -> 12.7)
+    const size_t share = std::max<size_t>(reduced / parts / 8 * 8, 8), needed = (reduced + share - 1) / share;
     const size_t step = needed >= 256 ? 32 : needed >= 16 ? 8 : 1;
-    parts = std::min(parts, (needed + step - 1) / step * step);
+    parts = std::min<size_t>((needed + step - 1) / step * step, 4096);
   }
   return parts < 2 ? 1 : parts;
 }
