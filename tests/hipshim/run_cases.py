@@ -126,8 +126,8 @@ STAGED_CASES = [name for name in CASES if name.startswith("staged ")]
 
 # programs whose kernels store bf16 results themselves (element-wise nests in strips)
 CASES["bias and threshold 21x35"] = (lambda: i("ij+j~ij||ij") >> i("ij>.~ij||ij0"), [(21, 35), (35,), ()])
-CASES["column normalize 37x72"] = (lambda: (I & i("+ij~j||ij")) >> i("ij/j~ij||1ij"), [(37, 72)])
-BF16_RESULT_CASES = ["pointwise chain", "scalar operand", "column normalize 37x72", "bias and threshold 21x35"]
+CASES["column max shift 37x72"] = (lambda: (I & i(">ij~j||ij")) >> i("ij-j~ij||1ij"), [(37, 72)])
+BF16_RESULT_CASES = ["pointwise chain", "scalar operand", "column max shift 37x72", "bias and threshold 21x35"]
 
 # the cases with a nest that has a wavefront-per-iteration form (reduction loops spread over 64 lanes)
 WAVE_CASES = ["naive attention ragged", "batched naive attention", "mm_t", "mm_t empty", "matmul unfused",
