@@ -15,7 +15,8 @@ def _components():
         "column_max": (i(">ij~j"), lambda x: x.max(0).values),
         "column_sum": (i("+ij~j"), lambda x: x.sum(0)),
         "row_sum": (i("+ij~i"), lambda x: x.sum(1)),
-        "square_over_rows": (i("ij*ij~ij||ij") >> i("+ij~j"), lambda x: (x * x).sum(0)),
+        # (one nest, with a fused temporary that is private to every work-item)
+        "staged_exponentials": (i("^ij~ij||ji") >> i("+ij~j||ji0"), lambda x: x.exp().sum(0)),
     }
 
 
@@ -23,7 +24,7 @@ _BITS = {t.float32: 0.0, t.bfloat16: 2.0 ** -8}
 
 
 @pytest.mark.parametrize("types", ["f32-f32", "bf16-f32", "bf16-bf16", "f32-bf16"])
-@pytest.mark.parametrize("name", ["column_normalize", "column_max", "column_sum", "row_sum"])
+@pytest.mark.parametrize("name", ["column_normalize", "column_max", "column_sum", "row_sum", "staged_exponentials"])
 def test_reductions_and_their_quotients(name, types):
     src, dst = ({"bf16": t.bfloat16, "f32": t.float32}[x] for x in types.split("-"))
     component, oracle = _components()[name]
@@ -38,7 +39,7 @@ def test_reductions_and_their_quotients(name, types):
             out = out_buf[off:off + ref.numel()].view(ref.shape)
             component.into(out, x)
             # a sum of n positive terms in f32 is off by at most n 2^-24 of itself (in whatever order), a quotient by as
-            # much and its own rounding; a bf16 result by one more rounding
+            # much and its own rounding, an exponential by two units in the last place; a bf16 result by one more rounding
             bound = ref.abs() * ((max(rows, cols) + 4) * 2.0 ** -24 + _BITS[dst])
             what = dict(name=name, types=types, rows=rows, cols=cols, off=off, report=component.report())
             assert bool(((out.double() - ref).abs() <= bound).all()), what
@@ -106,3 +107,31 @@ def test_rounding_to_bf16_is_to_nearest_even_and_keeps_nan():
     want = (x + 0.0).to(t.bfloat16)
     assert t.equal(t.isnan(out), t.isnan(x))
     assert t.equal(out[~t.isnan(x)], want[~t.isnan(x)])
+
+
+@pytest.mark.parametrize("static", [False, True])
+def test_the_first_call_with_bf16_operands_may_be_under_capture(static):
+    """A program that has run on f32 operands is captured on bf16 ones: the forms that read those are built then."""
+    from i_amd import Component as i
+
+    scaled, sums = i("ij+j~ij||ij") >> i("ij*.~ij||ij0"), i("+ij~j")
+    two = t.full((), 2.0, device="cuda")
+    x, b = t.randint(-8, 9, (300, 512), device="cuda").float(), t.randint(-8, 9, (512,), device="cuda").float()
+    scaled.exec_torch(x, b, two)
+    sums.exec_torch(x)
+    xb, bb = x.bfloat16(), b.bfloat16()
+    out, total = t.empty(300, 512, device="cuda", dtype=t.bfloat16), t.empty(512, device="cuda")
+    t.cuda.synchronize()
+    graph = t.cuda.CUDAGraph()
+    with t.cuda.graph(graph):
+        scaled.into(out, xb, bb, two, static_workspace=static)
+        sums.into(total, xb, static_workspace=static)
+    for _ in range(3):
+        xb.copy_(t.randint(-8, 9, (300, 512), device="cuda"))
+        out.zero_()
+        total.zero_()
+        t.cuda.synchronize()
+        graph.replay()
+        t.cuda.synchronize()
+        assert t.equal(out, ((xb.float() + bb.float()) * 2).bfloat16()), scaled.report()
+        assert t.equal(total, xb.float().sum(0)), sums.report()
