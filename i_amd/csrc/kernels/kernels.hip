@@ -5,6 +5,7 @@
 #include "attention_bf16_direct.h"
 #include "attention_f32.h"
 #include "attention_f32_direct.h"
+#include "attention_f32_waves.h"
 #include "gemm_narrow.h"
 #include "gemm_nt_bf16.h"
 #include "gemm_nt_f32_direct.h"
@@ -96,6 +97,17 @@ ATTN_F32_DIRECT(128)
   }
 ATTN_F32_DIRECT_PAD(64)
 ATTN_F32_DIRECT_PAD(128)
+// ... 16 query rows per workgroup, the keys in parts over its wavefronts (attention_f32_waves.h)
+#define ATTN_F32_WAVES(DPAD, NW)                                                                                \
+  extern "C" __global__ void __launch_bounds__(NW * 64) attn_fwd_f32_d##DPAD##_bn32_direct_waves##NW(AttnParams p) { \
+    attn_fwd_f32_waves_body<DPAD, NW, false>(p);                                                                \
+  }                                                                                                             \
+  extern "C" __global__ void __launch_bounds__(NW * 64) attn_fwd_f32_d##DPAD##_bn32_direct_pad_waves##NW(AttnParams p) { \
+    attn_fwd_f32_waves_body<DPAD, NW, true>(p);                                                                 \
+  }
+ATTN_F32_WAVES(64, 4)
+ATTN_F32_WAVES(64, 8)
+ATTN_F32_WAVES(128, 4)
 ATTN_F32(32, 32, 4)
 ATTN_F32(64, 32, 4)
 ATTN_F32(128, 32, 4)

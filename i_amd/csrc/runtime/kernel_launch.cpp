@@ -105,6 +105,49 @@ bool attention_supported(DType in_dtype, size_t d, size_t dv, const KernelOption
   return true;
 }
 
+// f32 attention: which kernel, and into how many parts over workgroups the keys go.
+struct F32AttentionPlan {
+  unsigned waves;   // 4 | 8: the kernel whose wavefronts take a part of the keys each (attention_f32_waves.h); 0: query tiles of 128
+  unsigned splits;
+};
+static unsigned attention_tile_splits(DType in_dtype, size_t bh, size_t nq, size_t nk, const AttentionOptions& options);
+static bool f32_waves_supported(size_t nk, size_t d, size_t dv, const KernelOptions& knobs) {
+  const size_t dmax = d > dv ? d : dv;
+  return d % 4 == 0 && dv % 4 == 0 && dmax <= 128 && nk * dmax * 4 < (size_t(1) << 32) && knobs.attention_direct && knobs.attention_kv_parts == 0;
+}
+// A model of the time in us.  Query tiles of 128: 4, and per trip of 32 keys 2.7 (4.7 above 64 columns, 2.4 up to 32) for a
+// CU's only workgroup, 2.3 (4.3, 1.75) for each of several.  16 rows per workgroup: a CU's only one is a chain of steps of 32
+// keys per wavefront; of several, each costs its share of the matrix instructions and of a step.  A split over workgroups
+// costs 6 for the second launch and its pass at 3 TB/s.  Over 1212 shapes from 1 x 1 x 21 x 8 to 512 x 700 x 700 x 128 this choice is 1.98 times as fast as query
+// tiles alone in the mean, and nowhere slower by more than 4 % but for calls of 10 us that wait for the host.  Both sides at
+// the line, us: 160 heads of 512 x 128 219 on tiles, 241 on rows; 16 of 1024 x 64 54 and 47.
+static F32AttentionPlan f32_attention_plan(size_t bh, size_t nq, size_t nk, size_t d, size_t dv, const AttentionOptions& options, bool may_split) {
+  const size_t dmax = d > dv ? d : dv;
+  auto merge = [&](size_t splits) { return splits > 1 ? 6.0 + (double)(bh * splits * nq * dv * 4) / 3e6 : 0.0; };
+  auto of_cu = [](size_t workgroups) { return (double)((workgroups + 255) / 256); };
+  F32AttentionPlan best{0, dmax > 32 && may_split ? attention_tile_splits(F32, bh, nq, nk, options) : 1};
+  if (!f32_waves_supported(nk, d, dv, options.knobs)) return best;
+  const double tiles = of_cu(bh * ((nq + 127) / 128) * best.splits), trips = (double)(((nk + best.splits - 1) / best.splits + 31) / 32);
+  const double alone = dmax <= 32 ? 2.4 : dmax <= 64 ? 2.7 : 4.7, shared = dmax <= 32 ? 1.75 : dmax <= 64 ? 2.3 : 4.3;
+  double least = 0.97 * (4.0 + trips * std::max(alone, shared * tiles) + merge(best.splits));
+  const size_t rows = bh * ((nq + 15) / 16);
+  for (unsigned waves : {8u, 4u}) {
+    if (waves == 8 && dmax > 64) continue;
+    //                      fixed, a step of a CU's only workgroup, per workgroup of several, and per step of it
+    const double cost[4] = {dmax > 64 ? 7.0 : waves == 8 ? 4.2 : 4.0, dmax > 64 ? 2.6 : waves == 8 ? 2.65 : 1.56,
+                            dmax > 64 ? 2.4 : waves == 8 ? 0.8 : 0.45, dmax > 64 ? 2.35 : waves == 8 ? 2.5 : 1.27};
+    for (size_t s = 1; s <= 32 && (s == 1 || (may_split && nk / s >= 32 * waves && rows * s <= 1024)); ++s) {
+      const size_t chunk = s == 1 ? nk : ((nk + s - 1) / s + 63) / 64 * 64, parts = (nk + chunk - 1) / chunk, blocks = (chunk + 31) / 32;
+      const double t = cost[0] + std::max((double)((blocks + waves - 1) / waves) * cost[1], of_cu(rows * parts) * (cost[2] + (double)blocks / waves * cost[3])) + merge(parts);
+      if (t < least) {
+        least = t;
+        best = {waves, (unsigned)parts};
+      }
+    }
+  }
+  return best;
+}
+
 Err launch_attention(const void* q, const void* k, const void* v, void* o, DType in_dtype, DType out_dtype, size_t bh,
                      size_t nq, size_t nk, size_t d, size_t dv, const float* scale_ptr, float scale, hipStream_t stream,
                      const AttentionOptions& options, LaunchNote* note) {
@@ -192,6 +235,11 @@ Err launch_attention(const void* q, const void* k, const void* v, void* o, DType
   const bool f32_direct = in_dtype == F32 && d % 4 == 0 && dv % 4 == 0 && dmax > 32 && dmax <= 128 &&
                           nk * dmax * 4 < (size_t(1) << 32) && aligned16(q) && aligned16(k) && aligned16(v) && aligned16(o) &&
                           knobs.attention_direct;
+  // ... or, where its tiles of 128 query rows leave the CUs little to do, the kernel with 16 rows per workgroup
+  unsigned f32_waves = 0;
+  if (in_dtype == F32 && f32_waves_supported(nk, d, dv, knobs) && aligned16(q) && aligned16(k) && aligned16(v) && aligned16(o))
+    f32_waves = f32_attention_plan(bh, nq, nk, d, dv, options, options.kv_splits > 1).waves;
+  if (f32_waves) bm = 16;
   AttnParams p{};
   p.q = q; p.k = k; p.v = v; p.o = o;
   p.bh = (uint32_t)bh; p.nq = (uint32_t)nq; p.nk = (uint32_t)nk; p.d = (uint32_t)d; p.dv = (uint32_t)dv;
@@ -204,7 +252,7 @@ Err launch_attention(const void* q, const void* k, const void* v, void* o, DType
   // caller's temporaries; attn_kv_merge follows.  (A request that the kernel chosen above cannot honour, the
   // register-staged ones and the 64-queries-per-wave kernel, is ignored: the result is the same.)
   unsigned splits = 1;
-  if (options.kv_splits > 1 && ((in_dtype == BF16 && direct && !q64) || f32_direct)) {
+  if (options.kv_splits > 1 && ((in_dtype == BF16 && direct && !q64) || f32_direct || f32_waves)) {
     if (!options.partial_o || !options.partial_lse) return "attention kernel: a split needs its temporaries";
     p.kv_chunk = (uint32_t)(((nk + options.kv_splits - 1) / options.kv_splits + 63) / 64 * 64);
     splits = (unsigned)((nk + p.kv_chunk - 1) / p.kv_chunk);  // (rounding the parts up to whole tiles may leave fewer)
@@ -233,7 +281,10 @@ Err launch_attention(const void* q, const void* k, const void* v, void* o, DType
     } else if (exact) name = d == 64 ? "attn_fwd_bf16_d64_bn64" : "attn_fwd_bf16_d128_bn64";
     else name = dmax <= 64 ? "attn_fwd_bf16_d64_bn64_any" : "attn_fwd_bf16_d128_bn64_any";
   } else {
-    if (f32_direct) {
+    if (f32_waves) {
+      name = (dmax <= 64 ? "attn_fwd_f32_d64_bn32_direct" : "attn_fwd_f32_d128_bn32_direct") + std::string(d == dv && (d == 64 || d == 128) ? "" : "_pad") + "_waves" + std::to_string(f32_waves);
+      threads = 64 * f32_waves;
+    } else if (f32_direct) {
       // (head sizes other than d == dv in {64, 128}: the same kernel with its LDS rows padded to 64 or 128 columns)
       name = dmax <= 64 ? "attn_fwd_f32_d64_bn32_direct" : "attn_fwd_f32_d128_bn32_direct";
       if (!(d == dv && (d == 64 || d == 128))) name += "_pad";
@@ -243,7 +294,8 @@ Err launch_attention(const void* q, const void* k, const void* v, void* o, DType
   }
   // padded head sizes of which 96 columns cover d and dv: the form that computes no more (its report names it so)
   const bool columns96 = in_dtype == BF16 && direct && padded && !wide && dmax > 64 && dmax <= 96;
-  if (note) *note = LaunchNote{name + (columns96 ? " (96 columns)" : "") + (splits > 1 ? " (keys in " + std::to_string(splits) + " parts)" : ""), bm, bn};
+  const std::string parts = f32_waves ? (splits > 1 ? std::to_string(splits) + " x " : "") + std::to_string(f32_waves) : std::to_string(splits);
+  if (note) *note = LaunchNote{name + (columns96 ? " (96 columns)" : "") + (splits > 1 || f32_waves ? " (keys in " + parts + " parts)" : ""), bm, bn};
   if (columns96) name += "96";
 
   const size_t grid = (size_t(p.bh) * p.nqt + 7) / 8 * 8;  // the query tiles of all heads in 8 equal runs, one per XCD
@@ -265,20 +317,11 @@ Err launch_attention(const void* q, const void* k, const void* v, void* o, DType
 // split gains).  Measured, enqueued back to back, d = 128: one head of 8192 x 8192 92 -> 46 us (4 parts), of
 // 4096 x 4096 48 -> 27, 128 queries x 8192 keys 91 -> 23 (16 parts), 8 heads of 128 x 16384 176 -> 32; from 256
 // workgroups on nothing is gained (16 heads of 4096: 127 -> 146 us with 2 parts).  An f32 workgroup spends four times
-// as long on half the keys, so f32 loops are split from 256 keys on, into parts of at least 64: the reference's
-// demo, one head of 512 x 64, 45 -> 16 us in 8 parts; 2 heads of 128 queries x 8192 keys of 128, 1136 -> 64 in 32.  Only where the direct kernels run (launch_attention's own
-// conditions).
-unsigned attention_kv_splits(DType in_dtype, size_t bh, size_t nq, size_t nk, size_t d, size_t dv, const AttentionOptions& options) {
+// as long on half the keys, so f32 loops on these tiles are split from 256 keys on, into parts of at least 64: 2 heads of
+// 128 queries x 8192 keys of 128, 1136 -> 64 us in 32.  Only where the direct kernels run (launch_attention's own
+// conditions); f32_attention_plan has the last word on f32.
+static unsigned attention_tile_splits(DType in_dtype, size_t bh, size_t nq, size_t nk, const AttentionOptions& options) {
   const KernelOptions& knobs = options.knobs;
-  if (bh == 0 || nq == 0 || d == 0 || dv == 0 || !knobs.attention_direct || knobs.attention_kv_parts == 1) return 1;
-  const size_t dmax = d > dv ? d : dv;
-  if (in_dtype == BF16) {
-    if (d % 8 != 0 || dv % 8 != 0 || d > 256 || dv > 256 || !(nk * dmax * 2 < (size_t(1) << 32))) return 1;
-    if (knobs.attention_waves == 64) return 1;
-    if (options.query_tile == 512) return 1;  // (may select the 64-queries-per-wave kernel)
-  } else if (d % 4 != 0 || dv % 4 != 0 || dmax <= 32 || dmax > 128 || !(nk * dmax * 4 < (size_t(1) << 32))) {
-    return 1;  // (f32: the direct kernel's head sizes; operands it cannot take for their alignment run unsplit)
-  }
   // an f32 workgroup takes about 2.8 us per 32 keys (a bf16 one 0.7 us per 64): much shorter loops are worth parts
   const size_t least_loop = in_dtype == BF16 ? 2048 : 256, least_part = in_dtype == BF16 ? 512 : 64;
   size_t want;
@@ -295,6 +338,22 @@ unsigned attention_kv_splits(DType in_dtype, size_t bh, size_t nq, size_t nk, si
   if (want < 2) return 1;
   const size_t chunk = ((nk + want - 1) / want + 63) / 64 * 64;
   return (unsigned)((nk + chunk - 1) / chunk);
+}
+
+unsigned attention_kv_splits(DType in_dtype, size_t bh, size_t nq, size_t nk, size_t d, size_t dv, const AttentionOptions& options) {
+  const KernelOptions& knobs = options.knobs;
+  if (bh == 0 || nq == 0 || nk == 0 || d == 0 || dv == 0 || !knobs.attention_direct || knobs.attention_kv_parts == 1) return 1;
+  const size_t dmax = d > dv ? d : dv;
+  if (in_dtype == BF16) {
+    if (d % 8 != 0 || dv % 8 != 0 || d > 256 || dv > 256 || !(nk * dmax * 2 < (size_t(1) << 32))) return 1;
+    if (knobs.attention_waves == 64) return 1;
+    if (options.query_tile == 512) return 1;  // (may select the 64-queries-per-wave kernel)
+    return attention_tile_splits(in_dtype, bh, nq, nk, options);
+  }
+  if (f32_waves_supported(nk, d, dv, knobs)) return f32_attention_plan(bh, nq, nk, d, dv, options, true).splits;
+  // (f32: the direct kernels' head sizes; operands they cannot take for their alignment run unsplit)
+  if (d % 4 != 0 || dv % 4 != 0 || dmax <= 32 || dmax > 128 || !(nk * dmax * 4 < (size_t(1) << 32))) return 1;
+  return attention_tile_splits(in_dtype, bh, nq, nk, options);
 }
 
 bool gemm_nt_bf16_supported(size_t k) { return k > 0 && k % 8 == 0; }
