@@ -89,7 +89,14 @@
 // of a padded row is zeros on either side of the products (96 of 128 columns: 2 x 12 heads of 1000 x 1000, d = 80, 22.0 ->
 // 20.0 us; 8 x 16 heads of 2048, d = 96, 232 -> 205; a kernel of its own, since the choice inside the kernel cost the
 // larger head sizes 2 %).
-template <int DPAD, int BN, int NWAVES, bool PRECISE = false, bool PADDED = false, int QB = 1, int DUSE = DPAD>
+//
+// KG: the workgroup's wavefronts form KG groups of NWAVES; every group walks its own KG-th of the keys, with tile memory
+// of its own, and group 0 puts the results together through LDS.  For calls whose time is the chain of a wavefront over all
+// keys, a CU having one workgroup at most: two wavefronts of 32 rows walk an eighth of the tiles each that four walked, and
+// four times the bytes are in flight (84 heads of 1 x 1500, d = 64: 18.5 -> 11.9 us; one head of 1500 x 128: 24.5 -> 18.5).
+// Where the chip is full the shared barrier costs more than it gives (24 heads of 1000, d = 80, in two groups of 128 rows:
+// 21.4 and 20.5; 160 heads 74 and 97): the launcher's rule says when.
+template <int DPAD, int BN, int NWAVES, bool PRECISE = false, bool PADDED = false, int QB = 1, int DUSE = DPAD, int KG = 1>
 __device__ __forceinline__ void attn_fwd_bf16_direct_body(const AttnParams& p) {
   static_assert(DUSE == DPAD || (PADDED && DUSE < DPAD && DUSE % 32 == 0), "columns in use");
   constexpr int BM = 32 * QB * NWAVES;
@@ -110,7 +117,7 @@ __device__ __forceinline__ void attn_fwd_bf16_direct_body(const AttnParams& p) {
   constexpr int WLW = SPLIT ? 1 : WL / NWAVES;  // ... per wave
   static_assert(RB == 128 || RB == 256 || RB == 512, "row size");
   static_assert(SPLIT ? 2 * WL == NWAVES : WL % NWAVES == 0, "tile / wave shape");
-  __shared__ __attribute__((aligned(1024))) char smem[2][2][TILE_BYTES];  // [buffer][K, V]
+  __shared__ __attribute__((aligned(1024))) char smem_all[KG][2][2][TILE_BYTES];  // [group][buffer][K, V]
 
   uint32_t head, qt;
   xcd_map(blockIdx.x, p.nqt, p.bh, head, qt);
@@ -119,7 +126,9 @@ __device__ __forceinline__ void attn_fwd_bf16_direct_body(const AttnParams& p) {
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave_id = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave = KG == 1 ? wave_id : wave_id % NWAVES, group = KG == 1 ? 0 : wave_id / NWAVES;
+  char (&smem)[2][2][TILE_BYTES] = smem_all[group];
   const int c = lane & 31;  // query column within the wave / A-operand row
   const int h = lane >> 5;  // half-wave
   const uint32_t d = PADDED ? p.d : (uint32_t)DPAD;    // elements per row of Q and K in global memory
@@ -136,6 +145,15 @@ __device__ __forceinline__ void attn_fwd_bf16_direct_body(const AttnParams& p) {
     qhead = head / p.kv_splits;
     first_key = (head - qhead * p.kv_splits) * p.kv_chunk;
     nk = p.nk - first_key < p.kv_chunk ? p.nk - first_key : p.kv_chunk;
+  }
+  // The group's tiles of 64 or 32 keys (at least one: the launcher sees to it).  Loops with barriers run as often for every
+  // group: as many steady trips as the group with the fewest full tiles has, as many trips as the one with the most tiles.
+  const uint32_t all_tiles = (nk + BN - 1) / BN;
+  [[maybe_unused]] const uint32_t fewest_full = all_tiles / KG - (nk % BN != 0 ? 1 : 0);  // (the last group holds a partial tile)
+  if constexpr (KG > 1) {
+    const uint32_t t0 = all_tiles * group / KG, t1 = all_tiles * (group + 1) / KG;
+    first_key += t0 * BN;
+    nk = t1 * BN < nk ? (t1 - t0) * BN : nk - t0 * BN;
   }
   const bf16_t* __restrict__ Q = reinterpret_cast<const bf16_t*>(p.q) + (size_t)qhead * p.nq * d;
   const char* __restrict__ K = reinterpret_cast<const char*>(p.k) + ((size_t)qhead * p.nk + first_key) * RBG;
@@ -353,7 +371,8 @@ __device__ __forceinline__ void attn_fwd_bf16_direct_body(const AttnParams& p) {
       const bool move = first || (mx - m_run[b]) * scale_log2 > RESCALE_LOG2;
       const float m_new = move ? mx : m_run[b];
       const float alpha = first ? 0.0f : fast_exp2((m_run[b] - m_new) * scale_log2);  // 1 when the reference stays
-      const float mb = m_new * scale_log2;
+      // (KG > 1: a group whose scores are all -inf weighs nothing)
+      const float mb = KG > 1 && m_new == -INFINITY ? 0.0f : m_new * scale_log2;
       m_run[b] = m_new;
 
       // P = exp(S - m) rounded to bf16 (the PV operand); the row sum is taken over the rounded values
@@ -411,6 +430,8 @@ __device__ __forceinline__ void attn_fwd_bf16_direct_body(const AttnParams& p) {
   using Yes = std::integral_constant<bool, true>;
   const uint32_t ntiles = (nk + BN - 1) / BN;
   const uint32_t nfull = nk / BN;  // tiles that lie entirely inside nk
+  const uint32_t trips = KG == 1 ? ntiles : (all_tiles + KG - 1) / KG;
+  const uint32_t nfull_trips = KG == 1 ? nfull : fewest_full;
 
   // Software pipeline: the scores of tile j+1 are computed (matrix pipe) in the same iteration as the
   // softmax of tile j (vector pipe).  K is therefore consumed one iteration before V: K(j+2) and V(j+1)
@@ -450,7 +471,7 @@ __device__ __forceinline__ void attn_fwd_bf16_direct_body(const AttnParams& p) {
   constexpr int NPRE = QB * (DT + NQK); // slots that carry the exponentials (all before the first PV slot of the tile)
   constexpr int NMAIN = NPV - DT;       // V operands of the trip that owns the tile
   constexpr int XLEAD = QB > 1 ? ATTN_Q64_XLEAD : ATTN_XLEAD;
-  static_assert(NPAIR % 4 == 0 && 2 * WLW <= NPRE && XLEAD >= 0 && XLEAD < NQK, "slot shape");
+  static_assert(NPAIR % 4 == 0 && XLEAD >= 0 && XLEAD < NQK, "slot shape");
 
   struct Carry {
     bf16x8 a[DT];  // V^T operands of the last 16-key group
@@ -529,15 +550,21 @@ __device__ __forceinline__ void attn_fwd_bf16_direct_body(const AttnParams& p) {
       }
       if (g + XLEAD < NOP) fetch(g + XLEAD);
     };
-    // request g of the 2 WLW global -> LDS requests of the trip
+    // request g of the 2 WLW global -> LDS requests of the trip, one per slot
+    auto request_one = [&](int g) {
+      if (g < WLW) {
+        if constexpr (decltype(any_k_tag)::value) request_k_one(j + 2, buf, g);
+        else request_full_one(j + 2, buf, g, Yes{});
+      } else {
+        request_full_one(j + 1, buf ^ 1, g - WLW, No{});
+      }
+    };
     auto request_for_slot = [&](int g) {
-      if (g < 2 * WLW) {
-        if (g < WLW) {
-          if constexpr (decltype(any_k_tag)::value) request_k_one(j + 2, buf, g);
-          else request_full_one(j + 2, buf, g, Yes{});
-        } else {
-          request_full_one(j + 1, buf ^ 1, g - WLW, No{});
-        }
+      if constexpr (2 * WLW <= NPRE) {
+        if (g < 2 * WLW) request_one(g);
+      } else {  // (a wavefront that brings a whole tile by itself: more than one per slot)
+#pragma unroll
+        for (int r = g * 2 * WLW / NPRE; r < (g + 1) * 2 * WLW / NPRE; ++r) request_one(r);
       }
     };
 
@@ -672,8 +699,8 @@ __device__ __forceinline__ void attn_fwd_bf16_direct_body(const AttnParams& p) {
   // tiles 0 and 1 of K and tile 0 of V into LDS, then S(0)
   if constexpr (PADDED) {
     // the tile memory, cleared once: what no transfer ever writes (the columns past d) then reads as zero
-    for (uint32_t at = 16 * tid; at < 4 * TILE_BYTES; at += 16 * 64 * NWAVES)
-      *reinterpret_cast<u32x4*>(&smem[0][0][0] + at) = u32x4{0, 0, 0, 0};
+    for (uint32_t at = 16 * tid; at < KG * 4 * TILE_BYTES; at += 16 * 64 * NWAVES * KG)
+      *reinterpret_cast<u32x4*>(&smem_all[0][0][0][0] + at) = u32x4{0, 0, 0, 0};
     __syncthreads();
   }
   auto first_tiles = [&]() {
@@ -693,11 +720,11 @@ __device__ __forceinline__ void attn_fwd_bf16_direct_body(const AttnParams& p) {
   // for the second pass of an item), and a second score tile alive next to the softmax's temporaries is what
   // would push the kernel over its register budget.
   auto general_loop = [&](uint32_t j) {
-    for (; j < ntiles; ++j) {
+    for (; j < trips; ++j) {
       const int buf = j & 1;
       if (j + 2 < ntiles) request_k(j + 2, buf);
       if (j + 1 < ntiles) request_v(j + 1, buf ^ 1);
-      softmax_pv(sa, j, buf, j >= nfull);
+      if (KG == 1 || j < ntiles) softmax_pv(sa, j, buf, j >= nfull);
       if (j + 1 < ntiles) qk(sa, buf ^ 1);
       dma_wait_all();
       __syncthreads();
@@ -706,7 +733,17 @@ __device__ __forceinline__ void attn_fwd_bf16_direct_body(const AttnParams& p) {
   first_tiles();
 
   uint32_t j = 0;
-  const bool steady = nfull >= 4;
+  bool steady = nfull_trips >= 4;
+  if constexpr (KG > 1 && !NOREF) {
+    // a wavefront whose first tile has a row of nothing but -inf has no reference to start from: the general loop finds one
+    // (the same requests and barriers, trip by trip)
+    float mx = sa[0][0][0];
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) mx = fmaxf(mx, sa[0][kt][i]);
+    if (__builtin_amdgcn_ballot_w64(half_max(mx) == -INFINITY)) steady = false;
+  }
   if (steady) {
 #pragma unroll
     for (int b = 0; b < QB; ++b) {
@@ -745,7 +782,7 @@ __device__ __forceinline__ void attn_fwd_bf16_direct_body(const AttnParams& p) {
     for (int t = 0; t < DT; ++t) ca.a[t] = __builtin_bit_cast(bf16x8, u32x4{0, 0, 0, 0});
 #pragma unroll
     for (int b = 0; b < QB; ++b) ca.p[b] = u32x4{0, 0, 0, 0};
-    for (; j + 4 <= nfull; j += 2) {  // j + 3 <= nfull - 1
+    for (; j + 4 <= nfull_trips; j += 2) {  // j + 3 <= nfull - 1
       fast_step(j, 0, sa, sb, ca, cb, No{});
       fast_step(j + 1, 1, sb, sa, cb, ca, No{});
     }
@@ -787,12 +824,12 @@ __device__ __forceinline__ void attn_fwd_bf16_direct_body(const AttnParams& p) {
         lane_bad = lane_bad || !(row_sum > 0x1p-100f && row_sum < INFINITY);
       }
       // one word per wave in the tile memory, which nobody reads any more after the loop's last barrier
-      int* wave_flags = reinterpret_cast<int*>(&smem[0][0][0]);
-      if (lane == 0) wave_flags[wave] = __builtin_amdgcn_ballot_w64(lane_bad) != 0;
+      int* wave_flags = reinterpret_cast<int*>(&smem_all[0][0][0][0]);
+      if (lane == 0) wave_flags[wave_id] = __builtin_amdgcn_ballot_w64(lane_bad) != 0;
       __syncthreads();
       int redo = 0;
 #pragma unroll
-      for (int w = 0; w < NWAVES; ++w) redo |= wave_flags[w];
+      for (int w = 0; w < NWAVES * KG; ++w) redo |= wave_flags[w];
       __syncthreads();  // every wave has read the flags before tile requests or the epilogue overwrite them
       if (redo != 0) {
         // throw the pass away and compute the item again, every tile through the general loop
@@ -809,6 +846,55 @@ __device__ __forceinline__ void attn_fwd_bf16_direct_body(const AttnParams& p) {
         general_loop(0);
       }
     }
+  }
+
+  if constexpr (KG > 1) {
+    // ---- the groups put together.  Tile memory is free after the loop's last barrier: per group but the first, (reference,
+    // row sum) and O of its wavefronts as they hold them, 16 bytes per lane and access.
+    static_assert(QB == 1 && (KG - 1) * NWAVES * (DT * 4096 + 512) <= KG * 4 * TILE_BYTES, "tile memory holds the groups' results");
+    constexpr int PER_WAVE = DT * 4096 + 512;
+    char* const left = &smem_all[0][0][0][0];
+    const float sum = half_sum(l_run[0]);
+    if (group > 0) {
+      char* to = left + ((group - 1) * NWAVES + wave) * PER_WAVE;
+#pragma unroll
+      for (int t = 0; t < DT; ++t)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) *reinterpret_cast<f32x4*>(to + (4 * t + g) * 1024 + 16 * lane) = f32x4{o[0][t][4 * g], o[0][t][4 * g + 1], o[0][t][4 * g + 2], o[0][t][4 * g + 3]};
+      *reinterpret_cast<float*>(to + DT * 4096 + 4 * lane) = m_run[0];
+      *reinterpret_cast<float*>(to + DT * 4096 + 256 + 4 * lane) = sum;
+    }
+    __syncthreads();
+    if (group == 0) {
+      float top = m_run[0];
+#pragma unroll
+      for (int n = 0; n < KG - 1; ++n) top = fmaxf(top, *reinterpret_cast<const float*>(left + (n * NWAVES + wave) * PER_WAVE + DT * 4096 + 4 * lane));
+      auto weight_of = [&](float m) { return m == -INFINITY ? 0.0f : fast_exp2((m - top) * scale_log2); };
+      const float own = weight_of(m_run[0]);
+      l_run[0] = sum * own;
+#pragma unroll
+      for (int t = 0; t < DT; ++t)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[0][t][i] *= own;
+#pragma unroll
+      for (int n = 0; n < KG - 1; ++n) {
+        const char* from = left + (n * NWAVES + wave) * PER_WAVE;
+        const float weight = weight_of(*reinterpret_cast<const float*>(from + DT * 4096 + 4 * lane));
+        l_run[0] += weight * *reinterpret_cast<const float*>(from + DT * 4096 + 256 + 4 * lane);
+#pragma unroll
+        for (int t = 0; t < DT; ++t)
+#pragma unroll
+          for (int g = 0; g < 4; ++g) {
+            const f32x4 x = *reinterpret_cast<const f32x4*>(from + (4 * t + g) * 1024 + 16 * lane);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[0][t][4 * g + e] += weight * x[e];
+          }
+      }
+      m_run[0] = top;
+    }
+    __syncthreads();  // (the store below stages rows in the same memory)
+    if (group > 0) return;
+    l_run[0] *= 0.5f;  // (both halves of the wavefront hold the whole row's sum: the store adds them up)
   }
 
   // ---- epilogue: normalise and store.  Lane (c, h) holds O[q = c][32 t + 8 g + 4 h + e] of each of its blocks.

@@ -74,6 +74,22 @@ ATTN_BF16_DIRECT(256, 32, 4, 1, , false)
 ATTN_BF16_DIRECT_PAD(256, 32, 4, 1, , false)
 ATTN_BF16_DIRECT(256, 32, 4, 1, _f32scale, true)
 ATTN_BF16_DIRECT_PAD(256, 32, 4, 1, _f32scale, true)
+// KG groups of NW waves, each on its own part of the keys: few query rows per workgroup, one workgroup per CU (K/V tiles of
+// all groups fill its LDS)
+#define ATTN_BF16_GROUPS(DPAD, BN, NW, KG)                                                                       \
+  extern "C" __global__ void __launch_bounds__(NW * KG * 64, 1) attn_fwd_bf16_d##DPAD##_bn##BN##_direct_w##NW##_k##KG(AttnParams p) { \
+    attn_fwd_bf16_direct_body<DPAD, BN, NW, false, false, 1, DPAD, KG>(p);                                        \
+  }                                                                                                              \
+  extern "C" __global__ void __launch_bounds__(NW * KG * 64, 1) attn_fwd_bf16_d##DPAD##_bn##BN##_direct_w##NW##_k##KG##_pad(AttnParams p) { \
+    attn_fwd_bf16_direct_body<DPAD, BN, NW, false, true, 1, DPAD, KG>(p);                                         \
+  }
+ATTN_BF16_GROUPS(64, 32, 1, 8)
+ATTN_BF16_GROUPS(64, 64, 2, 4)
+ATTN_BF16_GROUPS(128, 32, 2, 4)
+ATTN_BF16_GROUPS(256, 32, 2, 2)
+extern "C" __global__ void __launch_bounds__(512, 1) attn_fwd_bf16_d128_bn32_direct_w2_k4_pad96(AttnParams p) {
+  attn_fwd_bf16_direct_body<128, 32, 2, false, true, 1, 96, 4>(p);
+}
 // d = 64 with 64 queries per wave (two query blocks): 8 waves, 512 query rows per workgroup, 32-key tiles
 extern "C" __global__ void __launch_bounds__(512, 1) attn_fwd_bf16_d64_bn32_q64(AttnParams p) {
   attn_fwd_bf16_direct_body<64, 32, 8, false, false, 2>(p);

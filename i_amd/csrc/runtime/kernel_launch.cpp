@@ -148,6 +148,29 @@ static F32AttentionPlan f32_attention_plan(size_t bh, size_t nq, size_t nk, size
   return best;
 }
 
+// bf16: into how many parts a workgroup's waves take the keys (1: all waves walk all keys).  A model of the time in us
+// where every CU has at most one workgroup: a fixed part and a chain of trips, of 64 keys (32 above 128 columns) for the kernels
+// with 128 query rows, of 32 or 64 keys times the groups for these.  Their K/V tiles fill the LDS of a CU, so grids of more
+// workgroups than CUs stay where they are (400 heads of 1 x 1500 x 128: 55 us, in groups 61), and so do loops that are long
+// enough for parts over workgroups.  Measured, us: one head of 1500 x
+// 128 24.5 -> 18.5, x 64 18.3 -> 12; 84 heads of 1 x 1500, d = 64 18.5 -> 11.9, 128 24.3 -> 19.8, 184 42.7 -> 36; but 200 of 1 x
+// 2048 x 128, where reading K and V is the bound, 34.2 and 35.8.
+static unsigned attention_key_groups(size_t bh, size_t nq, size_t nk, size_t dmax, const AttentionOptions& options) {
+  const KernelOptions& knobs = options.knobs;
+  const size_t tile = options.query_tile;
+  if (knobs.attention_f32_scale || knobs.attention_waves || knobs.attention_kv_parts || tile == 64 || tile == 128 || tile == 256 || tile == 512) return 1;
+  const size_t rows64 = bh * ((nq + 63) / 64), rows32 = bh * ((nq + 31) / 32);
+  if (rows64 > 256 || attention_tile_splits(BF16, bh, nq, nk, options) > 1) return 1;
+  auto chain = [nk](double fixed, size_t keys, double trip) { return fixed + (double)((nk + keys - 1) / keys) * trip; };
+  if (dmax <= 64) {
+    const double whole = chain(4.5, 64, 0.56);
+    if (rows32 <= 256 && nk >= 256 && chain(7.2, 256, 0.53) < 0.97 * whole) return 8;
+    return nk >= 256 && chain(8.0, 256, 0.7) < 0.97 * whole ? 4 : 1;
+  }
+  if (dmax <= 128) return nk >= 128 && rows64 <= 192 && chain(8.5, 128, 0.66) < 0.97 * chain(6.3, 64, 0.72) ? 4 : 1;
+  return nk >= 64 && chain(14.0, 64, 0.9) < 0.97 * chain(8.8, 32, 0.72) ? 2 : 1;
+}
+
 Err launch_attention(const void* q, const void* k, const void* v, void* o, DType in_dtype, DType out_dtype, size_t bh,
                      size_t nq, size_t nk, size_t d, size_t dv, const float* scale_ptr, float scale, hipStream_t stream,
                      const AttentionOptions& options, LaunchNote* note) {
@@ -229,6 +252,12 @@ Err launch_attention(const void* q, const void* k, const void* v, void* o, DType
     }
     if (q64) { bm = 512; bn = 32; }
   }
+  // ... and where nothing is asked for and a chain over all keys is what a call waits for: groups of waves on parts of the keys
+  const unsigned groups = direct && !q64 && options.kv_splits <= 1 ? attention_key_groups(bh, nq, nk, dmax, options) : 1;
+  if (groups > 1) {
+    bm = groups == 8 ? 32 : 64;
+    bn = groups == 4 && dmax <= 64 ? 64 : 32;
+  }
   // f32: the direct-to-LDS kernel for d, dv multiples of 4 up to 128, the larger above 32 (16-byte aligned operands,
   // 32-bit byte offsets inside a head; up to 32 the register-staged kernel with 32-column tiles is the faster one), the
   // register-staged kernel with guarded columns otherwise (and with knobs.attention_direct == 0)
@@ -274,7 +303,11 @@ Err launch_attention(const void* q, const void* k, const void* v, void* o, DType
       threads = bm;
     } else if (direct) {
       name = "attn_fwd_bf16_d" + std::to_string(wide ? 256 : padded ? (dmax <= 64 ? 64 : 128) : d) + "_bn" + std::to_string(bn) + "_direct";
-      if (bm == 64) name += "_w2";
+      if (bm <= 64) name += bm == 64 ? "_w2" : "_w1";
+      if (groups > 1) {
+        name += "_k" + std::to_string(groups);
+        threads *= groups;
+      }
       if (bm == 256) name += "_w8";
       if (f32_scale) name += "_f32scale";
       if (padded) name += "_pad";
