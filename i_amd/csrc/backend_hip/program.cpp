@@ -386,7 +386,7 @@ ihip::Err launch_product_f32(Run& run, const void* a, const void* b, void* c, si
                              ihip::LaunchNote* note, size_t b_cols = 0) {
   void* partial = nullptr;
   unsigned splits = ihip::gemm_nt_f32_split_k(bh, m, n, k, run.knobs);
-  if (splits > 1 && ((m * n) % 4 != 0 || !run.alloc_optional(&partial, bh * splits * m * n * 4))) splits = 1;
+  if (splits > 1 && !run.alloc_optional(&partial, bh * splits * m * n * 4)) splits = 1;
   return ihip::launch_gemm_nt_f32(static_cast<const float*>(a), static_cast<const float*>(b), static_cast<float*>(c), bh, m, n, k,
                                   run.stream, note, static_cast<float*>(partial), splits, run.knobs, b_cols);
 }
@@ -653,7 +653,7 @@ ihip::Err launch_hand_noted(Run& run, const Recognized& r, const Step& step, ihi
       if (t == DType::F32) return launch_product_f32(run, pa, pb, out, bh, a[nb], b[nb], k, note);
       // few output tiles under a long k loop: the loop is split over workgroups, partial products in a temporary
       if (const unsigned splits = tile_asked && run.knobs.gemm_k_parts < 2 ? 1u : ihip::gemm_nt_bf16_split_k(bh, a[nb], b[nb], k, run.knobs);
-          splits > 1 && (a[nb] * b[nb]) % 4 == 0) {
+          splits > 1) {
         void* partial = nullptr;
         if (run.alloc_optional(&partial, bh * splits * a[nb] * b[nb] * 4))  // (no room for it: the unsplit kernel)
           return ihip::launch_gemm_nt_bf16_split_k(pa, pb, out, static_cast<float*>(partial), splits, bh, a[nb], b[nb], k, run.stream,
@@ -700,7 +700,7 @@ ihip::Err launch_hand_noted(Run& run, const Recognized& r, const Step& step, ihi
         if (f32) return launch_product_f32(run, pa, pb, out, bh, m, n, kp, note, b_cols);
         unsigned splits = tile_asked && run.knobs.gemm_k_parts < 2 ? 1u : ihip::gemm_nt_bf16_split_k(bh, m, n, kp, run.knobs);
         void* partial = nullptr;
-        if (splits > 1 && ((m * n) % 4 != 0 || !run.alloc_optional(&partial, bh * splits * m * n * 4))) splits = 1;
+        if (splits > 1 && !run.alloc_optional(&partial, bh * splits * m * n * 4)) splits = 1;
         return ihip::launch_gemm_nn_bf16(pa, pb, out, bh, m, n, kp, run.stream, r.tile_i, r.tile_j, note, out_dt,
                                          static_cast<float*>(partial), splits, run.knobs, b_cols);
       }

@@ -326,22 +326,35 @@ __device__ __forceinline__ void transpose_body(const TransposeParams& p) {
   for (uint32_t y = y0; y < 64; y += 4)
     if (c0 + y < p.cols && r0 + x < p.rows) dst[(size_t)(c0 + y) * p.rows + r0 + x] = tile[x][y];
 }
-// the partial products of a GEMM whose k loop was split over workgroups, added up in split order
+// The partial products of a GEMM whose k loop was split over workgroups, added up in split order, four to a work-item.  Any
+// count: the accesses need the alignment of the elements only, and the last four of a product may be fewer (before, a
+// product of m n outputs ran its k loop whole unless 4 divided m n: bf16 161 x 211 x 4022 64 us, now 21).
 extern "C" __global__ void __launch_bounds__(256) splitk_reduce(SplitReduceParams p) {
-  const uint64_t quads = p.count / 4, total = (uint64_t)p.batches * quads;
+  typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+  typedef __bf16 bf16x4_any __attribute__((ext_vector_type(4), aligned(2)));
+  const uint64_t quads = (p.count + 3) / 4, total = (uint64_t)p.batches * quads;
   for (uint64_t at = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; at < total; at += (uint64_t)gridDim.x * blockDim.x) {
-    const uint64_t b = at / quads, i = at - b * quads;
-    const f32x4* src = reinterpret_cast<const f32x4*>(p.partial + (size_t)b * p.splits * p.count) + i;
-    f32x4 sum = src[0];
+    const uint64_t b = at / quads, i = 4 * (at - b * quads), to = b * p.count + i;
+    const float* src = p.partial + (size_t)b * p.splits * p.count + i;
+    if (i + 4 > p.count) {
+      for (uint32_t e = 0; e < p.count - i; ++e) {
+        float sum = src[e];
+        for (uint32_t s = 1; s < p.splits; ++s) sum += src[(size_t)s * p.count + e];
+        if (p.out_bf16) reinterpret_cast<bf16_t*>(p.out)[to + e] = (bf16_t)sum;
+        else reinterpret_cast<float*>(p.out)[to + e] = sum;
+      }
+      continue;
+    }
+    f32x4 sum = *reinterpret_cast<const f32x4_any*>(src);
 #pragma unroll 8
-    for (uint32_t s = 1; s < p.splits; ++s) sum += src[(size_t)s * quads];  // (unrolled: eight loads in flight per lane)
+    for (uint32_t s = 1; s < p.splits; ++s) sum += *reinterpret_cast<const f32x4_any*>(src + (size_t)s * p.count);  // (unrolled: eight loads in flight per lane)
     if (p.out_bf16) {
       bf16x4 v;
 #pragma unroll
       for (int e = 0; e < 4; ++e) v[e] = (bf16_t)sum[e];
-      reinterpret_cast<bf16x4*>(p.out)[at] = v;
+      *reinterpret_cast<bf16x4_any*>(reinterpret_cast<bf16_t*>(p.out) + to) = v;
     } else {
-      reinterpret_cast<f32x4*>(p.out)[at] = sum;
+      *reinterpret_cast<f32x4_any*>(reinterpret_cast<float*>(p.out) + to) = sum;
     }
   }
 }

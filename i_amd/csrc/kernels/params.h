@@ -62,7 +62,7 @@ struct GemmParams {
   uint32_t b_cols;    // row-major right operand (NN): elements per row of B, at least n (n, or n rounded up by a padded copy)
 };
 
-// out[b][i] = sum over s < splits of partial[b][s][i], i < count (count a multiple of 4); out f32 or bf16
+// out[b][i] = sum over s < splits of partial[b][s][i], i < count; out f32 or bf16
 struct SplitReduceParams {
   const float* partial;
   void* out;

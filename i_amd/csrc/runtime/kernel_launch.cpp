@@ -496,53 +496,59 @@ Err launch_gemm_nt_bf16(const void* a, const void* b, void* c, size_t bh, size_t
   return launch(fn, (unsigned)grid, 1, 1, 256, &p, sizeof(p), stream);
 }
 
-// Tile of a split product: the large tile needs both extents to fill most of it
-static unsigned split_k_tile(size_t m, size_t n) { return m >= 192 && n >= 192 ? 256 : 128; }
+// A model of a product's time in us on 128 x 128 or 256 x 256 tiles with k in `parts` of `slabs` 64-wide slabs: a workgroup
+// spends 0.7 us per slab on a 128 x 128 tile (0.8 when the operands, beyond the 32 MB of the L2s, come from HBM, whose latency a
+// CU's only workgroup waits for; 0.95 when two share a CU) plus two slabs' worth before and after its loop, 1.4 us per slab and
+// 9 on a 256 x 256 tile; the chip holds 512 / 256 of them at a time; the second launch costs 5 us and the pass over the
+// partial products runs at 3 TB/s.  The workgroups that count are those launched, the tiles of a batch and part rounded up to
+// one per XCD (fewer than four small ones: to four): the empty ones leave at once but leave holes (8 x 27 x 704 x 7960, 6 tiles
+// a batch: 25 us in 8 parts = 512 workgroups, 34 in 9; 64 x 16 x 512 x 1024, 4 tiles: 16 whole, 22 in 2).
+static double split_k_time(unsigned tile, size_t bh, size_t m, size_t n, size_t k, size_t parts, size_t slabs) {
+  const size_t tiles = ((m + tile - 1) / tile) * ((n + tile - 1) / tile);  // of a batch
+  const size_t workgroups = (tile == 128 && tiles < 4 ? 4 : (tiles + 7) / 8 * 8) * bh * parts;
+  const double rounds = (double)((workgroups + (tile == 128 ? 511 : 255)) / (tile == 128 ? 512 : 256));
+  const bool far = bh * (m + n) * k * 2 > (size_t(32) << 20);
+  const double loop = tile == 256 ? (double)slabs * 1.4 + 9.0 : (double)(slabs + 2) * (workgroups > 256 ? 0.95 : far ? 0.8 : 0.7);
+  return rounds * loop + (parts > 1 ? 5.0 + (double)(bh * parts * m * n * 4) / 3e6 : 0.0);
+}
 
+// Tile of a product whose k loop is in parts.  The large one only where both extents fill it and the parts are long: on 110
+// products from 20 x 100 x 512 to 3500 x 3500 x 12000 the best of all parts of 128-tiles is 1.19 times as fast as the best of
+// 256-tiles, which lead on one (2854 x 1184 x 3880, 50.5 against 51.4 us; 402 x 896 x 2080 takes 14.2 on 128-tiles, 26.4 on those).
+static unsigned split_k_tile(size_t bh, size_t m, size_t n, size_t k, unsigned splits) {
+  if (m < 192 || n < 192) return 128;
+  const size_t slabs = ((k + splits - 1) / splits + 63) / 64;
+  return split_k_time(256, bh, m, n, k, splits, slabs) < split_k_time(128, bh, m, n, k, splits, slabs) ? 256 : 128;
+}
+
+// Into how many parts to cut k: by the model, parts of at least two slabs, where that gains 10 %.  Examples (whole -> parts):
+// 64 x 8192 x 8192 79 -> 30 us in 8, 512 x 512 x 4096 52 -> 16, 461 x 1535 x 4592 55 -> 24 in 5, 256 x 256 x 65536 576 -> 32 in
+// 32, 2 x 9304 x 2904 37 -> 17 in 5; left whole: 1024^3 (10 us), 2048^3 (28; 40 in 2).  The choice is 2.7 % behind the best of
+// all parts in the mean of those 110 products; with 256-tiles wherever they fit and parts of at least 512 it was 20 %.
 unsigned gemm_nt_bf16_split_k(size_t bh, size_t m, size_t n, size_t k, const KernelOptions& knobs) {
   if (bh == 0 || m == 0 || n == 0 || k % 8 != 0 || knobs.gemm_k_parts == 1) return 1;
-  const unsigned tile = split_k_tile(m, n);
-  if (knobs.gemm_k_parts > 1) {  // (tests, searches and measurements: that many parts, whole slabs each)
+  auto chunk_of = [k](size_t want) { return (k / want + 63) / 64 * 64; };  // what one part contracts: whole slabs
+  if (knobs.gemm_k_parts > 1) {  // (tests, searches and measurements: that many parts)
     const size_t want = std::min<size_t>((size_t)knobs.gemm_k_parts, k / 64);
     if (want < 2 || bh * want > 65535) return 1;
-    const size_t chunk = (k / want + 63) / 64 * 64;
-    return (unsigned)((k + chunk - 1) / chunk);
+    return (unsigned)((k + chunk_of(want) - 1) / chunk_of(want));
   }
-  // A model of the time in us: a workgroup spends 0.7 us per 64-wide slab on a 128 x 128 tile (0.9 when the operands, beyond
-  // the 32 MB of the L2s, come from HBM, whose latency a CU's only workgroup waits for; 1.1 when two share a CU), 1.4 us on
-  // a 256 x 256 tile, plus two slabs' worth before and after its loop; the chip holds 512 / 256 of them at a time; the
-  // second launch costs 4 us and the pass over the partial products runs at 3 TB/s.  The workgroups that count are those
-  // launched, the tiles of a batch and part rounded up to one per XCD (fewer than four small ones: to four): the empty ones
-  // leave at once but leave holes (8 x 27 x 704 x 7960, 6 tiles a batch: 25 us in 8 parts = 512 workgroups, 34 in 9; 64 x 16 x 512 x
-  // 1024, 4 tiles: 16 whole, 22 in 2).  On 150 products of either layout from 16 x 1072 x 48 to 4 x 88 x 6504 x 6904 the
-  // choice is 3.9 % behind the best of all parts in the mean (10 % with tiles counted instead of workgroups, and 10 % with
-  // parts that are powers of two only).  Examples (unsplit -> split): 64 x 8192 x 8192 79 -> 30 us in 8 parts, 512 x 512 x
-  // 4096 52 -> 27 in 8, 256 x 4096 x 4096 41 -> 29 in 8, 256 x 256 x 65536 576 -> 49 in 32, 2 x 9304 x 2904 37 -> 17 in 5;
-  // left whole: 1024^3 (10 us; 25 in 2 parts), 2048^3 (28; 40).
-  if (k > (size_t(1) << 22)) return 1;
-  const size_t slabs = (k + 63) / 64;
-  const size_t t128 = ((m + 127) / 128) * ((n + 127) / 128), t256 = ((m + 255) / 256) * ((n + 255) / 256);  // of a batch
-  const bool far = bh * (m + n) * k * 2 > (size_t(32) << 20);
-  auto time_of = [far, bh](unsigned tile_, size_t tiles_, size_t parts, size_t slabs_) {
-    const size_t workgroups = (tile_ == 128 && tiles_ < 4 ? 4 : (tiles_ + 7) / 8 * 8) * bh * parts;
-    const double rounds = (double)((workgroups + (tile_ == 128 ? 511 : 255)) / (tile_ == 128 ? 512 : 256));
-    return rounds * (double)(slabs_ + 2) * (tile_ == 256 ? 1.4 : workgroups > 256 ? 1.1 : far ? 0.9 : 0.7);
-  };
-  double best = time_of(128, t128, 1, slabs);
-  if (t256 * bh >= 64) best = std::min(best, time_of(256, t256, 1, slabs));
-  best *= 0.9;  // a split has to gain at least 10 %
+  if (k < 1024 || k > (size_t(1) << 22)) return 1;  // (short loops: 45 x 936 x 880 9.9 us whole, 11.1 in 5 parts)
+  const size_t slabs = (k + 63) / 64, t256 = ((m + 255) / 256) * ((n + 255) / 256);
+  double best = split_k_time(128, bh, m, n, k, 1, slabs);
+  if (t256 * bh >= 64) best = std::min(best, split_k_time(256, bh, m, n, k, 1, slabs));
+  best *= 0.9;
   size_t splits = 1;
-  for (size_t s = 2; s <= 32 && k / s >= 512 && bh * s <= 65535; ++s) {
-    const size_t chunk = (k / s + 63) / 64 * 64, parts = (k + chunk - 1) / chunk;
-    const double t = time_of(tile, tile == 256 ? t256 : t128, parts, chunk / 64) + 4.0 + (double)(bh * parts * m * n * 4) / 3e6;
+  for (size_t s = 2; s <= 32 && k / s >= 128 && bh * s <= 65535; ++s) {
+    const size_t chunk = chunk_of(s), parts = (k + chunk - 1) / chunk;
+    double t = split_k_time(128, bh, m, n, k, parts, chunk / 64);
+    if (m >= 192 && n >= 192) t = std::min(t, split_k_time(256, bh, m, n, k, parts, chunk / 64));
     if (t < best) {
       best = t;
-      splits = s;
+      splits = parts;
     }
   }
-  if (splits < 2) return 1;
-  const size_t chunk = (k / splits + 63) / 64 * 64;  // what one split contracts: whole 64-wide slabs
-  return (unsigned)((k + chunk - 1) / chunk);
+  return (unsigned)splits;
 }
 
 Err launch_gemm_nt_bf16_split_k(const void* a, const void* b, void* c, float* partial, unsigned splits, size_t bh, size_t m,
@@ -551,7 +557,6 @@ Err launch_gemm_nt_bf16_split_k(const void* a, const void* b, void* c, float* pa
   if (splits < 2 || bh * splits > 65535 || !fits_u32(m) || !fits_u32(n) || k > (size_t(1) << 22)) return "gemm_nt kernel: bad split";
   if (!a || !b || !c || !partial) return "gemm_nt kernel: null device pointer";
   if (!aligned16(a) || !aligned16(b)) return "gemm_nt kernel: operands must be 16-byte aligned";
-  if ((m * n) % 4 != 0) return "gemm_nt kernel: a split product needs m * n to be a multiple of 4";
   GemmParams p{};
   p.a = a; p.b = b; p.c = partial;
   p.bh = (uint32_t)bh; p.m = (uint32_t)m; p.n = (uint32_t)n; p.k = (uint32_t)k;
@@ -559,7 +564,7 @@ Err launch_gemm_nt_bf16_split_k(const void* a, const void* b, void* c, float* pa
   splits = (unsigned)((k + p.k_chunk - 1) / p.k_chunk);  // (rounding the parts up to whole slabs may leave fewer of them)
   if (splits < 2) return "gemm_nt kernel: bad split";
   p.splits = splits;
-  const unsigned tile = split_k_tile(m, n);
+  const unsigned tile = split_k_tile(bh, m, n, k, splits);
   p.tiles_m = (uint32_t)((m + tile - 1) / tile);
   p.tiles_n = (uint32_t)((n + tile - 1) / tile);
   const size_t grid = (size_t(p.tiles_m) * p.tiles_n + 7) / 8 * 8;
@@ -573,7 +578,7 @@ Err launch_gemm_nt_bf16_split_k(const void* a, const void* b, void* c, float* pa
   if (Err e = launch(fn, (unsigned)grid, (unsigned)(bh * splits), 1, 256, &p, sizeof(p), stream); !e.empty()) return e;
   SplitReduceParams r{partial, c, (uint32_t)bh, splits, (uint64_t)m * n, out_dtype == BF16 ? 1u : 0u};
   if (Err e = builtin_function("splitk_reduce", &fn); !e.empty()) return e;
-  size_t rgrid = (bh * m * n / 4 + 255) / 256;
+  size_t rgrid = (bh * ((m * n + 3) / 4) + 255) / 256;
   if (rgrid > 65536) rgrid = 65536;
   return launch(fn, (unsigned)rgrid, 1, 1, 256, &r, sizeof(r), stream);
 }
@@ -612,7 +617,6 @@ Err launch_gemm_nn_bf16(const void* a, const void* b, void* c, size_t bh, size_t
   // in the caller's temporary, added up by splitk_reduce
   if (splits > 1) {
     if (!partial) return "gemm_nn kernel: a split needs its temporary";
-    if ((m * n) % 4 != 0) return "gemm_nn kernel: a split product needs m * n to be a multiple of 4";
     p.k_chunk = (uint32_t)(((k + splits - 1) / splits + 63) / 64 * 64);
     splits = (unsigned)((k + p.k_chunk - 1) / p.k_chunk);  // (rounding the parts up to whole slabs may leave fewer of them)
     if (bh * splits > 65535) return "gemm_nn kernel: extent too large";
@@ -621,7 +625,7 @@ Err launch_gemm_nn_bf16(const void* a, const void* b, void* c, size_t bh, size_t
     p.splits = splits;
     p.c = partial;
     p.out_bf16 = 0;
-    tile = split_k_tile(m, n);
+    tile = split_k_tile(bh, m, n, k, splits);
   }
   p.tiles_m = (uint32_t)((m + tile - 1) / tile);
   p.tiles_n = (uint32_t)((n + tile - 1) / tile);
@@ -638,7 +642,7 @@ Err launch_gemm_nn_bf16(const void* a, const void* b, void* c, size_t bh, size_t
     return e;
   SplitReduceParams r{partial, c, (uint32_t)bh, splits, (uint64_t)m * n, out_dtype == BF16 ? 1u : 0u};
   if (Err e = builtin_function("splitk_reduce", &fn); !e.empty()) return e;
-  size_t rgrid = (bh * m * n / 4 + 255) / 256;
+  size_t rgrid = (bh * ((m * n + 3) / 4) + 255) / 256;
   if (rgrid > 65536) rgrid = 65536;
   return launch(fn, (unsigned)rgrid, 1, 1, 256, &r, sizeof(r), stream);
 }
@@ -672,7 +676,7 @@ bool gemm_narrow_usable(DType dtype, bool nn, size_t bh, size_t m, size_t n, siz
 // parts of at least 256, added up by a second launch, until there are three workgroups per CU (16 x 9808 x 4288 is
 // 153 column tiles: 50 us in 2 parts, 41 in 6; 20 x 9000 x 6000 108 and 78).
 unsigned gemm_narrow_parts(bool nn, size_t bh, size_t m, size_t n, size_t k) {
-  if (!nn || (m * n) % 4 != 0) return 1;
+  if (!nn) return 1;
   const size_t tiles = (n + 63) / 64 * bh;
   if (tiles >= 576 || (tiles >= 192 && k < 2048)) return 1;  // (1 x 16384 x 1024: 14 us whole, 17 in 3 parts)
   const size_t want = std::min<size_t>(std::min<size_t>((768 + tiles - 1) / tiles, k / 256), 32);
@@ -693,7 +697,7 @@ Err launch_gemm_narrow(const void* a, const void* b, void* c, DType dtype, bool 
   p.bh = (uint32_t)bh; p.m = (uint32_t)m; p.n = (uint32_t)n; p.k = (uint32_t)k;
   p.out_bf16 = out_dtype == BF16 ? 1u : 0u;
   if (splits > 1) {
-    if (!partial || (m * n) % 4 != 0) return "narrow gemm kernel: a split needs its temporary and m * n a multiple of 4";
+    if (!partial) return "narrow gemm kernel: a split needs its temporary";
     p.k_chunk = (uint32_t)(((k + splits - 1) / splits + 63) / 64 * 64);
     splits = (unsigned)((k + p.k_chunk - 1) / p.k_chunk);  // (rounding the parts up may leave fewer of them)
   }
@@ -714,7 +718,7 @@ Err launch_gemm_narrow(const void* a, const void* b, void* c, DType dtype, bool 
     return e;
   SplitReduceParams r{partial, c, (uint32_t)bh, splits, (uint64_t)m * n, out_dtype == BF16 ? 1u : 0u};
   if (Err e = builtin_function("splitk_reduce", &fn); !e.empty()) return e;
-  const size_t rgrid = std::min<size_t>((bh * m * n / 4 + 255) / 256, 65536);
+  const size_t rgrid = std::min<size_t>((bh * ((m * n + 3) / 4) + 255) / 256, 65536);
   return launch(fn, (unsigned)rgrid, 1, 1, 256, &r, sizeof(r), stream);
 }
 
@@ -787,7 +791,6 @@ Err launch_gemm_nt_f32(const float* a, const float* b, float* c, size_t bh, size
   // the k loop in parts over workgroups (gemm_nt_f32_split_k says when): partial products in the caller's temporary
   if (splits > 1) {
     if (!partial) return "gemm_nt f32 kernel: a split needs its temporary";
-    if ((m * n) % 4 != 0) return "gemm_nt f32 kernel: a split product needs m * n to be a multiple of 4";
     p.k_chunk = (uint32_t)(((k + splits - 1) / splits + 63) / 64 * 64);
     splits = (unsigned)((k + p.k_chunk - 1) / p.k_chunk);  // (rounding the parts up to whole slabs may leave fewer of them)
     if (bh * splits > 65535) return "gemm_nt f32 kernel: extent too large";
@@ -811,7 +814,7 @@ Err launch_gemm_nt_f32(const float* a, const float* b, float* c, size_t bh, size
     return e;
   SplitReduceParams r{partial, c, (uint32_t)bh, splits, (uint64_t)m * n, 0u};
   if (Err e = builtin_function("splitk_reduce", &fn); !e.empty()) return e;
-  size_t rgrid = (bh * m * n / 4 + 255) / 256;
+  size_t rgrid = (bh * ((m * n + 3) / 4) + 255) / 256;
   if (rgrid > 65536) rgrid = 65536;
   return launch(fn, (unsigned)rgrid, 1, 1, 256, &r, sizeof(r), stream);
 }
