@@ -1223,6 +1223,10 @@ GenericModule emit_generic_hip(const ExecPlan& plan, const Module& module, const
       for (size_t b = 0; b < info.n_reads; ++b)
         if (reads_along(stmts, b, inner)) phase.strip_reads.push_back(b);
     }
+    Uses uses;
+    collect(body, uses);
+    for (size_t w = 0; w < info.n_writes; ++w)
+      if (!uses.written.count(Param{true, w})) phase.only_read_writes.push_back(w);
     // (a buffer that the nest also reads, or accumulates into, keeps its f32 copy)
     for (size_t w = 0; phase.strip && w < info.n_writes; ++w) {
       bool direct = w < 8 * sizeof(size_t) && (private_inds.count(w) || !reads_writeable(stmts, w));

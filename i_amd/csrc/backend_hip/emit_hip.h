@@ -91,6 +91,7 @@ struct GenericPhase {
   bool sequential_loops = false;          // there are loops besides the parallel ones
   std::vector<size_t> strip_reads;        // readonlys that the strip form reads four elements at a time (and every writeable)
   std::vector<size_t> strip_direct_writes;  // writeables that the strip form may store in bf16: stored only, never read
+  std::vector<size_t> only_read_writes;   // writeables (buffers that another nest of the kernel writes) that this one only reads
   std::vector<size_t> same_element_reads; // readonlys of which every iteration reads the one element that it then writes, as
                                           // its last act, and nothing else: such an operand may be the output itself
   std::vector<size_t> bf16_reads;         // readonlys that are program inputs of rank 1 and more: bf16 in the forms <name>..._b

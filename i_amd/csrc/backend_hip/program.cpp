@@ -858,7 +858,7 @@ bool strips_usable(const Run& run, const GenericPhase& ph, const Step& dispatch,
   if (inner % 4 == 0) return true;
   // (sums that the nest starts itself, in registers, are the same again in every strip form)
   if (!(ph.grid.starts_fresh && ph.grid.accumulators.size() == dispatch.writes.size()) &&
-      (ph.sequential_loops || ph.strip_direct_writes.size() != dispatch.writes.size()))
+      (ph.sequential_loops || ph.strip_direct_writes.size() + ph.only_read_writes.size() != dispatch.writes.size()))
     return false;
   for (BufferRef w : dispatch.writes)
     for (BufferRef r : dispatch.reads)
