@@ -50,10 +50,10 @@ struct PrivateBuffer {
 // one before it, and two work-items store the same elements: that is left to nests that read nothing of what they
 // write.  Sums that the nest starts itself are such nests, since their registers start as the reduction's identity
 // (GridForm::starts_fresh; started through memory, a sum could be read back by the neighbour and counted twice).  The element-wise forms are bound by HBM and the plain ones by the number
-// of accesses in flight: 16384 x 4096 f32 divided by its column sums 213 -> 166 us (the division alone 145 -> 87, 6
+// of accesses in flight: 16384 x 4096 f32 divided by its column sums 213 -> 162 us (the division alone 145 -> 87, 6
 // TB/s), a bias and a threshold 193 -> 102.  And every form that reads program inputs exists once more, <name>..._b, with
 // those inputs' elements in bf16, which would otherwise be widened into temporaries first (16384 x 4096
-// bf16, results in bf16: 450 -> 100 and 447 -> 56 us; row sums 182 -> 32, where a lane takes four elements at a time).
+// bf16, results in bf16: 450 -> 96 and 447 -> 56 us; row sums 182 -> 32, where a lane takes four elements at a time).
 struct WaveLoop {
   size_t loop = 0;    // a loop of the parallel body: its accumulators are lane shares, combined after it
   size_t spread = 0;  // the loop whose iterations are dealt out over the lanes: `loop`, or one nested perfectly in it
@@ -126,8 +126,8 @@ struct GenericModule {
 ic::ExecPlan split_nests(const ic::ExecPlan& plan, std::vector<size_t>* origin);
 
 // Names of the helper kernels that every module with a GridForm carries: filling a temporary with a reduction's
-// identity; folding the parts' copies into the accumulated buffer, with a work-item per element (many elements) or a
-// wavefront per element whose lanes run over the parts (few elements, many parts).
+// identity; folding the parts' copies into the accumulated buffer, with a work-item per element (few parts) or a
+// wavefront for one or two elements, whose lanes run over the parts.
 constexpr const char* kFillKernel = "ilang_fill";
 constexpr const char* kCombineKernel = "ilang_combine";
 constexpr const char* kCombineWaveKernel = "ilang_combine_w";

@@ -791,9 +791,9 @@ ihip::Err generic_function(Program& p, const std::string& name, hipFunction_t* f
 // most of the chip idle: enough of them for 16 wavefronts per compute unit, each part with at least 16 iterations of
 // a loop that a work-item runs by itself, 4 rounds of the 64 lanes when the loop in parts is the one over the lanes,
 // one iteration when the lanes run over a loop inside it; at most 4096, from 16 on a multiple of 8 and from 256 on
-// of 32 (the copies of buffers of 64 elements and more are then folded in two passes).
+// of 32.
 // `strips`: a work-item takes four iterations of the innermost parallel loop and `total` counts those.
-size_t generated_parts(const ihip::KernelOptions& knobs, const GridForm& grid, bool wave, size_t total, size_t reduced, bool strips) {
+size_t generated_parts(const ihip::KernelOptions& knobs, const GridForm& grid, bool wave, size_t total, size_t reduced, bool strips, bool bf16) {
   if (!grid.available || (wave && !grid.wave) || knobs.generated_parts == 1 || total == 0) return 1;
   const size_t least = !wave ? 16 : grid.loop_is_spread ? 256 : 1;
   size_t parts;
@@ -802,12 +802,18 @@ size_t generated_parts(const ihip::KernelOptions& knobs, const GridForm& grid, b
   } else {
     const size_t target = wave ? 4096 : strips ? 98304 : 262144;  // wavefronts / work-items that fill the chip
     if (total * 2 > target) return 1;
-    // (strips have four times the bytes in flight: long loops read fastest with 49152 to 65536 of them.  65536 makes as many
-    // parts as the form without strips has, so that no sum is longer.  Column sums with 65536 and 98304 work-items, and without
-    // strips: 16384 x 4096 47.8, 49.0 and 46.4 us, 4096 x 4096 19.5, 20.5 and 19.4, 65536 x 1024 51.3, 54.2 and 52.1, 5042 x
-    // 2561 19.4, 20.7 and 22.1, 1000 x 50000 33.9, 34.8 and 39.2; short loops are bound by their rounds of loads instead, 64
-    // batches of 64 x 1024 10.7 us in 4 parts, 11.6 in 3)
-    parts = std::min<size_t>(strips && reduced > 256 ? std::max<size_t>(65536 / total, 2) : target / total, reduced / least);
+    // (strips have four times the bytes in flight: long loops read fastest with 49152 to 65536 of them, in bf16, where they have
+    // twice, with 98304: 16384 x 4096 in 64 and 96 parts 51.2 and 50.3 us in f32, 34.8 and 28.9 in bf16, 8404 x 3802 bf16 19.1
+    // and 18.0.  65536 makes as many parts as the form without strips has, so that no sum is longer; beyond 256 parts only
+    // as many as leave 64 iterations each, for the sake of the pass over them: 16384 x 64 in 1024 11.5, in 256 10.1.  Short loops are bound by their rounds of loads instead, 64 batches of 64 x 1024 10.7 us in 4
+    // parts, 11.6 in 3.)
+    if (strips && reduced > 256) {
+      parts = std::max<size_t>((bf16 ? 98304 : 65536) / total, 2);
+      if (parts > 256) parts = std::max<size_t>(256, std::min<size_t>(parts, reduced / 64));
+    } else {
+      parts = target / total;
+    }
+    parts = std::min<size_t>(parts, reduced / least);
   }
   // (at most 4096 parts; 2048 of wavefronts when left to this rule: the pass over the parts of a sum to one element
   // is one wavefront's work and grows with their number, 4096^2 to one element 29.7 us in 4096 parts, 23.8 in 2048)
@@ -924,12 +930,12 @@ ihip::Err launch_generic(Run& run, size_t k, const Step& dispatch) {
   if (!ph.wave_loops.empty()) {
     const size_t reduced = extent_of(ph.wave_extent);
     // (a nest with a form in parts fills the chip with work-items, whose lanes read along the parallel index)
-    wave = reduced >= 128 && (ph.wave_contiguous || (total < 65536 && !ph.grid.available));
+    wave = reduced >= (ph.wave_contiguous ? 64 : 128) && (ph.wave_contiguous || (total < 65536 && !ph.grid.available));
     if (run.knobs.generated_wave >= 0) wave = run.knobs.generated_wave == 1;
   }
   const size_t reduced = ph.grid.available ? extent_of(ph.grid.extent) : 0;
   auto parts_for = [&](bool in_strips) {
-    return generated_parts(run.knobs, ph.grid, wave, in_strips ? total / inner * ((inner + 3) / 4) : total, reduced, in_strips);
+    return generated_parts(run.knobs, ph.grid, wave, in_strips ? total / inner * ((inner + 3) / 4) : total, reduced, in_strips, bf16_inputs);
   };
   bool strips = !wave && ph.strip && inner >= 4;
   size_t parts = parts_for(strips && ph.grid.held_accumulators);
@@ -937,8 +943,17 @@ ihip::Err launch_generic(Run& run, size_t k, const Step& dispatch) {
     strips = false;
     parts = parts_for(false);
   }
-  // the outputs that a strip form stores in bf16 itself; any other bf16 output goes through an f32 temporary
-  size_t bf16_writes = 0;
+  bool dynamic_private = false;  // (per-work-item slices of a device buffer are sized for the plain form's grid)
+  for (const PrivateBuffer& pb : ph.privates) dynamic_private = dynamic_private || !pb.is_static;
+  if (dynamic_private) parts = 1;
+  auto accumulated_afresh = [&](size_t w) {
+    for (const GridAccumulator& acc : ph.grid.accumulators)
+      if (acc.writeable == w) return acc.init_here;
+    return false;
+  };
+  // the outputs that a strip form stores in bf16 itself, and those that the pass over the parts does; any other bf16 output
+  // goes through an f32 temporary
+  size_t bf16_writes = 0, folded_to_bf16 = 0;
   std::vector<void*> write_ptrs(dispatch.writes.size(), nullptr);
   for (size_t i = 0; i < dispatch.writes.size(); ++i) {
     const BufferRef w = dispatch.writes[i];
@@ -948,6 +963,10 @@ ihip::Err launch_generic(Run& run, size_t k, const Step& dispatch) {
         store_in_place(run, run.p.nest_plan, dispatch, w.id, same_element)) {
       write_ptrs[i] = run.raw_ptr(w);
       bf16_writes |= size_t(1) << i;
+    } else if (parts > 1 && i < 8 * sizeof(size_t) && accumulated_afresh(i) && run.dtype_of(w) == DType::BF16 && written_once(run, w) &&
+               store_in_place(run, run.p.nest_plan, dispatch, w.id, [](size_t) { return false; })) {
+      write_ptrs[i] = run.raw_ptr(w);
+      folded_to_bf16 |= size_t(1) << i;
     } else if (!gk.is_private(i)) {
       if (ihip::Err e = run.write_f32(w, &write_ptrs[i]); !e.empty()) return e;
     }
@@ -955,9 +974,6 @@ ihip::Err launch_generic(Run& run, size_t k, const Step& dispatch) {
   }
   if (total == 0) return {};
   const size_t items = strips ? total / inner * ((inner + 3) / 4) : total;  // work-items
-  bool dynamic_private = false;  // (per-work-item slices of a device buffer are sized for the plain form's grid)
-  for (const PrivateBuffer& pb : ph.privates) dynamic_private = dynamic_private || !pb.is_static;
-  if (dynamic_private) parts = 1;
   hipFunction_t fn;
   if (parts > 1) {
     // every part accumulates into a copy of its own of each accumulated buffer (filled with the reduction's
@@ -968,29 +984,24 @@ ihip::Err launch_generic(Run& run, size_t k, const Step& dispatch) {
       counts.push_back(std::max<size_t>(1, product(run.layout_of(dispatch.writes.at(acc.writeable)))));
       floats += counts.back() * parts;
     }
-    // How the copies fold.  A buffer of fewer than 64 elements: one pass, a wavefront per element with its lanes
-    // over the parts.  Larger ones: a work-item per element, and from 16 parts on in two passes (the copies, read as
-    // [parts / w][w * count], fold into w = 8 or 32 copies first), which puts w times as many work-items on the
-    // first pass.
-    const size_t width = parts >= 256 && parts % 32 == 0 ? 32 : parts >= 16 && parts % 8 == 0 ? 8 : 0;
-    size_t most = 0;
-    for (size_t c : counts)
-      if (c >= 64) most = std::max(most, c);
-    const bool two_passes = width != 0 && most != 0;
-    if (two_passes) floats += width * most;
+    // How the copies fold, in one pass: a work-item per element; from 16 parts on as many lanes as have eight parts each, 8 to
+    // 64, and a wavefront where there are fewer than 64 elements.  Column
+    // sums, in two passes of a work-item per element -> so, us: 5042 x 2561 19.8 -> 14.5, 16384 x 512 21.2 -> 11.9, 7426 x 243 bf16
+    // 18.6 -> 10.3; 4096 x 4096 to one element 24.2 -> 18.7, whose 2048 parts were folded one load after the other.
+    const bool lanes_per_element = parts >= 16;
+    const int shift = parts > 256 ? 0 : parts > 128 ? 1 : parts > 64 ? 2 : 3;  // 2^shift elements per wavefront
     void* partial = nullptr;
     if (run.alloc_optional(&partial, floats * 4)) {
       std::vector<unsigned char> gargs(args);
       gargs.resize(args.size() + 8 * nw + 8 + (strips ? 8 : 0), 0);  // (the strip form's bf16_writes: none, the copies are f32)
       float* at = static_cast<float*>(partial);
       struct FillArgs { float* data; size_t count; float value; };
-      struct CombineArgs { const float* partial; float* data; size_t parts; size_t count; int op; int keep; };
+      struct CombineArgs { const float* partial; float* data; size_t parts; size_t count; int op; int keep; int bf16; int shift; };
       hipFunction_t fill_fn, combine_fn, combine_wave_fn;
       if (ihip::Err e = generic_function(p, kFillKernel, &fill_fn); !e.empty()) return e;
       if (ihip::Err e = generic_function(p, kCombineKernel, &combine_fn); !e.empty()) return e;
       if (ihip::Err e = generic_function(p, kCombineWaveKernel, &combine_wave_fn); !e.empty()) return e;
-      std::vector<std::pair<CombineArgs, bool>> combines;  // (arguments, a wavefront per element)
-      float* const folded = static_cast<float*>(partial) + (floats - (two_passes ? width * most : 0));
+      std::vector<CombineArgs> combines;
       for (size_t a = 0; a < ph.grid.accumulators.size(); ++a) {
         const GridAccumulator& acc = ph.grid.accumulators[a];
         std::memcpy(gargs.data() + args.size() + 8 * acc.writeable, &at, 8);
@@ -1005,14 +1016,7 @@ ihip::Err launch_generic(Run& run, size_t k, const Step& dispatch) {
         }
         const int op = acc.op == Op::Add ? 0 : acc.op == Op::Mul ? 1 : acc.op == Op::Max ? 2 : 3;
         float* const dst = static_cast<float*>(write_ptrs.at(acc.writeable));
-        if (counts[a] < 64) {
-          combines.push_back({{at, dst, parts, counts[a], op, acc.init_here ? 0 : 1}, true});
-        } else if (two_passes) {
-          combines.push_back({{at, folded, parts / width, width * counts[a], op, 0}, false});
-          combines.push_back({{folded, dst, width, counts[a], op, acc.init_here ? 0 : 1}, false});
-        } else {
-          combines.push_back({{at, dst, parts, counts[a], op, acc.init_here ? 0 : 1}, false});
-        }
+        combines.push_back({at, dst, parts, counts[a], op, acc.init_here ? 0 : 1, folded_to_bf16 >> acc.writeable & 1 ? 1 : 0, counts[a] < 64 ? 0 : shift});
         at += counts[a] * parts;
       }
       std::memcpy(gargs.data() + args.size() + 8 * nw, &parts, 8);
@@ -1026,14 +1030,20 @@ ihip::Err launch_generic(Run& run, size_t k, const Step& dispatch) {
       if (ihip::Err e = ihip::launch(fn, (unsigned)groups, 1, 1, wave ? GenericPhase::kWaveThreads : 64, gargs.data(), gargs.size(), run.stream);
           !e.empty())
         return e;
-      for (const auto& [ca, by_wave] : combines) {
-        const size_t cgrid = std::min<size_t>(by_wave ? (ca.count + 3) / 4 : (ca.count + 255) / 256, 4096);
+      for (const CombineArgs& ca : combines) {
+        const bool by_wave = lanes_per_element || ca.count < 64;
+        const size_t lanes = by_wave ? ca.count * size_t(64 >> ca.shift) : ca.count, cgrid = std::min<size_t>((lanes + 255) / 256, 4096);
         if (ihip::Err e = ihip::launch(by_wave ? combine_wave_fn : combine_fn, (unsigned)cgrid, 1, 1, 256, &ca, sizeof(ca), run.stream);
             !e.empty())
           return e;
       }
       return {};
     }
+    for (size_t i = 0; i < dispatch.writes.size(); ++i)  // (no room for the parts: the nest stores f32)
+      if (folded_to_bf16 >> i & 1) {
+        if (ihip::Err e = run.write_f32(dispatch.writes[i], &write_ptrs[i]); !e.empty()) return e;
+        fill(nr + i, write_ptrs[i], dispatch.writes[i]);
+      }
   }
   if (wave) {
     const size_t waves = std::min<size_t>(total, size_t(1) << 16);
