@@ -76,18 +76,48 @@ std::vector<std::vector<size_t>> host_shapes(const ihipc::Program& p, const i_te
 // Device memory for the operands of host calls: one block per device that the library keeps from call to call
 // (a host call returns after the GPU has finished, so the block is free again), as large as the largest call needed,
 // at most ILANG_HIP_STAGING_MB (default 1024; 0: every operand is allocated, copied and freed on its own).  Calls
-// whose operands fit 8 MiB go through a page-locked host mirror of the block as well: the inputs are gathered
-// there and cross in one asynchronous copy, the outputs come back in one, instead of a blocking copy from pageable
-// memory per operand.  Larger operands cross in page-locked chunks that several host threads fill and empty while
+// whose operands are less than 64 MiB go through a page-locked host mirror of the block as well (run_mirrored).  Larger
+// operands cross in page-locked chunks that several host threads fill and empty while
 // the chunk before is in flight (runtime/host_copy.h).  A call that finds the block in use by another thread, or
 // needs more, allocates as before.
 struct Staging {
   void* base = nullptr;
   size_t capacity = 0;
-  void* pinned = nullptr;  // a page-locked host mirror of the first kPinnedBytes of the block (small calls)
+  void* pinned = nullptr;  // a page-locked host mirror of the first pinned_bytes of the block
+  size_t pinned_bytes = 0;
+  std::vector<hipEvent_t> events;  // kept with it
   std::mutex busy;
+
+  // a mirror of at least `bytes` (a power of two, 8 MiB and more), made larger if need be; false: there is none to be had
+  bool mirror(size_t bytes) {
+    if (pinned_bytes >= bytes) return true;
+    size_t size = size_t(8) << 20;
+    while (size < bytes) size *= 2;
+    if (pinned) (void)hipHostFree(pinned);
+    pinned = nullptr;
+    pinned_bytes = 0;
+    if (hipHostMalloc(&pinned, size, hipHostMallocDefault) != hipSuccess) {
+      pinned = nullptr;
+      (void)hipGetLastError();
+      return false;
+    }
+    pinned_bytes = size;
+    return true;
+  }
+  bool event(size_t n, hipEvent_t* e) {
+    while (events.size() <= n) {
+      hipEvent_t made = nullptr;
+      if (hipEventCreateWithFlags(&made, hipEventDisableTiming) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+      }
+      events.push_back(made);
+    }
+    *e = events[n];
+    return true;
+  }
 };
-constexpr size_t kPinnedBytes = size_t(8) << 20;
+constexpr size_t kMirroredBytes = size_t(64) << 20;  // calls of less go through the mirror
 
 struct StagingTable {
   std::mutex mu;
@@ -121,10 +151,12 @@ size_t release_staging_blocks() {
     }
     if (block->pinned) {
       (void)hipHostFree(block->pinned);
-      released += kPinnedBytes;
+      released += block->pinned_bytes;
     }
+    for (hipEvent_t e : block->events) (void)hipEventDestroy(e);
+    block->events.clear();
     block->base = block->pinned = nullptr;
-    block->capacity = 0;
+    block->capacity = block->pinned_bytes = 0;
   }
   return released;
 }
@@ -310,6 +342,170 @@ bool run_host_in_slices(ihipc::Program& p, const i_tensor* inputs, const std::ve
   return finish({}, true);
 }
 
+// A call whose operands lie in the kept block with a page-locked mirror of it.  Several host threads gather the inputs in
+// the mirror, and every MiB that is there starts across while the next is gathered; the outputs come back the
+// same way.  A program that only maps over its leading index runs in slices of about 8 MiB from 6 on, as above: the
+// kernels of a slice, and its outputs on their way down, run beside the uploads of those after it.  One thread drives
+// all of it: what has come down is copied out between two slices.  Attention of 8 x 2
+// heads of 2048 x 64 (33 MB) 1170 -> 840 us a call, 5 x 7 of 777 x 72 1530 -> 760, 2 x 8 of 412 x 64 340 -> 300, 2 x 3 of 398 x 32
+// 160 -> 105; the link alone takes 610, 570, 123 and 22.
+constexpr size_t kMirrorPiece = size_t(1) << 20, kMirroredSlicedBytes = size_t(6) << 20, kMirroredSliceBytes = size_t(8) << 20;
+std::string run_mirrored(ihipc::Program& p, const i_tensor* inputs, const std::vector<ihipc::DeviceTensor>& in,
+                         const std::vector<ihipc::DeviceTensor>& out, const std::vector<float*>& out_ptrs, Staging& block, hipStream_t stream) {
+  char* const base = static_cast<char*>(block.base);
+  char* const mirror = static_cast<char*>(block.pinned);
+  auto elements = [](const ihipc::DeviceTensor& t) {
+    size_t n = 1;
+    for (size_t d : t.shape) n *= d;
+    return n;
+  };
+  // slices of the leading index, if the program allows it and there is enough to move
+  std::vector<char> sliced;
+  size_t rows = out.empty() || out[0].shape.empty() ? 0 : out[0].shape[0], moving = 0, whole = 0;
+  bool in_slices = rows >= 2 && ihipc::row_sliceable(p, &sliced) && sliced.size() == in.size();
+  for (size_t i = 0; in_slices && i < in.size(); ++i) {
+    in_slices = !sliced[i] || (!in[i].shape.empty() && in[i].shape[0] == rows);
+    (sliced[i] ? moving : whole) += 4 * elements(in[i]);
+  }
+  for (size_t o = 0; in_slices && o < out.size(); ++o) {
+    in_slices = !out[o].shape.empty() && out[o].shape[0] == rows && (out_ptrs[o] || elements(out[o]) == 0);
+    moving += 4 * elements(out[o]);
+  }
+  hipStream_t up = stream, down = stream;
+  if (in_slices && moving >= kMirroredSlicedBytes && moving >= whole) {
+    up = side_stream_of_current_device(0);
+    down = side_stream_of_current_device(1);
+  }
+  in_slices = in_slices && up && down && up != stream;
+  if (!in_slices) up = down = stream;
+  const size_t wanted = in_slices ? std::min<size_t>(std::min<size_t>(8, rows), std::max<size_t>(2, moving / kMirroredSliceBytes)) : 1;
+  const size_t each = in_slices ? (rows + wanted - 1) / wanted : 0, slices = in_slices ? (rows + each - 1) / each : 1;
+
+  // ---- up: the pieces in the order in which they cross, and how many there are up to the end of each slice
+  std::vector<ihip::CopyPiece> gathered;
+  std::vector<size_t> gathered_until;
+  auto offset = [&](const ihipc::DeviceTensor& t) { return (size_t)(static_cast<char*>(t.data) - base); };
+  auto gather = [&](const void* data, size_t at, size_t bytes) {  // into bytes of the mirror from `at` on
+    for (size_t done = 0; done < bytes; done += kMirrorPiece)
+      gathered.push_back({mirror + at + done, static_cast<const char*>(data) + done, std::min(bytes - done, kMirrorPiece)});
+  };
+  for (size_t i = 0; i < in.size(); ++i)
+    if (!in_slices || !sliced[i]) gather(inputs[i].data, offset(in[i]), 4 * elements(in[i]));
+  for (size_t s = 0; s < slices; ++s) {
+    const size_t r0 = s * each, r1 = std::min(rows, r0 + each);
+    for (size_t i = 0; in_slices && i < in.size(); ++i)
+      if (sliced[i]) {
+        const size_t row = 4 * elements(in[i]) / rows;
+        gather(reinterpret_cast<const char*>(inputs[i].data) + r0 * row, offset(in[i]) + r0 * row, (r1 - r0) * row);
+      }
+    gathered_until.push_back(gathered.size());
+  }
+  ihip::CopyAhead ahead(gathered);
+  // sends the pieces before `until`, each as soon as it is there; small neighbours go together
+  size_t sent = 0;
+  auto send = [&](size_t until) -> ihip::Err {
+    while (sent < until) {
+      const size_t lo = (size_t)(static_cast<char*>(gathered[sent].dst) - mirror);
+      size_t hi = lo;
+      const size_t least = lo == 0 ? 2 * kMirrorPiece : 4 * kMirrorPiece;  // (9 us of every transfer are its own)
+      for (; sent < until && hi - lo < least; ++sent) {
+        const size_t at = (size_t)(static_cast<char*>(gathered[sent].dst) - mirror);
+        if (at < hi || at - hi >= 256) break;  // (operands start on the next 256 bytes after the one before)
+        ahead.wait(sent);
+        hi = at + gathered[sent].bytes;
+      }
+      if (ihip::Err e = ihip::h2d(base + lo, mirror + lo, hi - lo, up); !e.empty()) return e;
+    }
+    return {};
+  };
+  // ---- down: pieces on their way, copied out in order
+  struct Piece {
+    size_t at, bytes;
+    char* to;
+    hipEvent_t landed;
+  };
+  std::vector<Piece> pieces;
+  size_t copied = 0, events = 2 * slices;
+  auto bring = [&](size_t at, size_t bytes, char* to) -> ihip::Err {
+    const size_t step = std::max(2 * kMirrorPiece, (bytes / 4 + 4095) / 4096 * 4096);
+    for (size_t done = 0; done < bytes; done += step) {
+      Piece piece{at + done, std::min(step, bytes - done), to + done, nullptr};
+      if (ihip::Err e = ihip::d2h(mirror + piece.at, base + piece.at, piece.bytes, down); !e.empty()) return e;
+      if (in_slices || done + step < bytes) {  // (the last of all is awaited with the stream)
+        if (!block.event(events++, &piece.landed)) return "no event for a transfer";
+        if (ihip::Err e = ihip::check(hipEventRecord(piece.landed, down), "hipEventRecord"); !e.empty()) return e;
+      }
+      pieces.push_back(piece);
+    }
+    return {};
+  };
+  auto copy_out = [&](size_t until) -> ihip::Err {
+    for (; copied < until; ++copied) {
+      const Piece& piece = pieces[copied];
+      if (ihip::Err e = piece.landed ? ihip::check(hipEventSynchronize(piece.landed), "hipEventSynchronize") : ihip::sync(down); !e.empty()) return e;
+      ihip::copy_by_threads(piece.to, mirror + piece.at, piece.bytes);
+    }
+    return {};
+  };
+
+  auto run = [&]() -> ihip::Err {
+    std::vector<size_t> pieces_at;  // how many there were before each slice
+    for (size_t s = 0; s < slices; ++s) {
+      const size_t r0 = s * each, r1 = std::min(rows, r0 + each);
+      std::vector<ihipc::DeviceTensor> in_s(in), out_s(out);
+      auto cut = [&](ihipc::DeviceTensor& t) {  // rows r0 .. r1; returns the byte offset of the first
+        const size_t skip = 4 * elements(t) / rows * r0;
+        t.data = static_cast<char*>(t.data) + skip;
+        t.shape[0] = r1 - r0;
+        return skip;
+      };
+      std::vector<size_t> out_skip(out.size(), 0);
+      for (size_t i = 0; in_slices && i < in.size(); ++i) {
+        if (sliced[i]) (void)cut(in_s[i]);
+      }
+      for (size_t o = 0; in_slices && o < out.size(); ++o) out_skip[o] = cut(out_s[o]);
+      if (ihip::Err e = send(gathered_until[s]); !e.empty()) return e;
+      hipEvent_t landed = nullptr, ran = nullptr;
+      if (in_slices) {
+        if (!block.event(2 * s, &landed) || !block.event(2 * s + 1, &ran)) return "no event for a slice";
+        if (ihip::Err e = ihip::check(hipEventRecord(landed, up), "hipEventRecord"); !e.empty()) return e;
+        if (ihip::Err e = ihip::check(hipStreamWaitEvent(stream, landed, 0), "hipStreamWaitEvent"); !e.empty()) return e;
+      }
+      if (ihip::Err e = ihipc::execute(p, in_s, out_s, stream); !e.empty()) return e;
+      if (in_slices) {
+        if (ihip::Err e = ihip::check(hipEventRecord(ran, stream), "hipEventRecord"); !e.empty()) return e;
+        if (ihip::Err e = ihip::check(hipStreamWaitEvent(down, ran, 0), "hipStreamWaitEvent"); !e.empty()) return e;
+      }
+      pieces_at.push_back(pieces.size());
+      for (size_t o = 0; o < out.size(); ++o) {
+        if (elements(out[o]) == 0) continue;
+        if (!out_ptrs[o]) return "output " + std::to_string(o) + " has no data";
+        if (ihip::Err e = bring(offset(out_s[o]), 4 * elements(out_s[o]), reinterpret_cast<char*>(out_ptrs[o]) + out_skip[o]); !e.empty()) return e;
+      }
+      // (two slices back: down by now, unless the kernels are what takes the time, and then nothing waits for this thread)
+      if (s >= 2)
+        if (ihip::Err e = copy_out(pieces_at[s - 1]); !e.empty()) return e;
+    }
+    return copy_out(pieces.size());
+  };
+  std::string err;
+  try {
+    err = run();
+  } catch (const std::exception& e) {
+    err = e.what();
+  }
+  if (in_slices && !err.empty()) {  // (nothing may still be using the kept block)
+    (void)hipStreamSynchronize(up);
+    (void)hipStreamSynchronize(down);
+  }
+  const ihip::Err sync_err = ihip::sync(stream);
+  if (err.empty()) err = sync_err;
+  if (in_slices && err.empty())
+    ihipc::append_to_report(p, "host: operands in " + std::to_string(slices) + " slices of " + std::to_string(each) +
+                                   " rows, the kernels above are those of the last slice\n");
+  return err;
+}
+
 // Host entry: upload f32 operands, run, download, wait.  Mirrors the
 // blocking behaviour of the reference's exec (core/src/lib.rs:200-225).
 std::string run_host(ihipc::Program& p, const i_tensor* inputs, size_t input_count, const std::vector<float*>& out_ptrs) {
@@ -334,7 +530,7 @@ std::string run_host(ihipc::Program& p, const i_tensor* inputs, size_t input_cou
   for (const auto& shape : out_shapes) wanted += bytes_of(shape);
   std::unique_lock<std::mutex> staging_lock;
   char* carve = nullptr;
-  char *mirror = nullptr, *block_base = nullptr;  // mirror != nullptr: host data passes through the page-locked mirror
+  Staging* mirrored = nullptr;  // host data passes through the page-locked mirror of the kept block
   if (wanted <= staging_limit()) {
     if (Staging* block = staging_of_current_device()) {
       staging_lock = std::unique_lock<std::mutex>(block->busy, std::try_to_lock);
@@ -348,14 +544,7 @@ std::string run_host(ihipc::Program& p, const i_tensor* inputs, size_t input_cou
         if (block->capacity >= wanted) {
           carve = static_cast<char*>(block->base);
           staged = true;
-          if (wanted <= kPinnedBytes) {
-            if (!block->pinned && hipHostMalloc(&block->pinned, kPinnedBytes, hipHostMallocDefault) != hipSuccess) {
-              block->pinned = nullptr;
-              (void)hipGetLastError();
-            }
-            mirror = static_cast<char*>(block->pinned);
-          }
-          block_base = carve;
+          if (wanted < kMirroredBytes && block->mirror(wanted)) mirrored = block;
         }
       }
     }
@@ -386,15 +575,7 @@ std::string run_host(ihipc::Program& p, const i_tensor* inputs, size_t input_cou
       cleanup();
       return e;
     }
-    if (mirror && n) std::memcpy(mirror + (static_cast<char*>(t.data) - block_base), inputs[i].data, n * 4);
     in.push_back(std::move(t));
-  }
-  const size_t input_bytes = carve ? (size_t)(carve - block_base) : 0;  // (the inputs lie first in the block)
-  if (mirror && input_bytes) {
-    if (ihip::Err e = ihip::h2d(block_base, mirror, input_bytes, stream); !e.empty()) {
-      cleanup();
-      return e;
-    }
   }
   for (size_t o = 0; o < out_shapes.size(); ++o) {
     size_t n = 1;
@@ -408,10 +589,15 @@ std::string run_host(ihipc::Program& p, const i_tensor* inputs, size_t input_cou
     out.push_back(std::move(t));
   }
   std::string err;
+  if (mirrored) {
+    err = run_mirrored(p, inputs, in, out, out_ptrs, *mirrored, stream);
+    cleanup();
+    return err;
+  }
   // large operands: in slices when the program allows it, else one after the other and then the program
-  const bool in_slices = !mirror && run_host_in_slices(p, inputs, in, out, out_ptrs, stream, &err);  // (outputs included)
+  const bool in_slices = run_host_in_slices(p, inputs, in, out, out_ptrs, stream, &err);  // (outputs included)
   if (!in_slices) {
-    for (size_t i = 0; !mirror && err.empty() && i < input_count; ++i) {
+    for (size_t i = 0; err.empty() && i < input_count; ++i) {
       size_t n = 1;
       for (size_t d : in_shapes[i]) n *= d;
       err = ihip::upload_pipelined(in[i].data, inputs[i].data, n * 4, stream);
@@ -426,17 +612,10 @@ std::string run_host(ihipc::Program& p, const i_tensor* inputs, size_t input_cou
     size_t n = 1;
     for (size_t d : out_shapes[o]) n *= d;
     if (n && !out_ptrs[o]) err = "output " + std::to_string(o) + " has no data";
-    else if (!mirror) err = ihip::download_pipelined(out_ptrs[o], out[o].data, n * 4, stream);
+    else err = ihip::download_pipelined(out_ptrs[o], out[o].data, n * 4, stream);
   }
-  if (mirror && err.empty() && carve - block_base > (ptrdiff_t)input_bytes)
-    err = ihip::d2h(mirror + input_bytes, block_base + input_bytes, (size_t)(carve - block_base) - input_bytes, stream);
   const ihip::Err sync_err = ihip::sync(stream);
   if (err.empty()) err = sync_err;
-  for (size_t o = 0; mirror && err.empty() && o < out.size(); ++o) {
-    size_t n = 1;
-    for (size_t d : out_shapes[o]) n *= d;
-    if (n) std::memcpy(out_ptrs[o], mirror + (static_cast<char*>(out[o].data) - block_base), n * 4);
-  }
   cleanup();
   return err;
 }

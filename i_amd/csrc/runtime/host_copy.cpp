@@ -1,9 +1,11 @@
 #include "host_copy.h"
 
 #include <algorithm>
+#include <atomic>
 #include <condition_variable>
 #include <cstdlib>
 #include <cstring>
+#include <deque>
 #include <map>
 #include <memory>
 #include <mutex>
@@ -13,38 +15,76 @@
 namespace ihip {
 namespace {
 
-// A few threads that copy slices of one block of host memory at a time (one thread moves 10-15 GB/s, the link
-// to the device four times that).  ILANG_HIP_COPY_THREADS sets their number (default 8, the caller included;
-// 1: the caller alone).  The threads are started on first use and live until the process ends.
+// Pieces of host memory to copy, cut into shares that whoever has time takes in order.
+struct Job {
+  std::vector<CopyPiece> pieces;
+  std::vector<std::pair<size_t, size_t>> shares;  // (piece, offset)
+  std::unique_ptr<std::atomic<size_t>[]> left;    // shares of a piece that are not done
+  std::atomic<size_t> next{0}, active{0};         // the share that is taken next; threads that are in step()
+
+  // A share is what a thread copies in about 10 us, the time it takes to wake one; 1 MiB of the 8 MiB chunks that both
+  // directions of a large call fill and empty side by side (row softmax of 16384 x 4096 through the host entry: 7.5 ms, with
+  // shares of 128 KiB 8.1; 33 MB through the mirror 0.82 ms with those, 0.92 with 1 MiB).
+  static size_t share_of(const CopyPiece& piece) { return piece.bytes >= size_t(8) << 20 ? size_t(1) << 20 : size_t(128) << 10; }
+  explicit Job(std::vector<CopyPiece> given) : pieces(std::move(given)), left(new std::atomic<size_t>[pieces.size() + 1]) {
+    for (size_t p = 0; p < pieces.size(); ++p) {
+      size_t count = 0;
+      for (size_t at = 0; at < pieces[p].bytes; at += share_of(pieces[p]), ++count) shares.push_back({p, at});
+      left[p].store(count);
+    }
+  }
+  // takes the next share, if there is one
+  bool step() {
+    active.fetch_add(1);
+    const size_t n = next.fetch_add(1);
+    if (n >= shares.size()) {
+      active.fetch_sub(1);
+      return false;
+    }
+    const auto [p, at] = shares[n];
+    const CopyPiece& piece = pieces[p];
+    std::memcpy(static_cast<char*>(piece.dst) + at, static_cast<const char*>(piece.src) + at, std::min(share_of(piece), piece.bytes - at));
+    left[p].fetch_sub(1, std::memory_order_release);
+    active.fetch_sub(1);
+    return true;
+  }
+  // no share is begun any more, and none is being copied
+  void stop() {
+    next.store(shares.size());
+    while (active.load() != 0) std::this_thread::yield();
+  }
+  bool done(size_t p) const { return left[p].load(std::memory_order_acquire) == 0; }
+  // returns when piece p is copied; the caller copies too
+  void wait(size_t p) {
+    while (!done(p))
+      if (!step()) std::this_thread::yield();  // (its last shares are with other threads, which need 10 us for one)
+  }
+};
+
+// A few threads that copy shares of the jobs at hand (one thread moves 10-15 GB/s, the link to the device four times
+// that).  ILANG_HIP_COPY_THREADS sets their number (default 8, the caller included; 1: the caller alone).  The threads
+// are started on first use and live until the process ends.
 class CopyCrew {
  public:
   static CopyCrew& get() {
     static CopyCrew* crew = new CopyCrew();  // (never destroyed: its threads may outlive static destructors)
     return *crew;
   }
-  void copy(void* dst, const void* src, size_t bytes) {
-    const size_t slices = std::min<size_t>(workers_.size() + 1, std::max<size_t>(1, bytes >> 20));  // at least 1 MiB each
-    if (slices <= 1) {
-      std::memcpy(dst, src, bytes);
-      return;
-    }
-    std::lock_guard<std::mutex> one_job(job_mu_);  // one block at a time
-    const size_t each = (bytes / slices + 63) / 64 * 64;
+  static constexpr size_t kWorthWaking = size_t(512) << 10;  // waking the others costs the caller 15 us, as copying half of this
+  void post(const std::shared_ptr<Job>& job) {
+    size_t bytes = 0;
+    for (const CopyPiece& piece : job->pieces) bytes += piece.bytes;
+    if (threads_ == 0 || bytes < kWorthWaking) return;  // (the caller copies as it waits)
     {
       std::lock_guard<std::mutex> lock(mu_);
-      dst_ = static_cast<char*>(dst);
-      src_ = static_cast<const char*>(src);
-      bytes_ = bytes;
-      each_ = each;
-      next_ = 1;  // slice 0 is the caller's
-      pending_ = slices - 1;
-      slices_ = slices;
-      ++generation_;
+      jobs_.push_back(job);
     }
     wake_.notify_all();
-    std::memcpy(dst, src, std::min(each, bytes));
-    std::unique_lock<std::mutex> lock(mu_);
-    done_.wait(lock, [&] { return pending_ == 0; });
+  }
+  void copy(void* dst, const void* src, size_t bytes) {
+    auto job = std::make_shared<Job>(std::vector<CopyPiece>{{dst, src, bytes}});
+    post(job);
+    job->wait(0);
   }
 
  private:
@@ -52,32 +92,27 @@ class CopyCrew {
     size_t n = 8;
     if (const char* v = std::getenv("ILANG_HIP_COPY_THREADS")) n = (size_t)std::max(1, std::atoi(v));
     n = std::min<size_t>(n, std::max(1u, std::thread::hardware_concurrency()));
-    for (size_t t = 1; t < n; ++t) workers_.emplace_back([this] { work(); }).detach();
-  }
-  void work() {
-    size_t seen = 0;
-    std::unique_lock<std::mutex> lock(mu_);
-    for (;;) {
-      wake_.wait(lock, [&] { return generation_ != seen && next_ < slices_; });
-      while (next_ < slices_) {
-        const size_t slice = next_++;
-        const size_t at = slice * each_, len = at < bytes_ ? std::min(each_, bytes_ - at) : 0;
-        char* const d = dst_ + at;
-        const char* const s = src_ + at;
-        lock.unlock();
-        if (len) std::memcpy(d, s, len);
-        lock.lock();
-        if (--pending_ == 0) done_.notify_all();
-      }
-      seen = generation_;
+    for (size_t t = 1; t < n; ++t) {
+      std::thread([this] { work(); }).detach();
+      ++threads_;
     }
   }
-  std::vector<std::thread> workers_;
-  std::mutex job_mu_, mu_;
-  std::condition_variable wake_, done_;
-  char* dst_ = nullptr;
-  const char* src_ = nullptr;
-  size_t bytes_ = 0, each_ = 0, next_ = 0, slices_ = 0, pending_ = 0, generation_ = 0;
+  void work() {
+    std::unique_lock<std::mutex> lock(mu_);
+    for (;;) {
+      wake_.wait(lock, [&] { return !jobs_.empty(); });
+      const std::shared_ptr<Job> job = jobs_.front();
+      lock.unlock();
+      while (job->step()) {
+      }
+      lock.lock();
+      if (!jobs_.empty() && jobs_.front() == job) jobs_.pop_front();  // (every share is taken)
+    }
+  }
+  std::mutex mu_;
+  std::condition_variable wake_;
+  std::deque<std::shared_ptr<Job>> jobs_;
+  size_t threads_ = 0;
 };
 
 // A ring of page-locked chunks of one device (one for each direction): four chunks of 8 MiB (small enough that the first chunk's fill and
@@ -157,6 +192,15 @@ size_t release_copy_chunks() {
   }
   return released;
 }
+
+void copy_by_threads(void* dst, const void* src, size_t bytes) { CopyCrew::get().copy(dst, src, bytes); }
+
+struct CopyAhead::State {
+  std::shared_ptr<Job> job;
+};
+CopyAhead::CopyAhead(std::vector<CopyPiece> pieces) : state_(new State{std::make_shared<Job>(std::move(pieces))}) { CopyCrew::get().post(state_->job); }
+CopyAhead::~CopyAhead() { state_->job->stop(); }
+void CopyAhead::wait(size_t piece) { state_->job->wait(piece); }
 
 Err upload_pipelined(void* dst, const void* src, size_t bytes, hipStream_t stream) {
   Ring* ring = bytes >= kPipelinedCopyBytes ? ring_of_current_device(false) : nullptr;

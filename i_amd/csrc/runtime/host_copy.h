@@ -7,6 +7,8 @@
 // at once while the DMA of the chunk before is in flight.
 #pragma once
 #include <cstddef>
+#include <memory>
+#include <vector>
 
 #include "hip_rt.h"
 
@@ -20,6 +22,29 @@ Err upload_pipelined(void* dst, const void* src, size_t bytes, hipStream_t strea
 Err download_pipelined(void* dst, const void* src, size_t bytes, hipStream_t stream);
 // From this size on the two calls above pay (below it one plain copy does)
 constexpr size_t kPipelinedCopyBytes = size_t(8) << 20;
+
+// A block of host memory copied by the same threads; returns when it is.
+void copy_by_threads(void* dst, const void* src, size_t bytes);
+
+// Pieces of host memory that the same threads copy in order, starting at once; wait(n) returns when piece n is there (the
+// caller copies too meanwhile).  Nothing touches the memory any more when the object is gone.
+struct CopyPiece {
+  void* dst;
+  const void* src;
+  size_t bytes;
+};
+class CopyAhead {
+ public:
+  explicit CopyAhead(std::vector<CopyPiece> pieces);
+  ~CopyAhead();
+  CopyAhead(const CopyAhead&) = delete;
+  CopyAhead& operator=(const CopyAhead&) = delete;
+  void wait(size_t piece);
+
+ private:
+  struct State;
+  std::unique_ptr<State> state_;
+};
 
 // Frees the page-locked chunks of every device (those that no transfer is using at this moment); returns the bytes.
 size_t release_copy_chunks();
