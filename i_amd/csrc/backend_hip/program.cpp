@@ -1059,7 +1059,11 @@ ihip::Err launch_generic(Run& run, size_t k, const Step& dispatch) {
   size_t slot_elems = 0;
   for (const PrivateBuffer& pb : ph.privates)
     if (!pb.is_static) slot_elems += std::max<size_t>(1, product(run.layout_of(dispatch.writes[pb.writeable])));
-  size_t max_threads = size_t(1) << 20;
+  // Work-items that take one strip after the other hide the digits of their index behind the accesses, but an f32 strip is enough
+  // to hide them by itself, and more of them are in flight so: 16384 x 4096 with a bias and a threshold 103 us with 2^20
+  // work-items, 97, 93 and 90 with 2, 4 and 8 times as many, divided by its column sums 161, 152, 149 and 147.  Strips of bf16
+  // are half as long: 56, 55, 55 and 62, and 13896 x 2406 divided 57, 58, 60 and 67.
+  size_t max_threads = size_t(1) << (strips && !ph.sequential_loops && !bf16_inputs ? 23 : 20);
   if (slot_elems) max_threads = std::max<size_t>(64, std::min(max_threads, (size_t(1) << 28) / (slot_elems * 4)));
   threads = std::min(threads, max_threads);
   const unsigned grid = (unsigned)((threads + 63) / 64);
