@@ -395,7 +395,7 @@ ihip::Err launch_product_f32(Run& run, const void* a, const void* b, void* c, si
 ihip::Err launch_product_narrow(Run& run, const void* a, const void* b, void* c, ihip::DType t, bool nn, size_t bh, size_t m, size_t n,
                                 size_t k, ihip::LaunchNote* note, ihip::DType out_dt) {
   void* partial = nullptr;
-  unsigned splits = ihip::gemm_narrow_parts(nn, bh, m, n, k);
+  unsigned splits = ihip::gemm_narrow_parts(t, nn, bh, m, n, k);
   if (splits > 1 && !run.alloc_optional(&partial, bh * splits * m * n * 4)) splits = 1;
   return ihip::launch_gemm_narrow(a, b, c, t, nn, bh, m, n, k, run.stream, note, out_dt, static_cast<float*>(partial), splits);
 }

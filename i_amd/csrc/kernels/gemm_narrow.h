@@ -8,7 +8,7 @@
 // wavefront that needs it, many loads in flight, and a workgroup's W wavefronts take every W-th piece of k of the
 // same columns; their sums meet in LDS at the end.  Measured, before -> now: f32 NN 16 x 9808 x 4288 198 -> 41 us
 // (4.1 TB/s), 64 x 8192 x 8192 256 -> 133 (the f32 matrix rate), 1 x 16384 x 1024 73 -> 14; f32 NT 16 x 8192 x 8192
-// 128 -> 66, 3 x 1688 x 8896 44 -> 31; bf16 NT 7 x 8040 x 1296 15.0 -> 11.8.
+// 128 -> 66, 3 x 1688 x 8896 44 -> 21 (in 4 parts of k); bf16 NT 7 x 8040 x 1296 15.0 -> 11.8.
 //
 //   matrix      v_mfma_f32_16x16x32_bf16 / 16x16x4_f32, B's columns of C as the first operand and A's rows as the
 //               second: a lane ends up with C[m = lane % 16][4 columns]

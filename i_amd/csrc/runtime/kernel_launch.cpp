@@ -672,11 +672,39 @@ bool gemm_narrow_usable(DType dtype, bool nn, size_t bh, size_t m, size_t n, siz
   return k % 4 == 0 && (nn ? m <= 64 && n % 4 == 0 : m <= 32);
 }
 
-// NT workgroups take 16 or 32 columns and are as many as n gives; an NN workgroup takes 64, and the k loop is cut into
-// parts of at least 256, added up by a second launch, until there are three workgroups per CU (16 x 9808 x 4288 is
-// 153 column tiles: 50 us in 2 parts, 41 in 6; 20 x 9000 x 6000 108 and 78).
-unsigned gemm_narrow_parts(bool nn, size_t bh, size_t m, size_t n, size_t k) {
-  if (!nn) return 1;
+// Columns of an NT workgroup: 32 (A is read half as often) where that leaves 192 workgroups or k is in parts, else 16: 16
+// x 8192 x 8192 f32 79 us with 16, 66 with 32.
+static size_t narrow_nt_tile(size_t bh, size_t n, unsigned splits) { return splits <= 1 && (n + 31) / 32 * bh < 192 ? 16 : 32; }
+
+// f32 NT: the k loop in parts over workgroups of 32 columns, added up by a second launch, where the columns alone leave CUs
+// idle or a last round nearly empty.  A workgroup's 16 wavefronts fill a CU, so the time goes by whole rounds of 256
+// workgroups: 4 us, and per element of k 3.2 ns on 16 columns, 6 on 32 (5.6 and 9.5 above 16 rows); a split costs 4.5 more,
+// and its many workgroups read B at 5 TB/s at most.  Whole -> in parts, us: 12 x 4904 x 6696 60 -> 43, 3 x 1688 x 8896
+// 31 -> 21, 5 x 2000 x 16000 56 -> 34, 24 x 1500 x 9000 54 -> 29, 31 x 1024 x 16000 98 -> 29; left whole: 30 x 4096 x 4096
+// (28; 28 in 2), 16 x 8192 x 8192 (65; 73), 1 x 12952 x 6288 (69; 75 in 11).
+static unsigned narrow_nt_f32_parts(size_t bh, size_t m, size_t n, size_t k) {
+  auto time_of = [&](size_t tile, size_t parts) {
+    const double rounds = (double)(((n + tile - 1) / tile * bh * parts + 255) / 256);
+    const double loops = rounds * (double)(k / parts) * 1e-3 * (m <= 16 ? (tile == 16 ? 3.2 : 6.0) : (tile == 16 ? 5.6 : 9.5));
+    return parts > 1 ? 8.5 + std::max(loops, (double)(bh * n * k) * 4 / 5e6) : 4 + loops;
+  };
+  double least = 0.9 * time_of(narrow_nt_tile(bh, n, 1), 1);
+  unsigned best = 1;
+  for (size_t s = 2; s <= 16 && k / s >= 512 && bh * s <= 65535; ++s)
+    if (const double t = time_of(32, s); t < least) {
+      least = t;
+      best = (unsigned)s;
+    }
+  if (best < 2) return 1;
+  const size_t chunk = ((k + best - 1) / best + 63) / 64 * 64;
+  return (unsigned)((k + chunk - 1) / chunk);
+}
+
+// An NN workgroup takes 64 columns, and the k loop is cut into parts of at least 256, added up by a second launch, until
+// there are three workgroups per CU (16 x 9808 x 4288 is 153 column tiles: 50 us in 2 parts, 41 in 6; 20 x 9000 x 6000
+// 108 and 78).
+unsigned gemm_narrow_parts(DType dtype, bool nn, size_t bh, size_t m, size_t n, size_t k) {
+  if (!nn) return dtype == F32 ? narrow_nt_f32_parts(bh, m, n, k) : 1;
   const size_t tiles = (n + 63) / 64 * bh;
   if (tiles >= 576 || (tiles >= 192 && k < 2048)) return 1;  // (1 x 16384 x 1024: 14 us whole, 17 in 3 parts)
   const size_t want = std::min<size_t>(std::min<size_t>((768 + tiles - 1) / tiles, k / 256), 32);
@@ -706,8 +734,7 @@ Err launch_gemm_narrow(const void* a, const void* b, void* c, DType dtype, bool 
     p.c = partial;
     p.out_bf16 = 0;
   }
-  // 32 columns (A is read half as often) where that leaves 192 workgroups: 16 x 8192 x 8192 f32 79 us with 16, 66 with 32
-  const size_t tile = nn ? 64 : (n + 31) / 32 * bh < 192 ? 16 : 32;
+  const size_t tile = nn ? 64 : narrow_nt_tile(bh, n, splits);
   const std::string name = std::string(nn ? "gemm_nn_" : "gemm_nt_") + (dtype == BF16 ? "bf16" : "f32") + "_narrow" +
                            (m <= 16 ? "16x" : m <= 32 ? "32x" : "64x") + std::to_string(tile);
   if (note) *note = LaunchNote{splits > 1 ? name + " (k in " + std::to_string(splits) + " parts)" : name, 0, 0};

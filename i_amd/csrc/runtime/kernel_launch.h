@@ -116,7 +116,7 @@ bool gemm_nt_f32_supported(size_t k);
 // gemm_narrow_parts into how many parts its k loop goes (then `partial` is room for bh * splits * m * n floats);
 // operands 16-byte aligned.
 bool gemm_narrow_usable(DType dtype, bool nn, size_t bh, size_t m, size_t n, size_t k, const KernelOptions& knobs);
-unsigned gemm_narrow_parts(bool nn, size_t bh, size_t m, size_t n, size_t k);
+unsigned gemm_narrow_parts(DType dtype, bool nn, size_t bh, size_t m, size_t n, size_t k);
 Err launch_gemm_narrow(const void* a, const void* b, void* c, DType dtype, bool nn, size_t bh, size_t m, size_t n, size_t k,
                        hipStream_t stream, LaunchNote* note, DType out_dtype, float* partial = nullptr, unsigned splits = 1);
 
