@@ -370,6 +370,12 @@ std::string run_mirrored(ihipc::Program& p, const i_tensor* inputs, const std::v
   for (size_t o = 0; in_slices && o < out.size(); ++o) {
     in_slices = !out[o].shape.empty() && out[o].shape[0] == rows && (out_ptrs[o] || elements(out[o]) == 0);
     moving += 4 * elements(out[o]);
+    // (an output in memory that an input has as well must not be written before all of that input is gathered)
+    const uintptr_t to = reinterpret_cast<uintptr_t>(out_ptrs[o]), to_end = to + 4 * elements(out[o]);
+    for (size_t i = 0; in_slices && i < in.size(); ++i) {
+      const uintptr_t from = reinterpret_cast<uintptr_t>(inputs[i].data), from_end = from + 4 * elements(in[i]);
+      in_slices = to >= from_end || from >= to_end;
+    }
   }
   hipStream_t up = stream, down = stream;
   if (in_slices && moving >= kMirroredSlicedBytes && moving >= whole) {

@@ -1,6 +1,10 @@
 """Host calls whose operands are less than 64 MiB: gathered by several threads in page-locked memory, in slices where the program
 only maps over its leading index, copied out while the rest is under way."""
+import os
+import subprocess
+import sys
 import threading
+from pathlib import Path
 
 import numpy as np
 import pytest
@@ -35,6 +39,29 @@ def test_elements_arrive_where_they_belong(rows, cols):
         flipped = i("ij~ji")
         assert np.array_equal(flipped.exec_numpy(a), a.T)
         assert "host:" not in flipped.report()
+
+
+OVERLAPPING = """
+import numpy as np
+from i_amd import Component as i
+rows, cols = 2600, 2000
+for shift in (0, 1000, -1000, 1200 * cols, 1600 * cols, 2000 * cols, -1600 * cols):
+    memory = np.random.default_rng(5).uniform(-1, 1, 3 * rows * cols).astype(np.float32)
+    a = memory[rows * cols:][:rows * cols].reshape(rows, cols)
+    out = memory[rows * cols + shift:][:rows * cols].reshape(rows, cols)
+    expected = a + a
+    i("ij+ij~ij").into(out, a, a)
+    assert np.array_equal(out, expected), shift
+"""
+
+
+# outputs in memory that an input has too: the input itself, and rows before and behind it.  (With one thread that copies, every
+# row is gathered as late as it can be.)
+@pytest.mark.parametrize("threads", ["1", "8"])
+def test_outputs_over_inputs(threads):
+    done = subprocess.run([sys.executable, "-c", OVERLAPPING], env={**os.environ, "ILANG_HIP_COPY_THREADS": threads}, cwd=Path(__file__).parents[1],
+                          capture_output=True, text=True, timeout=100)
+    assert done.returncode == 0, done.stderr[-1500:]
 
 
 def test_products_and_reductions():
