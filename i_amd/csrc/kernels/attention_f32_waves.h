@@ -213,7 +213,10 @@ __device__ __forceinline__ void attn_fwd_f32_waves_body(const AttnParams& p) {
     const float m = ml_lds[0][w][c];
     total += (m == -INFINITY ? 0.0f : fast_exp2((m - top) * scale_log2)) * ml_lds[1][w][c];
   }
-  const float weight = (m_run == -INFINITY ? 0.0f : fast_exp2((m_run - top) * scale_log2)) / total;
+  // (A part over workgroups that sums to nothing, its scores all -inf, leaves O = 0 beside its lse of -inf: the merge weighs it
+  // with 0, and a NaN would survive that.  Without parts, or with all of them so, the row is NaN.)
+  const float divisor = p.kv_splits > 1 && total == 0.0f ? 1.0f : total;
+  const float weight = (m_run == -INFINITY ? 0.0f : fast_exp2((m_run - top) * scale_log2)) / divisor;
 #pragma unroll
   for (int u = 0; u < U; ++u)
 #pragma unroll

@@ -90,3 +90,25 @@ def test_scores_of_minus_infinity_infinity_and_nan():
         assert bool(t.isnan(component.exec_torch(q, k2, t.tensor(1.0, device="cuda"), v)).all()), bad
     k[0, :, 0] = -float("inf")
     assert bool(t.isnan(component.exec_torch(q, k, t.tensor(1.0, device="cuda"), v)).all())
+
+
+# (bh, nq, nk, d): every shape goes into several parts over workgroups
+@pytest.mark.parametrize("bh, nq, nk, d", [(1, 16, 8192, 32), (1, 64, 4096, 20), (64, 1, 1024, 32), (1, 5, 4100, 64), (200, 1, 4096, 64), (1, 64, 5000, 128)])
+def test_parts_over_workgroups_that_score_minus_infinity_weigh_nothing(bh, nq, nk, d):
+    """Whole parts at the end, at the beginning and in the middle; where every part is so, the row is NaN."""
+    component = _component()
+    g = t.Generator(device="cuda").manual_seed(nk)
+    q = t.randn(bh, nq, d, device="cuda", generator=g)
+    q[:, :, 0] = 1.0
+    k, v = (t.randn(bh, nk, d, device="cuda", generator=g) for _ in range(2))
+    one = t.tensor(1.0, device="cuda")
+    for first, last in ((nk // 3, nk), (0, nk - 40), (nk // 8, nk // 8 * 7)):
+        k2 = k.clone()
+        k2[:, first:last, 0] = -float("inf")
+        out = component.exec_torch(q, k2, one, v)
+        assert " x " in component.report().split("(keys in")[1], component.report()
+        keep = t.cat([t.arange(first), t.arange(last, nk)]).cuda()
+        ref, bound = _reference(q, k[:, keep], v[:, keep], 1.0)
+        assert bool(((out.double() - ref).abs() <= bound).all()), (first, last, component.report())
+    k[:, :, 0] = -float("inf")
+    assert bool(t.isnan(component.exec_torch(q, k, one, v)).all())
