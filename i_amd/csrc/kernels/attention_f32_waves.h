@@ -170,14 +170,17 @@ __device__ __forceinline__ void attn_fwd_f32_waves_body(const AttnParams& p) {
       for (int i = 0; i < 4; ++i) mx = fmaxf(mx, sc[b][i]);
     const float m_new = fmaxf(m_run, quarters_max(mx));
     const float alpha = m_run == -INFINITY ? 0.0f : fast_exp2((m_run - m_new) * scale_log2);
-    const float mb = m_new == -INFINITY ? 0.0f : m_new * scale_log2;  // (a part whose scores are all -inf weighs nothing)
+    // The difference is taken before the product with the scale: a score near the lowest f32 times the scale is infinite or
+    // far from what the rounded product of the maximum cancels, and a step of nothing but such scores would sum to infinity,
+    // which its weight of 0 in the end makes NaN.  (-inf: a step of nothing else weighs nothing.)
+    const float m_from = m_new == -INFINITY ? 0.0f : m_new;
     m_run = m_new;
     float psum = 0.0f;
 #pragma unroll
     for (int b = 0; b < KB; ++b)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        float e = fast_exp2(__builtin_fmaf(sc[b][i], scale_log2, -mb));
+        float e = fast_exp2((sc[b][i] - m_from) * scale_log2);
         // spelled out rather than left to exp(-inf): a zero scale turns the masked score into 0 * inf
         if (masked && key0 + 16 * b + 4 * g + i >= end) e = 0.0f;
         sc[b][i] = e;

@@ -112,3 +112,24 @@ def test_parts_over_workgroups_that_score_minus_infinity_weigh_nothing(bh, nq, n
         assert bool(((out.double() - ref).abs() <= bound).all()), (first, last, component.report())
     k[:, :, 0] = -float("inf")
     assert bool(t.isnan(component.exec_torch(q, k, one, v)).all())
+
+
+@pytest.mark.parametrize("bh, nq, nk, d", [(48, 700, 700, 64), (1, 300, 700, 32), (1, 64, 512, 128), (1, 64, 4096, 32), (200, 1, 4096, 64)])
+@pytest.mark.parametrize("scale", [1.0, 3.0, 0.125])
+def test_scores_of_the_lowest_value_weigh_nothing(bh, nq, nk, d, scale):
+    """Times log2(e) they are beyond f32 from a scale of 0.7 on.  They lie on the keys of whole wavefronts, and of whole parts over
+    workgroups where there are such."""
+    component = _component()
+    g = t.Generator(device="cuda").manual_seed(d)
+    q = t.randn(bh, nq, d, device="cuda", generator=g)
+    q[:, :, 0] = 1.0
+    k, v = (t.randn(bh, nk, d, device="cuda", generator=g) for _ in range(2))
+    for first, last in ((nk // 2, nk), (0, nk // 2)):
+        for low in (t.finfo(t.float32).min, t.finfo(t.bfloat16).min):
+            k2 = k.clone()
+            k2[:, first:last, 0] = low
+            out = component.exec_torch(q, k2, t.tensor(scale, device="cuda"), v)
+            assert "_waves" in component.report()
+            keep = t.cat([t.arange(first), t.arange(last, nk)]).cuda()
+            ref, bound = _reference(q, k[:, keep], v[:, keep], scale)
+            assert bool(((out.double() - ref).abs() <= bound).all()), (first, low, component.report())
