@@ -371,8 +371,8 @@ __device__ __forceinline__ void attn_fwd_bf16_direct_body(const AttnParams& p) {
       const bool move = first || (mx - m_run[b]) * scale_log2 > RESCALE_LOG2;
       const float m_new = move ? mx : m_run[b];
       const float alpha = first ? 0.0f : fast_exp2((m_run[b] - m_new) * scale_log2);  // 1 when the reference stays
-      // (KG > 1: a group whose scores are all -inf weighs nothing)
-      const float mb = KG > 1 && m_new == -INFINITY ? 0.0f : m_new * scale_log2;
+      // (a tile or a group whose scores are all -inf weighs nothing)
+      const float mb = (KG > 1 || PRESCALE) && m_new == -INFINITY ? 0.0f : m_new * scale_log2;
       m_run[b] = m_new;
 
       // P = exp(S - m) rounded to bf16 (the PV operand); the row sum is taken over the rounded values
@@ -734,15 +734,17 @@ __device__ __forceinline__ void attn_fwd_bf16_direct_body(const AttnParams& p) {
 
   uint32_t j = 0;
   bool steady = nfull_trips >= 4;
-  if constexpr (KG > 1 && !NOREF) {
-    // a wavefront whose first tile has a row of nothing but -inf has no reference to start from: the general loop finds one
-    // (the same requests and barriers, trip by trip)
+  if constexpr (PRESCALE) {
+    // A wavefront with a row whose first tile scores nothing above -2^8 (in the exponent) takes the general loop, which finds
+    // a reference tile by tile (the same requests and barriers, trip by trip).  The scores of the two tiles after the
+    // first are accumulated on minus its maximum: on 2^8 that costs 2^-16 per addition, on the lowest values of masked
+    // keys all their bits; and -inf is no reference at all.
     float mx = sa[0][0][0];
 #pragma unroll
     for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
       for (int i = 0; i < 16; ++i) mx = fmaxf(mx, sa[0][kt][i]);
-    if (__builtin_amdgcn_ballot_w64(half_max(mx) == -INFINITY)) steady = false;
+    if (__builtin_amdgcn_ballot_w64(half_max(mx) < -256.0f)) steady = false;
   }
   if (steady) {
 #pragma unroll

@@ -98,6 +98,36 @@ def test_groups_whose_scores_lie_far_apart(d):
     assert bool(t.isnan(out).all())
 
 
+# few and many groups, and one group of all keys (head size 64 asks for it with a tile)
+@pytest.mark.parametrize("d, nq, kernel, options", [(64, 70, "_w1_k8", {}), (48, 70, "_w1_k8", {}), (64, 1500, "_w2_k4", {}), (128, 70, "_w2_k4", {}), (256, 70, "_w2_k2", {}),
+                                                    (64, 70, "_direct", {"attention.kv_parts": 1}), (56, 300, "_direct", {"attention.kv_parts": 1})])
+@pytest.mark.parametrize("offset", [-2e2, -2e3, -3e4, -1e9, t.finfo(t.bfloat16).min, -float("inf")])
+def test_first_tiles_far_below_the_rest(d, nq, kernel, options, offset):
+    """Masked keys are the first tile of a group, or the first of all, or both: the groups start on a reference far below
+    the scores that follow."""
+    component = _component()
+    for name, value in options.items():
+        component.option(name, value)
+    nk = 1792
+    q, k, v = _operands(8 if nq > 1000 else 2, nq, nk, d, d, 4)
+    q, k = q * 0.5, k * 0.5
+    q[:, :, 0] = 1.0
+    k[:, :, 0] = 0.0
+    # (tiles of 64 and 32 keys; groups of 224, 448 and 896)
+    for masked in ([(0, 64)], [(896, 960)], [(224, 288), (448, 512), (1344, 1408)], [(0, 64), (896, 1200)]):
+        k2, keep = k.clone(), t.ones(nk, dtype=t.bool, device="cuda")
+        for first, last in masked:
+            k2[:, first:last, 0] = offset
+            keep[first:last] = False
+        out = component.exec_torch(q, k2, t.tensor(1.0, device="cuda"), v)
+        assert kernel in component.report() and (not options or "_k" not in component.report().split()[1]), component.report()
+        q64, k64, v64 = q.double(), k[:, keep].double(), v[:, keep].double()  # (e^-200 weighs nothing)
+        p = t.softmax(q64 @ k64.transpose(1, 2), -1)
+        # (_bound, with the terms of the keys that weigh something)
+        worst = float(((out.double() - p @ v64).abs() / _bound(q64, k64, v64, 1.0, p)).max())
+        assert worst <= 1.0, (masked, worst, component.report())
+
+
 def test_who_asks_for_another_kernel_gets_it():
     q, k, v = _operands(2, 100, 1200, 128, 128, 5)
     for name, value in (("attention.kv_parts", 1), ("attention.f32_scale", 1), ("attention.waves", 4)):
