@@ -189,6 +189,34 @@ hipStream_t side_stream_of_current_device(int which) {
   return made;
 }
 
+// Calls in slices write rows of the outputs while later rows of the inputs are still to be read.  Does an output lie in
+// memory that an input, or another output, has as well?  (An output that starts where an input of as long rows starts is
+// fine, as for a call in place: a slice writes only rows that it has read.)
+bool slices_collide(const i_tensor* inputs, const std::vector<ihipc::DeviceTensor>& in, const std::vector<char>& sliced,
+                    const std::vector<ihipc::DeviceTensor>& out, const std::vector<float*>& out_ptrs) {
+  struct Range {
+    uintptr_t from, to;
+  };
+  auto range_of = [](const void* data, const ihipc::DeviceTensor& t) {
+    size_t bytes = 4;
+    for (size_t d : t.shape) bytes *= d;
+    const uintptr_t from = reinterpret_cast<uintptr_t>(data);
+    return Range{from, from + bytes};
+  };
+  auto meet = [](Range a, Range b) { return a.from < b.to && b.from < a.to && a.from != a.to && b.from != b.to; };
+  for (size_t o = 0; o < out.size(); ++o) {
+    const Range to = range_of(out_ptrs[o], out[o]);
+    for (size_t i = 0; i < in.size(); ++i) {
+      const Range from = range_of(inputs[i].data, in[i]);
+      const bool same_rows = sliced[i] && to.from == from.from && to.to == from.to;  // (and as many: the leading extents are equal)
+      if (!same_rows && meet(to, from)) return true;
+    }
+    for (size_t other = 0; other < o; ++other)
+      if (meet(to, range_of(out_ptrs[other], out[other]))) return true;
+  }
+  return false;
+}
+
 // A call in slices (large operands of a program that only maps over its leading index, ihipc::row_sliceable): the
 // inputs that every slice needs whole are uploaded first; then, slice after slice, the rows of the other inputs go
 // up on the upload stream and the program is enqueued on `stream` behind them for just those rows, so the kernels
@@ -218,7 +246,7 @@ bool run_host_in_slices(ihipc::Program& p, const i_tensor* inputs, const std::ve
     if (out[o].shape.empty() || out[o].shape[0] != rows || !out_ptrs[o]) return false;
     moving += row_bytes(out[o]) * rows;
   }
-  if (rows < 2 || moving < kSlicedCallBytes || moving < whole) return false;
+  if (rows < 2 || moving < kSlicedCallBytes || moving < whole || slices_collide(inputs, in, sliced, out, out_ptrs)) return false;
   const size_t wanted = std::min<size_t>(std::min<size_t>(8, rows), std::max<size_t>(2, moving / kSliceBytes));
   const size_t each = (rows + wanted - 1) / wanted, slices = (rows + each - 1) / each;
   hipStream_t up = side_stream_of_current_device(0), down = side_stream_of_current_device(1);
@@ -370,13 +398,8 @@ std::string run_mirrored(ihipc::Program& p, const i_tensor* inputs, const std::v
   for (size_t o = 0; in_slices && o < out.size(); ++o) {
     in_slices = !out[o].shape.empty() && out[o].shape[0] == rows && (out_ptrs[o] || elements(out[o]) == 0);
     moving += 4 * elements(out[o]);
-    // (an output in memory that an input has as well must not be written before all of that input is gathered)
-    const uintptr_t to = reinterpret_cast<uintptr_t>(out_ptrs[o]), to_end = to + 4 * elements(out[o]);
-    for (size_t i = 0; in_slices && i < in.size(); ++i) {
-      const uintptr_t from = reinterpret_cast<uintptr_t>(inputs[i].data), from_end = from + 4 * elements(in[i]);
-      in_slices = to >= from_end || from >= to_end;
-    }
   }
+  in_slices = in_slices && !slices_collide(inputs, in, sliced, out, out_ptrs);
   hipStream_t up = stream, down = stream;
   if (in_slices && moving >= kMirroredSlicedBytes && moving >= whole) {
     up = side_stream_of_current_device(0);

@@ -42,24 +42,36 @@ def test_elements_arrive_where_they_belong(rows, cols):
 
 
 OVERLAPPING = """
+import sys
 import numpy as np
 from i_amd import Component as i
-rows, cols = 2600, 2000
-for shift in (0, 1000, -1000, 1200 * cols, 1600 * cols, 2000 * cols, -1600 * cols):
+rows, cols = int(sys.argv[1]), 2000
+for shift in (0, 1000, -1000, rows // 2 * cols, rows // 3 * 2 * cols, 100 * cols, -100 * cols, -(rows // 3 * 2) * cols):
     memory = np.random.default_rng(5).uniform(-1, 1, 3 * rows * cols).astype(np.float32)
     a = memory[rows * cols:][:rows * cols].reshape(rows, cols)
     out = memory[rows * cols + shift:][:rows * cols].reshape(rows, cols)
     expected = a + a
-    i("ij+ij~ij").into(out, a, a)
+    component = i("ij+ij~ij")
+    component.into(out, a, a)
+    assert np.array_equal(out, expected), shift
+    # (in place, a slice overwrites what it has read)
+    assert ("host: operands in" in component.report()) == (shift == 0), (shift, component.report())
+    # rows of the result shorter than those of the operand
+    a = memory[rows * cols:][:rows * cols].reshape(rows, cols)
+    expected = a[:, 0].copy()
+    out = a.reshape(-1)[:rows] if shift == 0 else memory[rows * cols + abs(shift):][:rows]
+    a[:, 1:] = 0.0
+    i("+ij~i").into(out, a)
     assert np.array_equal(out, expected), shift
 """
 
 
-# outputs in memory that an input has too: the input itself, and rows before and behind it.  (With one thread that copies, every
-# row is gathered as late as it can be.)
+# outputs in memory that an input has too: the input itself, and rows before and behind it, for calls through the mirror (62 MB)
+# and larger ones.  (With one thread that copies, every row is gathered as late as it can be.)
+@pytest.mark.parametrize("rows", [2600, 9000])
 @pytest.mark.parametrize("threads", ["1", "8"])
-def test_outputs_over_inputs(threads):
-    done = subprocess.run([sys.executable, "-c", OVERLAPPING], env={**os.environ, "ILANG_HIP_COPY_THREADS": threads}, cwd=Path(__file__).parents[1],
+def test_outputs_over_inputs(threads, rows):
+    done = subprocess.run([sys.executable, "-c", OVERLAPPING, str(rows)], env={**os.environ, "ILANG_HIP_COPY_THREADS": threads}, cwd=Path(__file__).parents[1],
                           capture_output=True, text=True, timeout=100)
     assert done.returncode == 0, done.stderr[-1500:]
 
