@@ -619,7 +619,11 @@ std::string run_host(ihipc::Program& p, const i_tensor* inputs, size_t input_cou
   }
   std::string err;
   if (mirrored) {
-    err = run_mirrored(p, inputs, in, out, out_ptrs, *mirrored, stream);
+    try {
+      err = run_mirrored(p, inputs, in, out, out_ptrs, *mirrored, stream);
+    } catch (const std::exception& e) {  // (out of memory before anything was enqueued)
+      err = e.what();
+    }
     cleanup();
     return err;
   }

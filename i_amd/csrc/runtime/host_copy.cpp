@@ -9,6 +9,7 @@
 #include <map>
 #include <memory>
 #include <mutex>
+#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -63,7 +64,8 @@ struct Job {
 
 // A few threads that copy shares of the jobs at hand (one thread moves 10-15 GB/s, the link to the device four times
 // that).  ILANG_HIP_COPY_THREADS sets their number (default 8, the caller included; 1: the caller alone).  The threads
-// are started on first use and live until the process ends.
+// are started by the first job that is worth waking them and live until the process ends; where the system has no more
+// threads to give, those that there are do the work, or the caller alone.
 class CopyCrew {
  public:
   static CopyCrew& get() {
@@ -74,7 +76,9 @@ class CopyCrew {
   void post(const std::shared_ptr<Job>& job) {
     size_t bytes = 0;
     for (const CopyPiece& piece : job->pieces) bytes += piece.bytes;
-    if (threads_ == 0 || bytes < kWorthWaking) return;  // (the caller copies as it waits)
+    if (bytes < kWorthWaking) return;  // (the caller copies as it waits)
+    std::call_once(started_, [this] { start(); });
+    if (threads_ == 0) return;
     {
       std::lock_guard<std::mutex> lock(mu_);
       jobs_.push_back(job);
@@ -88,12 +92,17 @@ class CopyCrew {
   }
 
  private:
-  CopyCrew() {
+  CopyCrew() = default;
+  void start() {
     size_t n = 8;
     if (const char* v = std::getenv("ILANG_HIP_COPY_THREADS")) n = (size_t)std::max(1, std::atoi(v));
     n = std::min<size_t>(n, std::max(1u, std::thread::hardware_concurrency()));
     for (size_t t = 1; t < n; ++t) {
-      std::thread([this] { work(); }).detach();
+      try {
+        std::thread([this] { work(); }).detach();
+      } catch (const std::system_error&) {
+        return;
+      }
       ++threads_;
     }
   }
@@ -112,6 +121,7 @@ class CopyCrew {
   std::mutex mu_;
   std::condition_variable wake_;
   std::deque<std::shared_ptr<Job>> jobs_;
+  std::once_flag started_;
   size_t threads_ = 0;
 };
 
