@@ -127,7 +127,7 @@ ic::ExecPlan split_nests(const ic::ExecPlan& plan, std::vector<size_t>* origin);
 
 // Names of the helper kernels that every module with a GridForm carries: filling a temporary with a reduction's
 // identity; folding the parts' copies into the accumulated buffer, with a work-item per element (few parts) or a
-// wavefront for one or two elements, whose lanes run over the parts.
+// wavefront for one, two, four or eight elements, whose lanes run over the parts.
 constexpr const char* kFillKernel = "ilang_fill";
 constexpr const char* kCombineKernel = "ilang_combine";
 constexpr const char* kCombineWaveKernel = "ilang_combine_w";

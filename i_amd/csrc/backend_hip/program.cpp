@@ -790,8 +790,9 @@ ihip::Err generic_function(Program& p, const std::string& name, hipFunction_t* f
 // the two forms (a work-item or a wavefront per iteration) would run.  Parts pay when the parallel loops alone leave
 // most of the chip idle: enough of them for 16 wavefronts per compute unit, each part with at least 16 iterations of
 // a loop that a work-item runs by itself, 4 rounds of the 64 lanes when the loop in parts is the one over the lanes,
-// one iteration when the lanes run over a loop inside it; at most 4096, from 16 on a multiple of 8 and from 256 on
-// of 32.
+// one iteration when the lanes run over a loop inside it; at most 4096.  (Any number folds in one pass: rounded down to
+// multiples of 8 and 32, 1000 x 50000 to one element took 992 parts, eight of them twice as long as the others, and 136 us; in
+// 1000 it takes 73.)
 // `strips`: a work-item takes four iterations of the innermost parallel loop and `total` counts those.
 size_t generated_parts(const ihip::KernelOptions& knobs, const GridForm& grid, bool wave, size_t total, size_t reduced, bool strips, bool bf16) {
   if (!grid.available || (wave && !grid.wave) || knobs.generated_parts == 1 || total == 0) return 1;
@@ -816,16 +817,14 @@ size_t generated_parts(const ihip::KernelOptions& knobs, const GridForm& grid, b
     parts = std::min<size_t>(parts, reduced / least);
   }
   // (at most 4096 parts; 2048 of wavefronts when left to this rule: the pass over the parts of a sum to one element
-  // is one wavefront's work and grows with their number, 4096^2 to one element 29.7 us in 4096 parts, 23.8 in 2048)
+  // is one wavefront's work and grows with their number: 4096^2 to one element 21.3 us in 4096 parts, 19.0 in 2048; only sums of
+  // four times as much gain by more, 16384 x 4096 57.2 in 2048 and 53.3 in 4096)
   parts = std::min<size_t>(std::min<size_t>(parts, wave && knobs.generated_parts <= 1 ? 2048 : 4096), std::max<size_t>(reduced, 1));
-  if (parts >= 256) parts = parts / 32 * 32;
-  else if (parts >= 16) parts = parts / 8 * 8;
   if (strips && knobs.generated_parts <= 1 && parts >= 2) {
     // (their shares are multiples of eight iterations, whole rounds of the loads in flight, and no longer than these parts
     // would have: 100000 x 64 30.6 -> 24.1 us, 4096 x 1024 13.9 -> 12.7)
-    const size_t share = std::max<size_t>(reduced / parts / 8 * 8, 8), needed = (reduced + share - 1) / share;
-    const size_t step = needed >= 256 ? 32 : needed >= 16 ? 8 : 1;
-    parts = std::min<size_t>((needed + step - 1) / step * step, 4096);
+    const size_t share = std::max<size_t>(reduced / parts / 8 * 8, 8);
+    parts = std::min<size_t>((reduced + share - 1) / share, 4096);
   }
   return parts < 2 ? 1 : parts;
 }

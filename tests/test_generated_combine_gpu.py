@@ -19,7 +19,8 @@ def _into(component, ref, terms, x, out, rows, parts=0):
     assert bool(t.isnan(ring[:16]).all()) and bool(t.isnan(ring[-16:]).all()), what
 
 
-# buffers of one, a few, 63 to 65 and many elements; parts just below and above where the pass takes lanes (16) and all of them (512)
+# buffers of one, a few, 63 to 65 and many elements (odd numbers leave a wavefront's last group of elements incomplete); parts on both
+# sides of where the pass takes lanes at all (16) and more of them per element (65, 129, 257)
 @pytest.mark.parametrize("dtype, out", [("f32", "f32"), ("bf16", "bf16"), ("bf16", "f32"), ("f32", "bf16")])
 @pytest.mark.parametrize("cols", [1, 3, 63, 64, 65, 130, 1000])
 def test_column_sums_in_any_number_of_parts(dtype, out, cols):
@@ -29,9 +30,10 @@ def test_column_sums_in_any_number_of_parts(dtype, out, cols):
     g = t.Generator(device="cuda").manual_seed(cols)
     for rows in (64, 1100, 9000):
         x = t.randn(rows, cols, device="cuda", generator=g).to(_T[dtype])
-        for parts in (0, 2, 15, 16, 17, 31, 33, 100, 511, 512, 700):
+        for parts in (0, 2, 15, 16, 17, 33, 64, 65, 128, 129, 256, 257, 511, 700):
             component.option("generated.parts", parts)
             _into(component, x.double().sum(0), x.double().abs().sum(0), x, out, rows, parts)
+            assert parts == 0 or f" in {min(parts, rows)} parts" in component.report(), component.report()
 
 
 @pytest.mark.parametrize("op, ref", [(">", lambda x: x.amax(0)), ("<", lambda x: x.amin(0)), ("*", lambda x: x.prod(0))])

@@ -47,8 +47,8 @@ def test_generated_kernels_match_the_emitted_c_on_the_cpu(shim_lib):
 def test_reduction_nests_with_their_outer_loop_in_parts_match_too(shim_lib):
     """The program option generated.parts (ILANG_SHIM_PARTS to the case runner) deals the outermost sequential loop of
     every nest that only accumulates out over that many groups of work-items, each with copies of its own of the
-    accumulated buffers, and a second kernel folds the copies: 3 parts (one pass of the fold, ragged shares), 256
-    parts (two passes; most parts get no iteration at these sizes), both forms of a nest (a work-item or a wavefront
+    accumulated buffers, and a second kernel folds the copies: 3 parts (ragged shares), 16 (lanes
+    share an element), as many as there are iterations, both forms of a nest (a work-item or a wavefront
     per iteration), and work-items last to first.  (3 parts on every case; the other settings on a few.)"""
     run_cases(shim_lib, {"ILANG_SHIM_PARTS": "3", "ILANG_SHIM_TOLERANCE": "1e-4"})
     few = ["total", "column max", "row sum 5x300", "column normalize (two nests)", "fused matrix-vector product", "mm_t"]
