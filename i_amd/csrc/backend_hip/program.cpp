@@ -1059,10 +1059,16 @@ ihip::Err launch_generic(Run& run, size_t k, const Step& dispatch) {
   for (const PrivateBuffer& pb : ph.privates)
     if (!pb.is_static) slot_elems += std::max<size_t>(1, product(run.layout_of(dispatch.writes[pb.writeable])));
   // Work-items that take one strip after the other hide the digits of their index behind the accesses, but an f32 strip is enough
-  // to hide them by itself, and more of them are in flight so: 16384 x 4096 with a bias and a threshold 103 us with 2^20
-  // work-items, 97, 93 and 90 with 2, 4 and 8 times as many, divided by its column sums 161, 152, 149 and 147.  Strips of bf16
-  // are half as long: 56, 55, 55 and 62, and 13896 x 2406 divided 57, 58, 60 and 67.
-  size_t max_threads = size_t(1) << (strips && !ph.sequential_loops && !bf16_inputs ? 23 : 20);
+  // to hide them by itself, and more of them are in flight so.  f32 with 2^20, 2^21, 2^22 and 2^23 work-items, us: 16384 x 4096
+  // with a bias and a threshold in one nest 103, 97, 93, 90; in two, as the sum of two operands and divided by its column
+  // sums 8192 x 3000 66, 63, 61, 62; 47, 45, 44, 44; 52, 51, 51, 52; 8000 x 20000 518, 522, 489, 459; 402, 402, 380, 356; 379,
+  // 370, 362, 358; the sum of two stored in bf16 37, 36, 36, 35 and 324, 323, 313, 298.  Strips of bf16 operands are half
+  // as long: 56, 55, 55, 62 at 16384 x 4096, the sum of two at 8192 x 3000 24, 24, 26, 31.  So is it where a nest stores bf16 and
+  // reads what another one wrote, as long as the 256 MB of the Infinity Cache still hold that: the threshold of the two
+  // nests 18, 19, 19, 19 at 2000 x 3001, 48, 47, 49, 52 at 8192 x 3000, 39, 40, 41, 42 at 65536 x 300, but 159, 150, 148, 146 at
+  // 16384 x 4096 and 402, 405, 386, 377 at 8000 x 20000.
+  const bool cached_to_bf16 = bf16_writes != 0 && ph.bf16_reads.empty() && total < (size_t(1) << 26);
+  size_t max_threads = size_t(1) << (!strips || ph.sequential_loops || bf16_inputs || cached_to_bf16 ? 20 : 23);
   if (slot_elems) max_threads = std::max<size_t>(64, std::min(max_threads, (size_t(1) << 28) / (slot_elems * 4)));
   threads = std::min(threads, max_threads);
   const unsigned grid = (unsigned)((threads + 63) / 64);
