@@ -50,8 +50,8 @@ struct PrivateBuffer {
 // one before it, and two work-items store the same elements: that is left to nests that read nothing of what they
 // write.  Sums that the nest starts itself are such nests, since their registers start as the reduction's identity
 // (GridForm::starts_fresh; started through memory, a sum could be read back by the neighbour and counted twice).  The element-wise forms are bound by HBM and the plain ones by the number
-// of accesses in flight: 16384 x 4096 f32 divided by its column sums 213 -> 162 us (the division alone 145 -> 87, 6
-// TB/s), a bias and a threshold 193 -> 102.  And every form that reads program inputs exists once more, <name>..._b, with
+// of accesses in flight: 16384 x 4096 f32 divided by its column sums 213 -> 147 us (the division alone 145 -> 78, 6.9
+// TB/s), a bias and a threshold 193 -> 90.  And every form that reads program inputs exists once more, <name>..._b, with
 // those inputs' elements in bf16, which would otherwise be widened into temporaries first (16384 x 4096
 // bf16, results in bf16: 450 -> 96 and 447 -> 56 us; row sums 182 -> 32, where a lane takes four elements at a time).
 struct WaveLoop {
