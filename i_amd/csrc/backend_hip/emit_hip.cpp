@@ -1408,8 +1408,10 @@ GenericModule emit_generic_hip(const ExecPlan& plan, const Module& module, const
     src << "  return op == 0 ? a + b : op == 1 ? a * b : op == 2 ? fmaxf(a, b) : fminf(a, b);\n}\n";
     src << "static __device__ __forceinline__ float ilang_identity(int op) { return op == 0 ? 0.0f : op == 1 ? 1.0f : op == 2 ? (-INFINITY) : INFINITY; }\n";
     // the elements from `at` on, every `step`-th before `end`, folded into `acc`: eight loads in flight, those past the end
-    // re-reading the first and counting as the identity
+    // re-reading the first and counting as the identity.  (A lane with one element has one load: with all eight, column sums of 50 x 30
+    // in 4 parts, waited for, 21.6 us, and 20.7 without.)
     src << "static __device__ __forceinline__ float ilang_fold_range(int op, float acc, const float* data, size_t at, size_t step, size_t end) {\n";
+    src << "  if (at >= end) return acc;\n  if (end - at <= step) return ilang_fold(op, acc, data[at]);\n";
     src << "  for (; at < end; at += 8 * step) {\n    float v[8];\n    #pragma unroll\n    for (int u = 0; u < 8; ++u) v[u] = data[at + u * step < end ? at + u * step : at];\n";
     src << "    #pragma unroll\n    for (int u = 0; u < 8; ++u) v[u] = at + u * step < end ? v[u] : ilang_identity(op);\n";
     src << "    #pragma unroll\n    for (int u = 0; u < 8; ++u) acc = ilang_fold(op, acc, v[u]);\n  }\n  return acc;\n}\n";
