@@ -2,6 +2,7 @@
 // Reference behaviour: core/src/lib.rs:61-121, 289-351.
 #include "../../../include/i.h"
 
+#include <cstdint>
 #include <cstdlib>
 #include <cstring>
 #include <algorithm>
@@ -382,7 +383,8 @@ bool run_host_in_slices(ihipc::Program& p, const i_tensor* inputs, const std::ve
 // 160 -> 105; the link alone takes 610, 570, 123 and 22.
 constexpr size_t kMirrorPiece = size_t(1) << 20, kMirroredSlicedBytes = size_t(6) << 20, kMirroredSliceBytes = size_t(8) << 20;
 std::string run_mirrored(ihipc::Program& p, const i_tensor* inputs, const std::vector<ihipc::DeviceTensor>& in,
-                         const std::vector<ihipc::DeviceTensor>& out, const std::vector<float*>& out_ptrs, Staging& block, hipStream_t stream) {
+                         const std::vector<ihipc::DeviceTensor>& out, const std::vector<float*>& out_ptrs, size_t call_bytes, Staging& block,
+                         hipStream_t stream) {
   char* const base = static_cast<char*>(block.base);
   char* const mirror = static_cast<char*>(block.pinned);
   auto elements = [](const ihipc::DeviceTensor& t) {
@@ -393,7 +395,7 @@ std::string run_mirrored(ihipc::Program& p, const i_tensor* inputs, const std::v
   // slices of the leading index, if the program allows it and there is enough to move
   std::vector<char> sliced;
   size_t rows = out.empty() || out[0].shape.empty() ? 0 : out[0].shape[0], moving = 0, whole = 0;
-  bool in_slices = rows >= 2 && ihipc::row_sliceable(p, &sliced) && sliced.size() == in.size();
+  bool in_slices = rows >= 2 && call_bytes >= kMirroredSlicedBytes && ihipc::row_sliceable(p, &sliced) && sliced.size() == in.size();
   for (size_t i = 0; in_slices && i < in.size(); ++i) {
     in_slices = !sliced[i] || (!in[i].shape.empty() && in[i].shape[0] == rows);
     (sliced[i] ? moving : whole) += 4 * elements(in[i]);
@@ -413,6 +415,9 @@ std::string run_mirrored(ihipc::Program& p, const i_tensor* inputs, const std::v
   const size_t wanted = in_slices ? std::min<size_t>(std::min<size_t>(8, rows), std::max<size_t>(2, moving / kMirroredSliceBytes)) : 1;
   const size_t each = in_slices ? (rows + wanted - 1) / wanted : 0, slices = in_slices ? (rows + each - 1) / each : 1;
 
+  // (transfers of whole operands end on a multiple of 256 bytes, which every operand has room for: 120 and 200 bytes cost a call of
+  // 32 us one more)
+  auto rounded = [in_slices](size_t end) { return in_slices ? end : (end + 255) / 256 * 256; };
   // ---- up: the pieces in the order in which they cross, and how many there are up to the end of each slice
   std::vector<ihip::CopyPiece> gathered;
   std::vector<size_t> gathered_until;
@@ -446,35 +451,59 @@ std::string run_mirrored(ihipc::Program& p, const i_tensor* inputs, const std::v
         ahead.wait(sent);
         hi = at + gathered[sent].bytes;
       }
-      if (ihip::Err e = ihip::h2d(base + lo, mirror + lo, hi - lo, up); !e.empty()) return e;
+      if (ihip::Err e = ihip::h2d(base + lo, mirror + lo, rounded(hi) - lo, up); !e.empty()) return e;
     }
     return {};
   };
-  // ---- down: pieces on their way, copied out in order
+  // ---- down: pieces on their way, copied out in order.  Small neighbours cross together here too.
   struct Piece {
     size_t at, bytes;
     char* to;
-    hipEvent_t landed;
+    bool first;          // of its transfer: copying it out waits for that
+    hipEvent_t landed;   // nullptr: the last transfer of all, awaited with the stream
   };
   std::vector<Piece> pieces;
-  size_t copied = 0, events = 2 * slices;
+  size_t copied = 0, events = 2 * slices, enqueued = 0;  // pieces that are copied out; events in use; pieces that are on their way
+  size_t unmarked = SIZE_MAX;                            // the first piece of the last transfer, as long as no event follows that
+  bool waited = false;                                   // for the stream, with nothing enqueued after
+  auto mark = [&]() -> ihip::Err {
+    if (unmarked == SIZE_MAX) return {};
+    if (!block.event(events++, &pieces[unmarked].landed)) return "no event for a transfer";
+    if (ihip::Err e = ihip::check(hipEventRecord(pieces[unmarked].landed, down), "hipEventRecord"); !e.empty()) return e;
+    unmarked = SIZE_MAX;
+    return {};
+  };
+  auto enqueue = [&]() -> ihip::Err {  // the pieces that are not on their way yet, in one transfer
+    if (enqueued == pieces.size()) return {};
+    if (ihip::Err e = mark(); !e.empty()) return e;
+    Piece& first = pieces[enqueued];
+    const size_t end = rounded(pieces.back().at + pieces.back().bytes);
+    first.first = true;
+    if (ihip::Err e = ihip::d2h(mirror + first.at, base + first.at, end - first.at, down); !e.empty()) return e;
+    unmarked = enqueued;
+    enqueued = pieces.size();
+    return {};
+  };
   auto bring = [&](size_t at, size_t bytes, char* to) -> ihip::Err {
     const size_t step = std::max(2 * kMirrorPiece, (bytes / 4 + 4095) / 4096 * 4096);
     for (size_t done = 0; done < bytes; done += step) {
-      Piece piece{at + done, std::min(step, bytes - done), to + done, nullptr};
-      if (ihip::Err e = ihip::d2h(mirror + piece.at, base + piece.at, piece.bytes, down); !e.empty()) return e;
-      if (in_slices || done + step < bytes) {  // (the last of all is awaited with the stream)
-        if (!block.event(events++, &piece.landed)) return "no event for a transfer";
-        if (ihip::Err e = ihip::check(hipEventRecord(piece.landed, down), "hipEventRecord"); !e.empty()) return e;
+      const size_t here = at + done, size = std::min(step, bytes - done);
+      if (enqueued < pieces.size()) {
+        const size_t end = pieces.back().at + pieces.back().bytes;  // (outputs, too, start on the next 256 bytes after the one before)
+        if (in_slices || here < end || here - end >= 256 || here + size - pieces[enqueued].at > 2 * kMirrorPiece)
+          if (ihip::Err e = enqueue(); !e.empty()) return e;
       }
-      pieces.push_back(piece);
+      pieces.push_back({here, size, to + done, false, nullptr});
     }
     return {};
   };
   auto copy_out = [&](size_t until) -> ihip::Err {
     for (; copied < until; ++copied) {
       const Piece& piece = pieces[copied];
-      if (ihip::Err e = piece.landed ? ihip::check(hipEventSynchronize(piece.landed), "hipEventSynchronize") : ihip::sync(down); !e.empty()) return e;
+      if (piece.first && !waited) {
+        if (ihip::Err e = piece.landed ? ihip::check(hipEventSynchronize(piece.landed), "hipEventSynchronize") : ihip::sync(down); !e.empty()) return e;
+        waited = !piece.landed;
+      }
       ihip::copy_by_threads(piece.to, mirror + piece.at, piece.bytes);
     }
     return {};
@@ -484,7 +513,12 @@ std::string run_mirrored(ihipc::Program& p, const i_tensor* inputs, const std::v
     std::vector<size_t> pieces_at;  // how many there were before each slice
     for (size_t s = 0; s < slices; ++s) {
       const size_t r0 = s * each, r1 = std::min(rows, r0 + each);
-      std::vector<ihipc::DeviceTensor> in_s(in), out_s(out);
+      std::vector<ihipc::DeviceTensor> in_cut, out_cut;
+      if (in_slices) {
+        in_cut = in;
+        out_cut = out;
+      }
+      const std::vector<ihipc::DeviceTensor>&in_s = in_slices ? in_cut : in, &out_s = in_slices ? out_cut : out;
       auto cut = [&](ihipc::DeviceTensor& t) {  // rows r0 .. r1; returns the byte offset of the first
         const size_t skip = 4 * elements(t) / rows * r0;
         t.data = static_cast<char*>(t.data) + skip;
@@ -493,9 +527,9 @@ std::string run_mirrored(ihipc::Program& p, const i_tensor* inputs, const std::v
       };
       std::vector<size_t> out_skip(out.size(), 0);
       for (size_t i = 0; in_slices && i < in.size(); ++i) {
-        if (sliced[i]) (void)cut(in_s[i]);
+        if (sliced[i]) (void)cut(in_cut[i]);
       }
-      for (size_t o = 0; in_slices && o < out.size(); ++o) out_skip[o] = cut(out_s[o]);
+      for (size_t o = 0; in_slices && o < out.size(); ++o) out_skip[o] = cut(out_cut[o]);
       if (ihip::Err e = send(gathered_until[s]); !e.empty()) return e;
       hipEvent_t landed = nullptr, ran = nullptr;
       if (in_slices) {
@@ -514,6 +548,9 @@ std::string run_mirrored(ihipc::Program& p, const i_tensor* inputs, const std::v
         if (!out_ptrs[o]) return "output " + std::to_string(o) + " has no data";
         if (ihip::Err e = bring(offset(out_s[o]), 4 * elements(out_s[o]), reinterpret_cast<char*>(out_ptrs[o]) + out_skip[o]); !e.empty()) return e;
       }
+      if (ihip::Err e = enqueue(); !e.empty()) return e;
+      if (in_slices)
+        if (ihip::Err e = mark(); !e.empty()) return e;
       // (two slices back: down by now, unless the kernels are what takes the time, and then nothing waits for this thread)
       if (s >= 2)
         if (ihip::Err e = copy_out(pieces_at[s - 1]); !e.empty()) return e;
@@ -530,8 +567,10 @@ std::string run_mirrored(ihipc::Program& p, const i_tensor* inputs, const std::v
     (void)hipStreamSynchronize(up);
     (void)hipStreamSynchronize(down);
   }
-  const ihip::Err sync_err = ihip::sync(stream);
-  if (err.empty()) err = sync_err;
+  if (!waited || !err.empty()) {
+    const ihip::Err sync_err = ihip::sync(stream);
+    if (err.empty()) err = sync_err;
+  }
   if (in_slices && err.empty())
     ihipc::append_to_report(p, "host: operands in " + std::to_string(slices) + " slices of " + std::to_string(each) +
                                    " rows, the kernels above are those of the last slice\n");
@@ -623,7 +662,7 @@ std::string run_host(ihipc::Program& p, const i_tensor* inputs, size_t input_cou
   std::string err;
   if (mirrored) {
     try {
-      err = run_mirrored(p, inputs, in, out, out_ptrs, *mirrored, stream);
+      err = run_mirrored(p, inputs, in, out, out_ptrs, wanted, *mirrored, stream);
     } catch (const std::exception& e) {  // (out of memory before anything was enqueued)
       err = e.what();
     }

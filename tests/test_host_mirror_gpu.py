@@ -41,6 +41,25 @@ def test_elements_arrive_where_they_belong(rows, cols):
         assert "host:" not in flipped.report()
 
 
+
+# several outputs: small neighbours that cross together, with an empty one between them, up to pieces of their own
+@pytest.mark.parametrize("rows, cols", [(1, 1), (3, 5), (63, 65), (0, 4), (300, 1001), (525, 999), (1100, 1000), (9, 150001)])
+def test_several_outputs_arrive_where_they_belong(rows, cols):
+    from i_amd import Component as i
+
+    a, b = _data((rows, cols), 1), _data((rows, cols), 2)
+    component = ((i("ij+ij~ij") & i("ij~ji")) & i("-ij~ij")) & i("ij~ji")
+    shapes = [(rows, cols), (cols, rows), (rows, cols), (cols, rows)]
+    expected = [a + b, a.T, -a, a.T]
+    for _ in range(2):
+        rings = [np.full(rows * cols + 32, np.nan, np.float32) for _ in shapes]
+        outs = [ring[16:16 + rows * cols].reshape(shape) for ring, shape in zip(rings, shapes)]
+        component.into(outs, a, b)
+        for out, want, ring in zip(outs, expected, rings):
+            assert np.array_equal(out, want)
+            assert np.isnan(ring[:16]).all() and np.isnan(ring[-16:]).all()
+
+
 OVERLAPPING = """
 import sys
 import numpy as np
