@@ -1067,8 +1067,10 @@ ihip::Err launch_generic(Run& run, size_t k, const Step& dispatch) {
   // reads what another one wrote, as long as the 256 MB of the Infinity Cache still hold that: the threshold of the two
   // nests 18, 19, 19, 19 at 2000 x 3001, 48, 47, 49, 52 at 8192 x 3000, 39, 40, 41, 42 at 65536 x 300, but 159, 150, 148, 146 at
   // 16384 x 4096 and 402, 405, 386, 377 at 8000 x 20000.
-  const bool cached_to_bf16 = bf16_writes != 0 && ph.bf16_reads.empty() && total < (size_t(1) << 26);
-  size_t max_threads = size_t(1) << (!strips || ph.sequential_loops || bf16_inputs || cached_to_bf16 ? 20 : 23);
+  // Below 2^24 iterations a second round of 2^20 work-items is not yet worth more of them: with 2^20 and 2^23, 6500 x 1000 with a bias and a
+  // threshold 9.9 and 10.9, 11000 x 1000 14.4 and 15.5, 5000 x 3001 21.2 and 21.1, 18000 x 1000 22.8 and 22.4, 27000 x 1000 36.5 and 34.6.
+  const int least = bf16_writes != 0 && ph.bf16_reads.empty() ? 26 : 24;  // (log2)
+  size_t max_threads = size_t(1) << (!strips || ph.sequential_loops || bf16_inputs || total < (size_t(1) << least) ? 20 : 23);
   if (slot_elems) max_threads = std::max<size_t>(64, std::min(max_threads, (size_t(1) << 28) / (slot_elems * 4)));
   threads = std::min(threads, max_threads);
   const unsigned grid = (unsigned)((threads + 63) / 64);
