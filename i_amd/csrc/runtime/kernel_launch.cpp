@@ -679,12 +679,15 @@ static size_t narrow_nt_tile(size_t bh, size_t n, unsigned splits) { return spli
 // f32 NT: the k loop in parts over workgroups of 32 columns, added up by a second launch, where the columns alone leave CUs
 // idle or a last round nearly empty.  A workgroup's 16 wavefronts fill a CU, so the time goes by whole rounds of 256
 // workgroups: 4 us, and per element of k 3.2 ns on 16 columns, 6 on 32 (5.6 and 9.5 above 16 rows); a split costs 4.5 more,
-// and its many workgroups read B at 5 TB/s at most.  Whole -> in parts, us: 12 x 4904 x 6696 60 -> 43, 3 x 1688 x 8896
+// and its many workgroups read B at 5 TB/s at most.  A single round has to hold every workgroup that is launched, the tiles of a batch and
+// part rounded up to one per XCD (85 tiles in 3 parts are 264, and some CU gets two: 2 x 2713 x 14136 59 us so, 48 in 6 or whole);
+// in later rounds the empty ones cost nothing (2 x 2345 x 9628, 74 tiles: 24.2 in 10 parts, 29.0 in 3).  Whole -> in parts, us: 12 x 4904 x 6696 60 -> 43, 3 x 1688 x 8896
 // 31 -> 21, 5 x 2000 x 16000 56 -> 34, 24 x 1500 x 9000 54 -> 29, 31 x 1024 x 16000 98 -> 29; left whole: 30 x 4096 x 4096
 // (28; 28 in 2), 16 x 8192 x 8192 (65; 73), 1 x 12952 x 6288 (69; 75 in 11).
 static unsigned narrow_nt_f32_parts(size_t bh, size_t m, size_t n, size_t k) {
   auto time_of = [&](size_t tile, size_t parts) {
-    const double rounds = (double)(((n + tile - 1) / tile * bh * parts + 255) / 256);
+    const size_t tiles = (n + tile - 1) / tile, launched = (tiles + 7) / 8 * 8 * bh * parts;
+    const double rounds = std::max((double)((tiles * bh * parts + 255) / 256), launched > 256 ? 2.0 : 1.0);
     const double loops = rounds * (double)(k / parts) * 1e-3 * (m <= 16 ? (tile == 16 ? 3.2 : 6.0) : (tile == 16 ? 5.6 : 9.5));
     return parts > 1 ? 8.5 + std::max(loops, (double)(bh * n * k) * 4 / 5e6) : 4 + loops;
   };
