@@ -785,7 +785,11 @@ static F32Plan f32_plan(size_t bh, size_t m, size_t n, size_t k, const KernelOpt
     if (asked ? tile != asked : tile == 256) continue;
     const size_t tiles = ((m + tile - 1) / tile) * ((n + tile - 1) / tile) * bh;
     for (size_t s = 1; s <= 32 && (s == 1 || (!whole && knobs.gemm_k_parts != 1 && k / s >= 64 && bh * s <= 65535)); ++s) {
-      const double resident = (double)((tiles * s + 255) / 256);
+      // (A single round of parts of large tiles has to hold every workgroup that is launched, the tiles of a batch and part rounded up
+      // to one per XCD: 85 tiles of 128 in 3 parts are 264, and some CU gets two.  605 x 2151 x 3224 136 us so, 90 on 64-tiles.  Of
+      // those a second one costs little: 815 x 122 x 1560, 26 tiles, 12.3 in 9 parts, 14.2 in 7.)
+      const bool crowded = tile >= 128 && s > 1 && (tiles / bh + 7) / 8 * 8 * bh * s > 256;
+      const double resident = std::max((double)((tiles * s + 255) / 256), crowded ? 2.0 : 1.0);
       double t = (double)((slabs + s - 1) / s + 2) * std::max(resident * (tile == 256 ? 6.8 : tile == 128 ? 1.7 : 0.46), far ? 0.7 : 0.0);
       if (s > 1) t = (t + 4.0 + (double)(bh * s * m * n * 4) / 3e6) / 0.85;
       if (t < best_time) {
