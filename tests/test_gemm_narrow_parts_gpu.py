@@ -26,3 +26,22 @@ def test_parts_of_k(m, n, k, parts):
     assert t.equal(c, (a.double() @ b.double().t()).float()), what
     assert bool(t.isnan(ring[m * n:]).all()), what
     assert "_narrow" in component.report() and ("parts)" in component.report()) == parts, what
+
+
+# 80, 81 and 85 column or output tiles: 240 workgroups in three parts are a round, 264 (the tiles of a part go up to a multiple of eight)
+# are not, in the kernel for few rows and on 128-tiles
+@pytest.mark.parametrize("m, n, k, three", [(2, 2560, 8000, True), (2, 2592, 8000, False), (1, 2713, 9001, False), (605, 2151, 3224, False), (601, 2050, 3001, False)])
+def test_a_round_of_parts_holds_every_workgroup(m, n, k, three):
+    from i_amd import Component as i
+
+    component = i("ik*jk~ijk | i:16,j:16 | jii'j'k") >> i("+ijk~ij | i:16,j:16 | jii'j'k0")
+    g = t.Generator(device="cuda").manual_seed(m + k)
+    a, b = (t.randint(-4, 5, (rows, k), device="cuda", generator=g).float() for rows in (m, n))
+    ring = t.full((m * n + 8,), float("nan"), device="cuda")
+    c = ring[:m * n].view(m, n)
+    component.into(c, a, b)
+    what = dict(m=m, n=n, k=k, report=component.report())
+    assert t.equal(c, (a.double() @ b.double().t()).float()), what
+    assert bool(t.isnan(ring[m * n:]).all()), what
+    crowded = "in 3 parts" in component.report() and "64x64" not in component.report()
+    assert crowded == three, what
